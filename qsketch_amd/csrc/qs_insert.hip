@@ -42,7 +42,9 @@
 //             kernel, unlinked ones to the replay first.
 //   k_ordered one wavefront per queued segment replays it in stream order until
 //             its allocation (at most ceil(28*129/3) inserts can precede it).
-//   k_assign  allocation ids per sketch, in stream order of the triggering inserts.
+//   k_assign  allocation ids per sketch, in stream order of the triggering inserts:
+//             an allocation's rank is the number of set bits before its position
+//             in a bitmap over the chunk (set by k_ordered).
 //   k_tail    long segments after their allocation point: per-lane LDS counter
 //             rows over windows of sorted items, one atomic per counter per
 //             window and bucket.  Only the runs at the two ends of a 64-item
@@ -94,6 +96,16 @@ __device__ static inline uint32_t find_sid(const uint64_t *__restrict__ offs, ui
             hi = mid;
     }
     return lo;
+}
+
+// first chunk position of sketch sid's part of the chunk that starts at batch
+// position base (offsets past the chunk stay past it: a batch position less
+// base fits 32 bits only up to there, so larger ones are cut to the largest)
+__device__ static inline uint32_t sid_chunk_start(const uint64_t *__restrict__ offs, uint32_t sid, uint64_t base)
+{
+    const uint64_t a = offs[sid];
+    const uint64_t p = a > base ? a - base : 0ull;
+    return p < 0xffffffffull ? (uint32_t)p : 0xffffffffu;
 }
 
 // ===========================================================================
@@ -196,14 +208,17 @@ __device__ static inline RawT<KB, FIRST> load_raw(const void *in, uint32_t i, ui
 }
 
 // Tile counts of the first pass, from the keys: each item is built on the way
-// (the scatter builds it again rather than reading it back)
+// (the scatter builds it again rather than reading it back).  It also clears
+// the chunk's allocation bitmap and its span counts.
+static_assert(QS_TSPAN % OS_TILE == 0 && OS_TILE % 32 == 0 && OS_TILE / 32 <= OS_THREADS, "bitmap words per tile");
 template <int KB, bool MULTI>
 __global__ __launch_bounds__(OS_THREADS) void k_bs_up(const void *__restrict__ in, uint32_t n, uint64_t base,
                                                       qs_sdesc d0, const qs_sdesc *__restrict__ D,
                                                       const uint64_t *__restrict__ offs, uint32_t nsk,
                                                       qs_pack pk, int shift, uint32_t dmask,
                                                       uint32_t nbins, uint32_t ntiles,
-                                                      uint16_t *__restrict__ hist)
+                                                      uint16_t *__restrict__ hist, uint32_t *__restrict__ tbit,
+                                                      uint32_t *__restrict__ tsum)
 {
     __shared__ uint32_t s_h[OS_BINS];
     __shared__ uint64_t s_off[MULTI ? SIDW + 1 : 1];
@@ -212,6 +227,11 @@ __global__ __launch_bounds__(OS_THREADS) void k_bs_up(const void *__restrict__ i
     if (t < OS_BINS)
         s_h[t] = 0;
     const uint32_t tb = blockIdx.x * OS_TILE;
+    // this tile's part of the allocation bitmap starts the chunk clear
+    if (t < OS_TILE / 32u)
+        tbit[blockIdx.x * (OS_TILE / 32u) + t] = 0;
+    if (t == 0 && tb % QS_TSPAN == 0)
+        tsum[tb / QS_TSPAN] = 0;
     sid_window win{s_off, 0u, 0u};
     if (MULTI) {
         const uint32_t te = (n - tb) < OS_TILE ? n : tb + OS_TILE;
@@ -1309,6 +1329,8 @@ __global__ __launch_bounds__(256) void k_ordered(const uint64_t *__restrict__ IT
                                                  uint32_t *__restrict__ longbm,
                                                  uint32_t *__restrict__ lng,
                                                  qs_trig *__restrict__ trig, uint32_t trig_cap,
+                                                 uint32_t *__restrict__ tbit, uint32_t *__restrict__ tsum,
+                                                 const uint64_t *__restrict__ offs, uint64_t base,
                                                  uint32_t one_masks, qs_dev_state *__restrict__ st)
 {
     __shared__ qs_trig s_tr[4][TBUF];
@@ -1409,6 +1431,12 @@ __global__ __launch_bounds__(256) void k_ordered(const uint64_t *__restrict__ IT
             if (lane < 32u)
                 s_tr[wv][ntb].hc[lane] = hc;
             if (lane == 0) {
+                // mark the trigger's chunk position (every insert has its own,
+                // so the counts of a span add up to its set bits)
+                if (!one_masks)
+                    t_idx += sid_chunk_start(offs, sid, base);
+                atomicOr(tbit + (t_idx >> 5), 1u << (t_idx & 31u));
+                atomicAdd(tsum + t_idx / QS_TSPAN, 1u);
                 s_tr[wv][ntb].idx = t_idx;
                 s_tr[wv][ntb].bucket = b;
                 s_tr[wv][ntb].tail_start = tail_start;
@@ -1467,38 +1495,90 @@ __global__ __launch_bounds__(256) void k_ordered(const uint64_t *__restrict__ IT
         lng[bl + lane] = s_ln[wv][lane];
 }
 
-// trigger sort key: sketch << ib | stream index (fits 32 bits by construction)
-__global__ void k_trig_keys(const qs_trig *__restrict__ trig, const qs_dev_state *__restrict__ st,
-                            uint32_t trig_cap, uint32_t ib, uint32_t *__restrict__ tk,
-                            uint32_t *__restrict__ tv)
+// Exclusive scan of the per-span trigger counts (one block), the total after
+// them.
+__global__ __launch_bounds__(1024) void k_trig_scan(uint32_t *__restrict__ tsum, uint32_t nspan,
+                                                    const qs_dev_state *__restrict__ st)
 {
-    const uint32_t n = min(st->n_trig, trig_cap);
-    for (uint32_t r = blockIdx.x * blockDim.x + threadIdx.x; r < n; r += gridDim.x * blockDim.x) {
-        tk[r] = (trig[r].sid << ib) | trig[r].idx;
-        tv[r] = r;
+    __shared__ uint32_t s_w[16];
+    if (st->n_trig == 0)
+        return; // nothing reads it
+    const uint32_t t = threadIdx.x, lane = t & 63u, wv = t >> 6;
+    uint32_t carry = 0;
+    for (uint32_t base = 0; base < nspan; base += 1024u * GSCAN_PT) {
+        const uint32_t g0 = base + t * GSCAN_PT;
+        uint32_t v[GSCAN_PT], sum = 0;
+#pragma unroll
+        for (uint32_t k = 0; k < GSCAN_PT; ++k) {
+            v[k] = g0 + k < nspan ? tsum[g0 + k] : 0u;
+            sum += v[k];
+        }
+        uint32_t x = sum;
+#pragma unroll
+        for (int o = 1; o < 64; o <<= 1) {
+            const uint32_t y = (uint32_t)__shfl_up((int)x, o, 64);
+            x += lane >= (uint32_t)o ? y : 0u;
+        }
+        if (lane == 63)
+            s_w[wv] = x;
+        __syncthreads();
+        uint32_t before = carry, total = carry;
+#pragma unroll
+        for (uint32_t w = 0; w < 16u; ++w) {
+            before += w < wv ? s_w[w] : 0u;
+            total += s_w[w];
+        }
+        uint32_t run = before + x - sum;
+#pragma unroll
+        for (uint32_t k = 0; k < GSCAN_PT; ++k) {
+            if (g0 + k < nspan)
+                tsum[g0 + k] = run;
+            run += v[k];
+        }
+        carry = total;
+        __syncthreads();
     }
+    if (t == 0)
+        tsum[nspan] = carry;
 }
 
-// first position of sketch sid among the sorted trigger keys
-__device__ static inline uint32_t group_start(const uint32_t *__restrict__ sk, uint32_t n, uint32_t key0)
+// Triggers before chunk position pos (<= cn), computed by a whole wavefront:
+// the scanned span count plus the set bits of the span before pos (four
+// bitmap words per lane).
+static_assert(QS_TSPAN == 64u * 4u * 32u, "one 16-byte load per lane covers a span");
+__device__ static inline uint32_t trig_rank(const uint32_t *__restrict__ tbit, const uint32_t *__restrict__ tsum,
+                                            uint32_t pos, uint32_t cn)
 {
-    uint32_t lo = 0, hi = n; // first index with sk[i] >= key0
-    while (lo < hi) {
-        uint32_t mid = (lo + hi) >> 1;
-        if (sk[mid] < key0)
-            lo = mid + 1;
-        else
-            hi = mid;
+    if (pos >= cn)
+        return tsum[(cn + QS_TSPAN - 1u) / QS_TSPAN];
+    const uint32_t lane = threadIdx.x & 63u, span = pos / QS_TSPAN, w = (pos % QS_TSPAN) >> 5;
+    const uint4 q = reinterpret_cast<const uint4 *>(tbit + (size_t)span * (QS_TSPAN / 32u))[lane];
+    const uint32_t b[4] = {q.x, q.y, q.z, q.w};
+    uint32_t c = 0;
+#pragma unroll
+    for (uint32_t k = 0; k < 4u; ++k) {
+        const uint32_t i = lane * 4u + k;
+        const uint32_t m = i < w ? b[k] : i == w ? b[k] & ((1u << (pos & 31u)) - 1u) : 0u;
+        c += (uint32_t)__popc(m);
     }
-    return lo;
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1)
+        c += (uint32_t)__shfl_xor((int)c, o, 64);
+    return tsum[span] + c;
 }
 
 // Ids in stream order of the triggering inserts, per sketch (the sequential
-// bump allocator of v3:68-85, next starting at 1025).
-__global__ __launch_bounds__(256) void k_assign(const qs_trig *__restrict__ trig,
-                                                const uint32_t *__restrict__ skey,
-                                                const uint32_t *__restrict__ order, uint32_t trig_cap,
-                                                uint32_t ib, const qs_sdesc *__restrict__ D,
+// bump allocator of v3:68-85, next starting at 1025).  The sketches' parts of
+// a chunk follow one another, so a trigger's rank within its sketch is its
+// rank in the chunk less that of its sketch's first position.
+// (The order came from a pair sort of the triggers before: three launches per
+// digit pass.  At 2^22 keys that was 57 us of kernels and 12 launches; the
+// bitmap costs one 8 us scan and no sort.)
+__global__ __launch_bounds__(256) void k_assign(const qs_trig *__restrict__ trig, uint32_t trig_cap,
+                                                const uint32_t *__restrict__ tbit,
+                                                const uint32_t *__restrict__ tsum, uint32_t cn,
+                                                const uint64_t *__restrict__ offs, uint64_t base,
+                                                const qs_sdesc *__restrict__ D, uint32_t nsk,
                                                 uint32_t *__restrict__ low_pool,
                                                 uint32_t *__restrict__ high_pool,
                                                 uint32_t *__restrict__ tail_pool,
@@ -1510,13 +1590,13 @@ __global__ __launch_bounds__(256) void k_assign(const qs_trig *__restrict__ trig
     const uint32_t gw = blockIdx.x * 4u + (threadIdx.x >> 6);
     const uint32_t nw = gridDim.x * 4u;
     for (uint32_t r = gw; r < n_trig; r += nw) {
-        const qs_trig *tr = trig + order[r];
+        const qs_trig *tr = trig + r;
         const uint32_t sid = tr->sid;
-        // sketch 0's keys sort first: its group starts at 0 (every trigger of a
-        // single sketch skips the search)
-        const uint32_t start = sid == 0 ? 0u : group_start(skey, n_trig, sid << ib);
+        uint32_t rank = trig_rank(tbit, tsum, tr->idx, cn);
+        if (nsk > 1)
+            rank -= trig_rank(tbit, tsum, sid_chunk_start(offs, sid, base), cn);
         const qs_sdesc &d = D[sid];
-        const uint32_t id = next[sid] + (r - start);
+        const uint32_t id = next[sid] + rank;
         const uint32_t row = id - QS_LINK_START;
         if (row >= d.n_high) {
             if (lane == 0)
@@ -1803,21 +1883,27 @@ __global__ void k_clear_long(const uint32_t *__restrict__ lng, const uint64_t *_
     }
 }
 
-// next[sid] += allocations of sid in this chunk: the last trigger of each
-// sketch group writes its id + 1.
-__global__ void k_next(const qs_trig *__restrict__ trig, const uint32_t *__restrict__ skey,
-                       const uint32_t *__restrict__ order, uint32_t trig_cap, uint32_t ib,
-                       uint32_t *__restrict__ next, const qs_dev_state *__restrict__ st)
+// next[sid] += allocations of sid in this chunk (a wavefront per sketch)
+__global__ __launch_bounds__(256) void k_next(const uint32_t *__restrict__ tbit, const uint32_t *__restrict__ tsum,
+                                              uint32_t cn, const uint64_t *__restrict__ offs, uint64_t base,
+                                              uint32_t nsk, uint32_t *__restrict__ next,
+                                              const qs_dev_state *__restrict__ st)
 {
-    const uint32_t n_trig = min(st->n_trig, trig_cap);
-    if (st->err)
+    if (st->err || st->n_trig == 0)
         return;
-    for (uint32_t r = blockIdx.x * blockDim.x + threadIdx.x; r < n_trig; r += gridDim.x * blockDim.x) {
-        const uint32_t sid = skey[r] >> ib;
-        if (r + 1 == n_trig || (skey[r + 1] >> ib) != sid) {
-            const uint32_t start = group_start(skey, n_trig, sid << ib);
-            next[sid] += r - start + 1;
+    const uint32_t lane = threadIdx.x & 63u;
+    const uint32_t nw = gridDim.x * 4u;
+    for (uint32_t sid = blockIdx.x * 4u + (threadIdx.x >> 6); sid < nsk; sid += nw) {
+        uint32_t c = st->n_trig;
+        if (nsk > 1) {
+            // (the chunk may begin or end inside a sketch's part, or hold none of it)
+            const uint64_t end = offs[sid + 1], lo = end > base ? sid_chunk_start(offs, sid, base) : cn;
+            const uint64_t hi = end > base ? end - base : cn;
+            c = lo < cn ? trig_rank(tbit, tsum, hi < cn ? (uint32_t)hi : cn, cn) - trig_rank(tbit, tsum, (uint32_t)lo, cn)
+                        : 0u;
         }
+        if (lane == 0 && c)
+            next[sid] += c;
     }
 }
 
@@ -1842,19 +1928,26 @@ uint64_t qs_scratch_hist_words(uint64_t chunk)
     if (tiles == 0)
         tiles = 1;
     // tile-major counts + group sums + digit totals
-    uint64_t a = OS_BINS * tiles + OS_BINS * ((tiles + SCAN_TPB - 1) / SCAN_TPB) + OS_BINS;
-    uint64_t b = qs_sort_hist_words((uint32_t)(chunk < 0xffffffffull ? chunk : 0xffffffffull));
-    return a > b ? a : b;
+    return OS_BINS * tiles + OS_BINS * ((tiles + SCAN_TPB - 1) / SCAN_TPB) + OS_BINS;
+}
+
+// bytes of the allocation bitmap (whole spans) and words of its span counts
+static uint64_t tbit_bytes(uint64_t chunk)
+{
+    return (chunk + QS_TSPAN - 1) / QS_TSPAN * (QS_TSPAN / 8u);
+}
+static uint64_t tsum_words(uint64_t chunk)
+{
+    return (chunk + QS_TSPAN - 1) / QS_TSPAN + 1;
 }
 
 void qs_free_scratch(qs_sketch *s)
 {
     qs_scratch &sc = s->sc;
-    for (int k = 0; k < 2; ++k) {
+    for (int k = 0; k < 2; ++k)
         hipFree(sc.it[k]);
-        hipFree(sc.tk[k]);
-        hipFree(sc.tv[k]);
-    }
+    hipFree(sc.tbit);
+    hipFree(sc.tsum);
     hipFree(sc.hist);
     hipFree(sc.dig);
     hipFree(sc.ord);
@@ -1889,10 +1982,8 @@ uint64_t qs_scratch_bytes(uint64_t chunk, uint32_t tcap, qs_scratch *sc, uint8_t
     t.ord = (uint32_t *)take(sizeof(uint32_t) * chunk);
     t.lng = (uint32_t *)take(sizeof(uint32_t) * (chunk / 8 + 64));
     t.trig = (qs_trig *)take(sizeof(qs_trig) * tcap);
-    for (int k = 0; k < 2; ++k) {
-        t.tk[k] = (uint32_t *)take(sizeof(uint32_t) * tcap);
-        t.tv[k] = (uint32_t *)take(sizeof(uint32_t) * tcap);
-    }
+    t.tbit = (uint32_t *)take(tbit_bytes(chunk));
+    t.tsum = (uint32_t *)take(sizeof(uint32_t) * tsum_words(chunk));
     t.chunk = chunk;
     t.trig_cap = tcap;
     if (sc)
@@ -1909,12 +2000,12 @@ int qs_ensure_scratch(qs_sketch *s, uint64_t chunk)
     const uint32_t tcap = qs_trig_cap(s, chunk);
     qs_scratch &sc = s->sc;
     sc.trig_cap = tcap;
-    for (int k = 0; k < 2; ++k) {
-        if (hipMalloc(&sc.it[k], sizeof(uint64_t) * chunk) != hipSuccess ||
-            hipMalloc(&sc.tk[k], sizeof(uint32_t) * tcap) != hipSuccess ||
-            hipMalloc(&sc.tv[k], sizeof(uint32_t) * tcap) != hipSuccess)
+    for (int k = 0; k < 2; ++k)
+        if (hipMalloc(&sc.it[k], sizeof(uint64_t) * chunk) != hipSuccess)
             return QS_ERR_NOMEM;
-    }
+    if (hipMalloc(&sc.tbit, tbit_bytes(chunk)) != hipSuccess ||
+        hipMalloc(&sc.tsum, sizeof(uint32_t) * tsum_words(chunk)) != hipSuccess)
+        return QS_ERR_NOMEM;
     if (hipMalloc(&sc.hist, sizeof(uint32_t) * qs_scratch_hist_words(chunk)) != hipSuccess ||
         hipMalloc(&sc.dig, (chunk + OS_TILE - 1) / OS_TILE * OS_TILE) != hipSuccess ||
         hipMalloc(&sc.ord, sizeof(uint32_t) * chunk) != hipSuccess ||
@@ -1963,7 +2054,7 @@ static int sort_chunk(qs_sketch *s, const KeyT<KB> *keys, uint32_t cn, uint64_t 
         if (ps == 0)
             hipLaunchKernelGGL((k_bs_up<KB, MULTI>), dim3(ntiles), dim3(OS_THREADS), 0, stream, in, cn,
                                base, d0, s->d_desc, bc.d_offs, s->nsk, s->pk, shift, dmask, nbins, ntiles,
-                               tcount);
+                               tcount, sc.tbit, sc.tsum);
         else
             hipLaunchKernelGGL(k_bs_up_dig, dim3((ntiles + UP_TILES - 1) / UP_TILES), dim3(OS_THREADS), 0, stream,
                                sc.dig, cn, ntiles, nbins, tcount);
@@ -2060,22 +2151,14 @@ static int insert_chunk(qs_sketch *s, const KeyT<KB> *keys, uint32_t cn, uint64_
     }
     hipLaunchKernelGGL(k_ordered, dim3(grid_cap(((uint64_t)cn + 255) / 256, 8)), dim3(256), 0, stream, IT, cn,
                        sc.ord, s->d_desc, s->d_low, s->d_masks, s->pk, s->d_longbm, sc.lng, sc.trig,
-                       sc.trig_cap, s->nsk == 1 ? s->h_desc[0].n_masks : 0u, s->d_st);
+                       sc.trig_cap, sc.tbit, sc.tsum, bc.d_offs, base, MULTI ? 0u : nm0, s->d_st);
     if (bc.timed) {
         qs_tim_next(s, eo, ea, QS_TK_ASSIGN, cn, stream);
     }
-    hipLaunchKernelGGL(k_trig_keys, dim3(grid_cap(((uint64_t)sc.trig_cap + 255) / 256, 4)), dim3(256), 0, stream,
-                       sc.trig, s->d_st, sc.trig_cap, s->pk.ib, sc.tk[0], sc.tv[0]);
-    // a single sketch's trigger keys are stream indices below cn (one digit
-    // pass fewer for a chunk of at most 2^24 keys)
-    const int tbits = s->nsk == 1 ? (int)qs_bits_for(cn) : (int)(s->pk.sb + s->pk.ib);
-    uint32_t *tk[2] = {sc.tk[0], sc.tk[1]}, *tv[2] = {sc.tv[0], sc.tv[1]};
-    const int tc = qs_sort_pairs_dev(tk, tv, sc.hist, &s->d_st->n_trig, sc.trig_cap,
-                                     tbits > 32 ? 32 : tbits, stream);
-    if (tc < 0)
-        return QS_ERR_HIP;
+    hipLaunchKernelGGL(k_trig_scan, dim3(1), dim3(1024), 0, stream, sc.tsum, (cn + QS_TSPAN - 1u) / QS_TSPAN,
+                       s->d_st);
     hipLaunchKernelGGL(k_assign, dim3(grid_cap(((uint64_t)sc.trig_cap + 3) / 4, 8)), dim3(256), 0, stream,
-                       sc.trig, sc.tk[tc], sc.tv[tc], sc.trig_cap, s->pk.ib, s->d_desc, s->d_low,
+                       sc.trig, sc.trig_cap, sc.tbit, sc.tsum, cn, bc.d_offs, base, s->d_desc, s->nsk, s->d_low,
                        s->d_high, s->d_tail_of, s->d_next, s->d_st);
     if (bc.timed) {
         qs_tim_next(s, ea, et, QS_TK_TAIL, cn, stream);
@@ -2094,8 +2177,8 @@ static int insert_chunk(qs_sketch *s, const KeyT<KB> *keys, uint32_t cn, uint64_
                            short_runs, s->d_st);
     hipLaunchKernelGGL(k_clear_long, dim3(grid_cap(((uint64_t)cn / 64 + 255) / 256, 4)), dim3(256), 0, stream,
                        sc.lng, IT, s->d_desc, s->pk, s->d_longbm, s->d_st);
-    hipLaunchKernelGGL(k_next, dim3(grid_cap(((uint64_t)sc.trig_cap + 255) / 256, 4)), dim3(256), 0, stream,
-                       sc.trig, sc.tk[tc], sc.tv[tc], sc.trig_cap, s->pk.ib, s->d_next, s->d_st);
+    hipLaunchKernelGGL(k_next, dim3(grid_cap(((uint64_t)s->nsk + 3) / 4, 4)), dim3(256), 0, stream, sc.tbit, sc.tsum,
+                       cn, bc.d_offs, base, s->nsk, s->d_next, s->d_st);
     hipLaunchKernelGGL(k_reset, dim3(1), dim3(64), 0, stream, s->d_st);
     if (bc.timed)
         qs_tim_end(s, et, stream);

@@ -255,12 +255,16 @@ static_assert(offsetof(qs_dev_state, n_ord) % 8 == 0 && offsetof(qs_dev_state, n
 
 // One allocation found by the in-order replay (filled before ids are known).
 struct qs_trig {
-    uint32_t idx;        // stream index of the triggering insert (within its sketch)
+    uint32_t idx;        // chunk position of the triggering insert
     uint32_t bucket;     // low bucket
     uint32_t tail_start; // first sorted position handled by the tail kernel
     uint32_t sid;        // sketch
     uint32_t hc[32];     // high counters accumulated up to tail_start (incl. trigger)
 };
+
+// chunk positions counted together in qs_scratch::tsum (one wavefront reads a
+// span of the bitmap as one 16-byte load per lane)
+#define QS_TSPAN 8192u
 
 // Device scratch of the insert pipeline for chunks of up to `chunk` keys.  A
 // handle allocates its own (qs_ensure_scratch); the allocation-free insert
@@ -269,14 +273,14 @@ struct qs_trig {
 struct qs_scratch {
     uint64_t chunk;         // capacity (keys)
     uint64_t *it[2];        // packed chunk items sorted by cell (double buffer)
-    uint32_t *hist;         // radix histograms (both sorts), qs_scratch_hist_words(chunk) words
+    uint32_t *hist;         // radix histograms, qs_scratch_hist_words(chunk) words
     uint8_t *dig;           // the next radix pass's digit of each sorted item (one byte per item)
     uint32_t *ord;          // heads of segments for the in-order replay
     uint32_t *lng;          // heads of long segments
     qs_trig *trig;          // allocations found by the replay
-    uint32_t trig_cap;      // entries of trig, tk, tv: at most the pool (sum of n_high) and the chunk
-    uint32_t *tk[2];        // trigger sort keys / values
-    uint32_t *tv[2];
+    uint32_t trig_cap;      // entries of trig: at most the pool (sum of n_high) and the chunk
+    uint32_t *tbit;         // one bit per chunk position: an allocation is triggered there
+    uint32_t *tsum;         // set bits per QS_TSPAN positions, then their exclusive scan (+ total)
 };
 
 // Host-side handle: a set of nsk sketches (nsk == 1 for the plain API).

@@ -1,9 +1,7 @@
 // qs_sort.hip -- stable LSD radix sort of (uint32 key, uint32 value) pairs.
 //
-// Used by the ordered fix-up of the insert path: the keys routed to the fix-up
-// arrive in stream order and are sorted by low bucket, so that each bucket's
-// inserts form one segment still in stream order (LSD radix sort is stable).
-// It is also used to order the allocations of one chunk by stream position.
+// Used by the hot-key filter (qs_hot.hip): its sample of keys, and the
+// candidates by their count.
 //
 // One pass = 8 key bits = three kernels:
 //   k_hist       per-tile digit histogram (LDS atomics), digit-major layout
