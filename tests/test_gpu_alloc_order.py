@@ -68,3 +68,17 @@ def test_set_ids_at_span_edges(gpu, chunk_keys):
         assert np.array_equal(st["low"], o.low()), i
         assert np.array_equal(st["high"], o.high()), i
         assert st["next"] == o.next, i
+
+
+@pytest.mark.parametrize("n", [65537, (1 << 20) + 1, (1 << 21) - 255, (3 << 20) + 63])
+def test_tail_windows_by_chunk_length(gpu, n):
+    """Long runs cross the tail pass's windows, whose length follows the chunk's
+    (256 items up to 2^20 keys, then more)."""
+    from tests.helpers import zipf_keys
+    print("CASE tail", n, flush=True)
+    keys = zipf_keys(1.3, 1 << 14, n, seed=n)
+    g, o = make_pair(12281, n_high=1 << 12)
+    for part in (keys, keys[: n // 3]):
+        g.insert(to_dev(part))
+        assert o.insert(part) == 0
+        assert_same_state(g, o, f"n={n}")
