@@ -351,6 +351,21 @@ __global__ __launch_bounds__(OS_THREADS) void k_bs_up_dig(const uint8_t *__restr
             hist[(size_t)(tile0 + k) * nbins + t] = (uint16_t)s_h[k][t];
 }
 
+// How a scatter finds its tile's offsets: by the two scan kernels below, or,
+// for few tiles, by summing counts itself (every launch costs about 5 us of
+// GPU time and a gap, more than reading a few rows in every block).
+//   SCAN_FULL   both scan kernels
+//   SCAN_LOCAL  k_hist_scan_local only; the scatter sums at most SCAN_SUM_GROUPS
+//               group rows
+//   SCAN_NONE   no scan kernel; it sums at most SCAN_SUM_TILES tile rows
+// Summing 33 tile rows (65537 keys) costs a scatter 3 us and saves two
+// launches; summing 64 group rows (2^22 keys) cost it 12 us and saved 4.
+#define SCAN_FULL 0
+#define SCAN_LOCAL 1
+#define SCAN_NONE 2
+#define SCAN_SUM_TILES 64u
+#define SCAN_SUM_GROUPS 16u
+
 // Two-level exclusive scan over tiles of the tile-major digit counts.
 // Level 1: each block takes SCAN_TPB consecutive tiles, thread d = digit d
 // (reads and writes are contiguous rows), and leaves group-local prefixes plus
@@ -470,8 +485,8 @@ __global__ __launch_bounds__(OS_THREADS) void k_bs_down(
     const void *__restrict__ in, uint32_t n, uint64_t base, qs_sdesc d0, const qs_sdesc *__restrict__ D,
     const uint64_t *__restrict__ offs, uint32_t nsk, qs_pack pk, int shift, uint32_t dmask,
     uint32_t nbins, uint32_t ntiles, const uint16_t *__restrict__ hist, const uint32_t *__restrict__ gsum,
-    const uint32_t *__restrict__ totals, uint64_t *__restrict__ out, uint8_t *__restrict__ dig, int nshift,
-    qs_dev_state *__restrict__ st)
+    const uint32_t *__restrict__ totals, int scan, uint64_t *__restrict__ out, uint8_t *__restrict__ dig,
+    int nshift, qs_dev_state *__restrict__ st)
 {
     __shared__ uint64_t s_item[OS_TILE];
     __shared__ uint32_t s_wh[OS_WAVES][OS_BINS];
@@ -499,9 +514,26 @@ __global__ __launch_bounds__(OS_THREADS) void k_bs_down(
         for (int w = 0; w < OS_WAVES; ++w)
             s_wh[w][t] = 0;
     const bool dv = t < nbins;
-    const uint32_t tot = dv ? totals[t] : 0u;
-    // items of digit t before this tile (tile-major counts, two-level scan)
-    const uint32_t hcur = dv ? hist[(size_t)tile * nbins + t] + gsum[(size_t)(tile / SCAN_TPB) * nbins + t] : 0u;
+    // items of digit t in the chunk and before this tile (tile-major counts)
+    uint32_t tot = 0, hcur = 0;
+    if (scan == SCAN_FULL) {
+        if (dv) {
+            tot = totals[t];
+            hcur = hist[(size_t)tile * nbins + t] + gsum[(size_t)(tile / SCAN_TPB) * nbins + t];
+        }
+    } else if (dv) {
+        const bool local = scan == SCAN_LOCAL;
+        const uint32_t rows = local ? (ntiles + SCAN_TPB - 1u) / SCAN_TPB : ntiles;
+        const uint32_t mine = local ? tile / SCAN_TPB : tile;
+#pragma unroll 8
+        for (uint32_t r = 0; r < rows; ++r) {
+            const uint32_t v = local ? gsum[(size_t)r * nbins + t] : (uint32_t)hist[(size_t)r * nbins + t];
+            tot += v;
+            hcur += r < mine ? v : 0u;
+        }
+        if (local)
+            hcur += hist[(size_t)tile * nbins + t];
+    }
     const uint32_t dbase = block_excl_scan(tot, s_red);
 
     const uint64_t lt = (1ull << lane) - 1ull;
@@ -1543,28 +1575,35 @@ __global__ __launch_bounds__(1024) void k_trig_scan(uint32_t *__restrict__ tsum,
 }
 
 // Triggers before chunk position pos (<= cn), computed by a whole wavefront:
-// the scanned span count plus the set bits of the span before pos (four
-// bitmap words per lane).
+// the span count's prefix plus the set bits of the span before pos (four
+// bitmap words per lane).  The counts of at most 64 spans are not scanned by a
+// kernel of their own: each lane takes one of them.
+#define TRIG_RAW_SPANS 64u
 static_assert(QS_TSPAN == 64u * 4u * 32u, "one 16-byte load per lane covers a span");
 __device__ static inline uint32_t trig_rank(const uint32_t *__restrict__ tbit, const uint32_t *__restrict__ tsum,
                                             uint32_t pos, uint32_t cn)
 {
-    if (pos >= cn)
-        return tsum[(cn + QS_TSPAN - 1u) / QS_TSPAN];
-    const uint32_t lane = threadIdx.x & 63u, span = pos / QS_TSPAN, w = (pos % QS_TSPAN) >> 5;
-    const uint4 q = reinterpret_cast<const uint4 *>(tbit + (size_t)span * (QS_TSPAN / 32u))[lane];
-    const uint32_t b[4] = {q.x, q.y, q.z, q.w};
-    uint32_t c = 0;
+    const uint32_t nspan = (cn + QS_TSPAN - 1u) / QS_TSPAN;
+    const bool scanned = nspan > TRIG_RAW_SPANS; // by k_trig_scan
+    if (scanned && pos >= cn)
+        return tsum[nspan];
+    const uint32_t lane = threadIdx.x & 63u, span = pos < cn ? pos / QS_TSPAN : nspan;
+    uint32_t c = !scanned && lane < span ? tsum[lane] : 0u;
+    if (pos < cn) {
+        const uint32_t w = (pos % QS_TSPAN) >> 5;
+        const uint4 q = reinterpret_cast<const uint4 *>(tbit + (size_t)span * (QS_TSPAN / 32u))[lane];
+        const uint32_t b[4] = {q.x, q.y, q.z, q.w};
 #pragma unroll
-    for (uint32_t k = 0; k < 4u; ++k) {
-        const uint32_t i = lane * 4u + k;
-        const uint32_t m = i < w ? b[k] : i == w ? b[k] & ((1u << (pos & 31u)) - 1u) : 0u;
-        c += (uint32_t)__popc(m);
+        for (uint32_t k = 0; k < 4u; ++k) {
+            const uint32_t i = lane * 4u + k;
+            const uint32_t m = i < w ? b[k] : i == w ? b[k] & ((1u << (pos & 31u)) - 1u) : 0u;
+            c += (uint32_t)__popc(m);
+        }
     }
 #pragma unroll
     for (int o = 32; o > 0; o >>= 1)
         c += (uint32_t)__shfl_xor((int)c, o, 64);
-    return tsum[span] + c;
+    return scanned ? tsum[span] + c : c;
 }
 
 // Ids in stream order of the triggering inserts, per sketch (the sequential
@@ -1871,52 +1910,57 @@ __global__ __launch_bounds__(256) void k_tail(const uint64_t *__restrict__ IT, u
     }
 }
 
-__global__ void k_clear_long(const uint32_t *__restrict__ lng, const uint64_t *__restrict__ IT,
-                             const qs_sdesc *__restrict__ D, qs_pack pk, uint32_t *__restrict__ longbm,
-                             const qs_dev_state *__restrict__ st)
+// The chunk's last kernel: the long-segment marks are taken back, next[sid]
+// moves on by the allocations of sid (a wavefront per sketch), and the block
+// that finishes last resets the chunk's counters and leaves the error bits in
+// the host's pinned mirror, so that a blocking call needs no copy.
+#define FIN_BLOCKS 64u // at most: every block ends with one atomic on st->done
+__global__ __launch_bounds__(256) void k_finish(const uint32_t *__restrict__ lng, const uint64_t *__restrict__ IT,
+                                                const qs_sdesc *__restrict__ D, qs_pack pk,
+                                                uint32_t *__restrict__ longbm, const uint32_t *__restrict__ tbit,
+                                                const uint32_t *__restrict__ tsum, uint32_t cn,
+                                                const uint64_t *__restrict__ offs, uint64_t base, uint32_t nsk,
+                                                uint32_t *__restrict__ next, qs_dev_state *__restrict__ st,
+                                                uint32_t *__restrict__ h_err)
 {
-    const uint32_t n_long = st->n_long;
+    const uint32_t n_long = st->n_long, n_trig = st->n_trig;
     for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < n_long; i += gridDim.x * blockDim.x) {
         const uint64_t it = IT[lng[i]];
         const uint64_t bit = D[it_sid(it, pk)].bm_off + it_b(it, pk);
         atomicAnd(longbm + (bit >> 5), ~(1u << (bit & 31u)));
     }
-}
-
-// next[sid] += allocations of sid in this chunk (a wavefront per sketch)
-__global__ __launch_bounds__(256) void k_next(const uint32_t *__restrict__ tbit, const uint32_t *__restrict__ tsum,
-                                              uint32_t cn, const uint64_t *__restrict__ offs, uint64_t base,
-                                              uint32_t nsk, uint32_t *__restrict__ next,
-                                              const qs_dev_state *__restrict__ st)
-{
-    if (st->err || st->n_trig == 0)
-        return;
-    const uint32_t lane = threadIdx.x & 63u;
-    const uint32_t nw = gridDim.x * 4u;
-    for (uint32_t sid = blockIdx.x * 4u + (threadIdx.x >> 6); sid < nsk; sid += nw) {
-        uint32_t c = st->n_trig;
-        if (nsk > 1) {
-            // (the chunk may begin or end inside a sketch's part, or hold none of it)
-            const uint64_t end = offs[sid + 1], lo = end > base ? sid_chunk_start(offs, sid, base) : cn;
-            const uint64_t hi = end > base ? end - base : cn;
-            c = lo < cn ? trig_rank(tbit, tsum, hi < cn ? (uint32_t)hi : cn, cn) - trig_rank(tbit, tsum, (uint32_t)lo, cn)
-                        : 0u;
+    if (n_trig && !st->err) {
+        const uint32_t lane = threadIdx.x & 63u;
+        for (uint32_t sid = blockIdx.x * 4u + (threadIdx.x >> 6); sid < nsk; sid += gridDim.x * 4u) {
+            uint32_t c = n_trig;
+            if (nsk > 1) {
+                // (the chunk may begin or end inside a sketch's part, or hold none of it)
+                const uint64_t end = offs[sid + 1];
+                const uint32_t lo = end > base ? sid_chunk_start(offs, sid, base) : cn;
+                c = 0;
+                if (lo < cn)
+                    c = trig_rank(tbit, tsum, end - base < cn ? (uint32_t)(end - base) : cn, cn) -
+                        trig_rank(tbit, tsum, lo, cn);
+            }
+            if (lane == 0 && c)
+                next[sid] += c;
         }
-        if (lane == 0 && c)
-            next[sid] += c;
     }
-}
-
-__global__ void k_reset(qs_dev_state *st)
-{
-    if (threadIdx.x == 0 && blockIdx.x == 0) {
-        st->ord_segments += st->n_ord;
-        st->long_segments += st->n_long;
-        st->chunks_ord += st->n_ord ? 1u : 0u;
-        st->n_ord = 0;
-        st->n_long = 0;
-        st->n_trig = 0;
-    }
+    __shared__ uint32_t s_last;
+    __syncthreads();
+    if (threadIdx.x == 0)
+        s_last = __hip_atomic_fetch_add(&st->done, 1u, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_AGENT);
+    __syncthreads();
+    if (s_last != gridDim.x - 1u || threadIdx.x != 0)
+        return;
+    st->ord_segments += st->n_ord;
+    st->long_segments += n_long;
+    st->chunks_ord += st->n_ord ? 1u : 0u;
+    st->n_ord = 0;
+    st->n_long = 0;
+    st->n_trig = 0;
+    st->done = 0;
+    __hip_atomic_store(h_err, st->err, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
 // ===========================================================================
@@ -2037,6 +2081,7 @@ static int sort_chunk(qs_sketch *s, const KeyT<KB> *keys, uint32_t cn, uint64_t 
     uint16_t *tcount = reinterpret_cast<uint16_t *>(sc.hist); // 16-bit tile counts (half the region)
     uint32_t *gsum = sc.hist + (size_t)OS_BINS * ntiles;
     uint32_t *totals = gsum + (size_t)OS_BINS * ngrp;
+    const int scan = ntiles <= SCAN_SUM_TILES ? SCAN_NONE : ngrp <= SCAN_SUM_GROUPS ? SCAN_LOCAL : SCAN_FULL;
     const qs_sdesc d0 = s->h_desc[0];
     const void *in = keys;
     int out = 0;
@@ -2060,18 +2105,20 @@ static int sort_chunk(qs_sketch *s, const KeyT<KB> *keys, uint32_t cn, uint64_t 
                                sc.dig, cn, ntiles, nbins, tcount);
         if (bc.timed)
             qs_tim_next(s, e0, e1, QS_TK_SORT_SCAN, cn, stream);
-        hipLaunchKernelGGL(k_hist_scan_local, dim3(ngrp), dim3(256), 0, stream, tcount, ntiles, nbins, gsum);
-        hipLaunchKernelGGL(k_hist_scan_groups, dim3(nbins), dim3(1024), 0, stream, gsum, ngrp, nbins, totals);
+        if (scan != SCAN_NONE)
+            hipLaunchKernelGGL(k_hist_scan_local, dim3(ngrp), dim3(256), 0, stream, tcount, ntiles, nbins, gsum);
+        if (scan == SCAN_FULL)
+            hipLaunchKernelGGL(k_hist_scan_groups, dim3(nbins), dim3(1024), 0, stream, gsum, ngrp, nbins, totals);
         if (bc.timed)
             qs_tim_next(s, e1, e2, QS_TK_SORT_DOWN, cn, stream);
         if (ps == 0)
             hipLaunchKernelGGL((k_bs_down<KB, true, MULTI>), dim3(ntiles), dim3(OS_THREADS), 0, stream, in, cn,
                                base, d0, s->d_desc, bc.d_offs, s->nsk, s->pk, shift, dmask, nbins, ntiles,
-                               tcount, gsum, totals, sc.it[out], sc.dig, nshift, s->d_st);
+                               tcount, gsum, totals, scan, sc.it[out], sc.dig, nshift, s->d_st);
         else
             hipLaunchKernelGGL((k_bs_down<KB, false, false>), dim3(ntiles), dim3(OS_THREADS), 0, stream, in, cn,
                                base, d0, s->d_desc, bc.d_offs, s->nsk, s->pk, shift, dmask, nbins, ntiles,
-                               tcount, gsum, totals, sc.it[out], sc.dig, nshift, s->d_st);
+                               tcount, gsum, totals, scan, sc.it[out], sc.dig, nshift, s->d_st);
         if (bc.timed) {
             if (ps + 1 == passes)
                 qs_tim_end(s, e2, stream);
@@ -2170,8 +2217,9 @@ static int insert_chunk(qs_sketch *s, const KeyT<KB> *keys, uint32_t cn, uint64_
     if (bc.timed) {
         qs_tim_next(s, eo, ea, QS_TK_ASSIGN, cn, stream);
     }
-    hipLaunchKernelGGL(k_trig_scan, dim3(1), dim3(1024), 0, stream, sc.tsum, (cn + QS_TSPAN - 1u) / QS_TSPAN,
-                       s->d_st);
+    const uint32_t nspan = (cn + QS_TSPAN - 1u) / QS_TSPAN;
+    if (nspan > TRIG_RAW_SPANS)
+        hipLaunchKernelGGL(k_trig_scan, dim3(1), dim3(1024), 0, stream, sc.tsum, nspan, s->d_st);
     hipLaunchKernelGGL(k_assign, dim3(grid_cap(((uint64_t)sc.trig_cap + 3) / 4, 8)), dim3(256), 0, stream,
                        sc.trig, sc.trig_cap, sc.tbit, sc.tsum, cn, bc.d_offs, base, s->d_desc, s->nsk, s->d_low,
                        s->d_high, s->d_tail_of, s->d_next, s->d_st);
@@ -2191,11 +2239,10 @@ static int insert_chunk(qs_sketch *s, const KeyT<KB> *keys, uint32_t cn, uint64_
         hipLaunchKernelGGL((k_tail<MULTI, uint64_t>), tgrid, dim3(256), tail_lds, stream, IT, cn, s->d_desc, nm0,
                            s->d_low, s->d_high, s->d_masks, s->pk, s->d_longbm, s->d_tail_of, s->d_next, sc.lng,
                            short_runs, twin, s->d_st);
-    hipLaunchKernelGGL(k_clear_long, dim3(grid_cap(((uint64_t)cn / 64 + 255) / 256, 4)), dim3(256), 0, stream,
-                       sc.lng, IT, s->d_desc, s->pk, s->d_longbm, s->d_st);
-    hipLaunchKernelGGL(k_next, dim3(grid_cap(((uint64_t)s->nsk + 3) / 4, 4)), dim3(256), 0, stream, sc.tbit, sc.tsum,
-                       cn, bc.d_offs, base, s->nsk, s->d_next, s->d_st);
-    hipLaunchKernelGGL(k_reset, dim3(1), dim3(64), 0, stream, s->d_st);
+    const uint64_t fin = (uint64_t)cn / 64 / 256 > (uint64_t)s->nsk / 4 ? (uint64_t)cn / 64 / 256 : (uint64_t)s->nsk / 4;
+    hipLaunchKernelGGL(k_finish, dim3((uint32_t)(fin < FIN_BLOCKS ? fin + 1 : FIN_BLOCKS)), dim3(256), 0, stream,
+                       sc.lng, IT, s->d_desc, s->pk, s->d_longbm, sc.tbit, sc.tsum, cn, bc.d_offs, base, s->nsk,
+                       s->d_next, s->d_st, &s->h_st->err);
     if (bc.timed)
         qs_tim_end(s, et, stream);
     CK(hipGetLastError());
@@ -2277,8 +2324,7 @@ static int insert_impl(qs_sketch *s, const void *d_keys, const uint64_t *offs, c
         done += cn;
     }
     if (blocking) {
-        CK(hipMemcpyAsync(s->h_st, s->d_st, sizeof(qs_dev_state), hipMemcpyDeviceToHost, stream));
-        CK(hipStreamSynchronize(stream));
+        CK(hipStreamSynchronize(stream)); // k_finish left the error bits in h_st
         if (s->h_st->err) {
             s->sticky_err = qs_err_code(s->h_st->err);
             return s->sticky_err;

@@ -248,6 +248,8 @@ struct qs_dev_state {
     unsigned long long ord_segments;  // segments sent to the replay
     unsigned long long long_segments; // segments handled by the tail kernel
     unsigned long long chunks_ord;    // chunks with at least one replayed segment
+    uint32_t done;      // blocks of the chunk's last kernel that have finished (its last block clears it)
+    uint32_t pad;
 };
 // k_segw reserves entries of both lists with one 64-bit atomic on (n_ord, n_long)
 static_assert(offsetof(qs_dev_state, n_ord) % 8 == 0 && offsetof(qs_dev_state, n_long) == offsetof(qs_dev_state, n_ord) + 4,

@@ -70,7 +70,8 @@ def test_set_ids_at_span_edges(gpu, chunk_keys):
         assert st["next"] == o.next, i
 
 
-@pytest.mark.parametrize("n", [65537, (1 << 20) + 1, (1 << 21) - 255, (3 << 20) + 63])
+# (also: 64 and 65 radix tiles, 16 and 17 groups of them, 64 and 65 spans)
+@pytest.mark.parametrize("n", [64 * 2048, 64 * 2048 + 1, 64 * SPAN, 64 * SPAN + 1, 16 * 32 * 2048 + 1, 65537, (1 << 20) + 1, (1 << 21) - 255, (3 << 20) + 63])
 def test_tail_windows_by_chunk_length(gpu, n):
     """Long runs cross the tail pass's windows, whose length follows the chunk's
     (256 items up to 2^20 keys, then more)."""
