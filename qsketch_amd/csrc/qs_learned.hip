@@ -4,11 +4,11 @@
 // is a 64 -> 64 -> 64 -> 1 MLP with ReLU on the 64 bits of a key, BF16 weights
 // and activations, FP32 accumulation:
 //   h1 = bf16(relu(W1 x + b1)),  h2 = bf16(relu(W2 h1 + b2)),  y = w3 . h2 + b3
-// Training kernels (VALU, one key per lane):
-//   k_mlp_grad  forward + backward of a minibatch, gradients summed per block
-//               in LDS-staged small GEMMs and added to an FP32 gradient buffer
-//   k_adam      Adam on the FP32 master weights; writes the BF16 copies and
-//               clears the gradient buffer
+// Training kernels (VALU, one unit per lane):
+//   k_mlp_grad  forward + backward of a minibatch, each block's gradients in a row
+//               of its own
+//   k_grad_sum  sums the blocks' partial gradients; Adam on the FP32 master weights
+//               and their BF16 copies
 // Serving kernels:
 //   k_mlp_mfma  the same forward on the matrix cores: a wavefront scores 32
 //               keys with v_mfma_f32_32x32x8_bf16, computing H^T = W X^T so that
@@ -61,8 +61,9 @@ struct qs_learned {
     float *d_p;        // FP32 master parameters
     uint16_t *d_pb;    // BF16 copies
     float *d_m, *d_v;  // Adam moments
-    float *d_g;        // gradient accumulator
-    float *d_loss;
+    float *d_part;     // partial gradients, a row per block of k_mlp_grad
+    float *d_g;        // gradient of the last batch (the row after d_part's)
+    float *d_loss;     // its loss (the element after the gradient)
     uint64_t step;
     float thr;
     uint32_t tlog2;
@@ -119,153 +120,247 @@ __device__ static inline uint64_t key64(const KeyT<KB> *keys, uint64_t i)
 }
 
 // ---------------------------------------------------------------------------
-// training: forward + backward of 64 keys per block (one per lane)
+// training: forward + backward
+//
+// A block takes groups of GK keys in turn.  In the forward and the deltas a
+// wavefront works on GK / 4 keys with one unit per lane (each unit's sum still
+// runs over its inputs in order, so activations and deltas equal the per-key
+// forward's bit for bit); the weights lie in LDS so that the lanes read
+// neighbouring words, and a read serves the wavefront's keys.  The
+// weight gradients are 64 x 64 outer-product sums over the group, GR elements of
+// each per thread, kept in registers over all of the block's groups and
+// written as the block's row of partial gradients (k_grad_sum adds the rows).  Bound by LDS reads (about five per 16
+// FMAs); the first form had one key per lane, 64 keys per block and one
+// wavefront per CU on a quarter of the chip: 356 us for 4096 keys, now 15.
 // ---------------------------------------------------------------------------
-#define GB 64 // keys per gradient block
+#define GK 16u        // keys per group
+#define GT 512u       // threads
+#define GNW (GT / 64u) // wavefronts
+#define GW (GK / GNW)  // keys per wavefront
+#define GR (64u / GNW) // rows of a weight gradient per wavefront
+static_assert(GR % 4u == 0 && GW * GNW == GK && 192u * GNW <= GK * 64u * 2u, "work per wavefront");
+#define GRAD_BLOCKS 256u // one per CU: rows of partial gradients at most
+#define PART_STRIDE 8448u // floats per row (parameters and loss, in whole 64s)
+static_assert(PART_STRIDE > NPAR && PART_STRIDE % 64u == 0, "a row holds the gradients and the loss");
+#define WT 66u        // row stride of a transposed weight matrix in LDS
 
-template <int KB>
-__global__ __launch_bounds__(GB) void k_mlp_grad(const KeyT<KB> *__restrict__ keys, const float *__restrict__ tgt,
-                                                 uint32_t n, const uint16_t *__restrict__ pb,
-                                                 const float *__restrict__ p, float inv_n, float *__restrict__ g,
-                                                 float *__restrict__ loss)
+// orders a wavefront's LDS writes before its later reads (the hardware keeps
+// one wavefront's LDS accesses in order; this holds the compiler to it)
+__device__ static inline void wave_lds_fence()
 {
-    __shared__ uint16_t sW1[64 * 64], sW2[64 * 64];
-    __shared__ float sb1[64], sb2[64], sw3[64];
-    __shared__ uint16_t sh1[GB][66], sh2[GB][66];
-    __shared__ float sd[GB][65]; // dh2, later dh1
-    __shared__ unsigned long long sx[GB];
-    __shared__ float sdy[GB];
-    const uint32_t t = threadIdx.x;
-    for (uint32_t e = t; e < 4096u; e += GB) {
-        sW1[e] = pb[OFF_W1 + e];
-        sW2[e] = pb[OFF_W2 + e];
-    }
-    sb1[t] = p[OFF_B1 + t];
-    sb2[t] = p[OFF_B2 + t];
-    sw3[t] = bf2f(pb[OFF_W3 + t]);
-    const float b3 = p[OFF_B3];
-    __syncthreads();
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+}
 
-    const uint32_t i = blockIdx.x * GB + t;
-    const bool valid = i < n;
-    const uint64_t x = valid ? key64<KB>(keys, i) : 0ull;
-    // forward; this lane's activations live in its LDS rows, the ReLU masks
-    // in registers
-    uint64_t m1 = 0, m2 = 0;
-    for (int j = 0; j < 64; ++j) {
-        float acc = sb1[j];
-        for (int k = 0; k < 64; ++k)
-            acc += ((x >> k) & 1ull) ? bf2f(sW1[j * 64 + k]) : 0.f;
-        m1 |= (uint64_t)(acc > 0.f) << j;
-        sh1[t][j] = f2bf(fmaxf(acc, 0.f));
-    }
-    float y = b3;
-    for (int j = 0; j < 64; ++j) {
-        float acc = sb2[j];
-        for (int k = 0; k < 64; ++k)
-            acc = fmaf(bf2f(sW2[j * 64 + k]), bf2f(sh1[t][k]), acc);
-        m2 |= (uint64_t)(acc > 0.f) << j;
-        const uint16_t h2 = f2bf(fmaxf(acc, 0.f));
-        sh2[t][j] = h2;
-        y = fmaf(sw3[j], bf2f(h2), y);
-    }
-    const float diff = valid ? (y - tgt[i]) : 0.f;
-    const float dy = diff * inv_n;
-    // backward to the hidden layers
-    for (int j = 0; j < 64; ++j)
-        sd[t][j] = ((m2 >> j) & 1ull) ? dy * sw3[j] : 0.f;
-    float dh1[64];
-#pragma unroll
-    for (int k = 0; k < 64; ++k) {
-        float acc = 0.f;
-        for (int j = 0; j < 64; ++j)
-            acc = fmaf(bf2f(sW2[j * 64 + k]), sd[t][j], acc);
-        dh1[k] = ((m1 >> k) & 1ull) ? acc : 0.f;
-    }
-    sx[t] = x;
-    sdy[t] = dy;
-    // loss: sum over the block, one atomic
-    float l = 0.5f * diff * diff * inv_n;
+__device__ static inline float wave_sum(float v)
+{
 #pragma unroll
     for (int o = 32; o > 0; o >>= 1)
-        l += __shfl_xor(l, o, 64);
-    if (t == 0)
-        atomicAdd(loss, l);
+        v += __shfl_xor(v, o, 64);
+    return v;
+}
+
+template <int KB>
+__global__ __launch_bounds__(GT) void k_mlp_grad(const KeyT<KB> *__restrict__ keys, const float *__restrict__ tgt,
+                                                 uint32_t n, const uint16_t *__restrict__ pb,
+                                                 const float *__restrict__ p, float inv_n,
+                                                 float *__restrict__ part)
+{
+    __shared__ uint16_t sW1t[64 * WT], sW2t[64 * WT]; // [input][unit]
+    __shared__ uint16_t sW2[64 * 64];                 // [unit][input]
+    __shared__ float4 srows[3][GK][16]; // per key: h1, and the deltas of layers 2 and 1
+    float4(*const sh1)[16] = srows[0], (*const sd2)[16] = srows[1], (*const sd1)[16] = srows[2];
+    __shared__ unsigned long long sx[GK];
+    const uint32_t t = threadIdx.x, lane = t & 63u, wv = t >> 6;
+    for (uint32_t e = t; e < 2048u; e += GT) { // two weights of row j at a time
+        const uint32_t j = e >> 5, k = 2u * (e & 31u);
+        const uint32_t a = reinterpret_cast<const uint32_t *>(pb + OFF_W1)[e];
+        const uint32_t b = reinterpret_cast<const uint32_t *>(pb + OFF_W2)[e];
+        sW1t[k * WT + j] = (uint16_t)a;
+        sW1t[(k + 1u) * WT + j] = (uint16_t)(a >> 16);
+        sW2t[k * WT + j] = (uint16_t)b;
+        sW2t[(k + 1u) * WT + j] = (uint16_t)(b >> 16);
+        reinterpret_cast<uint32_t *>(sW2)[e] = b;
+    }
+    const float b1 = p[OFF_B1 + lane], b2 = p[OFF_B2 + lane], w3 = bf2f(pb[OFF_W3 + lane]), b3 = p[OFF_B3];
+    // gradient sums of this thread: W2 and W1 elements (row GR wv + i, column
+    // lane), and this wavefront's part of unit lane's b1, b2, w3
+    float a2[GR], a1[GR], gb1 = 0.f, gb2 = 0.f, gw3 = 0.f, gb3 = 0.f, l = 0.f;
+#pragma unroll
+    for (uint32_t i = 0; i < GR; ++i)
+        a2[i] = a1[i] = 0.f;
     __syncthreads();
-    // W2 (row j, column k), b2, w3, b3
-    for (uint32_t e = t; e < 4225u; e += GB) {
-        float acc = 0.f;
-        if (e < 4096u) {
-            const uint32_t j = e >> 6, k = e & 63u;
-            for (uint32_t s = 0; s < GB; ++s)
-                acc = fmaf(sd[s][j], bf2f(sh1[s][k]), acc);
-            atomicAdd(g + OFF_W2 + e, acc);
-        } else if (e < 4160u) {
-            const uint32_t j = e - 4096u;
-            for (uint32_t s = 0; s < GB; ++s)
-                acc += sd[s][j];
-            atomicAdd(g + OFF_B2 + j, acc);
-        } else if (e < 4224u) {
-            const uint32_t j = e - 4160u;
-            for (uint32_t s = 0; s < GB; ++s)
-                acc = fmaf(sdy[s], bf2f(sh2[s][j]), acc);
-            atomicAdd(g + OFF_W3 + j, acc);
-        } else {
-            for (uint32_t s = 0; s < GB; ++s)
-                acc += sdy[s];
-            atomicAdd(g + OFF_B3, acc);
+    for (uint64_t g0 = (uint64_t)blockIdx.x * GK; g0 < n; g0 += (uint64_t)gridDim.x * GK) {
+        uint64_t x[GW];
+        float z[GW], h1[GW];
+        bool m1[GW];
+#pragma unroll
+        for (uint32_t q = 0; q < GW; ++q) {
+            const uint64_t i = g0 + wv * GW + q;
+            const uint64_t xv = i < n ? key64<KB>(keys, i) : 0ull; // one address per wavefront:
+            x[q] = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)xv) | // in scalar registers
+                   (uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(xv >> 32)) << 32;
+            if (lane == 0)
+                sx[wv * GW + q] = x[q];
+            z[q] = b1;
         }
+#pragma unroll 8
+        for (uint32_t k = 0; k < 64u; ++k) {
+            const float w = bf2f(sW1t[k * WT + lane]);
+#pragma unroll
+            for (uint32_t q = 0; q < GW; ++q)
+                z[q] += ((x[q] >> k) & 1ull) ? w : 0.f;
+        }
+#pragma unroll
+        for (uint32_t q = 0; q < GW; ++q) {
+            m1[q] = z[q] > 0.f;
+            h1[q] = bf2f(f2bf(fmaxf(z[q], 0.f)));
+            reinterpret_cast<float *>(sh1[wv * GW + q])[lane] = h1[q];
+            z[q] = b2;
+        }
+        wave_lds_fence(); // a wavefront reads back its own rows only
+#pragma unroll 4
+        for (uint32_t k4 = 0; k4 < 16u; ++k4) {
+            float4 h[GW];
+#pragma unroll
+            for (uint32_t q = 0; q < GW; ++q)
+                h[q] = sh1[wv * GW + q][k4];
+#pragma unroll
+            for (uint32_t e = 0; e < 4u; ++e) {
+                const float w = bf2f(sW2t[(4u * k4 + e) * WT + lane]);
+#pragma unroll
+                for (uint32_t q = 0; q < GW; ++q)
+                    z[q] = fmaf(w, e == 0 ? h[q].x : e == 1 ? h[q].y : e == 2 ? h[q].z : h[q].w, z[q]);
+            }
+        }
+        float d1[GW];
+#pragma unroll
+        for (uint32_t q = 0; q < GW; ++q) {
+            const uint64_t i = g0 + wv * GW + q;
+            const float h2 = bf2f(f2bf(fmaxf(z[q], 0.f)));
+            const float y = wave_sum(w3 * h2) + b3;
+            const float diff = i < n ? y - tgt[i] : 0.f;
+            const float dy = diff * inv_n;
+            const float d2 = z[q] > 0.f ? dy * w3 : 0.f;
+            l += 0.5f * diff * diff * inv_n;
+            gw3 = fmaf(dy, h2, gw3);
+            gb3 += dy;
+            gb2 += d2;
+            reinterpret_cast<float *>(sd2[wv * GW + q])[lane] = d2;
+            d1[q] = 0.f;
+        }
+        wave_lds_fence();
+#pragma unroll 4
+        for (uint32_t j4 = 0; j4 < 16u; ++j4) {
+            float4 d[GW];
+#pragma unroll
+            for (uint32_t q = 0; q < GW; ++q)
+                d[q] = sd2[wv * GW + q][j4];
+#pragma unroll
+            for (uint32_t e = 0; e < 4u; ++e) {
+                const float w = bf2f(sW2[(4u * j4 + e) * 64u + lane]);
+#pragma unroll
+                for (uint32_t q = 0; q < GW; ++q)
+                    d1[q] = fmaf(w, e == 0 ? d[q].x : e == 1 ? d[q].y : e == 2 ? d[q].z : d[q].w, d1[q]);
+            }
+        }
+#pragma unroll
+        for (uint32_t q = 0; q < GW; ++q) {
+            const float d = m1[q] ? d1[q] : 0.f;
+            gb1 += d;
+            reinterpret_cast<float *>(sd1[wv * GW + q])[lane] = d;
+        }
+        __syncthreads(); // every wavefront's keys
+        for (uint32_t s = 0; s < GK; ++s) {
+            const float h = reinterpret_cast<const float *>(sh1[s])[lane];
+            const bool on = (sx[s] >> lane) & 1ull;
+#pragma unroll
+            for (uint32_t c = 0; c < GR / 4u; ++c) {
+                const float4 u = sd2[s][GR / 4u * wv + c], v = sd1[s][GR / 4u * wv + c];
+                a2[4 * c + 0] = fmaf(u.x, h, a2[4 * c + 0]);
+                a2[4 * c + 1] = fmaf(u.y, h, a2[4 * c + 1]);
+                a2[4 * c + 2] = fmaf(u.z, h, a2[4 * c + 2]);
+                a2[4 * c + 3] = fmaf(u.w, h, a2[4 * c + 3]);
+                a1[4 * c + 0] += on ? v.x : 0.f;
+                a1[4 * c + 1] += on ? v.y : 0.f;
+                a1[4 * c + 2] += on ? v.z : 0.f;
+                a1[4 * c + 3] += on ? v.w : 0.f;
+            }
+        }
+        __syncthreads(); // the next group rewrites the rows
+    }
+    // this block's row of partial gradients, with its loss in the element after
+    // them; the wavefronts' unit sums meet in LDS (the rows are free now)
+    float *const red = reinterpret_cast<float *>(srows), *const row = part + (size_t)blockIdx.x * PART_STRIDE;
+    red[wv * 192u + lane] = gb1;
+    red[wv * 192u + 64u + lane] = gb2;
+    red[wv * 192u + 128u + lane] = gw3;
+    float *const red2 = reinterpret_cast<float *>(sd1);
+    if (lane == 0) {
+        red2[2u * wv] = gb3;
+        red2[2u * wv + 1u] = l;
+    }
+#pragma unroll
+    for (uint32_t i = 0; i < GR; ++i) {
+        row[OFF_W2 + (GR * wv + i) * 64u + lane] = a2[i];
+        row[OFF_W1 + (GR * wv + i) * 64u + lane] = a1[i];
     }
     __syncthreads();
+    if (t < 194u) {
+        float v = 0.f;
 #pragma unroll
-    for (int k = 0; k < 64; ++k)
-        sd[t][k] = dh1[k];
-    __syncthreads();
-    // W1 (row j, column = key bit k), b1
-    for (uint32_t e = t; e < 4160u; e += GB) {
-        float acc = 0.f;
-        if (e < 4096u) {
-            const uint32_t j = e >> 6, k = e & 63u;
-            for (uint32_t s = 0; s < GB; ++s)
-                acc += ((sx[s] >> k) & 1ull) ? sd[s][j] : 0.f;
-            atomicAdd(g + OFF_W1 + e, acc);
-        } else {
-            const uint32_t j = e - 4096u;
-            for (uint32_t s = 0; s < GB; ++s)
-                acc += sd[s][j];
-            atomicAdd(g + OFF_B1 + j, acc);
-        }
+        for (uint32_t w = 0; w < GNW; ++w)
+            v += t < 192u ? red[w * 192u + t] : red2[2u * w + (t - 192u)];
+        row[t < 64u ? OFF_B1 + t : t < 128u ? OFF_B2 + t - 64u : t < 192u ? OFF_W3 + t - 128u : t == 192u ? OFF_B3 : NPAR] = v;
     }
 }
 
-// Adam on the master weights; refreshes the BF16 copies and clears the gradients
-__global__ void k_adam(float *__restrict__ p, uint16_t *__restrict__ pb, float *__restrict__ m,
-                       float *__restrict__ v, float *__restrict__ g, float lr, float b1, float b2, float eps,
-                       float c1, float c2)
+// The blocks' partial gradients summed (64 elements per block, 16 wavefronts a
+// share of the rows each), left in g with the loss after them; with `update`,
+// Adam on the master weights and their BF16 copies follows.  (Adding the
+// partials with atomics to one gradient took 40 of a step's 49 us.)
+#define SUM_WAVES 16u
+__global__ __launch_bounds__(64 * SUM_WAVES) void k_grad_sum(const float *__restrict__ part, uint32_t nrows,
+                                                             float *__restrict__ g, bool update,
+                                                             float *__restrict__ p, uint16_t *__restrict__ pb,
+                                                             float *__restrict__ m, float *__restrict__ v, float lr,
+                                                             float b1, float b2, float eps, float c1, float c2)
+{
+    __shared__ float s[SUM_WAVES][64];
+    const uint32_t lane = threadIdx.x & 63u, wv = threadIdx.x >> 6;
+    const uint32_t e = blockIdx.x * 64u + lane; // < PART_STRIDE
+    float x = 0.f;
+#pragma unroll 8
+    for (uint32_t r = wv; r < nrows; r += SUM_WAVES)
+        x += part[(size_t)r * PART_STRIDE + e];
+    s[wv][lane] = x;
+    __syncthreads();
+    if (wv != 0 || e > NPAR)
+        return;
+    float gr = 0.f;
+#pragma unroll
+    for (uint32_t w = 0; w < SUM_WAVES; ++w)
+        gr += s[w][lane];
+    g[e] = gr;
+    if (!update || e == NPAR)
+        return;
+    const float mm = b1 * m[e] + (1.f - b1) * gr;
+    const float vv = b2 * v[e] + (1.f - b2) * gr * gr;
+    m[e] = mm;
+    v[e] = vv;
+    const float pp = p[e] - lr * (mm / c1) / (sqrtf(vv / c2) + eps);
+    p[e] = pp;
+    pb[e] = f2bf(pp);
+}
+
+// new parameters: their BF16 copies, and moments that start over
+__global__ void k_set_params(const float *__restrict__ p, uint16_t *__restrict__ pb, float *__restrict__ m,
+                             float *__restrict__ v)
 {
     for (uint32_t e = blockIdx.x * blockDim.x + threadIdx.x; e < NPAR; e += gridDim.x * blockDim.x) {
-        const float gr = g[e];
-        g[e] = 0.f;
-        const float mm = b1 * m[e] + (1.f - b1) * gr;
-        const float vv = b2 * v[e] + (1.f - b2) * gr * gr;
-        m[e] = mm;
-        v[e] = vv;
-        const float pp = p[e] - lr * (mm / c1) / (sqrtf(vv / c2) + eps);
-        p[e] = pp;
-        pb[e] = f2bf(pp);
-    }
-}
-
-__global__ void k_to_bf16(const float *__restrict__ p, uint16_t *__restrict__ pb)
-{
-    for (uint32_t e = blockIdx.x * blockDim.x + threadIdx.x; e < NPAR; e += gridDim.x * blockDim.x)
+        m[e] = v[e] = 0.f;
         pb[e] = f2bf(p[e]);
-}
-
-__global__ void k_zero_f32(float *__restrict__ a, uint32_t n)
-{
-    for (uint32_t e = blockIdx.x * blockDim.x + threadIdx.x; e < n; e += gridDim.x * blockDim.x)
-        a[e] = 0.f;
+    }
 }
 
 // per-key VALU forward (the training forward)
@@ -845,8 +940,7 @@ extern "C" void qs_learned_destroy(qs_learned *L)
     hipFree(L->d_pb);
     hipFree(L->d_m);
     hipFree(L->d_v);
-    hipFree(L->d_g);
-    hipFree(L->d_loss);
+    hipFree(L->d_part); // and d_g and d_loss, its tail
     hipFree(L->d_tkeys);
     hipFree(L->d_tcnt);
     hipFree(L->d_err);
@@ -882,7 +976,7 @@ extern "C" int qs_learned_create(const qs_params *p, uint32_t table_log2, uint64
     L->thr = INFINITY;
     bool ok = hipMalloc(&L->d_p, NPAR * 4) == hipSuccess && hipMalloc(&L->d_pb, NPAR * 2) == hipSuccess &&
               hipMalloc(&L->d_m, NPAR * 4) == hipSuccess && hipMalloc(&L->d_v, NPAR * 4) == hipSuccess &&
-              hipMalloc(&L->d_g, NPAR * 4) == hipSuccess && hipMalloc(&L->d_loss, 4) == hipSuccess &&
+              hipMalloc(&L->d_part, 4ull * PART_STRIDE * (GRAD_BLOCKS + 1u)) == hipSuccess &&
               hipMalloc(&L->d_tkeys, L->tcap * 8) == hipSuccess && hipMalloc(&L->d_tcnt, L->tcap * 4) == hipSuccess &&
               hipMalloc(&L->d_err, 8) == hipSuccess &&
               hipHostMalloc(&L->h_pin, 16, hipHostMallocDefault) == hipSuccess;
@@ -890,6 +984,8 @@ extern "C" int qs_learned_create(const qs_params *p, uint32_t table_log2, uint64
         qs_learned_destroy(L);
         return QS_ERR_NOMEM;
     }
+    L->d_g = L->d_part + (size_t)PART_STRIDE * GRAD_BLOCKS;
+    L->d_loss = L->d_g + NPAR;
     // initial weights: uniform in +-1/sqrt(64) from a SplitMix64 stream, biases 0
     std::vector<float> h(NPAR, 0.f);
     uint64_t st = init_seed;
@@ -934,27 +1030,30 @@ extern "C" int qs_mlp_set_params(qs_learned *L, const float *hp)
         return QS_ERR_STATE; // the routing of the keys already in would change
     CK(hipDeviceSynchronize());
     CK(hipMemcpy(L->d_p, hp, NPAR * 4, hipMemcpyHostToDevice));
-    CK(hipMemset(L->d_m, 0, NPAR * 4));
-    CK(hipMemset(L->d_v, 0, NPAR * 4));
-    CK(hipMemset(L->d_g, 0, NPAR * 4));
-    hipLaunchKernelGGL(k_to_bf16, dim3(33), dim3(256), 0, 0, L->d_p, L->d_pb);
+    hipLaunchKernelGGL(k_set_params, dim3(33), dim3(256), 0, 0, L->d_p, L->d_pb, L->d_m, L->d_v);
     CK(hipGetLastError());
     CK(hipDeviceSynchronize());
     L->step = 0;
     return QS_OK;
 }
 
-static int grad_launch(qs_learned *L, const void *d_keys, const float *d_t, uint32_t n)
+// the gradient of a batch and its loss, to d_g and d_loss; with `update`, one
+// Adam step on them
+static int grad_launch(qs_learned *L, const void *d_keys, const float *d_t, uint32_t n, bool update, float lr,
+                       float beta1, float beta2, float eps, float c1, float c2)
 {
-    hipLaunchKernelGGL(k_zero_f32, dim3(1), dim3(64), 0, 0, L->d_loss, 1u);
-    const dim3 grid((n + GB - 1) / GB), block(GB);
+    const uint32_t groups = n / GK + (n % GK != 0);
+    const uint32_t rows = groups < GRAD_BLOCKS ? groups : GRAD_BLOCKS;
+    const dim3 grid(rows), block(GT);
     const float inv = 1.0f / (float)n;
     if (L->key_bytes == 4)
         hipLaunchKernelGGL(k_mlp_grad<4>, grid, block, 0, 0, (const uint32_t *)d_keys, d_t, n, L->d_pb, L->d_p, inv,
-                           L->d_g, L->d_loss);
+                           L->d_part);
     else
         hipLaunchKernelGGL(k_mlp_grad<8>, grid, block, 0, 0, (const uint64_t *)d_keys, d_t, n, L->d_pb, L->d_p, inv,
-                           L->d_g, L->d_loss);
+                           L->d_part);
+    hipLaunchKernelGGL(k_grad_sum, dim3(PART_STRIDE / 64u), dim3(64 * SUM_WAVES), 0, 0, L->d_part, rows, L->d_g, update,
+                       L->d_p, L->d_pb, L->d_m, L->d_v, lr, beta1, beta2, eps, c1, c2);
     CK(hipGetLastError());
     return QS_OK;
 }
@@ -964,7 +1063,7 @@ extern "C" int qs_mlp_grad(qs_learned *L, const void *d_keys, const float *d_t, 
 {
     if (!L || !d_keys || !d_t || n == 0)
         return QS_ERR_PARAM;
-    int rc = grad_launch(L, d_keys, d_t, n);
+    int rc = grad_launch(L, d_keys, d_t, n, false, 0.f, 0.f, 0.f, 0.f, 1.f, 1.f);
     if (rc)
         return rc;
     CK(hipDeviceSynchronize());
@@ -972,9 +1071,6 @@ extern "C" int qs_mlp_grad(qs_learned *L, const void *d_keys, const float *d_t, 
         CK(hipMemcpy(loss, L->d_loss, 4, hipMemcpyDeviceToHost));
     if (h_grad)
         CK(hipMemcpy(h_grad, L->d_g, NPAR * 4, hipMemcpyDeviceToHost));
-    hipLaunchKernelGGL(k_zero_f32, dim3(33), dim3(256), 0, 0, L->d_g, (uint32_t)NPAR);
-    CK(hipGetLastError());
-    CK(hipDeviceSynchronize());
     return QS_OK;
 }
 
@@ -985,21 +1081,17 @@ extern "C" int qs_mlp_step(qs_learned *L, const void *d_keys, const float *d_t, 
         return QS_ERR_PARAM;
     if (L->inserted)
         return QS_ERR_STATE; // the routing of the keys already in would change
-    int rc = grad_launch(L, d_keys, d_t, n);
-    if (rc)
-        return rc;
-    if (h_grad) {
-        CK(hipDeviceSynchronize());
-        CK(hipMemcpy(h_grad, L->d_g, NPAR * 4, hipMemcpyDeviceToHost));
-    }
     L->step++;
     const float c1 = 1.f - powf(beta1, (float)L->step), c2 = 1.f - powf(beta2, (float)L->step);
-    hipLaunchKernelGGL(k_adam, dim3(33), dim3(256), 0, 0, L->d_p, L->d_pb, L->d_m, L->d_v, L->d_g, lr, beta1, beta2,
-                       eps, c1, c2);
-    CK(hipGetLastError());
-    if (loss) {
+    int rc = grad_launch(L, d_keys, d_t, n, true, lr, beta1, beta2, eps, c1, c2);
+    if (rc)
+        return rc;
+    if (loss || h_grad)
+        CK(hipDeviceSynchronize());
+    if (h_grad)
+        CK(hipMemcpy(h_grad, L->d_g, NPAR * 4, hipMemcpyDeviceToHost));
+    if (loss)
         CK(hipMemcpy(loss, L->d_loss, 4, hipMemcpyDeviceToHost));
-    }
     return QS_OK;
 }
 
