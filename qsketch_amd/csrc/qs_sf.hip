@@ -78,6 +78,7 @@ struct qs_sf {
 
 struct sf_par {
     qs_fastdiv fd_n, fd_masks, fd_times;
+    qs_fastdiv64 fd_n64, fd_masks64, fd_times64;
     uint64_t n;
     uint32_t n_masks, m, times;
     uint32_t s32[3];
@@ -106,15 +107,15 @@ template <> struct sf_idx<8> {
     __device__ static inline void get(uint64_t key, const sf_par &p, uint32_t &b, uint32_t &mu, uint32_t t[3])
     {
         const uint64_t h0 = key * p.s64[0];
-        b = (uint32_t)(h0 % p.n);
-        mu = (uint32_t)(h0 % (uint64_t)p.n_masks);
-        t[0] = (uint32_t)(h0 % (uint64_t)p.times);
-        t[1] = (uint32_t)((key * p.s64[1]) % (uint64_t)p.times);
-        t[2] = (uint32_t)((key * p.s64[2]) % (uint64_t)p.times);
+        b = qs_fastmod64(h0, p.fd_n64);
+        mu = qs_fastmod64(h0, p.fd_masks64);
+        t[0] = qs_fastmod64(h0, p.fd_times64);
+        t[1] = qs_fastmod64(key * p.s64[1], p.fd_times64);
+        t[2] = qs_fastmod64(key * p.s64[2], p.fd_times64);
     }
     __device__ static inline uint32_t bucket(uint64_t key, const sf_par &p)
     {
-        return (uint32_t)((key * p.s64[0]) % p.n);
+        return qs_fastmod64(key * p.s64[0], p.fd_n64);
     }
 };
 
@@ -705,6 +706,9 @@ static sf_par sf_par_of(const qs_sf *s)
     p.fd_n = qs_fastdiv_make(s->key_bytes == 4 ? (uint32_t)s->n : 1u);
     p.fd_masks = qs_fastdiv_make(s->n_masks);
     p.fd_times = qs_fastdiv_make(s->times);
+    p.fd_n64 = qs_fastdiv64_make((uint32_t)s->n); // n fits 32 bits (qs_sf_create)
+    p.fd_masks64 = qs_fastdiv64_make(s->n_masks);
+    p.fd_times64 = qs_fastdiv64_make(s->times);
     p.n = s->n;
     p.n_masks = s->n_masks;
     p.m = s->m;

@@ -362,6 +362,8 @@ static void set_hash(qs_sdesc &d, uint32_t seed)
     d.seed = seed;
     d.fd_low = qs_fastdiv_make(d.n_low);
     d.fd_masks = qs_fastdiv_make(d.n_masks);
+    d.fd_low64 = qs_fastdiv64_make(d.n_low);
+    d.fd_masks64 = qs_fastdiv64_make(d.n_masks);
 }
 
 extern "C" void qs_destroy(qs_sketch *s)
