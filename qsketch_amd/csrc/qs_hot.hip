@@ -537,6 +537,19 @@ __global__ __launch_bounds__(64 * FLUSH_WAVES) void k_hot_flush(const uint32_t *
 // ===========================================================================
 // host
 // ===========================================================================
+uint64_t qs_scan_sums(uint64_t n)
+{
+    return (n + SCAN_SPAN - 1) / SCAN_SPAN + 1;
+}
+
+void qs_scan_u32(uint32_t *a, uint32_t n, uint32_t *bsum, hipStream_t stream)
+{
+    const uint32_t nb = (uint32_t)(((uint64_t)n + SCAN_SPAN - 1) / SCAN_SPAN); // <= 8192
+    hipLaunchKernelGGL(k_scan_reduce, dim3(nb), dim3(1024), 0, stream, a, n, bsum);
+    hipLaunchKernelGGL(k_scan_top, dim3(1), dim3(1024), 0, stream, bsum, nb);
+    hipLaunchKernelGGL(k_scan_apply, dim3(nb), dim3(1024), 0, stream, a, n, bsum, nb);
+}
+
 void qs_hot_state_free(void *state)
 {
     qs_hot *h = (qs_hot *)state;
@@ -794,10 +807,7 @@ int qs_insert_hot(qs_sketch *s, const void *d_keys, uint64_t n, hipStream_t stre
                        h->tkey, h->tinfo, h->tmask, h->tfill, h->ctl);
     hipLaunchKernelGGL(k_hot_count, dim3(h->nblk), dim3(HOT_THREADS), 0, stream, keys + HOT_PREFIX, rest,
                        nchunks, h->tkey, h->part, h->stage, h->ccold);
-    const uint32_t nb = (nchunks + SCAN_SPAN - 1) / SCAN_SPAN; // <= 8192 for any u32 chunk count of a call
-    hipLaunchKernelGGL(k_scan_reduce, dim3(nb), dim3(1024), 0, stream, h->ccold, nchunks, h->bsum);
-    hipLaunchKernelGGL(k_scan_top, dim3(1), dim3(1024), 0, stream, h->bsum, nb);
-    hipLaunchKernelGGL(k_scan_apply, dim3(nb), dim3(1024), 0, stream, h->ccold, nchunks, h->bsum, nb);
+    qs_scan_u32(h->ccold, nchunks, h->bsum, stream);
     hipLaunchKernelGGL(k_hot_move, dim3(h->nblk * 8u), dim3(256), 0, stream, h->stage, nchunks, h->ccold, h->cold);
     hipLaunchKernelGGL(k_hot_flush, dim3(HOT_SLOTS / 64), dim3(64 * FLUSH_WAVES), 0, stream, h->part, h->nblk, h->tkey,
                        h->tinfo, h->tmask, s->d_high);
@@ -856,10 +866,7 @@ int qs_hot_split_keys(void **state, const uint32_t *keys, uint64_t n, hipStream_
     hipLaunchKernelGGL(k_hot_build_any, dim3(HOT_MAX / 256), dim3(256), 0, stream, cand, h->tkey, h->tfill, h->ctl);
     hipLaunchKernelGGL(k_hot_count, dim3(h->nblk), dim3(HOT_THREADS), 0, stream, keys, n, nchunks, h->tkey, h->part,
                        h->stage, h->ccold);
-    const uint32_t nb = (nchunks + SCAN_SPAN - 1) / SCAN_SPAN;
-    hipLaunchKernelGGL(k_scan_reduce, dim3(nb), dim3(1024), 0, stream, h->ccold, nchunks, h->bsum);
-    hipLaunchKernelGGL(k_scan_top, dim3(1), dim3(1024), 0, stream, h->bsum, nb);
-    hipLaunchKernelGGL(k_scan_apply, dim3(nb), dim3(1024), 0, stream, h->ccold, nchunks, h->bsum, nb);
+    qs_scan_u32(h->ccold, nchunks, h->bsum, stream);
     hipLaunchKernelGGL(k_hot_move, dim3(h->nblk * 8u), dim3(256), 0, stream, h->stage, nchunks, h->ccold, h->cold);
     CK(hipGetLastError());
     rc = hot_read(h, h->ccold + nchunks, 1, stream);

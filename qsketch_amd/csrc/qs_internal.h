@@ -394,6 +394,11 @@ size_t qs_sort_hist_words(uint32_t max_count);
 void qs_scan_digits(uint32_t *hist, uint32_t ntiles, uint32_t nbins, uint32_t *totals,
                     hipStream_t stream);
 
+// Exclusive scan of a[0 .. n) in place with the total in a[n], over many blocks
+// (qs_hot.hip); bsum holds qs_scan_sums(n) words of scratch.  n <= 2^26.
+void qs_scan_u32(uint32_t *a, uint32_t n, uint32_t *bsum, hipStream_t stream);
+uint64_t qs_scan_sums(uint64_t n);
+
 // insert pipeline (qs_insert.hip).  offs: host array of nsk + 1 batch offsets
 // (sketch i owns keys[offs[i], offs[i+1])).  blocking: synchronise at the end
 // and report a pool error; otherwise the call never waits on the device.

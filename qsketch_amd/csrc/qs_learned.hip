@@ -14,10 +14,11 @@
 //               keys with v_mfma_f32_32x32x8_bf16, computing H^T = W X^T so that
 //               the accumulator layout of one layer is the B-operand layout of
 //               the next (no transpose between layers)
-//   k_route     k_mlp_mfma + routing: keys with score >= threshold are counted
-//               in a per-block LDS table and flushed to the exact GPU table with
-//               one atomic per distinct key and block; the others are flagged
-//               for a stable compaction into the sketch's input
+//   k_route     k_mlp_mfma + routing: keys with score >= threshold and the others
+//               are packed apart, chunk by chunk
+//   k_heavy_*   the heavy keys counted in LDS tables, whose entries are added to
+//               the exact GPU table; long calls group them by bin first
+//   k_light_move  the light keys put together, in stream order: the sketch's input
 //   k_reflag    after a routing pass the table could not hold: heavy keys
 //               without a slot go to the sketch instead
 //   k_table_query / k_learned_query  the query: the table count of a key
@@ -50,10 +51,15 @@
 #define T_NONE 0xffffffffu
 #define T_PROBES 4096u
 
-#define ROUTE_THREADS 256
-#define ROUTE_TILE 8192u // keys per routing block: 4 waves x 64 steps x 32 keys
-#define LT_SLOTS 4096u   // per-block LDS aggregation table
-#define LT_PROBES 32u
+#define ROUTE_THREADS 1024
+#define ROUTE_CHUNK 1024u // keys per chunk, a wavefront's unit of routing
+#define HBINS 256u        // bins of heavy keys
+#define LT_BUCKETS 1024u  // per-block LDS table of heavy keys: buckets of 4 slots (48 KB)
+// Calls of at least this many keys group their heavy keys by bin before they
+// are counted: one launch more, but fewer updates of the exact table (whole
+// windows of 2^20 keys 302 us straight, 356 grouped; of 2^25 keys 1.9 and 1.46 ms;
+// the lines meet near 2^21, where both take about 370 us).
+#define HEAVY_PART_MIN (1u << 21)
 
 struct qs_learned {
     qs_sketch *sk;
@@ -70,15 +76,19 @@ struct qs_learned {
     uint64_t tcap;
     uint64_t *d_tkeys;
     uint32_t *d_tcnt;
-    uint32_t *d_err;   // [0] set by k_route when the table turned a key away, [1] slots in use
+    uint32_t *d_bins;  // heavy keys per bin and the bins' write cursors (both of one call)
+    uint32_t *d_err;   // (after them) [0] set when the table turned a key away, [1] slots in use
     uint64_t inserted; // keys inserted since create / clear
     uint32_t full;     // the table has turned a key away since create / clear
     uint32_t used;     // table slots in use after the last insert
     // routing scratch
     uint64_t rcap;     // keys
     uint8_t *d_flag;   // 1 = goes to the sketch
-    uint32_t *d_tiles; // light keys per routing tile (+ scan totals)
-    void *d_light;
+    uint32_t *d_count; // light keys per chunk, scanned in place (+ total)
+    uint32_t *d_bsum;  // block sums of that scan (+ total)
+    void *d_stage;     // per chunk: its light keys, packed at the front
+    void *d_light;     // the light keys of the call, in stream order
+    uint32_t cus;      // routing blocks at most
     uint32_t *h_pin;   // pinned: light total, error flag, slots in use
 };
 
@@ -578,6 +588,13 @@ __device__ static inline float mlp_mfma(const mlp_lds &S, uint64_t x)
     return acc3[0] + S.b3;
 }
 
+// the key that lane src of the wavefront holds
+__device__ static inline uint64_t lane_key(uint64_t x, uint32_t src)
+{
+    return (uint64_t)(uint32_t)__shfl((int)(uint32_t)x, (int)src, 64) |
+           (uint64_t)(uint32_t)__shfl((int)(uint32_t)(x >> 32), (int)src, 64) << 32;
+}
+
 template <int KB>
 __global__ __launch_bounds__(256) void k_mlp_mfma(const KeyT<KB> *__restrict__ keys, uint64_t n,
                                                   const uint16_t *__restrict__ pb, const float *__restrict__ p,
@@ -613,8 +630,8 @@ __device__ static inline uint32_t t_home(uint64_t key, uint32_t tlog2)
     return (uint32_t)((key * 0x9E3779B97F4A7C15ull) >> (64u - tlog2));
 }
 
-// slot of key, claiming a free one if it is absent (*used counts claims)
-__device__ static inline uint32_t t_insert(uint64_t *tkeys, uint32_t tlog2, uint64_t key, uint32_t *used)
+// slot of key, claiming a free one if it is absent (claims counts them)
+__device__ static inline uint32_t t_insert(uint64_t *tkeys, uint32_t tlog2, uint64_t key, uint32_t &claims)
 {
     const uint32_t mask = (1u << tlog2) - 1u;
     uint32_t s = t_home(key, tlog2);
@@ -625,8 +642,7 @@ __device__ static inline uint32_t t_insert(uint64_t *tkeys, uint32_t tlog2, uint
         if (cur == T_EMPTY) {
             unsigned long long prev =
                 atomicCAS((unsigned long long *)(tkeys + s), (unsigned long long)T_EMPTY, (unsigned long long)key);
-            if (prev == T_EMPTY)
-                atomicAdd(used, 1u);
+            claims += prev == T_EMPTY ? 1u : 0u;
             if (prev == T_EMPTY || prev == key)
                 return s;
         }
@@ -648,151 +664,379 @@ __device__ static inline uint32_t t_find(const uint64_t *tkeys, uint32_t tlog2, 
     return T_NONE;
 }
 
-// err[0]: set when the table has no slot for key; err[1]: slots in use
+// err[0]: set when the table has no slot for key
 __device__ static inline void t_add(uint64_t *tkeys, uint32_t *tcnt, uint32_t tlog2, uint64_t key, uint32_t c,
-                                    uint32_t *err)
+                                    uint32_t *err, uint32_t &claims)
 {
-    const uint32_t s = t_insert(tkeys, tlog2, key, err + 1);
+    const uint32_t s = t_insert(tkeys, tlog2, key, claims);
     if (s == T_NONE)
         atomicOr(err, 1u);
     else
         atomicAdd(tcnt + s, c);
 }
 
-// Route one tile of ROUTE_TILE keys per block: score, count heavy keys in the
-// block's LDS table (flushed to the exact table at the end), flag the others.
-template <int KB>
-__global__ __launch_bounds__(ROUTE_THREADS) void k_route(const KeyT<KB> *__restrict__ keys, uint64_t n,
-                                                         const uint16_t *__restrict__ pb,
-                                                         const float *__restrict__ p, float thr,
-                                                         uint64_t *__restrict__ tkeys, uint32_t *__restrict__ tcnt,
-                                                         uint32_t tlog2, uint8_t *__restrict__ flag,
-                                                         uint32_t *__restrict__ tiles, uint32_t *__restrict__ err)
+// the bin of a heavy key
+__device__ static inline uint32_t heavy_bin(uint64_t x)
 {
-    __shared__ unsigned long long s_key[LT_SLOTS];
-    __shared__ uint32_t s_cnt[LT_SLOTS];
-    __shared__ uint32_t s_light;
-    for (uint32_t e = threadIdx.x; e < LT_SLOTS; e += ROUTE_THREADS) {
-        s_key[e] = T_EMPTY;
-        s_cnt[e] = 0;
-    }
-    if (threadIdx.x == 0)
-        s_light = 0;
-    __shared__ mlp_lds S;
-    load_mlp(S, pb, p);
-    const uint32_t lane = threadIdx.x & 63u, wv = threadIdx.x >> 6;
-    const uint64_t tb = (uint64_t)blockIdx.x * ROUTE_TILE;
-    uint32_t light = 0;
-    uint64_t xn = 0;
-    {
-        const uint64_t i0 = tb + (uint64_t)wv * 32u + (lane & 31u);
-        xn = key_at<KB>(keys, i0, n);
-    }
-    for (uint32_t st = 0; st < ROUTE_TILE / 128u; ++st) {
-        const uint64_t i = tb + (uint64_t)(st * 4u + wv) * 32u + (lane & 31u);
-        const bool valid = i < n;
-        const uint64_t x = xn;
-        // the next step's key is loaded while this one is scored
-        const uint64_t in = i + 128u;
-        xn = key_at<KB>(keys, in, n);
-        const float y = mlp_mfma(S, x);
-        if (lane >= 32u || !valid)
-            continue;
-        const bool heavy = y >= thr && x != T_EMPTY;
-        flag[i] = heavy ? 0 : 1;
-        if (!heavy) {
-            ++light;
-            continue;
-        }
-        uint32_t sl = (uint32_t)((x * 0x9E3779B97F4A7C15ull) >> 52) & (LT_SLOTS - 1u);
-        bool done = false;
-        for (uint32_t pr = 0; pr < LT_PROBES && !done; ++pr, sl = (sl + 1u) & (LT_SLOTS - 1u)) {
-            unsigned long long cur = s_key[sl];
-            if (cur == T_EMPTY)
-                cur = atomicCAS(&s_key[sl], (unsigned long long)T_EMPTY, (unsigned long long)x);
-            if (cur == T_EMPTY || cur == x) {
-                atomicAdd(&s_cnt[sl], 1u);
-                done = true;
-            }
-        }
-        if (!done)
-            t_add(tkeys, tcnt, tlog2, x, 1u, err);
-    }
-    atomicAdd(&s_light, light);
-    __syncthreads();
-    for (uint32_t e = threadIdx.x; e < LT_SLOTS; e += ROUTE_THREADS)
-        if (s_cnt[e])
-            t_add(tkeys, tcnt, tlog2, s_key[e], s_cnt[e], err);
-    if (threadIdx.x == 0)
-        tiles[blockIdx.x] = s_light;
+    return (uint32_t)((x * 0x9E3779B97F4A7C15ull) >> 56);
 }
 
-// stable compaction of the flagged keys of each routing tile
+// Routing.  A wavefront owns chunks of ROUTE_CHUNK consecutive keys and takes 64
+// at a time: two matrix-core tiles score them, then every lane places one key:
+// light keys, in stream order, at the front of the chunk's own slots of
+// `stage`, heavy ones at the back (from the end), the light ones' number in
+// `ccount` and the heavy ones' per bin in `bins`.  The heavy keys are counted by
+// the kernels below; k_light_move puts the light ones together after a scan.
+// The chunks of a short call go to different CUs.  Counting in this kernel held
+// every wavefront to its slowest lane's probes between two scorings: 1.24 ms for
+// 2^25 keys, now 0.60 and 0.23 for the counting; the forward alone takes 0.55.
 template <int KB>
-__global__ __launch_bounds__(ROUTE_THREADS) void k_light_scatter(const KeyT<KB> *__restrict__ keys, uint64_t n,
-                                                                 const uint8_t *__restrict__ flag,
-                                                                 const uint32_t *__restrict__ tile_off,
-                                                                 KeyT<KB> *__restrict__ out)
+__global__ __launch_bounds__(ROUTE_THREADS) void k_route(const KeyT<KB> *__restrict__ keys, uint64_t n,
+                                                         uint32_t nchunks, const uint16_t *__restrict__ pb,
+                                                         const float *__restrict__ p, float thr,
+                                                         uint8_t *__restrict__ flag, KeyT<KB> *__restrict__ stage,
+                                                         uint32_t *__restrict__ ccount, uint32_t *__restrict__ bins)
 {
-    __shared__ uint32_t s_w[ROUTE_THREADS / 64];
-    const uint32_t lane = threadIdx.x & 63u, wv = threadIdx.x >> 6;
-    const uint64_t tb = (uint64_t)blockIdx.x * ROUTE_TILE;
-    uint32_t base = tile_off[blockIdx.x];
-    for (uint32_t st = 0; st < ROUTE_TILE / ROUTE_THREADS; ++st) {
-        const uint64_t i = tb + (uint64_t)st * ROUTE_THREADS + threadIdx.x;
-        const bool f = i < n && flag[i];
-        const uint64_t m = __ballot(f);
-        if (lane == 0)
-            s_w[wv] = (uint32_t)__popcll(m);
-        __syncthreads();
-        uint32_t off = 0, tot = 0;
-#pragma unroll
-        for (uint32_t w = 0; w < ROUTE_THREADS / 64; ++w) {
-            off += w < wv ? s_w[w] : 0u;
-            tot += s_w[w];
+    __shared__ mlp_lds S;
+    __shared__ uint32_t s_bin[HBINS]; // heavy keys per bin
+    for (uint32_t e = threadIdx.x; e < HBINS; e += ROUTE_THREADS)
+        s_bin[e] = 0;
+    load_mlp(S, pb, p); // ends with a barrier
+    const uint32_t lane = threadIdx.x & 63u, l32 = lane & 31u;
+    const uint64_t below = (1ull << lane) - 1ull;
+    const uint32_t nw = gridDim.x * (ROUTE_THREADS / 64u);
+    uint32_t c = (threadIdx.x >> 6) * gridDim.x + blockIdx.x;
+    uint64_t xn = key_at<KB>(keys, (uint64_t)c * ROUTE_CHUNK + lane, n);
+    for (; c < nchunks; c += nw) {
+        const uint64_t base = (uint64_t)c * ROUTE_CHUNK;
+        uint32_t light = 0;
+        for (uint32_t st = 0; st < ROUTE_CHUNK / 64u; ++st) {
+            const uint64_t i = base + st * 64u + lane;
+            if (base + st * 64u >= n) // uniform
+                break;
+            const bool valid = i < n;
+            const uint64_t x = xn;
+            // the next keys are loaded while these are scored
+            xn = key_at<KB>(keys, st + 1u < ROUTE_CHUNK / 64u ? i + 64u : base + (uint64_t)nw * ROUTE_CHUNK + lane, n);
+            const float ya = mlp_mfma(S, lane_key(x, l32));
+            const float yb = mlp_mfma(S, lane_key(x, 32u + l32));
+            const float y2 = __shfl(yb, (int)l32, 64);
+            const float y = lane < 32u ? ya : y2;
+            const bool heavy = y >= thr && x != T_EMPTY;
+            const uint64_t m = __ballot(valid && !heavy); // the whole wavefront, outside any branch
+            const uint32_t before = light + (uint32_t)__popcll(m & below); // light keys before this one
+            if (valid) {
+                flag[i] = heavy ? 0 : 1;
+                stage[base + (heavy ? ROUTE_CHUNK - 1u - (st * 64u + lane - before) : before)] = (KeyT<KB>)x;
+                if (heavy)
+                    atomicAdd(&s_bin[heavy_bin(x)], 1u);
+            }
+            light += (uint32_t)__popcll(m);
         }
-        if (f)
-            out[base + off + (uint32_t)__popcll(m & ((1ull << lane) - 1ull))] = keys[i];
-        base += tot;
-        __syncthreads();
+        if (lane == 0)
+            ccount[c] = light;
+    }
+    __syncthreads();
+    for (uint32_t e = threadIdx.x; e < HBINS; e += ROUTE_THREADS)
+        if (s_bin[e])
+            atomicAdd(bins + e, s_bin[e]);
+}
+
+// The block's LDS table of heavy keys: LT_BUCKETS buckets of 4 slots, a key in
+// the one bucket its hash names (two 16-byte reads and no loop but for a lost
+// race); a key whose bucket is full goes to the exact table directly.
+struct heavy_lds {
+    ulonglong2 key2[LT_BUCKETS * 2u];
+    uint32_t cnt[LT_BUCKETS * 4u];
+};
+
+__device__ static inline void heavy_clear(heavy_lds &T)
+{
+    unsigned long long *key = reinterpret_cast<unsigned long long *>(T.key2);
+    for (uint32_t e = threadIdx.x; e < LT_BUCKETS * 4u; e += blockDim.x) {
+        key[e] = T_EMPTY;
+        T.cnt[e] = 0;
+    }
+    __syncthreads();
+}
+
+// one insert of x by every lane with `act` (the whole wavefront calls it)
+__device__ static inline void heavy_add(heavy_lds &T, bool act, unsigned long long x, uint64_t *tkeys, uint32_t *tcnt,
+                                        uint32_t tlog2, uint32_t *err, uint32_t &claims)
+{
+    // The lanes that hold the same key as the first lane, and then as the first
+    // of the others, are counted by one of them: a hot key would serialise
+    // its lanes on one LDS counter.
+    const uint32_t lane = threadIdx.x & 63u;
+    uint32_t w = act ? 1u : 0u;
+    uint64_t left = __ballot(act);
+#pragma unroll
+    for (int peel = 0; peel < 2; ++peel) {
+        if (left == 0)
+            break;
+        const uint32_t first = (uint32_t)__builtin_ctzll(left);
+        const uint64_t same = __ballot(w == 1u && x == lane_key(x, first)) & left;
+        left &= ~same;
+        if ((same >> lane) & 1ull)
+            w = lane == first ? (uint32_t)__popcll(same) : 0u;
+    }
+    if (w == 0)
+        return;
+    const uint32_t b = (uint32_t)((x * 0x9E3779B97F4A7C15ull) >> 32) & (LT_BUCKETS - 1u); // (not the bin's bits)
+    unsigned long long *key = reinterpret_cast<unsigned long long *>(T.key2) + 4u * b;
+    int sl = -1;
+    for (int tries = 0; tries < 4; ++tries) { // again only when another lane took the free slot
+        const ulonglong2 p = T.key2[2u * b], q = T.key2[2u * b + 1u];
+        const unsigned long long v[4] = {p.x, p.y, q.x, q.y};
+        int fr = -1;
+#pragma unroll
+        for (int e = 3; e >= 0; --e) {
+            sl = v[e] == x ? e : sl;
+            fr = v[e] == T_EMPTY ? e : fr;
+        }
+        if (sl >= 0 || fr < 0)
+            break;
+        const unsigned long long old = atomicCAS(key + fr, (unsigned long long)T_EMPTY, x);
+        if (old == T_EMPTY || old == x) {
+            sl = fr;
+            break;
+        }
+    }
+    if (sl >= 0)
+        atomicAdd(&T.cnt[4u * b + sl], w);
+    else
+        t_add(tkeys, tcnt, tlog2, x, w, err, claims);
+}
+
+// The table's entries to the exact table; the slots the block claimed there
+// (also while counting) are added to err[1] at once (an atomic per claim on
+// that one word serialised: 0.24 ms for 1.1e5 keys).
+__device__ static inline void heavy_flush(heavy_lds &T, uint64_t *tkeys, uint32_t *tcnt, uint32_t tlog2, uint32_t *err,
+                                          uint32_t claims)
+{
+    __syncthreads();
+    const unsigned long long *key = reinterpret_cast<const unsigned long long *>(T.key2);
+    for (uint32_t e = threadIdx.x; e < LT_BUCKETS * 4u; e += blockDim.x)
+        if (T.cnt[e])
+            t_add(tkeys, tcnt, tlog2, key[e], T.cnt[e], err, claims);
+    __syncthreads();
+    uint32_t *total = T.cnt; // free now
+    if (threadIdx.x == 0)
+        *total = 0;
+    __syncthreads();
+    if (claims)
+        atomicAdd(total, claims);
+    __syncthreads();
+    if (threadIdx.x == 0 && *total)
+        atomicAdd(err + 1, *total);
+}
+
+// the heavy keys of chunk c, rows of 64 (0 past their number, returned)
+template <int KB>
+__device__ static inline uint32_t load_heavy(const KeyT<KB> *__restrict__ stage, uint64_t n, uint32_t c,
+                                             uint32_t nchunks, const uint32_t *__restrict__ ccount,
+                                             KeyT<KB> k[ROUTE_CHUNK / 64u])
+{
+    const uint32_t lane = threadIdx.x & 63u;
+    uint32_t heavy = 0;
+    const uint64_t base = (uint64_t)c * ROUTE_CHUNK;
+    if (c < nchunks)
+        heavy = (n - base < ROUTE_CHUNK ? (uint32_t)(n - base) : ROUTE_CHUNK) - ccount[c];
+    const KeyT<KB> *src = stage + base + ROUTE_CHUNK - heavy;
+#pragma unroll
+    for (uint32_t r = 0; r < ROUTE_CHUNK / 64u; ++r)
+        k[r] = r * 64u + lane < heavy ? __builtin_nontemporal_load(src + r * 64u + lane) : (KeyT<KB>)0;
+    return heavy;
+}
+
+// Heavy keys counted straight from the chunks (short calls): every block meets
+// every key, so each key costs an update of the exact table per block.
+template <int KB>
+__global__ __launch_bounds__(256) void k_heavy_count(const KeyT<KB> *__restrict__ stage, uint64_t n, uint32_t nchunks,
+                                                     const uint32_t *__restrict__ ccount,
+                                                     uint64_t *__restrict__ tkeys, uint32_t *__restrict__ tcnt,
+                                                     uint32_t tlog2, uint32_t *__restrict__ err)
+{
+    __shared__ heavy_lds T;
+    heavy_clear(T);
+    uint32_t claims = 0;
+    const uint32_t lane = threadIdx.x & 63u;
+    const uint32_t nw = gridDim.x * 4u;
+    for (uint32_t c = blockIdx.x * 4u + (threadIdx.x >> 6); c < nchunks; c += nw) {
+        KeyT<KB> k[ROUTE_CHUNK / 64u];
+        const uint32_t heavy = load_heavy<KB>(stage, n, c, nchunks, ccount, k);
+#pragma unroll
+        for (uint32_t r = 0; r < ROUTE_CHUNK / 64u; ++r)
+            if (r * 64u < heavy) // uniform
+                heavy_add(T, r * 64u + lane < heavy, (unsigned long long)k[r], tkeys, tcnt, tlog2, err,
+                          claims);
+    }
+    heavy_flush(T, tkeys, tcnt, tlog2, err, claims);
+}
+
+// Long calls group the heavy keys by bin first (any order within a bin), so
+// that a key's inserts meet in the LDS tables of few blocks: updates of the exact
+// table (about 5 M of them, 0.89 ms at 2^25 keys, when every block counted
+// whatever came) then number little more than its keys.
+// A block takes 8 chunks, one per wavefront, ranks their heavy keys per bin in
+// LDS, reserves each bin's run with one atomic, and writes the runs in order.
+#define HP_WAVES 8u
+template <int KB>
+__global__ __launch_bounds__(64 * HP_WAVES) void k_heavy_part(const KeyT<KB> *__restrict__ stage, uint64_t n,
+                                                              uint32_t nchunks, const uint32_t *__restrict__ ccount,
+                                                              const uint32_t *__restrict__ bins,
+                                                              uint32_t *__restrict__ cursor,
+                                                              KeyT<KB> *__restrict__ out)
+{
+    __shared__ KeyT<KB> s_key[HP_WAVES * ROUTE_CHUNK];
+    __shared__ uint32_t s_cnt[HBINS], s_start[HBINS], s_goff[HBINS], s_red[2][4];
+    const uint32_t t = threadIdx.x, lane = t & 63u, wv = t >> 6;
+    if (t < HBINS)
+        s_cnt[t] = 0;
+    __syncthreads();
+    KeyT<KB> k[ROUTE_CHUNK / 64u];
+    uint32_t rank[ROUTE_CHUNK / 64u];
+    const uint32_t heavy = load_heavy<KB>(stage, n, blockIdx.x * HP_WAVES + wv, nchunks, ccount, k);
+#pragma unroll
+    for (uint32_t r = 0; r < ROUTE_CHUNK / 64u; ++r)
+        rank[r] = r * 64u + lane < heavy ? atomicAdd(&s_cnt[heavy_bin((uint64_t)k[r])], 1u) : 0u;
+    __syncthreads();
+    // exclusive scans over the bins: of the block's counts and of the totals
+    uint32_t x = 0, y = 0, cx = 0, cy = 0;
+    if (t < HBINS) {
+        x = cx = s_cnt[t];
+        y = cy = bins[t];
+#pragma unroll
+        for (int o = 1; o < 64; o <<= 1) {
+            const uint32_t u = (uint32_t)__shfl_up((int)x, o, 64), v = (uint32_t)__shfl_up((int)y, o, 64);
+            x += lane >= (uint32_t)o ? u : 0u;
+            y += lane >= (uint32_t)o ? v : 0u;
+        }
+        if (lane == 63u) {
+            s_red[0][wv] = x;
+            s_red[1][wv] = y;
+        }
+    }
+    __syncthreads();
+    if (t < HBINS) {
+        for (uint32_t w = 0; w < wv; ++w) {
+            x += s_red[0][w];
+            y += s_red[1][w];
+        }
+        const uint32_t at = cx ? atomicAdd(cursor + t, cx) : 0u;
+        s_start[t] = x - cx;
+        s_goff[t] = y - cy + at - (x - cx);
+    }
+    __syncthreads();
+#pragma unroll
+    for (uint32_t r = 0; r < ROUTE_CHUNK / 64u; ++r)
+        if (r * 64u + lane < heavy)
+            s_key[s_start[heavy_bin((uint64_t)k[r])] + rank[r]] = k[r];
+    __syncthreads();
+    const uint32_t total = s_start[HBINS - 1u] + s_cnt[HBINS - 1u];
+    for (uint32_t q = t; q < total; q += 64u * HP_WAVES) {
+        const KeyT<KB> v = s_key[q];
+        const uint32_t dst = s_goff[heavy_bin((uint64_t)v)] + q;
+        if (dst < n) // the counts and the ranks agree; checked, never trusted
+            out[dst] = v;
+    }
+}
+
+// counts windows of HS_WINDOW grouped heavy keys (few bins each) per block
+#define HS_THREADS 512u
+#define HS_WINDOW (HS_THREADS * 64u)
+template <int KB>
+__global__ __launch_bounds__(HS_THREADS) void k_heavy_sum(const KeyT<KB> *__restrict__ keys,
+                                                          const uint32_t *__restrict__ bins,
+                                                          uint64_t *__restrict__ tkeys, uint32_t *__restrict__ tcnt,
+                                                          uint32_t tlog2, uint32_t *__restrict__ err)
+{
+    __shared__ heavy_lds T;
+    __shared__ uint32_t s_n;
+    if (threadIdx.x == 0)
+        s_n = 0;
+    __syncthreads();
+    if (threadIdx.x < HBINS)
+        atomicAdd(&s_n, bins[threadIdx.x]);
+    __syncthreads();
+    const uint32_t n = s_n; // heavy keys
+    const uint64_t w0 = (uint64_t)blockIdx.x * HS_WINDOW;
+    if (w0 >= n)
+        return;
+    heavy_clear(T);
+    uint32_t claims = 0;
+    for (uint32_t g = 0; g < HS_WINDOW; g += HS_THREADS * 8u) {
+        KeyT<KB> k[8];
+#pragma unroll
+        for (uint32_t r = 0; r < 8u; ++r) { // every load first, from clamped positions
+            const uint64_t i = w0 + g + r * HS_THREADS + threadIdx.x;
+            k[r] = __builtin_nontemporal_load(keys + (i < n ? i : n - 1u));
+        }
+#pragma unroll
+        for (uint32_t r = 0; r < 8u; ++r)
+            heavy_add(T, w0 + g + r * HS_THREADS + threadIdx.x < n, (unsigned long long)k[r], tkeys, tcnt, tlog2, err,
+                          claims);
+    }
+    heavy_flush(T, tkeys, tcnt, tlog2, err, claims);
+}
+
+// every chunk moves its staged light keys to its scanned offset
+template <int KB>
+__global__ __launch_bounds__(256) void k_light_move(const KeyT<KB> *__restrict__ stage, uint32_t nchunks,
+                                                    const uint32_t *__restrict__ coff, KeyT<KB> *__restrict__ out)
+{
+    const uint32_t lane = threadIdx.x & 63u;
+    const uint32_t nw = gridDim.x * 4u;
+    for (uint32_t c = blockIdx.x * 4u + (threadIdx.x >> 6); c < nchunks; c += nw) {
+        const uint32_t off = coff[c], cnt = coff[c + 1] - off; // cnt <= ROUTE_CHUNK
+        const KeyT<KB> *src = stage + (size_t)c * ROUTE_CHUNK;
+        KeyT<KB> v[ROUTE_CHUNK / 64u];
+#pragma unroll
+        for (uint32_t r = 0; r < ROUTE_CHUNK / 64u; ++r)
+            v[r] = r * 64u + lane < cnt ? __builtin_nontemporal_load(src + r * 64u + lane) : (KeyT<KB>)0;
+#pragma unroll
+        for (uint32_t r = 0; r < ROUTE_CHUNK / 64u; ++r)
+            if (r * 64u + lane < cnt)
+                out[(size_t)off + r * 64u + lane] = v[r];
     }
 }
 
 // After a routing pass in which the table turned keys away (*err set): every
 // key flagged heavy that is not in the table goes to the sketch instead, and
-// the tile's light count is redone.  A key is either in the table for all of
+// the chunks are staged again.  A key is either in the table for all of
 // its occurrences or for none: slots only fill, so a key's probe window that
 // had no room for it never gains room, and once the key holds a slot every
 // later probe finds it.  Blocks exit at once when *err is clear.
 template <int KB>
-__global__ __launch_bounds__(ROUTE_THREADS) void k_reflag(const KeyT<KB> *__restrict__ keys, uint64_t n,
-                                                          const uint64_t *__restrict__ tkeys, uint32_t tlog2,
-                                                          uint8_t *__restrict__ flag, uint32_t *__restrict__ tiles,
-                                                          const uint32_t *__restrict__ err)
+__global__ __launch_bounds__(256) void k_reflag(const KeyT<KB> *__restrict__ keys, uint64_t n, uint32_t nchunks,
+                                                const uint64_t *__restrict__ tkeys, uint32_t tlog2,
+                                                const uint8_t *__restrict__ flag, KeyT<KB> *__restrict__ stage,
+                                                uint32_t *__restrict__ ccount, const uint32_t *__restrict__ err)
 {
     if (*err == 0)
         return;
-    __shared__ uint32_t s_light;
-    if (threadIdx.x == 0)
-        s_light = 0;
-    __syncthreads();
-    const uint64_t tb = (uint64_t)blockIdx.x * ROUTE_TILE;
-    uint32_t light = 0;
-    for (uint32_t st = 0; st < ROUTE_TILE / ROUTE_THREADS; ++st) {
-        const uint64_t i = tb + (uint64_t)st * ROUTE_THREADS + threadIdx.x;
-        if (i >= n)
-            break;
-        uint8_t f = flag[i];
-        if (!f && t_find(tkeys, tlog2, key64<KB>(keys, i)) == T_NONE) {
-            f = 1;
-            flag[i] = 1;
+    const uint32_t lane = threadIdx.x & 63u;
+    const uint64_t below = (1ull << lane) - 1ull;
+    const uint32_t nw = gridDim.x * 4u;
+    for (uint32_t c = blockIdx.x * 4u + (threadIdx.x >> 6); c < nchunks; c += nw) {
+        const uint64_t base = (uint64_t)c * ROUTE_CHUNK;
+        uint32_t light = 0;
+        for (uint32_t st = 0; st < ROUTE_CHUNK / 64u; ++st) {
+            const uint64_t i = base + st * 64u + lane;
+            bool f = false;
+            KeyT<KB> x = 0;
+            if (i < n) {
+                x = keys[i];
+                f = flag[i] || t_find(tkeys, tlog2, (uint64_t)x) == T_NONE;
+            }
+            const uint64_t m = __ballot(f);
+            if (f)
+                stage[base + light + (uint32_t)__popcll(m & below)] = x;
+            light += (uint32_t)__popcll(m);
         }
-        light += f;
+        if (lane == 0)
+            ccount[c] = light;
     }
-    atomicAdd(&s_light, light);
-    __syncthreads();
-    if (threadIdx.x == 0)
-        tiles[blockIdx.x] = s_light;
 }
 
 // Queries of the learned form.  A key is counted entirely in one part: only
@@ -943,9 +1187,11 @@ extern "C" void qs_learned_destroy(qs_learned *L)
     hipFree(L->d_part); // and d_g and d_loss, its tail
     hipFree(L->d_tkeys);
     hipFree(L->d_tcnt);
-    hipFree(L->d_err);
+    hipFree(L->d_bins); // and d_err, its tail
     hipFree(L->d_flag);
-    hipFree(L->d_tiles);
+    hipFree(L->d_count);
+    hipFree(L->d_bsum);
+    hipFree(L->d_stage);
     hipFree(L->d_light);
     if (L->h_pin)
         hipHostFree(L->h_pin);
@@ -978,12 +1224,13 @@ extern "C" int qs_learned_create(const qs_params *p, uint32_t table_log2, uint64
               hipMalloc(&L->d_m, NPAR * 4) == hipSuccess && hipMalloc(&L->d_v, NPAR * 4) == hipSuccess &&
               hipMalloc(&L->d_part, 4ull * PART_STRIDE * (GRAD_BLOCKS + 1u)) == hipSuccess &&
               hipMalloc(&L->d_tkeys, L->tcap * 8) == hipSuccess && hipMalloc(&L->d_tcnt, L->tcap * 4) == hipSuccess &&
-              hipMalloc(&L->d_err, 8) == hipSuccess &&
+              hipMalloc(&L->d_bins, 4ull * (2u * HBINS + 2u)) == hipSuccess &&
               hipHostMalloc(&L->h_pin, 16, hipHostMallocDefault) == hipSuccess;
     if (!ok) {
         qs_learned_destroy(L);
         return QS_ERR_NOMEM;
     }
+    L->d_err = L->d_bins + 2u * HBINS;
     L->d_g = L->d_part + (size_t)PART_STRIDE * GRAD_BLOCKS;
     L->d_loss = L->d_g + NPAR;
     // initial weights: uniform in +-1/sqrt(64) from a SplitMix64 stream, biases 0
@@ -1158,17 +1405,29 @@ extern "C" int qs_learned_clear(qs_learned *L)
 
 static int ensure_route(qs_learned *L, uint64_t n)
 {
+    if (!L->cus) {
+        int cu = 0;
+        if (hipDeviceGetAttribute(&cu, hipDeviceAttributeMultiprocessorCount, L->sk->device) != hipSuccess || cu <= 0)
+            cu = 256;
+        L->cus = (uint32_t)cu;
+    }
     if (L->rcap >= n)
         return QS_OK;
     hipFree(L->d_flag);
-    hipFree(L->d_tiles);
+    hipFree(L->d_count);
+    hipFree(L->d_bsum);
+    hipFree(L->d_stage);
     hipFree(L->d_light);
     L->d_flag = nullptr;
-    L->d_tiles = nullptr;
+    L->d_count = nullptr;
+    L->d_bsum = nullptr;
+    L->d_stage = nullptr;
     L->d_light = nullptr;
     L->rcap = 0;
-    const uint64_t tiles = (n + ROUTE_TILE - 1) / ROUTE_TILE;
-    if (hipMalloc(&L->d_flag, n) != hipSuccess || hipMalloc(&L->d_tiles, (tiles + 1) * 4) != hipSuccess ||
+    const uint64_t chunks = (n + ROUTE_CHUNK - 1) / ROUTE_CHUNK;
+    if (hipMalloc(&L->d_flag, n) != hipSuccess || hipMalloc(&L->d_count, (chunks + 1) * 4) != hipSuccess ||
+        hipMalloc(&L->d_bsum, 4ull * qs_scan_sums(chunks)) != hipSuccess ||
+        hipMalloc(&L->d_stage, chunks * ROUTE_CHUNK * L->key_bytes) != hipSuccess ||
         hipMalloc(&L->d_light, n * L->key_bytes) != hipSuccess)
         return QS_ERR_NOMEM;
     L->rcap = n;
@@ -1181,18 +1440,33 @@ static int learned_insert(qs_learned *L, const KeyT<KB> *keys, uint64_t n, uint6
     int rc = ensure_route(L, n);
     if (rc)
         return rc;
-    const uint32_t tiles = (uint32_t)((n + ROUTE_TILE - 1) / ROUTE_TILE);
-    CK(hipMemsetAsync(L->d_err, 0, 4, 0)); // this call's flag
-    hipLaunchKernelGGL(k_route<KB>, dim3(tiles), dim3(ROUTE_THREADS), 0, 0, keys, n, L->d_pb, L->d_p, L->thr,
-                       L->d_tkeys, L->d_tcnt, L->tlog2, L->d_flag, L->d_tiles, L->d_err);
+    const uint32_t chunks = (uint32_t)((n + ROUTE_CHUNK - 1) / ROUTE_CHUNK); // n < 2^32
+    KeyT<KB> *stage = (KeyT<KB> *)L->d_stage;
+    CK(hipMemsetAsync(L->d_bins, 0, 4u * (2u * HBINS + 1u), 0)); // bins, cursors and this call's flag
+    hipLaunchKernelGGL(k_route<KB>, dim3(chunks < L->cus ? chunks : L->cus), dim3(ROUTE_THREADS), 0, 0, keys, n, chunks,
+                       L->d_pb, L->d_p, L->thr, L->d_flag, stage, L->d_count, L->d_bins);
+    if (n < HEAVY_PART_MIN) {
+        hipLaunchKernelGGL(k_heavy_count<KB>, dim3(lgrid((chunks + 3u) / 4u, 2u * L->cus)), dim3(256), 0, 0, stage, n,
+                           chunks, L->d_count, L->d_tkeys, L->d_tcnt, L->tlog2, L->d_err);
+    } else {
+        // (grouped in the buffer that takes the light keys afterwards)
+        KeyT<KB> *grouped = (KeyT<KB> *)L->d_light;
+        hipLaunchKernelGGL(k_heavy_part<KB>, dim3((chunks + HP_WAVES - 1u) / HP_WAVES), dim3(64 * HP_WAVES), 0, 0,
+                           stage, n, chunks, L->d_count, L->d_bins, L->d_bins + HBINS, grouped);
+        hipLaunchKernelGGL(k_heavy_sum<KB>, dim3((uint32_t)((n + HS_WINDOW - 1) / HS_WINDOW)), dim3(HS_THREADS), 0, 0,
+                           grouped, L->d_bins, L->d_tkeys, L->d_tcnt, L->tlog2, L->d_err);
+    }
+    const dim3 wgrid(lgrid((chunks + 3u) / 4u, 8u * L->cus)); // a wavefront per chunk
     // keys the table turned away go to the sketch (no work unless it did)
-    hipLaunchKernelGGL(k_reflag<KB>, dim3(tiles), dim3(ROUTE_THREADS), 0, 0, keys, n, L->d_tkeys, L->tlog2,
-                       L->d_flag, L->d_tiles, L->d_err);
-    qs_scan_digits(L->d_tiles, tiles, 1, L->d_tiles + tiles, 0);
-    hipLaunchKernelGGL(k_light_scatter<KB>, dim3(tiles), dim3(ROUTE_THREADS), 0, 0, keys, n, L->d_flag, L->d_tiles,
-                       (KeyT<KB> *)L->d_light);
+    hipLaunchKernelGGL(k_reflag<KB>, wgrid, dim3(256), 0, 0, keys, n, chunks, L->d_tkeys, L->tlog2, L->d_flag, stage,
+                       L->d_count, L->d_err);
+    if (chunks <= 16384u) // one launch while one block is quick enough
+        qs_scan_digits(L->d_count, chunks, 1, L->d_count + chunks, 0);
+    else
+        qs_scan_u32(L->d_count, chunks, L->d_bsum, 0);
+    hipLaunchKernelGGL(k_light_move<KB>, wgrid, dim3(256), 0, 0, stage, chunks, L->d_count, (KeyT<KB> *)L->d_light);
     CK(hipGetLastError());
-    CK(hipMemcpy(L->h_pin, L->d_tiles + tiles, 4, hipMemcpyDeviceToHost));
+    CK(hipMemcpy(L->h_pin, L->d_count + chunks, 4, hipMemcpyDeviceToHost));
     CK(hipMemcpy(L->h_pin + 1, L->d_err, 8, hipMemcpyDeviceToHost));
     const uint64_t n_light = L->h_pin[0];
     if (L->h_pin[1])
