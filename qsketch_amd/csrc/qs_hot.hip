@@ -6,8 +6,7 @@
 // inserts into unlinked buckets depend on their order (the promotion point,
 // v3:160-190).  So a long insert call runs as:
 //   1. the candidates: the keys occurring at least HOT_MIN_RUN times among the
-//      first HOT_SAMPLE keys (a sort of that sample, then its runs), ordered
-//      by count (ties by key) and capped at HOT_MAX; on a second stream, at
+//      first HOT_SAMPLE keys, the HOT_MAX most frequent of them; on a second stream, at
 //      the same time as
 //   2. the first HOT_PREFIX keys through the ordinary pipeline (qs_insert.hip),
 //      which links the buckets of the hot keys;
@@ -45,6 +44,7 @@
 #define HOT_SAMPLE (1u << 20)              // candidates come from the first HOT_SAMPLE keys
 #define HOT_MIN_RUN 8u                     // a candidate occurs at least this often there
 #define HOT_CAND_MAX (HOT_SAMPLE / HOT_MIN_RUN)
+static_assert(HOT_CAND_MAX % 1024u == 0, "blocks of k_samp_select");
 #define HOT_MAX 8192u                      // hot keys at most
 #define HOT_BUCKETS 4096u                  // buckets of 4 slots (load at most 1/2)
 #define HOT_SLOTS (HOT_BUCKETS * 4u)
@@ -58,17 +58,19 @@
 #define HOT_MIN_COVER_DEN 10u              //   3/10 of the sample
 
 // device control words
-#define HC_NCAND 0   // candidates found
-#define HC_COVER 1   // sample keys the first HOT_MAX candidates cover
+#define HC_NCAND 0   // candidates (at most HOT_MAX)
+#define HC_COVER 1   // sample keys they cover
 #define HC_NHOT 2    // keys in the hot table
-#define HC_WORDS 4
+#define HC_FOUND 3   // keys of the sample that occur often enough
+#define HC_TIES 4    // of those, the ones with the least count taken that were looked at
+#define HC_WORDS 5
 
 struct qs_hot {
-    uint32_t *sk[2], *sv[2];   // sample sort (keys, unused values)
-    uint32_t *ck[2], *cv[2];   // candidate sorts
-    uint32_t *hist;            // radix histograms of both sorts
-    uint32_t *cflag;           // candidate flags of the sorted sample, scanned in place (+ total)
-    uint32_t *cbsum;           // block sums of that scan (+ total)
+    uint32_t *samp;            // the sample grouped by bin
+    uint32_t *scnt;            // its keys per tile and bin, then the bins' starts
+    uint32_t *ccount;          // histogram of the counts of its frequent keys
+    uint32_t *ck, *cv;         // those keys and their counts
+    uint32_t *cand;            // the candidates
     uint32_t *ctl;             // HC_* words
     uint32_t *h_ctl;           // pinned copy
     uint32_t *tkey;            // hot table: key per slot
@@ -84,7 +86,6 @@ struct qs_hot {
     uint32_t *cold;            // the cold keys of the call, in stream order
     uint64_t cold_cap;
     uint32_t seq;              // sequence number of the last publication to h_ctl
-    const uint32_t *cand;      // the candidates, most frequent first (set by hot_cand_launch)
     hipStream_t side;          // the candidate phase of a plain insert runs here (default priority)
     hipEvent_t ev_fork;        // the caller's stream up to the call
     hipEvent_t ev_cand;        // the candidate phase done
@@ -135,101 +136,263 @@ __device__ static inline void hot_buckets(uint32_t key, uint32_t &b1, uint32_t &
     b2 = b2 == b1 ? b1 ^ 1u : b2;
 }
 
-__global__ void k_hot_sample(const uint32_t *__restrict__ keys, uint32_t n, uint32_t *__restrict__ sk,
-                             uint32_t *__restrict__ sv, uint32_t *__restrict__ ctl)
+// ---------------------------------------------------------------------------
+// Candidates: the sample's keys are split by hash into SAMP_BINS bins, one block
+// counts each bin's keys in an LDS table, and the HOT_MAX most frequent of
+// those that occur at least HOT_MIN_RUN times are selected by a histogram
+// of the counts.  Which keys become candidates moves time only, never the
+// result, so a key that finds the LDS table crowded is simply left out.
+// (The sample was sorted before, and the candidates sorted again by count:
+// 29 launches, about 270 us with their gaps; these four kernels take 72 us at
+// Zipf 1.1, 48 of them the block whose bin holds the hottest key.)
+// ---------------------------------------------------------------------------
+#define SAMP_TILE 8192u // sample keys per block of the split
+#define SAMP_TILES (HOT_SAMPLE / SAMP_TILE)
+#define SAMP_IPT (SAMP_TILE / 1024u)
+#define SAMP_BINS 256u
+#define SAMP_SLOTS 8192u   // LDS table of one bin (about 4096 keys)
+#define SAMP_PROBES 32u
+#define SAMP_ROWS 8u
+#define SAMP_COUNTS 4096u  // histogram of candidate counts (the last one holds all above)
+
+__device__ static inline uint32_t samp_hash(uint32_t k)
 {
-    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n) {
-        sk[i] = keys[i];
-        sv[i] = 0;
+    return k * 0x9E3779B1u;
+}
+__device__ static inline uint32_t samp_bin(uint32_t k)
+{
+    return samp_hash(k) >> 24;
+}
+
+// keys per bin of each tile; also clears the control words and the histogram
+__global__ __launch_bounds__(1024) void k_samp_hist(const uint32_t *__restrict__ keys, uint32_t *__restrict__ cnt,
+                                                    uint32_t *__restrict__ ccount, uint32_t *__restrict__ ctl)
+{
+    __shared__ uint32_t s_cnt[SAMP_BINS];
+    const uint32_t t = threadIdx.x, i0 = blockIdx.x * SAMP_TILE + t;
+    if (t < SAMP_BINS)
+        s_cnt[t] = 0;
+    if (blockIdx.x < SAMP_COUNTS / 1024u)
+        ccount[blockIdx.x * 1024u + t] = 0;
+    if (blockIdx.x == 0 && t < HC_WORDS)
+        ctl[t] = 0;
+    uint32_t k[SAMP_IPT];
+#pragma unroll
+    for (uint32_t r = 0; r < SAMP_IPT; ++r)
+        k[r] = keys[i0 + r * 1024u];
+    __syncthreads();
+#pragma unroll
+    for (uint32_t r = 0; r < SAMP_IPT; ++r)
+        atomicAdd(&s_cnt[samp_bin(k[r])], 1u);
+    __syncthreads();
+    if (t < SAMP_BINS)
+        cnt[blockIdx.x * SAMP_BINS + t] = s_cnt[t];
+}
+
+// the keys grouped by bin (any order within one); bin b is
+// out[start[b] .. start[b + 1])
+__global__ __launch_bounds__(1024) void k_samp_split(const uint32_t *__restrict__ keys,
+                                                     const uint32_t *__restrict__ cnt, uint32_t *__restrict__ out,
+                                                     uint32_t *__restrict__ start)
+{
+    __shared__ uint32_t s_pre[4][SAMP_BINS], s_tot[4][SAMP_BINS], s_pos[SAMP_BINS], s_red[4];
+    const uint32_t t = threadIdx.x, b = t & (SAMP_BINS - 1u), part = t / SAMP_BINS;
+    const uint32_t i0 = blockIdx.x * SAMP_TILE + t;
+    uint32_t k[SAMP_IPT];
+#pragma unroll
+    for (uint32_t r = 0; r < SAMP_IPT; ++r)
+        k[r] = keys[i0 + r * 1024u];
+    uint32_t pre = 0, tot = 0;
+#pragma unroll 8
+    for (uint32_t u = 0; u < SAMP_TILES / 4u; ++u) {
+        const uint32_t tile = part * (SAMP_TILES / 4u) + u, v = cnt[tile * SAMP_BINS + b];
+        tot += v;
+        pre += tile < blockIdx.x ? v : 0u;
     }
-    if (i < HC_WORDS)
-        ctl[i] = 0;
-}
-
-// The first index of the run that ends at i in the sorted sample a (the run
-// is at least HOT_MIN_RUN long): gallop back from the run end, then bisect;
-// the loads stay near i.
-__device__ static inline uint32_t run_start(const uint32_t *__restrict__ a, uint32_t i)
-{
-    const uint32_t k = a[i];
-    uint32_t hi = i + 1u - HOT_MIN_RUN, lo = hi, step = HOT_MIN_RUN;
-    while (lo > 0) { // a[lo] < k or lo = 0 ends the gallop
-        lo = lo > step ? lo - step : 0u;
-        if (a[lo] < k)
-            break;
-        hi = lo;
-        step <<= 1;
+    s_pre[part][b] = pre;
+    s_tot[part][b] = tot;
+    __syncthreads();
+    uint32_t x = 0;
+    if (t < SAMP_BINS) {
+        tot = s_tot[0][t] + s_tot[1][t] + s_tot[2][t] + s_tot[3][t];
+        pre = s_pre[0][t] + s_pre[1][t] + s_pre[2][t] + s_pre[3][t];
+        x = tot;
+#pragma unroll
+        for (int o = 1; o < 64; o <<= 1) {
+            const uint32_t y = (uint32_t)__shfl_up((int)x, o, 64);
+            x += (t & 63u) >= (uint32_t)o ? y : 0u;
+        }
+        if ((t & 63u) == 63u)
+            s_red[t >> 6] = x;
     }
-    if (a[lo] == k) // lo = 0 holds k: the run starts at 0
-        hi = lo;
-    while (lo + 1u < hi) { // a[lo] < k <= a[hi]
-        const uint32_t mid = (lo + hi) >> 1;
-        if (a[mid] < k)
-            lo = mid;
-        else
-            hi = mid;
+    __syncthreads();
+    if (t < SAMP_BINS) {
+        for (uint32_t w = 0; w < t >> 6; ++w)
+            x += s_red[w];
+        s_pos[t] = x - tot + pre;
+        if (blockIdx.x == 0) {
+            start[t] = x - tot;
+            if (t == SAMP_BINS - 1u)
+                start[SAMP_BINS] = x;
+        }
     }
-    return hi;
+    __syncthreads();
+#pragma unroll
+    for (uint32_t r = 0; r < SAMP_IPT; ++r)
+        out[atomicAdd(&s_pos[samp_bin(k[r])], 1u)] = k[r];
 }
 
-// whether i ends a run of the sorted sample that is at least HOT_MIN_RUN long
-__device__ static inline bool cand_end(const uint32_t *__restrict__ a, uint32_t n, uint32_t i)
+// counts one bin's keys; those with HOT_MIN_RUN or more are appended to (ck, cv),
+// their counts to the histogram
+__global__ __launch_bounds__(1024) void k_samp_count(const uint32_t *__restrict__ bins,
+                                                     const uint32_t *__restrict__ start, uint32_t *__restrict__ ck,
+                                                     uint32_t *__restrict__ cv, uint32_t *__restrict__ ccount,
+                                                     uint32_t *__restrict__ ctl)
 {
-    const uint32_t k = a[i];
-    return !(i + 1 < n && a[i + 1] == k) && i + 1 >= HOT_MIN_RUN && a[i + 1 - HOT_MIN_RUN] == k;
+    __shared__ uint32_t s_key[SAMP_SLOTS], s_cnt[SAMP_SLOTS], s_h[SAMP_COUNTS];
+    __shared__ uint32_t s_n, s_base;
+    const uint32_t t = threadIdx.x, lane = t & 63u;
+    for (uint32_t e = t; e < SAMP_SLOTS; e += 1024u) {
+        s_key[e] = HOT_EMPTY;
+        s_cnt[e] = 0;
+    }
+    for (uint32_t e = t; e < SAMP_COUNTS; e += 1024u)
+        s_h[e] = 0;
+    if (t == 0)
+        s_n = 0;
+    __syncthreads();
+    const uint32_t b0 = start[blockIdx.x], b1 = start[blockIdx.x + 1];
+    // (a hot key's bin can hold most of the sample: the loads of SAMP_ROWS rows
+    // are in flight together)
+    for (uint32_t i0 = b0; i0 < b1; i0 += 1024u * SAMP_ROWS) {
+        uint32_t kk[SAMP_ROWS];
+#pragma unroll
+        for (uint32_t r = 0; r < SAMP_ROWS; ++r) {
+            const uint32_t i = i0 + r * 1024u + t;
+            kk[r] = bins[i < b1 ? i : b1 - 1u];
+        }
+#pragma unroll
+        for (uint32_t r = 0; r < SAMP_ROWS; ++r) {
+            const uint32_t i = i0 + r * 1024u + t, k = kk[r];
+            // the lanes with the first lane's key, then those with the first key
+            // of the rest, are added by one lane each
+            uint32_t w = i < b1 && k != HOT_EMPTY ? 1u : 0u; // (the empty marker is never hot)
+            uint64_t left = __ballot(w != 0u);
+#pragma unroll
+            for (int peel = 0; peel < 2; ++peel) {
+                if (left == 0)
+                    break;
+                const uint32_t first = (uint32_t)__builtin_ctzll(left);
+                const uint32_t fk = (uint32_t)__shfl((int)k, (int)first, 64);
+                const uint64_t same = __ballot(k == fk) & left;
+                left &= ~same;
+                if ((same >> lane) & 1ull)
+                    w = lane == first ? (uint32_t)__popcll(same) : 0u;
+            }
+            if (!w)
+                continue;
+            uint32_t sl = (samp_hash(k) >> 11) & (SAMP_SLOTS - 1u);
+            for (uint32_t pr = 0; pr < SAMP_PROBES; ++pr, sl = (sl + 1u) & (SAMP_SLOTS - 1u)) {
+                uint32_t cur = s_key[sl];
+                if (cur == HOT_EMPTY)
+                    cur = atomicCAS(&s_key[sl], HOT_EMPTY, k);
+                if (cur == HOT_EMPTY || cur == k) {
+                    atomicAdd(&s_cnt[sl], w);
+                    break;
+                }
+            }
+        }
+    }
+    __syncthreads();
+    uint32_t mine = 0;
+    for (uint32_t e = t; e < SAMP_SLOTS; e += 1024u)
+        if (s_cnt[e] >= HOT_MIN_RUN) {
+            ++mine;
+            atomicAdd(&s_h[min(s_cnt[e], SAMP_COUNTS - 1u)], 1u);
+        }
+    uint32_t at = mine ? atomicAdd(&s_n, mine) : 0u;
+    __syncthreads();
+    if (t == 0)
+        s_base = s_n ? atomicAdd(ctl + HC_FOUND, s_n) : 0u;
+    __syncthreads();
+    at += s_base;
+    for (uint32_t e = t; e < SAMP_SLOTS; e += 1024u)
+        if (s_cnt[e] >= HOT_MIN_RUN) { // (at most HOT_SAMPLE / HOT_MIN_RUN in all bins)
+            ck[at] = s_key[e];
+            cv[at] = s_cnt[e];
+            ++at;
+        }
+    for (uint32_t e = t; e < SAMP_COUNTS; e += 1024u)
+        if (s_h[e])
+            atomicAdd(ccount + e, s_h[e]);
 }
 
-// flag[i] = 1 when i ends a candidate run (scanned next into offsets)
-__global__ void k_hot_cand_flag(const uint32_t *__restrict__ a, uint32_t n, uint32_t *__restrict__ flag)
+// The HOT_MAX most frequent candidates (of those with the least count among
+// them, as many as there is room for) to cand, their number and the sample keys
+// they cover to the control words.
+__global__ __launch_bounds__(1024) void k_samp_select(const uint32_t *__restrict__ ck, const uint32_t *__restrict__ cv,
+                                                      const uint32_t *__restrict__ ccount, uint32_t *__restrict__ cand,
+                                                      uint32_t *__restrict__ ctl)
 {
-    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n)
-        flag[i] = cand_end(a, n, i) ? 1u : 0u;
-}
-
-// Each candidate run's key and length at its scanned offset (off: exclusive
-// offsets, total at off[n]), so the candidates come out in key order, with no
-// atomic on a shared counter.
-__global__ void k_hot_cand(const uint32_t *__restrict__ a, uint32_t n, const uint32_t *__restrict__ off,
-                           uint32_t *__restrict__ ck, uint32_t *__restrict__ cv, uint32_t *__restrict__ ctl)
-{
-    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i == 0)
-        ctl[HC_NCAND] = off[n];
-    if (i >= n || off[i + 1] == off[i])
+    __shared__ uint32_t s_w[16], s_least, s_room, s_take, s_base, s_cover;
+    const uint32_t n = ctl[HC_FOUND];
+    if (blockIdx.x * 1024u >= n) // uniform
         return;
-    ck[off[i]] = a[i];
-    cv[off[i]] = i - run_start(a, i) + 1;
-}
-
-// candidates in key order -> (HOT_SAMPLE - count, key), so that a stable
-// sort of the first orders them by count, ties by key
-__global__ void k_hot_rekey(const uint32_t *__restrict__ ck, const uint32_t *__restrict__ cv,
-                            uint32_t *__restrict__ k2, uint32_t *__restrict__ v2, const uint32_t *__restrict__ ctl)
-{
-    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < ctl[HC_NCAND]) {
-        k2[i] = HOT_SAMPLE - cv[i];
-        v2[i] = ck[i];
+    const uint32_t t = threadIdx.x, lane = t & 63u, wv = t >> 6;
+    if (t == 0) {
+        s_least = 0; // every candidate is taken, unless found otherwise below
+        s_room = 0;
+        s_take = 0;
+        s_cover = 0;
     }
-}
-
-// sample keys the first HOT_MAX candidates cover (one block)
-__global__ __launch_bounds__(1024) void k_hot_cover(const uint32_t *__restrict__ k2, uint32_t *__restrict__ ctl)
-{
-    __shared__ uint32_t s;
-    if (threadIdx.x == 0)
-        s = 0;
+    // thread t holds the four counts from the top: 4095 - 4 t and the three below
+    uint32_t h[4], sum = 0;
+#pragma unroll
+    for (uint32_t k = 0; k < 4u; ++k) {
+        h[k] = ccount[SAMP_COUNTS - 1u - (4u * t + k)];
+        sum += h[k];
+    }
+    uint32_t x = sum;
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+        const uint32_t y = (uint32_t)__shfl_up((int)x, o, 64);
+        x += lane >= (uint32_t)o ? y : 0u;
+    }
+    if (lane == 63u)
+        s_w[wv] = x;
     __syncthreads();
-    const uint32_t m = min(ctl[HC_NCAND], HOT_MAX);
-    uint32_t sum = 0;
-    for (uint32_t i = threadIdx.x; i < m; i += blockDim.x)
-        sum += HOT_SAMPLE - k2[i];
-    atomicAdd(&s, sum);
+    uint32_t above = x - sum; // candidates with larger counts than h[0]'s
+    for (uint32_t w = 0; w < wv; ++w)
+        above += s_w[w];
+#pragma unroll
+    for (uint32_t k = 0; k < 4u; ++k) {
+        if (above <= HOT_MAX && above + h[k] > HOT_MAX) { // one count at most
+            s_least = SAMP_COUNTS - 1u - (4u * t + k);
+            s_room = HOT_MAX - above;
+        }
+        above += h[k];
+    }
     __syncthreads();
-    if (threadIdx.x == 0)
-        ctl[HC_COVER] = s;
+    const uint32_t i = blockIdx.x * 1024u + t;
+    const uint32_t c = i < n ? cv[i] : 0u, cl = min(c, SAMP_COUNTS - 1u);
+    bool take = i < n && cl > s_least;
+    if (i < n && s_least && cl == s_least)
+        take = atomicAdd(ctl + HC_TIES, 1u) < s_room;
+    const uint64_t m = __ballot(take);
+    uint32_t at = 0;
+    if (lane == 0 && m)
+        at = atomicAdd(&s_take, (uint32_t)__popcll(m));
+    at = (uint32_t)__shfl((int)at, 0, 64) + (uint32_t)__popcll(m & ((1ull << lane) - 1ull));
+    if (take)
+        atomicAdd(&s_cover, c);
+    __syncthreads();
+    if (t == 0 && s_take) {
+        s_base = atomicAdd(ctl + HC_NCAND, s_take);
+        atomicAdd(ctl + HC_COVER, s_cover);
+    }
+    __syncthreads();
+    if (take && s_base + at < HOT_MAX)
+        cand[s_base + at] = ck[i];
 }
 
 __global__ void k_hot_clear(uint32_t *__restrict__ tkey, uint32_t *__restrict__ tfill, uint32_t *__restrict__ ctl)
@@ -555,15 +718,7 @@ void qs_hot_state_free(void *state)
     qs_hot *h = (qs_hot *)state;
     if (!h)
         return;
-    for (int k = 0; k < 2; ++k) {
-        (void)hipFree(h->sk[k]);
-        (void)hipFree(h->sv[k]);
-        (void)hipFree(h->ck[k]);
-        (void)hipFree(h->cv[k]);
-    }
-    (void)hipFree(h->hist);
-    (void)hipFree(h->cflag);
-    (void)hipFree(h->cbsum);
+    (void)hipFree(h->samp); // and the candidate buffers after it
     (void)hipFree(h->ctl);
     (void)hipFree(h->tkey);
     (void)hipFree(h->tinfo);
@@ -606,15 +761,8 @@ static int hot_alloc(void **state, uint64_t rest)
             hipDeviceGetAttribute(&cu, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cu <= 0)
             cu = 256;
         h->nblk = (uint32_t)cu;
-        bool ok = true;
-        for (int k = 0; k < 2; ++k)
-            ok = ok && hipMalloc(&h->sk[k], 4ull * HOT_SAMPLE) == hipSuccess &&
-                 hipMalloc(&h->sv[k], 4ull * HOT_SAMPLE) == hipSuccess &&
-                 hipMalloc(&h->ck[k], 4ull * HOT_CAND_MAX) == hipSuccess &&
-                 hipMalloc(&h->cv[k], 4ull * HOT_CAND_MAX) == hipSuccess;
-        ok = ok && hipMalloc(&h->hist, 4ull * qs_sort_hist_words(HOT_SAMPLE)) == hipSuccess &&
-             hipMalloc(&h->cflag, 4ull * (HOT_SAMPLE + 1)) == hipSuccess &&
-             hipMalloc(&h->cbsum, 4ull * (HOT_SAMPLE / SCAN_SPAN + 1)) == hipSuccess &&
+        const uint64_t words = HOT_SAMPLE + (SAMP_TILES + 2u) * SAMP_BINS + SAMP_COUNTS + 2ull * HOT_CAND_MAX + HOT_MAX;
+        bool ok = hipMalloc(&h->samp, 4ull * words) == hipSuccess &&
              hipMalloc(&h->ctl, 4ull * HC_WORDS) == hipSuccess &&
              hipMalloc(&h->tkey, 4ull * HOT_SLOTS) == hipSuccess &&
              hipMalloc(&h->tinfo, 4ull * HOT_SLOTS) == hipSuccess &&
@@ -626,6 +774,11 @@ static int hot_alloc(void **state, uint64_t rest)
              hipEventCreateWithFlags(&h->ev_fork, hipEventDisableTiming) == hipSuccess &&
              hipEventCreateWithFlags(&h->ev_cand, hipEventDisableTiming) == hipSuccess;
         if (ok) {
+            h->scnt = h->samp + HOT_SAMPLE;
+            h->ccount = h->scnt + (SAMP_TILES + 2u) * SAMP_BINS;
+            h->ck = h->ccount + SAMP_COUNTS;
+            h->cv = h->ck + HOT_CAND_MAX;
+            h->cand = h->cv + HOT_CAND_MAX;
             memset(h->h_ctl, 0, 4ull * HOT_PUB_WORDS);
             h->seq = 0;
         }
@@ -658,34 +811,18 @@ static int hot_alloc(void **state, uint64_t rest)
     return QS_OK;
 }
 
-// Candidates from the first HOT_SAMPLE keys (step 1), queued on `stream`:
-// h->cand = the candidate keys, most frequent first (at most HOT_MAX are
-// used).  hot_cand_result then waits for their cover.
+// Candidates from the first HOT_SAMPLE keys (step 1), queued on `stream`, to
+// h->cand.  hot_cand_result then waits for their cover.
 static int hot_cand_launch(qs_hot *h, const uint32_t *keys, hipStream_t stream)
 {
-    hipLaunchKernelGGL(k_hot_sample, dim3(HOT_SAMPLE / 256), dim3(256), 0, stream, keys, HOT_SAMPLE, h->sk[0],
-                       h->sv[0], h->ctl);
-    const int r0 = qs_sort_pairs(h->sk, h->sv, h->hist, HOT_SAMPLE, 32, stream);
-    if (r0 < 0)
-        return QS_ERR_HIP;
-    // candidates in key order: flags, a scan, each at its offset
-    const uint32_t snb = HOT_SAMPLE / SCAN_SPAN;
-    hipLaunchKernelGGL(k_hot_cand_flag, dim3(HOT_SAMPLE / 256), dim3(256), 0, stream, h->sk[r0], HOT_SAMPLE,
-                       h->cflag);
-    hipLaunchKernelGGL(k_scan_reduce, dim3(snb), dim3(1024), 0, stream, h->cflag, HOT_SAMPLE, h->cbsum);
-    hipLaunchKernelGGL(k_scan_top, dim3(1), dim3(1024), 0, stream, h->cbsum, snb);
-    hipLaunchKernelGGL(k_scan_apply, dim3(snb), dim3(1024), 0, stream, h->cflag, HOT_SAMPLE, h->cbsum, snb);
-    hipLaunchKernelGGL(k_hot_cand, dim3(HOT_SAMPLE / 256), dim3(256), 0, stream, h->sk[r0], HOT_SAMPLE, h->cflag,
-                       h->ck[0], h->cv[0], h->ctl);
-    uint32_t *k2[2] = {h->ck[1], h->ck[0]}, *v2[2] = {h->cv[1], h->cv[0]};
-    hipLaunchKernelGGL(k_hot_rekey, dim3(HOT_CAND_MAX / 256), dim3(256), 0, stream, h->ck[0], h->cv[0], k2[0],
-                       v2[0], h->ctl);
-    const int r2 = qs_sort_pairs_dev(k2, v2, h->hist, h->ctl + HC_NCAND, HOT_CAND_MAX, 21, stream);
-    if (r2 < 0)
-        return QS_ERR_HIP;
-    hipLaunchKernelGGL(k_hot_cover, dim3(1), dim3(1024), 0, stream, k2[r2], h->ctl);
+    uint32_t *start = h->scnt + SAMP_TILES * SAMP_BINS; // SAMP_BINS + 1 words
+    hipLaunchKernelGGL(k_samp_hist, dim3(SAMP_TILES), dim3(1024), 0, stream, keys, h->scnt, h->ccount, h->ctl);
+    hipLaunchKernelGGL(k_samp_split, dim3(SAMP_TILES), dim3(1024), 0, stream, keys, h->scnt, h->samp, start);
+    hipLaunchKernelGGL(k_samp_count, dim3(SAMP_BINS), dim3(1024), 0, stream, h->samp, start, h->ck, h->cv, h->ccount,
+                       h->ctl);
+    hipLaunchKernelGGL(k_samp_select, dim3(HOT_CAND_MAX / 1024u), dim3(1024), 0, stream, h->ck, h->cv, h->ccount,
+                       h->cand, h->ctl);
     CK(hipGetLastError());
-    h->cand = v2[r2];
     return QS_OK;
 }
 

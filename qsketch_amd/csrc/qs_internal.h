@@ -380,16 +380,6 @@ struct qs_hot_split {
 int qs_hot_split_keys(void **state, const uint32_t *keys, uint64_t n, hipStream_t stream, qs_hot_split *out);
 void qs_hot_state_free(void *state);
 
-// Stable LSD radix sort of (key, value) uint32 pairs, 8 bits per pass, over the
-// low key_bits bits.  Input in keys[0]/vals[0]; returns the index (0 or 1) of
-// the buffer pair holding the sorted result.
-int qs_sort_pairs(uint32_t *keys[2], uint32_t *vals[2], uint32_t *d_hist, uint32_t count,
-                  int key_bits, hipStream_t stream);
-// Same, with the element count read from device memory at run time (max_count
-// sizes the grid); capture-safe: no host synchronisation.
-int qs_sort_pairs_dev(uint32_t *keys[2], uint32_t *vals[2], uint32_t *d_hist,
-                      const uint32_t *d_count, uint32_t max_count, int key_bits, hipStream_t stream);
-size_t qs_sort_hist_words(uint32_t max_count);
 // Exclusive scan of each row hist[d][0..ntiles) for d < nbins; totals[d] = row sum.
 void qs_scan_digits(uint32_t *hist, uint32_t ntiles, uint32_t nbins, uint32_t *totals,
                     hipStream_t stream);
