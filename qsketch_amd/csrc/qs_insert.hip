@@ -942,14 +942,34 @@ __device__ static inline uint32_t finish_run(bool act, uint32_t sid, uint32_t b,
 // lane finishes in one window are in flight together (the runs are distinct
 // cells, so no load depends on another run's store): load_run reads the
 // bucket's two 16-byte words, apply_run then does what finish_run does.
+//
+// In a batch, a wavefront's windows nearly always lie in one sketch's part of
+// the sorted items; its descriptor is then read once, into scalar registers
+// (one_sketch.on), instead of per item and per run.
+struct one_sketch {
+    bool on; // wave-uniform, like the rest
+    uint32_t n_low;
+    qs_fastdiv fd_masks;
+    seg_tables t;
+};
+
 template <bool MULTI>
-__device__ static inline void load_run(bool act, uint64_t cell, const qs_pack &pk, const qs_sdesc *__restrict__ D,
-                                       uint32_t *low_pool, uint32_t *high_pool, const uint32_t *mask_pool,
-                                       uint4 &x, uint4 &y)
+__device__ static inline seg_tables tables_at(const one_sketch &u, uint32_t sid, const qs_sdesc *__restrict__ D,
+                                              uint32_t *low_pool, uint32_t *high_pool, const uint32_t *mask_pool)
+{
+    if (MULTI && u.on)
+        return u.t;
+    return tables_of<MULTI>(sid, D, low_pool, high_pool, mask_pool);
+}
+
+template <bool MULTI>
+__device__ static inline void load_run(bool act, uint64_t cell, const qs_pack &pk, const one_sketch &u,
+                                       const qs_sdesc *__restrict__ D, uint32_t *low_pool, uint32_t *high_pool,
+                                       const uint32_t *mask_pool, uint4 &x, uint4 &y)
 {
     if (!act)
         return;
-    const seg_tables tb = tables_of<MULTI>((uint32_t)(cell >> pk.bb), D, low_pool, high_pool, mask_pool);
+    const seg_tables tb = tables_at<MULTI>(u, (uint32_t)(cell >> pk.bb), D, low_pool, high_pool, mask_pool);
     const uint4 *bp = reinterpret_cast<const uint4 *>(tb.low + (size_t)(uint32_t)(cell & pk.bmask) * 8u);
     x = bp[0];
     y = bp[1];
@@ -957,8 +977,8 @@ __device__ static inline void load_run(bool act, uint64_t cell, const qs_pack &p
 
 template <bool MULTI>
 __device__ static inline uint32_t apply_run(bool act, uint64_t cell, uint64_t len, const uint32_t a[7], uint4 x,
-                                            uint4 y, const qs_pack &pk, const qs_sdesc *__restrict__ D,
-                                            uint32_t *low_pool, uint32_t *high_pool, const uint32_t *mask_pool,
+                                            uint4 y, const qs_pack &pk, const one_sketch &u,
+                                            const qs_sdesc *__restrict__ D, uint32_t *low_pool, uint32_t *high_pool, const uint32_t *mask_pool,
                                             uint32_t *longbm)
 {
     if (!act)
@@ -968,14 +988,14 @@ __device__ static inline uint32_t apply_run(bool act, uint64_t cell, uint64_t le
         set_long<MULTI>(longbm, D, sid, b);
         return FR_LONG | (y.w <= QS_LINK_START ? FR_UNLINKED : 0u);
     }
-    const seg_tables tb = tables_of<MULTI>(sid, D, low_pool, high_pool, mask_pool);
+    const seg_tables tb = tables_at<MULTI>(u, sid, D, low_pool, high_pool, mask_pool);
     return apply_loaded(tb.low, tb.high, b, a, x, y) ? FR_RISKY : 0u;
 }
 
-// (A single sketch's shapes of up to 4 items per lane are held to 168
-// registers, three wavefronts per SIMD, which they fit without spilling.)
+// (Shapes of up to 4 items per lane are held to 168 registers, three
+// wavefronts per SIMD, which they fit without spilling.)
 template <bool MULTI, int W, int IPL>
-__global__ __launch_bounds__(SEG_THREADS) __attribute__((amdgpu_waves_per_eu(!MULTI && IPL <= 4 ? 3 : 1))) void k_segw(
+__global__ __launch_bounds__(SEG_THREADS) __attribute__((amdgpu_waves_per_eu(IPL <= 4 ? 3 : 1))) void k_segw(
     const uint64_t *__restrict__ IT, uint32_t n, const qs_sdesc *__restrict__ D, uint32_t n_masks0,
     uint32_t *__restrict__ low_pool, uint32_t *__restrict__ high_pool,
     const uint32_t *__restrict__ mask_pool, qs_pack pk, uint32_t *__restrict__ longbm,
@@ -1026,6 +1046,28 @@ __global__ __launch_bounds__(SEG_THREADS) __attribute__((amdgpu_waves_per_eu(!MU
 #pragma unroll
         for (int k = 0; k < IPL; ++k)
             itk[k] = nit[k];
+        // (items are sorted by sketch first: the lanes' first items and the
+        // items after the windows bound the rest)
+        one_sketch u;
+        u.on = false;
+        if (MULTI) {
+            const uint32_t su = (uint32_t)__builtin_amdgcn_readfirstlane((int)it_sid(itk[0], pk));
+            u.on = __ballot(it_sid(itk[0], pk) != su || it_sid(xit, pk) != su) == 0;
+            if (u.on) {
+                const qs_sdesc &d = D[su];
+                u.n_low = d.n_low;
+                u.fd_masks = d.fd_masks;
+                u.t.low = low_pool + d.low_off;
+                u.t.high = high_pool + d.high_off;
+                u.t.masks = mask_pool + d.masks_off;
+            }
+        }
+        auto mask_at = [&](uint64_t it) -> uint32_t {
+            if (MULTI && u.on)
+                return u.t.masks[pk.quot ? qs_fastmod(it_mu(it, pk) * u.n_low + it_b(it, pk), u.fd_masks)
+                                         : it_mu(it, pk)];
+            return mask_of<MULTI>(it_sid(it, pk), item_mu<MULTI>(it, pk, D), D, mask_pool, s_masks, pk.unm);
+        };
         {
             const uint64_t w1 = w0 + ngroups * T, p1 = w1 + (uint64_t)gl * IPL;
 #pragma unroll
@@ -1040,7 +1082,7 @@ __global__ __launch_bounds__(SEG_THREADS) __attribute__((amdgpu_waves_per_eu(!MU
             const bool v = p < n;
             const uint64_t it = itk[k];
             c[k] = v ? it_cell(it, pk) : NO_CELL;
-            M[k] = v ? mask_of<MULTI>(it_sid(it, pk), item_mu<MULTI>(it, pk, D), D, mask_pool, s_masks, pk.unm) : 0u;
+            M[k] = v ? mask_at(it) : 0u;
         }
         // cell before my first item and after my last one
         uint64_t cprev = shfl64w<W>(c[IPL - 1], (int)gl - 1);
@@ -1150,20 +1192,20 @@ __global__ __launch_bounds__(SEG_THREADS) __attribute__((amdgpu_waves_per_eu(!MU
         const uint64_t ce = shfl64w<W>(cl, W - 1);
         // the buckets of (a), the interior runs, (b) and (c), loaded together
         uint4 xa, ya, xb, yb, xe, ye, xi[NI], yi[NI];
-        load_run<MULTI>(ext && gl == 0, ce, pk, D, low_pool, high_pool, mask_pool, xe, ye);
-        load_run<MULTI>(act_a, c[0], pk, D, low_pool, high_pool, mask_pool, xa, ya);
+        load_run<MULTI>(ext && gl == 0, ce, pk, u, D, low_pool, high_pool, mask_pool, xe, ye);
+        load_run<MULTI>(act_a, c[0], pk, u, D, low_pool, high_pool, mask_pool, xa, ya);
 #pragma unroll
         for (int j = 0; j < NI; ++j)
-            load_run<MULTI>(iact[j], icell[j], pk, D, low_pool, high_pool, mask_pool, xi[j], yi[j]);
-        load_run<MULTI>(act_b, cl, pk, D, low_pool, high_pool, mask_pool, xb, yb);
-        const uint32_t fr_a = apply_run<MULTI>(act_a, c[0], act_a ? p0 + f1 - (head - 1u) : 0u, af, xa, ya, pk, D,
+            load_run<MULTI>(iact[j], icell[j], pk, u, D, low_pool, high_pool, mask_pool, xi[j], yi[j]);
+        load_run<MULTI>(act_b, cl, pk, u, D, low_pool, high_pool, mask_pool, xb, yb);
+        const uint32_t fr_a = apply_run<MULTI>(act_a, c[0], act_a ? p0 + f1 - (head - 1u) : 0u, af, xa, ya, pk, u, D,
                                                low_pool, high_pool, mask_pool, longbm);
         uint32_t fr_i[NI];
 #pragma unroll
         for (int j = 0; j < NI; ++j) // an interior run is shorter than IPL items: never long
-            fr_i[j] = apply_run<MULTI>(iact[j], icell[j], 1u, ia[j], xi[j], yi[j], pk, D, low_pool, high_pool,
+            fr_i[j] = apply_run<MULTI>(iact[j], icell[j], 1u, ia[j], xi[j], yi[j], pk, u, D, low_pool, high_pool,
                                        mask_pool, longbm);
-        const uint32_t fr_b = apply_run<MULTI>(act_b, cl, act_b ? p0 + IPL - (hp - 1u) : 0u, x, xb, yb, pk, D,
+        const uint32_t fr_b = apply_run<MULTI>(act_b, cl, act_b ? p0 + IPL - (hp - 1u) : 0u, x, xb, yb, pk, u, D,
                                                low_pool, high_pool, mask_pool, longbm);
         // (c): the run's items in the extension window [w0 + T, w0 + 2T) are
         // a prefix of it (the items are sorted by cell).  When fewer than W
@@ -1184,7 +1226,7 @@ __global__ __launch_bounds__(SEG_THREADS) __attribute__((amdgpu_waves_per_eu(!MU
             const bool in1 = w0 + T + gl < n && it_cell(xit, pk) == ce;
             if ((__ballot(in1) & gmask) != gmask) {
                 if (in1) {
-                    mask_to_words(mask_of<MULTI>(sid, item_mu<MULTI>(xit, pk, D), D, mask_pool, s_masks, pk.unm), sum);
+                    mask_to_words(mask_at(xit), sum);
                     cnt = 1;
                 }
             } else {
@@ -1194,8 +1236,7 @@ __global__ __launch_bounds__(SEG_THREADS) __attribute__((amdgpu_waves_per_eu(!MU
                     if (q < n) {
                         const uint64_t iq = IT[q];
                         if (it_cell(iq, pk) == ce) {
-                            mask_to_words(mask_of<MULTI>(sid, item_mu<MULTI>(iq, pk, D), D, mask_pool, s_masks, pk.unm),
-                                          tmp);
+                            mask_to_words(mask_at(iq), tmp);
                             add_words(sum, tmp);
                             ++cnt;
                         }
@@ -1217,7 +1258,7 @@ __global__ __launch_bounds__(SEG_THREADS) __attribute__((amdgpu_waves_per_eu(!MU
                     set_long<MULTI>(longbm, D, sid, b);
                     fr_e = FR_LONG | (ye.w <= QS_LINK_START ? FR_UNLINKED : 0u);
                 } else {
-                    fr_e = apply_run<MULTI>(true, ce, len, e, xe, ye, pk, D, low_pool, high_pool, mask_pool, longbm);
+                    fr_e = apply_run<MULTI>(true, ce, len, e, xe, ye, pk, u, D, low_pool, high_pool, mask_pool, longbm);
                 }
             }
             hpos_e = (uint32_t)(he - 1u);

@@ -248,6 +248,50 @@ __device__ static inline uint32_t query_sid(const uint64_t *__restrict__ offs, u
     return lo;
 }
 
+// Answers key i: two lanes, one 16-byte half of the bucket each.
+__device__ static inline void query_bucket(uint32_t M, uint32_t b, const uint32_t *__restrict__ low,
+                                           const uint32_t *__restrict__ high, uint32_t half, uint32_t *out)
+{
+    // read once: a non-temporal load (measured 0.433 -> 0.405 ms for 16.6 M keys)
+    const u32x4 vv = __builtin_nontemporal_load(reinterpret_cast<const u32x4 *>(low + (size_t)b * 8u) + half);
+    const uint4 v = make_uint4(vv[0], vv[1], vv[2], vv[3]);
+    const uint32_t Mh = half ? (M >> 16) : (M & 0xffffu);
+    uint32_t lo = 0xffffffffu;
+    for (uint32_t m = Mh; m; m &= m - 1u) {
+        const uint32_t jj = (uint32_t)__builtin_ctz(m);
+        lo = min(lo, (sel4(v, jj >> 2) >> ((jj & 3u) * 8u)) & 0xffu);
+    }
+    lo = min(lo, (uint32_t)__shfl_xor(lo, 1, 64));
+    const uint32_t wo = (uint32_t)__shfl_xor(v.w, 1, 64);
+    const uint32_t w = half ? v.w : wo;
+    uint32_t hi = 0;
+    if (w > QS_LINK_START) {
+        const uint32_t *g = high + (size_t)(w - QS_LINK_START) * 32u + 16u * half;
+        hi = 0xffffffffu;
+        for (uint32_t m = Mh; m; m &= m - 1u)
+            hi = min(hi, g[__builtin_ctz(m)]);
+        hi = min(hi, (uint32_t)__shfl_xor(hi, 1, 64));
+    }
+    if (!half)
+        *out = lo + hi;
+}
+
+// Keys of a batch that a block takes at a time.
+#define QUERY_TILE 1024u
+// Sketches of a tile that it takes one after the other; a tile of more (short
+// parts) finds each key's sketch by itself.
+#define QUERY_PARTS 8u
+// keys of a part from which its masks are worth copying to LDS
+#define QUERY_LDS_MIN 256u
+
+// A single sketch's blocks take keys in turn.  In a batch a block takes tiles of
+// consecutive keys and, sketch by sketch, answers the tile's parts as a single
+// sketch's: descriptor in scalar registers, masks in LDS.  The tiles of one XCD's
+// blocks (blocks go to the 8 XCDs in turn) are consecutive, so at any time they
+// read the buckets of one or two sketches, which its L2 holds.  18.8 M keys of
+// 512 sketches: 770 us with a search in the global offsets, a descriptor load and a
+// mask load per key; 609 without them but with one long range per block (every
+// sketch at once); now 553.
 template <int KB, bool MULTI>
 __global__ __launch_bounds__(INS_THREADS) void k_query(const KeyT<KB> *__restrict__ keys, uint32_t n, qs_sdesc d0,
                                                        const qs_sdesc *__restrict__ D,
@@ -257,50 +301,68 @@ __global__ __launch_bounds__(INS_THREADS) void k_query(const KeyT<KB> *__restric
                                                        const uint32_t *__restrict__ mask_pool,
                                                        uint32_t *__restrict__ out)
 {
-    __shared__ uint32_t s_masks[MULTI ? 1 : QS_MAX_MASKS];
-    if (!MULTI)
+    __shared__ uint32_t s_masks[QS_MAX_MASKS];
+    const uint32_t half = threadIdx.x & 1u;
+    if (!MULTI) {
         for (uint32_t i = threadIdx.x; i < d0.n_masks; i += INS_THREADS)
             s_masks[i] = mask_pool[i];
-    __syncthreads();
-    const uint32_t half = threadIdx.x & 1u;
-    const uint64_t stride = (uint64_t)gridDim.x * (INS_THREADS / 2);
-    for (uint64_t i = (uint64_t)blockIdx.x * (INS_THREADS / 2) + (threadIdx.x >> 1); i < n; i += stride) {
-        const KeyT<KB> key = keys[i];
-        const uint32_t *low = low_pool;
-        const uint32_t *high = high_pool;
-        uint32_t M, b;
-        if (MULTI) {
-            const qs_sdesc &d = D[query_sid(offs, nsk, i)];
-            M = mask_pool[d.masks_off + qs_maskidx_d(key, d)];
-            b = qs_bucket_d(key, d);
-            low += d.low_off;
-            high += d.high_off;
-        } else {
-            M = s_masks[qs_maskidx_d(key, d0)];
-            b = qs_bucket_d(key, d0);
+        __syncthreads();
+        const uint64_t stride = (uint64_t)gridDim.x * (INS_THREADS / 2);
+        for (uint64_t i = (uint64_t)blockIdx.x * (INS_THREADS / 2) + (threadIdx.x >> 1); i < n; i += stride) {
+            const KeyT<KB> key = keys[i];
+            query_bucket(s_masks[qs_maskidx_d(key, d0)], qs_bucket_d(key, d0), low_pool, high_pool, half, out + i);
         }
-        // read once: a non-temporal load (measured 0.433 -> 0.405 ms for 16.6 M keys)
-        const u32x4 vv = __builtin_nontemporal_load(reinterpret_cast<const u32x4 *>(low + (size_t)b * 8u) + half);
-        const uint4 v = make_uint4(vv[0], vv[1], vv[2], vv[3]);
-        const uint32_t Mh = half ? (M >> 16) : (M & 0xffffu);
-        uint32_t lo = 0xffffffffu;
-        for (uint32_t m = Mh; m; m &= m - 1u) {
-            const uint32_t jj = (uint32_t)__builtin_ctz(m);
-            lo = min(lo, (sel4(v, jj >> 2) >> ((jj & 3u) * 8u)) & 0xffu);
+        return;
+    }
+    __shared__ uint32_t s_sid[2];
+    const uint64_t stride = INS_THREADS / 2;
+    // XCD x's tiles are [tx, tz) (a bijection of all tiles whatever the placement)
+    const uint64_t tiles = ((uint64_t)n + QUERY_TILE - 1u) / QUERY_TILE;
+    const uint32_t x = blockIdx.x & 7u, xb = min(8u, gridDim.x); // XCDs in use
+    const uint64_t tx = tiles * x / xb, tz = tiles * (x + 1u) / xb;
+    const uint32_t nb = (gridDim.x - x + 7u) / 8u; // blocks of this XCD
+    uint32_t held = 0xffffffffu;                   // sketch whose masks are in LDS
+    for (uint64_t tile = tx + (blockIdx.x >> 3); tile < tz; tile += nb) {
+        const uint64_t i0 = tile * QUERY_TILE, i1 = i0 + QUERY_TILE < n ? i0 + QUERY_TILE : n;
+        __syncthreads();
+        if (threadIdx.x < 2u)
+            s_sid[threadIdx.x] = query_sid(offs, nsk, threadIdx.x ? i1 - 1u : i0);
+        __syncthreads();
+        const uint32_t sa = s_sid[0], sz = s_sid[1];
+        if (sz - sa >= QUERY_PARTS) {
+            for (uint64_t i = i0 + (threadIdx.x >> 1); i < i1; i += stride) {
+                const KeyT<KB> key = keys[i];
+                const qs_sdesc &d = D[sa + query_sid(offs + sa, sz - sa + 1u, i)];
+                query_bucket(mask_pool[d.masks_off + qs_maskidx_d(key, d)], qs_bucket_d(key, d),
+                             low_pool + d.low_off, high_pool + d.high_off, half, out + i);
+            }
+            continue;
         }
-        lo = min(lo, (uint32_t)__shfl_xor(lo, 1, 64));
-        const uint32_t wo = (uint32_t)__shfl_xor(v.w, 1, 64);
-        const uint32_t w = half ? v.w : wo;
-        uint32_t hi = 0;
-        if (w > QS_LINK_START) {
-            const uint32_t *g = high + (size_t)(w - QS_LINK_START) * 32u + 16u * half;
-            hi = 0xffffffffu;
-            for (uint32_t m = Mh; m; m &= m - 1u)
-                hi = min(hi, g[__builtin_ctz(m)]);
-            hi = min(hi, (uint32_t)__shfl_xor(hi, 1, 64));
+        for (uint32_t sid = sa; sid <= sz; ++sid) { // uniform
+            const uint64_t a = offs[sid] > i0 ? offs[sid] : i0, z = offs[sid + 1] < i1 ? offs[sid + 1] : i1;
+            if (a >= z)
+                continue;
+            const qs_sdesc d = D[sid];
+            const uint32_t *low = low_pool + d.low_off, *high = high_pool + d.high_off,
+                           *masks = mask_pool + d.masks_off;
+            if (held != sid && z - a >= QUERY_LDS_MIN) {
+                __syncthreads(); // the part before still reads its masks
+                for (uint32_t i = threadIdx.x; i < d.n_masks; i += INS_THREADS)
+                    s_masks[i] = masks[i];
+                __syncthreads();
+                held = sid;
+            }
+            if (held == sid)
+                for (uint64_t i = a + (threadIdx.x >> 1); i < z; i += stride) {
+                    const KeyT<KB> key = keys[i];
+                    query_bucket(s_masks[qs_maskidx_d(key, d)], qs_bucket_d(key, d), low, high, half, out + i);
+                }
+            else
+                for (uint64_t i = a + (threadIdx.x >> 1); i < z; i += stride) {
+                    const KeyT<KB> key = keys[i];
+                    query_bucket(masks[qs_maskidx_d(key, d)], qs_bucket_d(key, d), low, high, half, out + i);
+                }
         }
-        if (!half)
-            out[i] = lo + hi;
     }
 }
 
