@@ -773,24 +773,18 @@ __device__ static inline bool test_long(const uint32_t *longbm, const qs_sdesc *
     return (longbm[bit >> 5] >> (bit & 31u)) & 1u;
 }
 
-template <bool MULTI>
-__global__ __launch_bounds__(SEG_THREADS) void k_seg(
-    const uint64_t *__restrict__ IT, uint32_t n, const qs_sdesc *__restrict__ D, uint32_t n_masks0,
+// block bid of nblk, of NW wavefronts; s_masks: a single sketch's masks, in LDS
+template <bool MULTI, int NW>
+__device__ __forceinline__ void seg_pass(uint32_t bid, uint32_t nblk,
+    const uint64_t *__restrict__ IT, uint32_t n, const qs_sdesc *__restrict__ D, const uint32_t *s_masks,
     uint32_t *__restrict__ low_pool, uint32_t *__restrict__ high_pool,
     const uint32_t *__restrict__ mask_pool, qs_pack pk, uint32_t *__restrict__ longbm,
     uint32_t *__restrict__ ord, uint32_t *__restrict__ lng, qs_dev_state *__restrict__ st)
 {
-    // a single sketch keeps its masks in LDS; a batch reads each sketch's masks
-    // from the (cache-resident) pool
-    __shared__ uint32_t s_masks[MULTI ? 1 : QS_MAX_MASKS];
-    if (!MULTI)
-        for (uint32_t i = threadIdx.x; i < n_masks0; i += SEG_THREADS)
-            s_masks[i] = mask_pool[i];
-    __syncthreads();
     const uint32_t lane = threadIdx.x & 63u;
     const uint64_t le = (lane == 63u) ? ~0ull : ((2ull << lane) - 1ull);
-    const uint32_t gw = blockIdx.x * (SEG_THREADS / 64u) + (threadIdx.x >> 6);
-    const uint32_t nw = gridDim.x * (SEG_THREADS / 64u);
+    const uint32_t gw = bid * ((uint32_t)NW) + (threadIdx.x >> 6);
+    const uint32_t nw = nblk * ((uint32_t)NW);
     for (uint64_t w0 = (uint64_t)gw * 64u; w0 < n; w0 += (uint64_t)nw * 64u) {
         const uint32_t p = (uint32_t)w0 + lane;
         const bool valid = p < n;
@@ -890,6 +884,23 @@ __global__ __launch_bounds__(SEG_THREADS) void k_seg(
             }
         }
     }
+}
+
+template <bool MULTI>
+__global__ __launch_bounds__(SEG_THREADS) void k_seg(
+    const uint64_t *__restrict__ IT, uint32_t n, const qs_sdesc *__restrict__ D, uint32_t n_masks0,
+    uint32_t *__restrict__ low_pool, uint32_t *__restrict__ high_pool,
+    const uint32_t *__restrict__ mask_pool, qs_pack pk, uint32_t *__restrict__ longbm,
+    uint32_t *__restrict__ ord, uint32_t *__restrict__ lng, qs_dev_state *__restrict__ st)
+{
+    // a single sketch keeps its masks in LDS; a batch reads each sketch's masks
+    // from the (cache-resident) pool
+    __shared__ uint32_t s_masks[MULTI ? 1 : QS_MAX_MASKS];
+    if (!MULTI)
+        for (uint32_t i = threadIdx.x; i < n_masks0; i += SEG_THREADS)
+            s_masks[i] = mask_pool[i];
+    __syncthreads();
+    seg_pass<MULTI, SEG_THREADS / 64>(blockIdx.x, gridDim.x, IT, n, D, s_masks, low_pool, high_pool, mask_pool, pk, longbm, ord, lng, st);
 }
 
 // ---------------------------------------------------------------------------
@@ -1394,27 +1405,26 @@ __device__ static inline void flush_long(uint32_t (*s_ln)[TBUF], uint32_t wv, ui
         lng[base + lane] = s_ln[wv][lane];
     nlb = 0;
 }
-__global__ __launch_bounds__(256) void k_ordered(const uint64_t *__restrict__ IT, uint32_t n,
-                                                 const uint32_t *__restrict__ ord,
-                                                 const qs_sdesc *__restrict__ D,
-                                                 uint32_t *__restrict__ low_pool,
-                                                 const uint32_t *__restrict__ mask_pool, qs_pack pk,
-                                                 uint32_t *__restrict__ longbm,
-                                                 uint32_t *__restrict__ lng,
-                                                 qs_trig *__restrict__ trig, uint32_t trig_cap,
-                                                 uint32_t *__restrict__ tbit, uint32_t *__restrict__ tsum,
-                                                 const uint64_t *__restrict__ offs, uint64_t base,
-                                                 uint32_t one_masks, qs_dev_state *__restrict__ st)
+// block bid of nblk, of NW wavefronts; a single sketch's masks (one_masks of them)
+// are in LDS
+template <int NW>
+__device__ __forceinline__ void ordered_pass(uint32_t bid, uint32_t nblk, const uint64_t *__restrict__ IT, uint32_t n,
+                                             const uint32_t *__restrict__ ord,
+                                             const qs_sdesc *__restrict__ D,
+                                             uint32_t *__restrict__ low_pool,
+                                             const uint32_t *__restrict__ mask_pool, qs_pack pk,
+                                             uint32_t *__restrict__ longbm,
+                                             uint32_t *__restrict__ lng,
+                                             qs_trig *__restrict__ trig, uint32_t trig_cap,
+                                             uint32_t *__restrict__ tbit, uint32_t *__restrict__ tsum,
+                                             const uint64_t *__restrict__ offs, uint64_t base,
+                                             uint32_t one_masks, const uint32_t *s_masks, qs_dev_state *__restrict__ st)
 {
-    __shared__ qs_trig s_tr[4][TBUF];
-    __shared__ uint32_t s_ln[4][TBUF];
-    __shared__ uint32_t s_masks[QS_MAX_MASKS]; // a single sketch's masks (one_masks of them)
-    for (uint32_t i = threadIdx.x; i < one_masks; i += blockDim.x)
-        s_masks[i] = mask_pool[i];
-    __syncthreads();
+    __shared__ qs_trig s_tr[NW][TBUF];
+    __shared__ uint32_t s_ln[NW][TBUF];
     const uint32_t lane = threadIdx.x & 63u, wv = threadIdx.x >> 6;
-    const uint32_t gw = blockIdx.x * (blockDim.x / 64u) + (threadIdx.x >> 6);
-    const uint32_t nw = gridDim.x * (blockDim.x / 64u);
+    const uint32_t gw = bid * (uint32_t)NW + (threadIdx.x >> 6);
+    const uint32_t nw = nblk * (uint32_t)NW;
     const uint32_t n_ord = st->n_ord;
     uint32_t ntb = 0, nlb = 0;
     unsigned long long replayed_all = 0;
@@ -1540,8 +1550,8 @@ __global__ __launch_bounds__(256) void k_ordered(const uint64_t *__restrict__ IT
     // Final flush, one reservation per list per block: same-address atomics
     // serialise (~11 ns each), and one per wavefront and list costs more than
     // the replay itself.
-    __shared__ uint32_t s_nt[4], s_nl[4], s_base[2];
-    __shared__ unsigned long long s_rep[4];
+    __shared__ uint32_t s_nt[NW], s_nl[NW], s_base[2];
+    __shared__ unsigned long long s_rep[NW];
     if (lane == 0) {
         s_nt[wv] = ntb;
         s_nl[wv] = nlb;
@@ -1549,9 +1559,14 @@ __global__ __launch_bounds__(256) void k_ordered(const uint64_t *__restrict__ IT
     }
     __syncthreads();
     if (threadIdx.x == 0) {
-        const uint32_t tt = s_nt[0] + s_nt[1] + s_nt[2] + s_nt[3];
-        const uint32_t tl = s_nl[0] + s_nl[1] + s_nl[2] + s_nl[3];
-        const unsigned long long rk = s_rep[0] + s_rep[1] + s_rep[2] + s_rep[3];
+        uint32_t tt = 0, tl = 0;
+        unsigned long long rk = 0;
+#pragma unroll
+        for (int w = 0; w < NW; ++w) {
+            tt += s_nt[w];
+            tl += s_nl[w];
+            rk += s_rep[w];
+        }
         s_base[0] = tt ? atomicAdd(&st->n_trig, tt) : 0u;
         s_base[1] = tl ? atomicAdd(&st->n_long, tl) : 0u;
         if (rk)
@@ -1567,6 +1582,27 @@ __global__ __launch_bounds__(256) void k_ordered(const uint64_t *__restrict__ IT
     if (lane < nlb)
         lng[bl + lane] = s_ln[wv][lane];
 }
+
+__global__ __launch_bounds__(256) void k_ordered(const uint64_t *__restrict__ IT, uint32_t n,
+                                                 const uint32_t *__restrict__ ord,
+                                                 const qs_sdesc *__restrict__ D,
+                                                 uint32_t *__restrict__ low_pool,
+                                                 const uint32_t *__restrict__ mask_pool, qs_pack pk,
+                                                 uint32_t *__restrict__ longbm,
+                                                 uint32_t *__restrict__ lng,
+                                                 qs_trig *__restrict__ trig, uint32_t trig_cap,
+                                                 uint32_t *__restrict__ tbit, uint32_t *__restrict__ tsum,
+                                                 const uint64_t *__restrict__ offs, uint64_t base,
+                                                 uint32_t one_masks, qs_dev_state *__restrict__ st)
+{
+    __shared__ uint32_t s_masks[QS_MAX_MASKS];
+    for (uint32_t i = threadIdx.x; i < one_masks; i += blockDim.x)
+        s_masks[i] = mask_pool[i];
+    __syncthreads();
+    ordered_pass<4>(blockIdx.x, gridDim.x, IT, n, ord, D, low_pool, mask_pool, pk, longbm, lng, trig, trig_cap, tbit, tsum,
+                 offs, base, one_masks, s_masks, st);
+}
+
 
 // Exclusive scan of the per-span trigger counts (one block), the total after
 // them.
@@ -1654,21 +1690,23 @@ __device__ static inline uint32_t trig_rank(const uint32_t *__restrict__ tbit, c
 // (The order came from a pair sort of the triggers before: three launches per
 // digit pass.  At 2^22 keys that was 57 us of kernels and 12 launches; the
 // bitmap costs one 8 us scan and no sort.)
-__global__ __launch_bounds__(256) void k_assign(const qs_trig *__restrict__ trig, uint32_t trig_cap,
-                                                const uint32_t *__restrict__ tbit,
-                                                const uint32_t *__restrict__ tsum, uint32_t cn,
-                                                const uint64_t *__restrict__ offs, uint64_t base,
-                                                const qs_sdesc *__restrict__ D, uint32_t nsk,
-                                                uint32_t *__restrict__ low_pool,
-                                                uint32_t *__restrict__ high_pool,
-                                                uint32_t *__restrict__ tail_pool,
-                                                const uint32_t *__restrict__ next,
-                                                qs_dev_state *__restrict__ st)
+// block bid of nblk, of NW wavefronts
+template <int NW>
+__device__ __forceinline__ void assign_pass(uint32_t bid, uint32_t nblk, const qs_trig *__restrict__ trig, uint32_t trig_cap,
+                                            const uint32_t *__restrict__ tbit,
+                                            const uint32_t *__restrict__ tsum, uint32_t cn,
+                                            const uint64_t *__restrict__ offs, uint64_t base,
+                                            const qs_sdesc *__restrict__ D, uint32_t nsk,
+                                            uint32_t *__restrict__ low_pool,
+                                            uint32_t *__restrict__ high_pool,
+                                            uint32_t *__restrict__ tail_pool,
+                                            const uint32_t *__restrict__ next,
+                                            qs_dev_state *__restrict__ st)
 {
     const uint32_t n_trig = min(st->n_trig, trig_cap);
     const uint32_t lane = threadIdx.x & 63u;
-    const uint32_t gw = blockIdx.x * 4u + (threadIdx.x >> 6);
-    const uint32_t nw = gridDim.x * 4u;
+    const uint32_t gw = bid * (uint32_t)NW + (threadIdx.x >> 6);
+    const uint32_t nw = nblk * (uint32_t)NW;
     for (uint32_t r = gw; r < n_trig; r += nw) {
         const qs_trig *tr = trig + r;
         const uint32_t sid = tr->sid;
@@ -1691,6 +1729,22 @@ __global__ __launch_bounds__(256) void k_assign(const qs_trig *__restrict__ trig
         }
     }
 }
+
+__global__ __launch_bounds__(256) void k_assign(const qs_trig *__restrict__ trig, uint32_t trig_cap,
+                                                const uint32_t *__restrict__ tbit,
+                                                const uint32_t *__restrict__ tsum, uint32_t cn,
+                                                const uint64_t *__restrict__ offs, uint64_t base,
+                                                const qs_sdesc *__restrict__ D, uint32_t nsk,
+                                                uint32_t *__restrict__ low_pool,
+                                                uint32_t *__restrict__ high_pool,
+                                                uint32_t *__restrict__ tail_pool,
+                                                const uint32_t *__restrict__ next,
+                                                qs_dev_state *__restrict__ st)
+{
+    assign_pass<4>(blockIdx.x, gridDim.x, trig, trig_cap, tbit, tsum, cn, offs, base, D, nsk, low_pool, high_pool, tail_pool,
+                next, st);
+}
+
 
 // Long segments: every insert of a bucket linked before this chunk, and the
 // inserts after the allocation batch of a bucket linked in this chunk, are
@@ -1760,36 +1814,31 @@ template <> __device__ inline uint64_t shfl_cell<uint64_t>(uint64_t v, int src)
 
 // CT: the cell type, uint32_t when bucket and sketch bits fit in 31 (then the
 // sentinels NO_CELL, END_CELL truncated to 32 bits are above every cell)
-template <bool MULTI, typename CT>
-__global__ __launch_bounds__(256) void k_tail(const uint64_t *__restrict__ IT, uint32_t n,
-                                              const qs_sdesc *__restrict__ D, uint32_t n_masks0,
-                                              const uint32_t *__restrict__ low_pool,
-                                              uint32_t *__restrict__ high_pool,
-                                              const uint32_t *__restrict__ mask_pool, qs_pack pk,
-                                              const uint32_t *__restrict__ longbm,
-                                              const uint32_t *__restrict__ tail_pool,
-                                              const uint32_t *__restrict__ first_new,
-                                              const uint32_t *__restrict__ lng, bool short_runs, uint32_t window,
-                                              const qs_dev_state *__restrict__ st)
+// block bid of nblk, of NW wavefronts; s_masks: a single sketch's masks, in LDS (complete after the
+// barrier below)
+template <bool MULTI, typename CT, int NW>
+__device__ __forceinline__ void tail_pass(uint32_t bid, uint32_t nblk, const uint64_t *__restrict__ IT, uint32_t n,
+                                          const qs_sdesc *__restrict__ D, const uint32_t *s_masks,
+                                          const uint32_t *__restrict__ low_pool,
+                                          uint32_t *__restrict__ high_pool,
+                                          const uint32_t *__restrict__ mask_pool, qs_pack pk,
+                                          const uint32_t *__restrict__ longbm,
+                                          const uint32_t *__restrict__ tail_pool,
+                                          const uint32_t *__restrict__ first_new,
+                                          const uint32_t *__restrict__ lng, bool short_runs, uint32_t window,
+                                          const qs_dev_state *__restrict__ st)
 {
     if (st->n_long == 0)
         return;
-    // a single sketch's masks, n_masks0 words of dynamic LDS (sized by the
-    // launch: 16 KiB for the largest table would hold the kernel to five
-    // wavefronts per SIMD)
-    extern __shared__ uint32_t s_masks[];
-    if (!MULTI)
-        for (uint32_t i = threadIdx.x; i < n_masks0; i += blockDim.x)
-            s_masks[i] = mask_pool[i];
-    __shared__ uint32_t s_rows[4][64][TROW];
+    __shared__ uint32_t s_rows[NW][64][TROW];
     const uint32_t lane = threadIdx.x & 63u, wv = threadIdx.x >> 6;
     uint32_t(*rows)[TROW] = s_rows[wv];
 #pragma unroll
     for (int j = 0; j < 14; ++j)
         rows[lane][j] = 0;
     __syncthreads();
-    const uint32_t gw = blockIdx.x * 4u + wv;
-    const uint32_t nw = gridDim.x * 4u;
+    const uint32_t gw = bid * (uint32_t)NW + wv;
+    const uint32_t nw = nblk * (uint32_t)NW;
     for (uint64_t w0 = (uint64_t)gw * window; w0 < n; w0 += (uint64_t)nw * window) {
         const uint64_t wend = (w0 + window < n) ? w0 + window : n;
         uint32_t *cur = nullptr;
@@ -1951,28 +2000,55 @@ __global__ __launch_bounds__(256) void k_tail(const uint64_t *__restrict__ IT, u
     }
 }
 
+template <bool MULTI, typename CT>
+__global__ __launch_bounds__(256) void k_tail(const uint64_t *__restrict__ IT, uint32_t n,
+                                              const qs_sdesc *__restrict__ D, uint32_t n_masks0,
+                                              const uint32_t *__restrict__ low_pool,
+                                              uint32_t *__restrict__ high_pool,
+                                              const uint32_t *__restrict__ mask_pool, qs_pack pk,
+                                              const uint32_t *__restrict__ longbm,
+                                              const uint32_t *__restrict__ tail_pool,
+                                              const uint32_t *__restrict__ first_new,
+                                              const uint32_t *__restrict__ lng, bool short_runs, uint32_t window,
+                                              const qs_dev_state *__restrict__ st)
+{
+    if (st->n_long == 0)
+        return;
+    // n_masks0 words of dynamic LDS (sized by the launch: 16 KiB for the
+    // largest table would hold the kernel to five wavefronts per SIMD)
+    extern __shared__ uint32_t s_masks[];
+    if (!MULTI)
+        for (uint32_t i = threadIdx.x; i < n_masks0; i += blockDim.x)
+            s_masks[i] = mask_pool[i];
+    tail_pass<MULTI, CT, 4>(blockIdx.x, gridDim.x, IT, n, D, s_masks, low_pool, high_pool, mask_pool, pk, longbm, tail_pool,
+                         first_new, lng, short_runs, window, st);
+}
+
+
 // The chunk's last kernel: the long-segment marks are taken back, next[sid]
 // moves on by the allocations of sid (a wavefront per sketch), and the block
 // that finishes last resets the chunk's counters and leaves the error bits in
 // the host's pinned mirror, so that a blocking call needs no copy.
 #define FIN_BLOCKS 64u // at most: every block ends with one atomic on st->done
-__global__ __launch_bounds__(256) void k_finish(const uint32_t *__restrict__ lng, const uint64_t *__restrict__ IT,
-                                                const qs_sdesc *__restrict__ D, qs_pack pk,
-                                                uint32_t *__restrict__ longbm, const uint32_t *__restrict__ tbit,
-                                                const uint32_t *__restrict__ tsum, uint32_t cn,
-                                                const uint64_t *__restrict__ offs, uint64_t base, uint32_t nsk,
-                                                uint32_t *__restrict__ next, qs_dev_state *__restrict__ st,
-                                                uint32_t *__restrict__ h_err)
+// block bid of nblk, of NW wavefronts
+template <int NW>
+__device__ __forceinline__ void finish_pass(uint32_t bid, uint32_t nblk, const uint32_t *__restrict__ lng, const uint64_t *__restrict__ IT,
+                                            const qs_sdesc *__restrict__ D, qs_pack pk,
+                                            uint32_t *__restrict__ longbm, const uint32_t *__restrict__ tbit,
+                                            const uint32_t *__restrict__ tsum, uint32_t cn,
+                                            const uint64_t *__restrict__ offs, uint64_t base, uint32_t nsk,
+                                            uint32_t *__restrict__ next, qs_dev_state *__restrict__ st,
+                                            uint32_t *__restrict__ h_err)
 {
     const uint32_t n_long = st->n_long, n_trig = st->n_trig;
-    for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < n_long; i += gridDim.x * blockDim.x) {
+    for (uint32_t i = bid * blockDim.x + threadIdx.x; i < n_long; i += nblk * blockDim.x) {
         const uint64_t it = IT[lng[i]];
         const uint64_t bit = D[it_sid(it, pk)].bm_off + it_b(it, pk);
         atomicAnd(longbm + (bit >> 5), ~(1u << (bit & 31u)));
     }
     if (n_trig && !st->err) {
         const uint32_t lane = threadIdx.x & 63u;
-        for (uint32_t sid = blockIdx.x * 4u + (threadIdx.x >> 6); sid < nsk; sid += gridDim.x * 4u) {
+        for (uint32_t sid = bid * (uint32_t)NW + (threadIdx.x >> 6); sid < nsk; sid += nblk * (uint32_t)NW) {
             uint32_t c = n_trig;
             if (nsk > 1) {
                 // (the chunk may begin or end inside a sketch's part, or hold none of it)
@@ -1989,10 +2065,10 @@ __global__ __launch_bounds__(256) void k_finish(const uint32_t *__restrict__ lng
     }
     __shared__ uint32_t s_last;
     __syncthreads();
-    if (threadIdx.x == 0)
-        s_last = __hip_atomic_fetch_add(&st->done, 1u, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_AGENT);
+    if (threadIdx.x == 0) // (one block needs no count)
+        s_last = nblk > 1u ? __hip_atomic_fetch_add(&st->done, 1u, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_AGENT) : 0u;
     __syncthreads();
-    if (s_last != gridDim.x - 1u || threadIdx.x != 0)
+    if (s_last != nblk - 1u || threadIdx.x != 0)
         return;
     st->ord_segments += st->n_ord;
     st->long_segments += n_long;
@@ -2003,6 +2079,159 @@ __global__ __launch_bounds__(256) void k_finish(const uint32_t *__restrict__ lng
     st->done = 0;
     __hip_atomic_store(h_err, st->err, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
 }
+
+__global__ __launch_bounds__(256) void k_finish(const uint32_t *__restrict__ lng, const uint64_t *__restrict__ IT,
+                                                const qs_sdesc *__restrict__ D, qs_pack pk,
+                                                uint32_t *__restrict__ longbm, const uint32_t *__restrict__ tbit,
+                                                const uint32_t *__restrict__ tsum, uint32_t cn,
+                                                const uint64_t *__restrict__ offs, uint64_t base, uint32_t nsk,
+                                                uint32_t *__restrict__ next, qs_dev_state *__restrict__ st,
+                                                uint32_t *__restrict__ h_err)
+{
+    finish_pass<4>(blockIdx.x, gridDim.x, lng, IT, D, pk, longbm, tbit, tsum, cn, offs, base, nsk, next, st, h_err);
+}
+
+// ---------------------------------------------------------------------------
+// A short chunk of a single sketch: everything above in one block and one
+// launch.  The items are sorted in LDS (the same stable digit passes, a sixteenth of
+// the items per wavefront), and the passes run one after the other on them.  At
+// such lengths a chunk costs its launches and the gaps between them (1500 keys:
+// 12 launches, 49 us of GPU time; one block 26), not its work; 4096 keys take 41
+// us here and 49 the other way, which is why the line lies there.
+// ---------------------------------------------------------------------------
+#define SMALL_MAX 4096u
+#define SMALL_THREADS 1024u
+#define SMALL_WAVES 16
+#define SMALL_ROUNDS (SMALL_MAX / SMALL_THREADS)
+
+// Between two passes: what one wavefront wrote, the others read.  They share a
+// CU, so their plain stores need only be complete; the acquire drops the lines of
+// its first-level cache, since the atomics of a pass happen behind it.
+__device__ static inline void pass_fence()
+{
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
+}
+
+template <int KB>
+__global__ __launch_bounds__(SMALL_THREADS) void k_small(const KeyT<KB> *__restrict__ keys, uint32_t n, qs_sdesc d0,
+                                               const qs_sdesc *D, uint32_t *low, uint32_t *high,
+                                               const uint32_t *mask_pool, qs_pack pk, int dbits, int passes,
+                                               uint32_t *longbm, uint32_t *ord, uint32_t *lng, qs_trig *trig,
+                                               uint32_t trig_cap, uint32_t *tbit, uint32_t *tsum, uint32_t *tail_pool,
+                                               uint32_t *next, qs_dev_state *st, uint32_t *h_err)
+{
+    __shared__ uint64_t s_item[SMALL_MAX];
+    __shared__ uint32_t s_wh[SMALL_WAVES][OS_BINS], s_ls[OS_BINS], s_red[4];
+    __shared__ uint32_t s_masks[QS_MAX_MASKS];
+    const uint32_t t = threadIdx.x, lane = t & 63u, wv = t >> 6;
+    for (uint32_t i = t; i < d0.n_masks; i += SMALL_THREADS)
+        s_masks[i] = mask_pool[i];
+    for (uint32_t i = t; i < (n + 31u) / 32u; i += SMALL_THREADS)
+        tbit[i] = 0;
+    if (t == 0)
+        tsum[0] = 0;
+    const uint32_t rounds = (n + SMALL_THREADS - 1u) / SMALL_THREADS, wave0 = wv * rounds * 64u; // this wavefront's items
+    const uint64_t lt = (1ull << lane) - 1ull;
+    const uint32_t dmask = (1u << dbits) - 1u;
+    const sid_window win{nullptr, 0u, 0u};
+    uint64_t item[SMALL_ROUNDS];
+    uint32_t dr[SMALL_ROUNDS]; // digit | position within the wavefront's digit << 8
+#pragma unroll
+    for (uint32_t r = 0; r < SMALL_ROUNDS; ++r) {
+        const uint32_t i = wave0 + r * 64u + lane;
+        item[r] = r < rounds ? (uint64_t)keys[i < n ? i : n - 1u] : 0ull; // every load first
+    }
+#pragma unroll
+    for (uint32_t r = 0; r < SMALL_ROUNDS; ++r) {
+        const uint32_t i = wave0 + r * 64u + lane;
+        if (r < rounds && i < n)
+            item[r] = make_item<KB, false>((KeyT<KB>)item[r], i, 0, d0, D, nullptr, 1u, pk, win);
+    }
+    for (int ps = 0; ps < passes; ++ps) {
+        const int shift = dbits * ps;
+        for (uint32_t e = t; e < SMALL_WAVES * OS_BINS; e += SMALL_THREADS)
+            s_wh[e / OS_BINS][e % OS_BINS] = 0;
+        __syncthreads();
+#pragma unroll
+        for (uint32_t r = 0; r < SMALL_ROUNDS; ++r) {
+            if (r >= rounds) // uniform
+                break;
+            const bool valid = wave0 + r * 64u + lane < n;
+            const uint32_t d = (uint32_t)(it_cell(item[r], pk) >> shift) & dmask;
+            uint64_t m = __ballot(valid);
+#pragma unroll
+            for (int bit = 0; bit < 8; ++bit) {
+                if (bit < dbits) {
+                    const bool on = (d >> bit) & 1u;
+                    const uint64_t bb = __ballot(on);
+                    m &= on ? bb : ~bb;
+                }
+            }
+            const uint32_t rank = (uint32_t)__popcll(m & lt);
+            const int leader = valid ? (int)__builtin_ctzll(m) : 0;
+            uint32_t run = 0;
+            if (valid && rank == 0)
+                run = atomicAdd(&s_wh[wv][d], (uint32_t)__popcll(m));
+            run = (uint32_t)__shfl((int)run, leader, 64);
+            dr[r] = d | ((run + rank) << 8);
+        }
+        __syncthreads();
+        // thread d < OS_BINS: digit d's start and each wavefront's within it
+        uint32_t cnt = 0, x = 0;
+        if (t < OS_BINS) {
+#pragma unroll
+            for (int w = 0; w < SMALL_WAVES; ++w) {
+                const uint32_t c = s_wh[w][t];
+                s_wh[w][t] = cnt;
+                cnt += c;
+            }
+            x = cnt;
+#pragma unroll
+            for (int o = 1; o < 64; o <<= 1) {
+                const uint32_t y = (uint32_t)__shfl_up((int)x, o, 64);
+                x += lane >= (uint32_t)o ? y : 0u;
+            }
+            if (lane == 63u)
+                s_red[wv] = x;
+        }
+        __syncthreads();
+        if (t < OS_BINS) {
+            for (uint32_t w = 0; w < wv; ++w)
+                x += s_red[w];
+            s_ls[t] = x - cnt;
+        }
+        __syncthreads();
+#pragma unroll
+        for (uint32_t r = 0; r < SMALL_ROUNDS; ++r)
+            if (r < rounds && wave0 + r * 64u + lane < n)
+                s_item[s_ls[dr[r] & 0xffu] + s_wh[wv][dr[r] & 0xffu] + (dr[r] >> 8)] = item[r];
+        __syncthreads();
+        if (ps + 1 < passes)
+#pragma unroll
+            for (uint32_t r = 0; r < SMALL_ROUNDS; ++r) {
+                const uint32_t i = wave0 + r * 64u + lane;
+                if (r < rounds && i < n)
+                    item[r] = s_item[i];
+            }
+    }
+    seg_pass<false, SMALL_WAVES>(0u, 1u, s_item, n, D, s_masks, low, high, mask_pool, pk, longbm, ord, lng, st);
+    pass_fence();
+    const uint32_t n_ord = __hip_atomic_load(&st->n_ord, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if (n_ord) { // uniform
+        ordered_pass<SMALL_WAVES>(0u, 1u, s_item, n, ord, D, low, mask_pool, pk, longbm, lng, trig, trig_cap, tbit, tsum, nullptr, 0,
+                     d0.n_masks, s_masks, st);
+        pass_fence();
+        assign_pass<SMALL_WAVES>(0u, 1u, trig, trig_cap, tbit, tsum, n, nullptr, 0, D, 1u, low, high, tail_pool, next, st);
+        pass_fence();
+    }
+    tail_pass<false, uint64_t, SMALL_WAVES>(0u, 1u, s_item, n, D, s_masks, low, high, mask_pool, pk, longbm, tail_pool, next, lng, false,
+                               64u * TAIL_PF, st);
+    pass_fence();
+    finish_pass<SMALL_WAVES>(0u, 1u, lng, s_item, D, pk, longbm, tbit, tsum, n, nullptr, 0, 1u, next, st, h_err);
+}
+
 
 // ===========================================================================
 // host side
@@ -2238,6 +2467,16 @@ template <int KB, bool MULTI>
 static int insert_chunk(qs_sketch *s, const KeyT<KB> *keys, uint32_t cn, uint64_t base, const batch_ctx &bc,
                         hipStream_t stream)
 {
+    if (!MULTI && cn <= SMALL_MAX && !bc.timed) {
+        const qs_scratch &sc = *bc.sc;
+        const int bits = (int)s->pk.bb, passes = (bits + 7) / 8;
+        hipLaunchKernelGGL(k_small<KB>, dim3(1), dim3(SMALL_THREADS), 0, stream, keys, cn, s->h_desc[0], s->d_desc, s->d_low,
+                           s->d_high, s->d_masks, s->pk, (bits + passes - 1) / passes, passes, s->d_longbm, sc.ord,
+                           sc.lng, sc.trig, sc.trig_cap, sc.tbit, sc.tsum, s->d_tail_of, s->d_next, s->d_st,
+                           &s->h_st->err);
+        CK(hipGetLastError());
+        return QS_OK;
+    }
     int res = 0;
     int rc = sort_chunk<KB, MULTI>(s, keys, cn, base, bc, stream, res);
     if (rc)
