@@ -27,8 +27,8 @@
 //
 // Splits only grow, so a counter no add touched already holds its largest
 // split: after the call every counter is what update() leaves.  Inserts
-// shorter than SF_SORT_MIN skip the sort and go to k_sf_runs (runs of equal
-// adjacent keys, atomic adds that return the old value, an atomic max).
+// shorter than SF_SORT_MIN skip the sort and go to k_sf_tile (tiles of keys
+// counted in LDS, atomic adds that return the old value, an atomic max).
 // Long skewed calls of 4-byte keys first pass the hot-key filter of
 // qs_hot.hip (qs_hot_split_keys): the frequent keys are counted in LDS and
 // added once each by k_sf_hot_flush, and only the cold keys are sorted.
@@ -51,9 +51,11 @@
 
 #define SF_THREADS 256
 #define SF_WAVES (SF_THREADS / 64)
-#define SF_RUN_WAVES 8192u      // wavefronts of k_sf_runs (32 per CU)
-#define SF_ROW_RANGE 4096u     // keys per work item of k_sf_rows
+#define SF_ROW_WAVES 8192u      // wavefronts of k_sf_rows (32 per CU)
+#define SF_ROW_SPREAD 4096u     // work items that a short call is cut into
+#define SF_ROW_RANGE 4096u     // most keys per work item of k_sf_rows
 #define SF_SORT_MIN (1u << 16)  // shorter inserts are applied unsorted
+#define SF_TILE_SMALL_MAX (1u << 17) // up to here the unsorted tiles hold 512 keys, then 2048
 #define SF_CHUNK4 (1u << 28)    // keys per radix chunk: 4-byte keys
 #define SF_CHUNK8 (1u << 27)    //                       8-byte keys
 
@@ -313,64 +315,77 @@ __device__ static inline void sf_add(uint32_t *__restrict__ split, uint32_t *__r
     }
 }
 
-// Wavefront w takes keys [w * per_wave, (w + 1) * per_wave) and walks them
-// in steps of 64 (SF_RUN_PF steps loaded ahead).  In a step, a lane heads a
-// run when its key differs from its left neighbour's (lane 0 compares with
-// the carried run); a run that ends inside the step is flushed by its head,
-// the step's last run is carried on (wave-uniform key and length), and the
-// carried run is flushed when a step starts with another key and at the end.
+// Short inserts, unsorted: a block counts a tile of 256 * IPT keys in an LDS
+// table and adds each distinct key's count with sf_add, so that a frequent key
+// costs its counters one atomic per tile (20000 Zipf 1.1 keys: 149 us when
+// every run of equal neighbours was added by itself, now 44).  The all-ones
+// key is the table's empty marker and is counted apart.
 #define SF_RUN_PF 8
-template <int KB>
-__global__ __launch_bounds__(SF_THREADS) void k_sf_runs(const KeyT<KB> *__restrict__ keys, uint64_t n,
-                                                        uint64_t per_wave, sf_par p,
+template <int KB, int IPT>
+__global__ __launch_bounds__(SF_THREADS) void k_sf_tile(const KeyT<KB> *__restrict__ keys, uint64_t n, sf_par p,
                                                         const uint32_t *__restrict__ index,
                                                         uint32_t *__restrict__ split, uint32_t *__restrict__ search)
 {
-    const uint32_t lane = threadIdx.x & 63u;
-    const uint64_t wave = (uint64_t)blockIdx.x * SF_WAVES + (threadIdx.x >> 6);
-    const uint64_t r0 = wave * per_wave;
-    if (r0 >= n)
-        return;
-    const uint64_t r1 = r0 + per_wave < n ? r0 + per_wave : n;
-    KeyT<KB> ck = 0;  // carried run: key and length (0: none)
-    uint32_t cc = 0;
-    for (uint64_t g0 = r0; g0 < r1; g0 += 64u * SF_RUN_PF) {
-        KeyT<KB> kk[SF_RUN_PF];
+    constexpr uint32_t TILE = SF_THREADS * IPT, SLOTS = 2u * TILE; // at most half full
+    constexpr KeyT<KB> EMPTY = ~(KeyT<KB>)0;
+    __shared__ KeyT<KB> s_key[SLOTS];
+    __shared__ uint32_t s_cnt[SLOTS + 1u]; // the last one: the all-ones key's
+    const uint32_t t = threadIdx.x, lane = t & 63u;
+    const uint64_t tb = (uint64_t)blockIdx.x * TILE;
+    KeyT<KB> kk[IPT];
 #pragma unroll
-        for (int s = 0; s < SF_RUN_PF; ++s) { // every load first, from clamped positions
-            const uint64_t i = g0 + (uint64_t)s * 64u + lane;
-            kk[s] = __builtin_nontemporal_load(keys + (i < r1 ? i : r1 - 1u));
+    for (int r = 0; r < IPT; ++r) { // every load first, from clamped positions
+        const uint64_t i = tb + (uint64_t)r * SF_THREADS + t;
+        kk[r] = keys[i < n ? i : n - 1u];
+    }
+    for (uint32_t e = t; e < SLOTS; e += SF_THREADS) {
+        s_key[e] = EMPTY;
+        s_cnt[e] = 0;
+    }
+    if (t == 0)
+        s_cnt[SLOTS] = 0;
+    __syncthreads();
+#pragma unroll
+    for (int r = 0; r < IPT; ++r) {
+        const KeyT<KB> k = kk[r];
+        // the lanes with the first lane's key are added by that lane (a hot
+        // key would serialise them on one LDS word)
+        uint32_t w = tb + (uint64_t)r * SF_THREADS + t < n ? 1u : 0u;
+        const uint64_t act = __ballot(w != 0u);
+        if (act == 0)
+            continue;
+        const uint32_t first = (uint32_t)__builtin_ctzll(act);
+        const uint64_t same = __ballot(k == __shfl(k, (int)first, 64)) & act;
+        if ((same >> lane) & 1ull)
+            w = lane == first ? (uint32_t)__popcll(same) : 0u;
+        if (!w)
+            continue;
+        if (k == EMPTY) {
+            atomicAdd(&s_cnt[SLOTS], w);
+            continue;
         }
-#pragma unroll
-        for (int s = 0; s < SF_RUN_PF; ++s) {
-            const uint64_t s0 = g0 + (uint64_t)s * 64u;
-            if (s0 >= r1) // uniform
-                break;
-            const uint32_t nv = (uint32_t)(r1 - s0 < 64u ? r1 - s0 : 64u); // valid lanes: a prefix
-            const KeyT<KB> k = kk[s];
-            const KeyT<KB> left = __shfl_up(k, 1, 64);
-            const bool valid = lane < nv;
-            const bool head = valid && (lane == 0 ? !(cc && k == ck) : k != left);
-            const uint64_t H = __ballot(head);
-            if (head) {
-                const uint64_t later = H & ~((2ull << lane) - 1ull);
-                if (later) // the run ends inside this step
-                    sf_add<KB>(split, search, p, index, (uint64_t)k, (uint32_t)__builtin_ctzll(later) - lane);
+        uint32_t sl = (uint32_t)(((uint64_t)k * 0x9E3779B97F4A7C15ull) >> 40) & (SLOTS - 1u);
+        for (;; sl = (sl + 1u) & (SLOTS - 1u)) { // ends: half of the slots stay empty
+            KeyT<KB> cur = s_key[sl];
+            if (cur == EMPTY) {
+                if (KB == 4)
+                    cur = (KeyT<KB>)atomicCAS((unsigned int *)&s_key[sl], (unsigned int)EMPTY, (unsigned int)k);
+                else
+                    cur = (KeyT<KB>)atomicCAS((unsigned long long *)&s_key[sl], (unsigned long long)EMPTY,
+                                              (unsigned long long)k);
             }
-            if (H == 0) { // the whole step continues the carried run
-                cc += nv;
-            } else {
-                const uint32_t h0 = (uint32_t)__builtin_ctzll(H);
-                if (cc && lane == 0) // the carried run ends before the first head
-                    sf_add<KB>(split, search, p, index, (uint64_t)ck, cc + h0);
-                const uint32_t hl = 63u - (uint32_t)__builtin_clzll(H); // the step's last run
-                ck = __shfl(k, (int)hl, 64);
-                cc = nv - hl;
+            if (cur == EMPTY || cur == k) {
+                atomicAdd(&s_cnt[sl], w);
+                break;
             }
         }
     }
-    if (cc && lane == 0)
-        sf_add<KB>(split, search, p, index, (uint64_t)ck, cc);
+    __syncthreads();
+    for (uint32_t e = t; e < SLOTS; e += SF_THREADS)
+        if (s_cnt[e])
+            sf_add<KB>(split, search, p, index, (uint64_t)s_key[e], s_cnt[e]);
+    if (t == 0 && s_cnt[SLOTS])
+        sf_add<KB>(split, search, p, index, (uint64_t)EMPTY, s_cnt[SLOTS]);
 }
 
 // G = m / 4 lanes per key, one 16-byte quarter (m = 16), half (m = 8) or
@@ -517,8 +532,8 @@ __global__ __launch_bounds__(256) void k_sf_fix(const uint32_t *__restrict__ lis
 }
 
 // Keys sorted by bucket, cut into ranges of `range` keys that persistent
-// wavefronts take from the counter *work (zero at launch) and walk in steps
-// of 64.  Each bucket's keys are one run of the sorted keys, so a bucket that
+// wavefronts take (the first by their number, then from the counter *work,
+// zero at launch) and walk in steps of 64.  Each bucket's keys are one run of the sorted keys, so a bucket that
 // lies inside one range belongs to that range's wavefront alone; only the
 // range's first and last bucket can be shared with the neighbouring ranges:
 // those are added with atomics (sf_add_shared) and listed in shared[2 * range
@@ -548,13 +563,11 @@ __global__ __launch_bounds__(SF_THREADS) void k_sf_rows(const KeyT<KB> *__restri
     __syncthreads();
     const uint32_t lane = threadIdx.x & 63u, wv = threadIdx.x >> 6;
     const uint64_t nranges = (n + range - 1) / range;
-    for (;;) {
-        uint32_t rr = 0;
-        if (lane == 0)
-            rr = atomicAdd(work, 1u);
-        rr = (uint32_t)__shfl((int)rr, 0, 64);
-        if (rr >= nranges) // every wavefront leaves once the ranges are taken
-            break;
+    // The first range is the wavefront's own number, later ones come from the
+    // counter (an atomic per wavefront on that one word serialises: 8192 of
+    // them at the start, and again at the end, took 90 us each time).
+    const uint32_t nwaves = gridDim.x * SF_WAVES;
+    for (uint32_t rr = blockIdx.x * SF_WAVES + wv; rr < nranges;) { // every wavefront leaves once the ranges are taken
         const uint64_t r0 = (uint64_t)rr * range;
         const uint64_t r1 = r0 + range < n ? r0 + range : n;
         const uint32_t bfirst = sf_idx<KB>::bucket((uint64_t)keys[r0], p);
@@ -663,6 +676,12 @@ __global__ __launch_bounds__(SF_THREADS) void k_sf_rows(const KeyT<KB> *__restri
         }
         if (carry && lane == co)
             finish();
+        if (nranges <= nwaves) // all taken
+            break;
+        uint32_t nr = 0;
+        if (lane == 0)
+            nr = atomicAdd(work, 1u);
+        rr = nwaves + (uint32_t)__shfl((int)nr, 0, 64);
     }
 }
 
@@ -827,6 +846,24 @@ static uint32_t sf_grid(uint64_t want)
     return (uint32_t)(want < 1 ? 1 : (want > 8192 ? 8192 : want));
 }
 
+// Keys per work item of k_sf_rows.  A wavefront walks its range one 64-key step
+// after the other, so short calls take short ranges that occupy the chip; long
+// ones take the longest (each range's first and last bucket are shared, and
+// cost atomics).  Ranges of 4096 keys whatever the call took 290 us for 65536
+// keys (16 wavefronts), now 90.
+static uint64_t sf_range(uint64_t n)
+{
+    const uint64_t r = (n / SF_ROW_SPREAD + 63) / 64 * 64;
+    return r < 64 ? 64 : r < SF_ROW_RANGE ? r : SF_ROW_RANGE;
+}
+
+// most ranges of any call of at most n keys
+static uint64_t sf_max_ranges(uint64_t n)
+{
+    const uint64_t a = (n + SF_ROW_RANGE - 1) / SF_ROW_RANGE, b = (n + 63) / 64;
+    return a > SF_ROW_WAVES ? a : b < SF_ROW_WAVES ? b : SF_ROW_WAVES;
+}
+
 // radix scratch for chunks of up to `keys` keys (kept across calls)
 static int sf_ensure_scratch(qs_sf *s, uint64_t keys)
 {
@@ -847,7 +884,7 @@ static int sf_ensure_scratch(qs_sf *s, uint64_t keys)
     if (hipMalloc(&s->d_buf[0], keys * s->key_bytes) != hipSuccess ||
         hipMalloc(&s->d_buf[1], keys * s->key_bytes) != hipSuccess ||
         hipMalloc(&s->d_hist, 4ull * 256 * (ntiles + 1)) != hipSuccess ||
-        hipMalloc(&s->d_shared, 8ull * ((keys + SF_ROW_RANGE - 1) / SF_ROW_RANGE)) != hipSuccess)
+        hipMalloc(&s->d_shared, 8ull * sf_max_ranges(keys)) != hipSuccess)
         return QS_ERR_NOMEM;
     if (!s->d_err) {
         if (hipMalloc(&s->d_err, 8) != hipSuccess)
@@ -858,22 +895,19 @@ static int sf_ensure_scratch(qs_sf *s, uint64_t keys)
     return QS_OK;
 }
 
-// k_sf_runs (owned = false: any order, all atomics) or k_sf_rows (owned =
+// k_sf_tile (owned = false: any order, all atomics) or k_sf_rows (owned =
 // true: keys sorted by bucket)
 template <int KB>
 static void sf_launch_flush(qs_sf *s, const sf_par &p, const KeyT<KB> *keys, uint64_t n, bool owned)
 {
-    const uint64_t steps = (n + 63) / 64;
-    const uint64_t per_wave = (steps + SF_RUN_WAVES - 1) / SF_RUN_WAVES * 64; // whole steps
-    const uint64_t waves = (n + per_wave - 1) / per_wave;
-    const dim3 grid((uint32_t)((waves + SF_WAVES - 1) / SF_WAVES)), block(SF_THREADS);
+    const dim3 block(SF_THREADS);
     if (owned) {
-        const uint64_t ranges = (n + SF_ROW_RANGE - 1) / SF_ROW_RANGE;
-        const uint64_t w = ranges < SF_RUN_WAVES ? ranges : SF_RUN_WAVES;
+        const uint64_t range = sf_range(n), ranges = (n + range - 1) / range;
+        const uint64_t w = ranges < SF_ROW_WAVES ? ranges : SF_ROW_WAVES;
         (void)hipMemsetAsync(s->d_err + 1, 0, 4, 0);
         const dim3 g((uint32_t)((w + SF_WAVES - 1) / SF_WAVES));
 #define SF_ROWS(T)                                                                                               \
-    hipLaunchKernelGGL((k_sf_rows<KB, T>), g, block, 0, 0, keys, n, (uint64_t)SF_ROW_RANGE, p, s->d_index,       \
+    hipLaunchKernelGGL((k_sf_rows<KB, T>), g, block, 0, 0, keys, n, range, p, s->d_index,                        \
                        s->d_split, s->d_search, s->d_err + 1, s->d_shared)
         switch (s->times) {
         case 1: SF_ROWS(1); break;
@@ -886,9 +920,13 @@ static void sf_launch_flush(qs_sf *s, const sf_par &p, const KeyT<KB> *keys, uin
         const uint32_t listed = (uint32_t)(2 * ranges);
         hipLaunchKernelGGL(k_sf_fix, dim3((listed + 255) / 256), dim3(256), 0, 0, s->d_shared, listed, p, s->d_split,
                            s->d_search);
-    } else
-        hipLaunchKernelGGL(k_sf_runs<KB>, grid, block, 0, 0, keys, n, per_wave, p, s->d_index, s->d_split,
-                           s->d_search);
+    } else if (n <= SF_TILE_SMALL_MAX) {
+        hipLaunchKernelGGL((k_sf_tile<KB, 2>), dim3((uint32_t)((n + 2 * SF_THREADS - 1) / (2 * SF_THREADS))), block, 0, 0,
+                           keys, n, p, s->d_index, s->d_split, s->d_search);
+    } else {
+        hipLaunchKernelGGL((k_sf_tile<KB, 8>), dim3((uint32_t)((n + 8 * SF_THREADS - 1) / (8 * SF_THREADS))), block, 0, 0,
+                           keys, n, p, s->d_index, s->d_split, s->d_search);
+    }
 }
 
 // one chunk: sort by bucket (8-bit digits at most), then flush
