@@ -11,7 +11,7 @@
 //   2. the first HOT_PREFIX keys through the ordinary pipeline (qs_insert.hip),
 //      which links the buckets of the hot keys;
 //   3. the hot set: the candidates whose bucket is linked now, in a table of
-//      HOT_BUCKETS buckets of 4 slots where each key may sit in one of two
+//      HOT_BUCKETS buckets of 2 slots where each key may sit in one of two
 //      buckets (the emptier one when it is placed), so that a lookup is two
 //      16-byte reads and no loop; a key that finds both buckets full is left
 //      out of the set (it then takes the ordered path, which is always exact);
@@ -46,8 +46,9 @@
 #define HOT_CAND_MAX (HOT_SAMPLE / HOT_MIN_RUN)
 static_assert(HOT_CAND_MAX % 1024u == 0, "blocks of k_samp_select");
 #define HOT_MAX 8192u                      // hot keys at most
-#define HOT_BUCKETS 4096u                  // buckets of 4 slots (load at most 1/2)
-#define HOT_SLOTS (HOT_BUCKETS * 4u)
+#define HOT_BUCKETS 8192u                  // buckets of 2 slots (load at most 1/2)
+#define HOT_SLOTS (HOT_BUCKETS * 2u)
+#define HOT_FIRST_RUN 64u                  // candidates this frequent are placed before the others
 #define HOT_EMPTY 0xffffffffu              // empty slot (that key is never hot)
 #define HOT_THREADS 1024
 #define HOT_IPT 16u                        // rows of 64 keys per chunk
@@ -70,7 +71,7 @@ struct qs_hot {
     uint32_t *scnt;            // its keys per tile and bin, then the bins' starts
     uint32_t *ccount;          // histogram of the counts of its frequent keys
     uint32_t *ck, *cv;         // those keys and their counts
-    uint32_t *cand;            // the candidates
+    uint32_t *cand, *ccnt;     // the candidates and their counts
     uint32_t *ctl;             // HC_* words
     uint32_t *h_ctl;           // pinned copy
     uint32_t *tkey;            // hot table: key per slot
@@ -128,12 +129,14 @@ static int hot_read(qs_hot *h, const uint32_t *d_src, uint32_t nwords, hipStream
     return QS_OK;
 }
 
-// the two buckets a key may sit in (distinct)
+// The two buckets a key may sit in (now and then the same one): two fields of
+// one 24-bit product, a full-rate instruction where a 32-bit product takes four
+// times as long.
 __device__ static inline void hot_buckets(uint32_t key, uint32_t &b1, uint32_t &b2)
 {
-    b1 = (key * 0x9E3779B1u) >> 20; // HOT_BUCKETS = 2^12
-    b2 = (key * 0x85EBCA77u) >> 20;
-    b2 = b2 == b1 ? b1 ^ 1u : b2;
+    const uint32_t h = __umul24(key ^ (key >> 15), 0x9E3779u);
+    b1 = h >> 19; // HOT_BUCKETS = 2^13
+    b2 = (h >> 6) & (HOT_BUCKETS - 1u);
 }
 
 // ---------------------------------------------------------------------------
@@ -332,7 +335,7 @@ __global__ __launch_bounds__(1024) void k_samp_count(const uint32_t *__restrict_
 // they cover to the control words.
 __global__ __launch_bounds__(1024) void k_samp_select(const uint32_t *__restrict__ ck, const uint32_t *__restrict__ cv,
                                                       const uint32_t *__restrict__ ccount, uint32_t *__restrict__ cand,
-                                                      uint32_t *__restrict__ ctl)
+                                                      uint32_t *__restrict__ ccnt, uint32_t *__restrict__ ctl)
 {
     __shared__ uint32_t s_w[16], s_least, s_room, s_take, s_base, s_cover;
     const uint32_t n = ctl[HC_FOUND];
@@ -391,8 +394,10 @@ __global__ __launch_bounds__(1024) void k_samp_select(const uint32_t *__restrict
         atomicAdd(ctl + HC_COVER, s_cover);
     }
     __syncthreads();
-    if (take && s_base + at < HOT_MAX)
+    if (take && s_base + at < HOT_MAX) {
         cand[s_base + at] = ck[i];
+        ccnt[s_base + at] = c;
+    }
 }
 
 __global__ void k_hot_clear(uint32_t *__restrict__ tkey, uint32_t *__restrict__ tfill, uint32_t *__restrict__ ctl)
@@ -406,8 +411,12 @@ __global__ void k_hot_clear(uint32_t *__restrict__ tkey, uint32_t *__restrict__ 
         ctl[HC_NHOT] = 0;
 }
 
-// the candidates whose bucket is linked now enter the hot table
-__global__ void k_hot_build(const uint32_t *__restrict__ cand, qs_sdesc d0, const uint32_t *__restrict__ low,
+// The candidates whose bucket is linked now enter the hot table, those that the
+// sample holds at least lo and fewer than hi times (a key that finds both its
+// buckets full stays out, so the most frequent go first: with 8192 keys
+// about 1 % of the last placed do).
+__global__ void k_hot_build(const uint32_t *__restrict__ cand, const uint32_t *__restrict__ ccnt, uint32_t lo,
+                            uint32_t hi, qs_sdesc d0, const uint32_t *__restrict__ low,
                             const uint32_t *__restrict__ masks, uint32_t *__restrict__ tkey,
                             uint32_t *__restrict__ tinfo, uint32_t *__restrict__ tmask, uint32_t *tfill,
                             uint32_t *ctl)
@@ -416,7 +425,7 @@ __global__ void k_hot_build(const uint32_t *__restrict__ cand, qs_sdesc d0, cons
     if (c >= min(ctl[HC_NCAND], HOT_MAX))
         return;
     const uint32_t k = cand[c];
-    if (k == HOT_EMPTY)
+    if (k == HOT_EMPTY || ccnt[c] < lo || ccnt[c] >= hi)
         return;
     const uint32_t h = k * d0.seed;
     const uint32_t b = qs_fastmod(h, d0.fd_low);
@@ -434,13 +443,13 @@ __global__ void k_hot_build(const uint32_t *__restrict__ cand, qs_sdesc d0, cons
         b2 = t;
     }
     uint32_t pos = atomicAdd(tfill + b1, 1u), hb = b1;
-    if (pos >= 4u) {
+    if (pos >= 2u) {
         pos = atomicAdd(tfill + b2, 1u);
         hb = b2;
     }
-    if (pos >= 4u)
+    if (pos >= 2u)
         return; // both full: the key stays on the ordered path
-    const uint32_t slot = hb * 4u + pos;
+    const uint32_t slot = hb * 2u + pos;
     tkey[slot] = k;
     tinfo[slot] = w;
     tmask[slot] = M;
@@ -448,14 +457,14 @@ __global__ void k_hot_build(const uint32_t *__restrict__ cand, qs_sdesc d0, cons
 }
 
 // every candidate enters the hot table (a sink whose inserts all commute)
-__global__ void k_hot_build_any(const uint32_t *__restrict__ cand, uint32_t *__restrict__ tkey, uint32_t *tfill,
-                                uint32_t *ctl)
+__global__ void k_hot_build_any(const uint32_t *__restrict__ cand, const uint32_t *__restrict__ ccnt, uint32_t lo,
+                                uint32_t hi, uint32_t *__restrict__ tkey, uint32_t *tfill, uint32_t *ctl)
 {
     const uint32_t c = blockIdx.x * blockDim.x + threadIdx.x;
     if (c >= min(ctl[HC_NCAND], HOT_MAX))
         return;
     const uint32_t k = cand[c];
-    if (k == HOT_EMPTY)
+    if (k == HOT_EMPTY || ccnt[c] < lo || ccnt[c] >= hi)
         return;
     uint32_t b1, b2;
     hot_buckets(k, b1, b2);
@@ -466,32 +475,28 @@ __global__ void k_hot_build_any(const uint32_t *__restrict__ cand, uint32_t *__r
         b2 = t;
     }
     uint32_t pos = atomicAdd(tfill + b1, 1u), hb = b1;
-    if (pos >= 4u) {
+    if (pos >= 2u) {
         pos = atomicAdd(tfill + b2, 1u);
         hb = b2;
     }
-    if (pos >= 4u)
+    if (pos >= 2u)
         return; // both full: the key stays cold
-    tkey[hb * 4u + pos] = k;
+    tkey[hb * 2u + pos] = k;
     atomicAdd(ctl + HC_NHOT, 1u);
 }
 
 // slot of key k in the LDS copy of the hot table, or -1: both buckets read
 // at once, no loop (the empty marker is never looked up: it is never hot)
-__device__ static inline int hot_find(const uint4 *skey4, uint32_t k)
+__device__ static inline int hot_find(const uint2 *skey2, uint32_t k)
 {
     uint32_t b1, b2;
     hot_buckets(k, b1, b2);
-    const uint4 p = skey4[b1], q = skey4[b2];
+    const uint2 p = skey2[b1], q = skey2[b2];
     int s = -1;
-    s = p.x == k ? (int)(b1 * 4u + 0u) : s;
-    s = p.y == k ? (int)(b1 * 4u + 1u) : s;
-    s = p.z == k ? (int)(b1 * 4u + 2u) : s;
-    s = p.w == k ? (int)(b1 * 4u + 3u) : s;
-    s = q.x == k ? (int)(b2 * 4u + 0u) : s;
-    s = q.y == k ? (int)(b2 * 4u + 1u) : s;
-    s = q.z == k ? (int)(b2 * 4u + 2u) : s;
-    s = q.w == k ? (int)(b2 * 4u + 3u) : s;
+    s = p.x == k ? (int)(b1 * 2u) : s;
+    s = p.y == k ? (int)(b1 * 2u + 1u) : s;
+    s = q.x == k ? (int)(b2 * 2u) : s;
+    s = q.y == k ? (int)(b2 * 2u + 1u) : s;
     return k == HOT_EMPTY ? -1 : s;
 }
 
@@ -502,48 +507,59 @@ __device__ static inline int hot_find(const uint4 *skey4, uint32_t k)
 // HOT_CHUNK slots of `stage`, and their number to ccold.  Persistent blocks
 // (one per CU: the two LDS arrays take 128 KB) take chunks in turn and write
 // their row of per-slot counts at the end.
+// Bound by VALU issue (55 instructions per 64 keys kept it 80 % busy) and LDS
+// conflicts (the two 16-byte reads of a table with 4-slot buckets): buckets of two
+// slots, the cheaper hash and addresses from scalar bases took 252 M keys of a
+// 2^28-key Zipf 1.1 call from 435 us to 321.
 __global__ __launch_bounds__(HOT_THREADS) void k_hot_count(const uint32_t *__restrict__ keys, uint64_t n,
                                                            uint32_t nchunks, const uint32_t *__restrict__ tkey,
                                                            uint32_t *__restrict__ part,
                                                            uint32_t *__restrict__ stage,
                                                            uint32_t *__restrict__ ccold)
 {
-    __shared__ uint4 skey4[HOT_BUCKETS];
+    __shared__ uint2 skey2[HOT_BUCKETS];
     __shared__ uint32_t scnt[HOT_SLOTS];
     for (uint32_t e = threadIdx.x; e < HOT_BUCKETS; e += HOT_THREADS)
-        skey4[e] = reinterpret_cast<const uint4 *>(tkey)[e];
+        skey2[e] = reinterpret_cast<const uint2 *>(tkey)[e];
     for (uint32_t e = threadIdx.x; e < HOT_SLOTS; e += HOT_THREADS)
         scnt[e] = 0;
     __syncthreads();
     const uint32_t lane = threadIdx.x & 63u;
-    const uint64_t below = (1ull << lane) - 1ull;
     const uint32_t nw = gridDim.x * (HOT_THREADS / 64);
-    uint32_t c = blockIdx.x * (HOT_THREADS / 64) + (threadIdx.x >> 6);
+    // the chunk number and what follows from it stay in scalar registers
+    uint32_t c = (uint32_t)__builtin_amdgcn_readfirstlane((int)(blockIdx.x * (HOT_THREADS / 64) + (threadIdx.x >> 6)));
     uint32_t k[HOT_IPT], kn[HOT_IPT];
+    auto load = [&](uint32_t ch, uint32_t *v) {
+        const uint64_t base = (uint64_t)ch * HOT_CHUNK;
+        const uint32_t *src = keys + base;
+        if (ch < nchunks && base + HOT_CHUNK <= n) { // uniform: a whole chunk
 #pragma unroll
-    for (uint32_t r = 0; r < HOT_IPT; ++r) {
-        const uint64_t i = (uint64_t)c * HOT_CHUNK + r * 64u + lane;
-        k[r] = c < nchunks && i < n ? __builtin_nontemporal_load(keys + i) : HOT_EMPTY;
-    }
-    for (; c < nchunks; c += nw) {
-        const uint32_t cn = c + nw; // the next chunk, loaded while this one is probed
+            for (uint32_t r = 0; r < HOT_IPT; ++r)
+                v[r] = __builtin_nontemporal_load(src + (r * 64u + lane));
+        } else {
+            const uint32_t left = ch < nchunks ? (uint32_t)(n - base) : 0u;
 #pragma unroll
-        for (uint32_t r = 0; r < HOT_IPT; ++r) {
-            const uint64_t i = (uint64_t)cn * HOT_CHUNK + r * 64u + lane;
-            kn[r] = cn < nchunks && i < n ? __builtin_nontemporal_load(keys + i) : HOT_EMPTY;
+            for (uint32_t r = 0; r < HOT_IPT; ++r)
+                v[r] = r * 64u + lane < left ? __builtin_nontemporal_load(src + (r * 64u + lane)) : HOT_EMPTY;
         }
+    };
+    load(c, k);
+    for (; c < nchunks; c += nw) {
+        load(c + nw, kn); // the next chunk, loaded while this one is probed
+        const uint64_t base = (uint64_t)c * HOT_CHUNK;
+        const uint32_t left = n - base < HOT_CHUNK ? (uint32_t)(n - base) : HOT_CHUNK; // keys of this chunk
         uint32_t cold = 0;
-        uint32_t *dst = stage + (size_t)c * HOT_CHUNK;
+        uint32_t *dst = stage + base;
 #pragma unroll
         for (uint32_t r = 0; r < HOT_IPT; ++r) {
-            const uint64_t i = (uint64_t)c * HOT_CHUNK + r * 64u + lane;
-            const int s = hot_find(skey4, k[r]); // the key past the end is HOT_EMPTY: -1
+            const int s = hot_find(skey2, k[r]); // the key past the end is HOT_EMPTY: -1
             if (s >= 0)
                 atomicAdd(&scnt[s], 1u);
-            const bool is_cold = (i < n) & (s < 0);
+            const bool is_cold = (r * 64u + lane < left) & (s < 0);
             const uint64_t m = __ballot(is_cold); // every lane, outside any branch
             if (is_cold)
-                dst[cold + (uint32_t)__popcll(m & below)] = k[r];
+                dst[cold + __builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0u))] =
+                    k[r];
             cold += (uint32_t)__popcll(m);
         }
         if (lane == 0)
@@ -761,7 +777,8 @@ static int hot_alloc(void **state, uint64_t rest)
             hipDeviceGetAttribute(&cu, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cu <= 0)
             cu = 256;
         h->nblk = (uint32_t)cu;
-        const uint64_t words = HOT_SAMPLE + (SAMP_TILES + 2u) * SAMP_BINS + SAMP_COUNTS + 2ull * HOT_CAND_MAX + HOT_MAX;
+        const uint64_t words = HOT_SAMPLE + (SAMP_TILES + 2u) * SAMP_BINS + SAMP_COUNTS + 2ull * HOT_CAND_MAX +
+                               2ull * HOT_MAX;
         bool ok = hipMalloc(&h->samp, 4ull * words) == hipSuccess &&
              hipMalloc(&h->ctl, 4ull * HC_WORDS) == hipSuccess &&
              hipMalloc(&h->tkey, 4ull * HOT_SLOTS) == hipSuccess &&
@@ -779,6 +796,7 @@ static int hot_alloc(void **state, uint64_t rest)
             h->ck = h->ccount + SAMP_COUNTS;
             h->cv = h->ck + HOT_CAND_MAX;
             h->cand = h->cv + HOT_CAND_MAX;
+            h->ccnt = h->cand + HOT_MAX;
             memset(h->h_ctl, 0, 4ull * HOT_PUB_WORDS);
             h->seq = 0;
         }
@@ -821,7 +839,7 @@ static int hot_cand_launch(qs_hot *h, const uint32_t *keys, hipStream_t stream)
     hipLaunchKernelGGL(k_samp_count, dim3(SAMP_BINS), dim3(1024), 0, stream, h->samp, start, h->ck, h->cv, h->ccount,
                        h->ctl);
     hipLaunchKernelGGL(k_samp_select, dim3(HOT_CAND_MAX / 1024u), dim3(1024), 0, stream, h->ck, h->cv, h->ccount,
-                       h->cand, h->ctl);
+                       h->cand, h->ccnt, h->ctl);
     CK(hipGetLastError());
     return QS_OK;
 }
@@ -932,16 +950,16 @@ int qs_insert_hot(qs_sketch *s, const void *d_keys, uint64_t n, hipStream_t stre
             return rc;
         CK(hipEventRecord(h->ev_cand, stream)); // (the wait below is then already met)
     }
-    const uint32_t *cand = h->cand;
-
     // 3. the hot set, 4. the filter
     const uint32_t nchunks = (uint32_t)((rest + HOT_CHUNK - 1) / HOT_CHUNK);
     if (timed)
         qs_tim_begin(s, e1, QS_TK_HOT, 0, stream); // a wait for the candidates counts here
     CK(hipStreamWaitEvent(stream, h->ev_cand, 0));
     hipLaunchKernelGGL(k_hot_clear, dim3(HOT_SLOTS / 256), dim3(256), 0, stream, h->tkey, h->tfill, h->ctl);
-    hipLaunchKernelGGL(k_hot_build, dim3(HOT_MAX / 256), dim3(256), 0, stream, cand, d0, s->d_low, s->d_masks,
-                       h->tkey, h->tinfo, h->tmask, h->tfill, h->ctl);
+    for (int first = 1; first >= 0; --first)
+        hipLaunchKernelGGL(k_hot_build, dim3(HOT_MAX / 256), dim3(256), 0, stream, h->cand, h->ccnt,
+                           first ? HOT_FIRST_RUN : 0u, first ? ~0u : HOT_FIRST_RUN, d0, s->d_low, s->d_masks, h->tkey,
+                           h->tinfo, h->tmask, h->tfill, h->ctl);
     hipLaunchKernelGGL(k_hot_count, dim3(h->nblk), dim3(HOT_THREADS), 0, stream, keys + HOT_PREFIX, rest,
                        nchunks, h->tkey, h->part, h->stage, h->ccold);
     qs_scan_u32(h->ccold, nchunks, h->bsum, stream);
@@ -997,10 +1015,11 @@ int qs_hot_split_keys(void **state, const uint32_t *keys, uint64_t n, hipStream_
     rc = hot_cand_result(h, stream, &skewed);
     if (rc || !skewed)
         return rc;
-    const uint32_t *cand = h->cand;
     const uint32_t nchunks = (uint32_t)((n + HOT_CHUNK - 1) / HOT_CHUNK);
     hipLaunchKernelGGL(k_hot_clear, dim3(HOT_SLOTS / 256), dim3(256), 0, stream, h->tkey, h->tfill, h->ctl);
-    hipLaunchKernelGGL(k_hot_build_any, dim3(HOT_MAX / 256), dim3(256), 0, stream, cand, h->tkey, h->tfill, h->ctl);
+    for (int first = 1; first >= 0; --first)
+        hipLaunchKernelGGL(k_hot_build_any, dim3(HOT_MAX / 256), dim3(256), 0, stream, h->cand, h->ccnt,
+                           first ? HOT_FIRST_RUN : 0u, first ? ~0u : HOT_FIRST_RUN, h->tkey, h->tfill, h->ctl);
     hipLaunchKernelGGL(k_hot_count, dim3(h->nblk), dim3(HOT_THREADS), 0, stream, keys, n, nchunks, h->tkey, h->part,
                        h->stage, h->ccold);
     qs_scan_u32(h->ccold, nchunks, h->bsum, stream);
