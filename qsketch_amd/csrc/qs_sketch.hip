@@ -248,12 +248,14 @@ __device__ static inline uint32_t query_sid(const uint64_t *__restrict__ offs, u
     return lo;
 }
 
-// Answers key i: two lanes, one 16-byte half of the bucket each.
+// Answers a key: two lanes, one 16-byte half of the bucket each.  NT: the bucket
+// is read with a non-temporal load (query_launch says when).
+template <bool NT>
 __device__ static inline void query_bucket(uint32_t M, uint32_t b, const uint32_t *__restrict__ low,
                                            const uint32_t *__restrict__ high, uint32_t half, uint32_t *out)
 {
-    // read once: a non-temporal load (measured 0.433 -> 0.405 ms for 16.6 M keys)
-    const u32x4 vv = __builtin_nontemporal_load(reinterpret_cast<const u32x4 *>(low + (size_t)b * 8u) + half);
+    const u32x4 *src = reinterpret_cast<const u32x4 *>(low + (size_t)b * 8u) + half;
+    const u32x4 vv = NT ? __builtin_nontemporal_load(src) : *src;
     const uint4 v = make_uint4(vv[0], vv[1], vv[2], vv[3]);
     const uint32_t Mh = half ? (M >> 16) : (M & 0xffffu);
     uint32_t lo = 0xffffffffu;
@@ -292,7 +294,7 @@ __device__ static inline void query_bucket(uint32_t M, uint32_t b, const uint32_
 // 512 sketches: 770 us with a search in the global offsets, a descriptor load and a
 // mask load per key; 609 without them but with one long range per block (every
 // sketch at once); now 553.
-template <int KB, bool MULTI>
+template <int KB, bool MULTI, bool NT>
 __global__ __launch_bounds__(INS_THREADS) void k_query(const KeyT<KB> *__restrict__ keys, uint32_t n, qs_sdesc d0,
                                                        const qs_sdesc *__restrict__ D,
                                                        const uint64_t *__restrict__ offs, uint32_t nsk,
@@ -308,9 +310,12 @@ __global__ __launch_bounds__(INS_THREADS) void k_query(const KeyT<KB> *__restric
             s_masks[i] = mask_pool[i];
         __syncthreads();
         const uint64_t stride = (uint64_t)gridDim.x * (INS_THREADS / 2);
-        for (uint64_t i = (uint64_t)blockIdx.x * (INS_THREADS / 2) + (threadIdx.x >> 1); i < n; i += stride) {
-            const KeyT<KB> key = keys[i];
-            query_bucket(s_masks[qs_maskidx_d(key, d0)], qs_bucket_d(key, d0), low_pool, high_pool, half, out + i);
+        uint64_t i = (uint64_t)blockIdx.x * (INS_THREADS / 2) + (threadIdx.x >> 1);
+        KeyT<KB> next = keys[i < n ? i : n - 1u];
+        for (; i < n; i += stride) {
+            const KeyT<KB> key = next;
+            next = keys[i + stride < n ? i + stride : n - 1u]; // in flight beside this key's bucket
+            query_bucket<NT>(s_masks[qs_maskidx_d(key, d0)], qs_bucket_d(key, d0), low_pool, high_pool, half, out + i);
         }
         return;
     }
@@ -333,7 +338,7 @@ __global__ __launch_bounds__(INS_THREADS) void k_query(const KeyT<KB> *__restric
             for (uint64_t i = i0 + (threadIdx.x >> 1); i < i1; i += stride) {
                 const KeyT<KB> key = keys[i];
                 const qs_sdesc &d = D[sa + query_sid(offs + sa, sz - sa + 1u, i)];
-                query_bucket(mask_pool[d.masks_off + qs_maskidx_d(key, d)], qs_bucket_d(key, d),
+                query_bucket<NT>(mask_pool[d.masks_off + qs_maskidx_d(key, d)], qs_bucket_d(key, d),
                              low_pool + d.low_off, high_pool + d.high_off, half, out + i);
             }
             continue;
@@ -355,12 +360,12 @@ __global__ __launch_bounds__(INS_THREADS) void k_query(const KeyT<KB> *__restric
             if (held == sid)
                 for (uint64_t i = a + (threadIdx.x >> 1); i < z; i += stride) {
                     const KeyT<KB> key = keys[i];
-                    query_bucket(s_masks[qs_maskidx_d(key, d)], qs_bucket_d(key, d), low, high, half, out + i);
+                    query_bucket<NT>(s_masks[qs_maskidx_d(key, d)], qs_bucket_d(key, d), low, high, half, out + i);
                 }
             else
                 for (uint64_t i = a + (threadIdx.x >> 1); i < z; i += stride) {
                     const KeyT<KB> key = keys[i];
-                    query_bucket(masks[qs_maskidx_d(key, d)], qs_bucket_d(key, d), low, high, half, out + i);
+                    query_bucket<NT>(masks[qs_maskidx_d(key, d)], qs_bucket_d(key, d), low, high, half, out + i);
                 }
         }
     }
@@ -819,6 +824,9 @@ extern "C" int qs_multi_insert_async(qs_sketch *s, const void *d_keys, const uin
     return qs_insert_set(s, d_keys, h_offs, d_offs, (hipStream_t)stream, false, false);
 }
 
+// keys from which a query may read its buckets past the caches
+#define QUERY_NT_MIN (1u << 23)
+
 static int query_launch(qs_sketch *s, const void *d_keys, uint64_t n, const uint64_t *d_offs, uint32_t *d_counts,
                         hipStream_t stream)
 {
@@ -832,21 +840,32 @@ static int query_launch(qs_sketch *s, const void *d_keys, uint64_t n, const uint
     const dim3 grid(grid_for((uint64_t)nn * 2, INS_THREADS, 8)), block(INS_THREADS);
     qs_evpair ev;
     qs_tim_begin(s, ev, QS_TK_QUERY, nn, stream);
+    // Bucket reads are cached, so that a skewed stream finds its hot buckets again
+    // (12.6 M Zipf 1.1 lookups: 165 us with non-temporal reads, 92 so).  A large
+    // read-out of a table that it mostly touches once is the exception: with
+    // at least two lines per key nothing is found again, and non-temporal reads take
+    // 380 us instead of 410 for 15.8 M distinct keys of a 6.4 GB table.  (Short
+    // calls are left cached: they are bound by latency either way.)
+    const bool nt = !multi && nn >= QUERY_NT_MIN && s->low_words / 32u >= 2ull * nn;
+#define QS_QUERY(KB, MULTI, NT)                                                                                  \
+    hipLaunchKernelGGL((k_query<KB, MULTI, NT>), grid, block, 0, stream, (const KeyT<KB> *)d_keys, nn, d0, s->d_desc, \
+                       d_offs, s->nsk, s->d_low, s->d_high, s->d_masks, d_counts)
     if (s->key_bytes == 4) {
         if (multi)
-            hipLaunchKernelGGL((k_query<4, true>), grid, block, 0, stream, (const uint32_t *)d_keys, nn, d0,
-                               s->d_desc, d_offs, s->nsk, s->d_low, s->d_high, s->d_masks, d_counts);
+            QS_QUERY(4, true, false);
+        else if (nt)
+            QS_QUERY(4, false, true);
         else
-            hipLaunchKernelGGL((k_query<4, false>), grid, block, 0, stream, (const uint32_t *)d_keys, nn, d0,
-                               s->d_desc, d_offs, s->nsk, s->d_low, s->d_high, s->d_masks, d_counts);
+            QS_QUERY(4, false, false);
     } else {
         if (multi)
-            hipLaunchKernelGGL((k_query<8, true>), grid, block, 0, stream, (const uint64_t *)d_keys, nn, d0,
-                               s->d_desc, d_offs, s->nsk, s->d_low, s->d_high, s->d_masks, d_counts);
+            QS_QUERY(8, true, false);
+        else if (nt)
+            QS_QUERY(8, false, true);
         else
-            hipLaunchKernelGGL((k_query<8, false>), grid, block, 0, stream, (const uint64_t *)d_keys, nn, d0,
-                               s->d_desc, d_offs, s->nsk, s->d_low, s->d_high, s->d_masks, d_counts);
+            QS_QUERY(8, false, false);
     }
+#undef QS_QUERY
     qs_tim_end(s, ev, stream);
     CK(hipGetLastError());
     return QS_OK;
