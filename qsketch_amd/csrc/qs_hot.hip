@@ -8,8 +8,8 @@
 //   1. the candidates: the keys occurring at least HOT_MIN_RUN times among the
 //      first HOT_SAMPLE keys, the HOT_MAX most frequent of them; on a second stream, at
 //      the same time as
-//   2. the first HOT_PREFIX keys through the ordinary pipeline (qs_insert.hip),
-//      which links the buckets of the hot keys;
+//   2. the first keys of the call (hot_prefix) through the ordinary pipeline
+//      (qs_insert.hip), which links the buckets of the hot keys;
 //   3. the hot set: the candidates whose bucket is linked now, in a table of
 //      HOT_BUCKETS buckets of 2 slots where each key may sit in one of two
 //      buckets (the emptier one when it is placed), so that a lookup is two
@@ -53,10 +53,20 @@ static_assert(HOT_CAND_MAX % 1024u == 0, "blocks of k_samp_select");
 #define HOT_THREADS 1024
 #define HOT_IPT 16u                        // rows of 64 keys per chunk
 #define HOT_CHUNK (64u * HOT_IPT)          // keys per chunk (one wavefront's unit of work)
-#define HOT_PREFIX (1ull << 24)            // keys inserted the ordinary way first
 #define HOT_MIN_KEYS (1ull << 26)          // shorter calls are not filtered
 #define HOT_MIN_COVER_NUM 3u               // filter when the candidates cover at least
 #define HOT_MIN_COVER_DEN 10u              //   3/10 of the sample
+
+// Keys inserted the ordinary way first: a sixteenth of the call, 2^22 to 2^24.
+// A longer prefix links more of the candidates' buckets, but its keys all go
+// through the sort.  2^26 keys, Zipf 1.1: 1461 us with 2^24, 1381 with 2^23, 1336
+// with 2^22, 1359 with 2^21; 2^27: 2215, 2173, 2186, 2260; 2^28: 4072, 4173, 4310.
+// At Zipf 1.5 2^26 keys take 719 us with 2^22 and 868 with 2^24.
+static uint64_t hot_prefix(uint64_t n)
+{
+    const uint64_t p = n / 16;
+    return p < (1ull << 22) ? 1ull << 22 : p > (1ull << 24) ? 1ull << 24 : p;
+}
 
 // device control words
 #define HC_NCAND 0   // candidates (at most HOT_MAX)
@@ -863,10 +873,10 @@ static int hot_cand_result(qs_hot *h, hipStream_t stream, bool *skewed)
 int qs_insert_hot(qs_sketch *s, const void *d_keys, uint64_t n, hipStream_t stream, int *used)
 {
     *used = 0;
-    if (s->nsk != 1 || s->key_bytes != 4 || n < HOT_MIN_KEYS || n - HOT_PREFIX > 0xffffffffull)
+    if (s->nsk != 1 || s->key_bytes != 4 || n < HOT_MIN_KEYS || n - hot_prefix(n) > 0xffffffffull)
         return QS_OK;
     const uint32_t *keys = (const uint32_t *)d_keys;
-    const uint64_t rest = n - HOT_PREFIX;
+    const uint64_t prefix = hot_prefix(n), rest = n - prefix;
     int rc = hot_alloc(&s->hot, rest);
     if (rc)
         return rc;
@@ -886,7 +896,7 @@ int qs_insert_hot(qs_sketch *s, const void *d_keys, uint64_t n, hipStream_t stre
         const uint64_t cap = qs_chunk_keys(s, offs_n);
         return qs_ensure_scratch(s, n < cap ? n : cap);
     };
-    const uint64_t offs_p[2] = {0, HOT_PREFIX};
+    const uint64_t offs_p[2] = {0, prefix};
     bool skewed = false;
     if (!h->prev_flat) {
         // 2. the prefix goes through the ordinary pipeline on the caller's
@@ -917,7 +927,7 @@ int qs_insert_hot(qs_sketch *s, const void *d_keys, uint64_t n, hipStream_t stre
         if (!skewed) { // not skewed enough to pay for the filter: the rest the ordinary way
             CK(hipStreamWaitEvent(stream, h->ev_cand, 0));
             const uint64_t offs_r[2] = {0, rest};
-            return qs_insert_set(s, keys + HOT_PREFIX, offs_r, nullptr, stream, true, false);
+            return qs_insert_set(s, keys + prefix, offs_r, nullptr, stream, true, false);
         }
     } else {
         // The previous call showed no skew: 1. the candidates first, on the
@@ -960,7 +970,7 @@ int qs_insert_hot(qs_sketch *s, const void *d_keys, uint64_t n, hipStream_t stre
         hipLaunchKernelGGL(k_hot_build, dim3(HOT_MAX / 256), dim3(256), 0, stream, h->cand, h->ccnt,
                            first ? HOT_FIRST_RUN : 0u, first ? ~0u : HOT_FIRST_RUN, d0, s->d_low, s->d_masks, h->tkey,
                            h->tinfo, h->tmask, h->tfill, h->ctl);
-    hipLaunchKernelGGL(k_hot_count, dim3(h->nblk), dim3(HOT_THREADS), 0, stream, keys + HOT_PREFIX, rest,
+    hipLaunchKernelGGL(k_hot_count, dim3(h->nblk), dim3(HOT_THREADS), 0, stream, keys + prefix, rest,
                        nchunks, h->tkey, h->part, h->stage, h->ccold);
     qs_scan_u32(h->ccold, nchunks, h->bsum, stream);
     hipLaunchKernelGGL(k_hot_move, dim3(h->nblk * 8u), dim3(256), 0, stream, h->stage, nchunks, h->ccold, h->cold);
