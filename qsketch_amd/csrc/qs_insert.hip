@@ -1355,13 +1355,16 @@ __device__ static inline uint32_t kth_set_bit(uint64_t m, uint32_t k)
 // 28 ballots B_j, and the first insert that would see a selected byte > 128 is
 // the (129 - c_j)-th set bit of B_j, minimised over j.
 // A wavefront stages its allocations and newly long segments in LDS and
-// reserves their list slots TBUF at a time: one global atomic per segment on
-// a single counter would serialise (tens of thousands of segments replay in a
-// chunk that links the hot buckets).
-#define TBUF 8u
+// reserves their list slots TBUF at a time, both with one 64-bit atomic: same-word
+// atomics serialise at ~11 ns, and tens of thousands of segments replay in a
+// chunk that links the hot buckets (8 at a time on two counters the replay of
+// 76000 segments took 293 us, now 201).
+// (8 in the 16 wavefronts of k_small, whose LDS holds no more)
+template <int NW> constexpr uint32_t TBUF = NW > 4 ? 8u : 16u;
 
 // copy a wave's ntb staged allocations to list slots base, base + 1, ...
-__device__ static inline void write_trig(qs_trig (*s_tr)[TBUF], uint32_t wv, uint32_t lane, uint32_t ntb,
+template <int NW>
+__device__ static inline void write_trig(qs_trig (*s_tr)[TBUF<NW>], uint32_t wv, uint32_t lane, uint32_t ntb,
                                          uint32_t base, qs_trig *__restrict__ trig, uint32_t trig_cap,
                                          qs_dev_state *__restrict__ st)
 {
@@ -1378,31 +1381,21 @@ __device__ static inline void write_trig(qs_trig (*s_tr)[TBUF], uint32_t wv, uin
     }
 }
 
-__device__ static inline void flush_trig(qs_trig (*s_tr)[TBUF], uint32_t wv, uint32_t lane, uint32_t &ntb,
-                                         qs_trig *__restrict__ trig, uint32_t trig_cap,
-                                         qs_dev_state *__restrict__ st)
+// both buffers to their lists; the long segments go after the n_long of the
+// segment pass
+template <int NW>
+__device__ static inline void flush_lists(qs_trig (*s_tr)[TBUF<NW>], uint32_t (*s_ln)[TBUF<NW>], uint32_t wv, uint32_t lane,
+                                          uint32_t &ntb, uint32_t &nlb, qs_trig *__restrict__ trig, uint32_t trig_cap,
+                                          uint32_t *__restrict__ lng, uint32_t n_long, qs_dev_state *__restrict__ st)
 {
-    if (!ntb)
-        return;
-    uint32_t base = 0;
+    unsigned long long base = 0;
     if (lane == 0)
-        base = atomicAdd(&st->n_trig, ntb);
-    base = __shfl(base, 0, 64);
-    write_trig(s_tr, wv, lane, ntb, base, trig, trig_cap, st);
-    ntb = 0;
-}
-
-__device__ static inline void flush_long(uint32_t (*s_ln)[TBUF], uint32_t wv, uint32_t lane, uint32_t &nlb,
-                                         uint32_t *__restrict__ lng, qs_dev_state *__restrict__ st)
-{
-    if (!nlb)
-        return;
-    uint32_t base = 0;
-    if (lane == 0)
-        base = atomicAdd(&st->n_long, nlb);
-    base = __shfl(base, 0, 64);
+        base = atomicAdd(reinterpret_cast<unsigned long long *>(&st->n_trig), ((unsigned long long)nlb << 32) | ntb);
+    base = shfl64(base, 0);
+    write_trig<NW>(s_tr, wv, lane, ntb, (uint32_t)base, trig, trig_cap, st);
     if (lane < nlb)
-        lng[base + lane] = s_ln[wv][lane];
+        lng[n_long + (uint32_t)(base >> 32) + lane] = s_ln[wv][lane];
+    ntb = 0;
     nlb = 0;
 }
 // block bid of nblk, of NW wavefronts; a single sketch's masks (one_masks of them)
@@ -1420,12 +1413,12 @@ __device__ __forceinline__ void ordered_pass(uint32_t bid, uint32_t nblk, const 
                                              const uint64_t *__restrict__ offs, uint64_t base,
                                              uint32_t one_masks, const uint32_t *s_masks, qs_dev_state *__restrict__ st)
 {
-    __shared__ qs_trig s_tr[NW][TBUF];
-    __shared__ uint32_t s_ln[NW][TBUF];
+    __shared__ qs_trig s_tr[NW][TBUF<NW>];
+    __shared__ uint32_t s_ln[NW][TBUF<NW>];
     const uint32_t lane = threadIdx.x & 63u, wv = threadIdx.x >> 6;
     const uint32_t gw = bid * (uint32_t)NW + (threadIdx.x >> 6);
     const uint32_t nw = nblk * (uint32_t)NW;
-    const uint32_t n_ord = st->n_ord;
+    const uint32_t n_ord = st->n_ord, n_long = st->n_long;
     uint32_t ntb = 0, nlb = 0;
     unsigned long long replayed_all = 0;
     // Loaded ahead, unconditionally from clamped positions so that waits do
@@ -1541,16 +1534,14 @@ __device__ __forceinline__ void ordered_pass(uint32_t bid, uint32_t nblk, const 
                     ++nlb;
                 }
             }
-            if (ntb == TBUF)
-                flush_trig(s_tr, wv, lane, ntb, trig, trig_cap, st);
-            if (nlb == TBUF)
-                flush_long(s_ln, wv, lane, nlb, lng, st);
+            if (ntb == TBUF<NW>) // (at most one long segment per allocation)
+                flush_lists<NW>(s_tr, s_ln, wv, lane, ntb, nlb, trig, trig_cap, lng, n_long, st);
         }
     }
-    // Final flush, one reservation per list per block: same-address atomics
-    // serialise (~11 ns each), and one per wavefront and list costs more than
-    // the replay itself.
-    __shared__ uint32_t s_nt[NW], s_nl[NW], s_base[2];
+    // Final flush, one reservation per block: same-address atomics serialise
+    // (~11 ns each), and one per wavefront costs more than the replay itself.
+    __shared__ uint32_t s_nt[NW], s_nl[NW];
+    __shared__ unsigned long long s_base;
     __shared__ unsigned long long s_rep[NW];
     if (lane == 0) {
         s_nt[wv] = ntb;
@@ -1567,18 +1558,18 @@ __device__ __forceinline__ void ordered_pass(uint32_t bid, uint32_t nblk, const 
             tl += s_nl[w];
             rk += s_rep[w];
         }
-        s_base[0] = tt ? atomicAdd(&st->n_trig, tt) : 0u;
-        s_base[1] = tl ? atomicAdd(&st->n_long, tl) : 0u;
+        s_base = tt ? atomicAdd(reinterpret_cast<unsigned long long *>(&st->n_trig), ((unsigned long long)tl << 32) | tt)
+                    : 0ull; // (no long segment without an allocation)
         if (rk)
             atomicAdd(&st->replay_keys, rk);
     }
     __syncthreads();
-    uint32_t bt = s_base[0], bl = s_base[1];
+    uint32_t bt = (uint32_t)s_base, bl = n_long + (uint32_t)(s_base >> 32);
     for (uint32_t w = 0; w < wv; ++w) {
         bt += s_nt[w];
         bl += s_nl[w];
     }
-    write_trig(s_tr, wv, lane, ntb, bt, trig, trig_cap, st);
+    write_trig<NW>(s_tr, wv, lane, ntb, bt, trig, trig_cap, st);
     if (lane < nlb)
         lng[bl + lane] = s_ln[wv][lane];
 }
@@ -1595,7 +1586,7 @@ __global__ __launch_bounds__(256) void k_ordered(const uint64_t *__restrict__ IT
                                                  const uint64_t *__restrict__ offs, uint64_t base,
                                                  uint32_t one_masks, qs_dev_state *__restrict__ st)
 {
-    __shared__ uint32_t s_masks[QS_MAX_MASKS];
+    extern __shared__ uint32_t s_masks[]; // one_masks words, sized by the launch
     for (uint32_t i = threadIdx.x; i < one_masks; i += blockDim.x)
         s_masks[i] = mask_pool[i];
     __syncthreads();
@@ -1828,7 +1819,8 @@ __device__ __forceinline__ void tail_pass(uint32_t bid, uint32_t nblk, const uin
                                           const uint32_t *__restrict__ lng, bool short_runs, uint32_t window,
                                           const qs_dev_state *__restrict__ st)
 {
-    if (st->n_long == 0)
+    const uint32_t n_long = st->n_long + st->n_tail;
+    if (n_long == 0)
         return;
     __shared__ uint32_t s_rows[NW][64][TROW];
     const uint32_t lane = threadIdx.x & 63u, wv = threadIdx.x >> 6;
@@ -1967,7 +1959,6 @@ __device__ __forceinline__ void tail_pass(uint32_t bid, uint32_t nblk, const uin
     // outside a run that fits in one step.
     if (!short_runs)
         return;
-    const uint32_t n_long = st->n_long;
     for (uint32_t e = gw; e < n_long; e += nw) {
         const uint32_t h = lng[e]; // head of the run
         const uint32_t p = h + lane;
@@ -2012,7 +2003,7 @@ __global__ __launch_bounds__(256) void k_tail(const uint64_t *__restrict__ IT, u
                                               const uint32_t *__restrict__ lng, bool short_runs, uint32_t window,
                                               const qs_dev_state *__restrict__ st)
 {
-    if (st->n_long == 0)
+    if (st->n_long + st->n_tail == 0)
         return;
     // n_masks0 words of dynamic LDS (sized by the launch: 16 KiB for the
     // largest table would hold the kernel to five wavefronts per SIMD)
@@ -2040,7 +2031,7 @@ __device__ __forceinline__ void finish_pass(uint32_t bid, uint32_t nblk, const u
                                             uint32_t *__restrict__ next, qs_dev_state *__restrict__ st,
                                             uint32_t *__restrict__ h_err)
 {
-    const uint32_t n_long = st->n_long, n_trig = st->n_trig;
+    const uint32_t n_long = st->n_long + st->n_tail, n_trig = st->n_trig;
     for (uint32_t i = bid * blockDim.x + threadIdx.x; i < n_long; i += nblk * blockDim.x) {
         const uint64_t it = IT[lng[i]];
         const uint64_t bit = D[it_sid(it, pk)].bm_off + it_b(it, pk);
@@ -2076,6 +2067,7 @@ __device__ __forceinline__ void finish_pass(uint32_t bid, uint32_t nblk, const u
     st->n_ord = 0;
     st->n_long = 0;
     st->n_trig = 0;
+    st->n_tail = 0;
     st->done = 0;
     __hip_atomic_store(h_err, st->err, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
 }
@@ -2491,7 +2483,8 @@ static int insert_chunk(qs_sketch *s, const KeyT<KB> *keys, uint32_t cn, uint64_
     if (bc.timed) {
         qs_tim_next(s, es, eo, QS_TK_ORDERED, cn, stream);
     }
-    hipLaunchKernelGGL(k_ordered, dim3(grid_cap(((uint64_t)cn + 255) / 256, 8)), dim3(256), 0, stream, IT, cn,
+    hipLaunchKernelGGL(k_ordered, dim3(grid_cap(((uint64_t)cn + 255) / 256, 8)), dim3(256),
+                       MULTI ? 0 : (size_t)nm0 * sizeof(uint32_t), stream, IT, cn,
                        sc.ord, s->d_desc, s->d_low, s->d_masks, s->pk, s->d_longbm, sc.lng, sc.trig,
                        sc.trig_cap, sc.tbit, sc.tsum, bc.d_offs, base, MULTI ? 0u : nm0, s->d_st);
     if (bc.timed) {

@@ -273,20 +273,23 @@ static inline int qs_err_code(uint32_t err)
 
 struct qs_dev_state {
     uint32_t n_ord;     // bucket segments queued for the in-order replay
-    uint32_t n_long;    // long bucket segments (handled by the windowed tail kernel)
+    uint32_t n_long;    // long bucket segments found by the segment pass (for the windowed tail kernel)
     uint32_t n_trig;    // allocations triggered in the current chunk
+    uint32_t n_tail;    // long segments found by the replay (listed after the n_long)
     uint32_t err;       // sticky error bits (QS_EF_*)
+    uint32_t done;      // blocks of the chunk's last kernel that have finished (its last block clears it)
     // running totals since create / clear (statistics only)
     unsigned long long replay_keys;   // inserts replayed in stream order
     unsigned long long ord_segments;  // segments sent to the replay
     unsigned long long long_segments; // segments handled by the tail kernel
     unsigned long long chunks_ord;    // chunks with at least one replayed segment
-    uint32_t done;      // blocks of the chunk's last kernel that have finished (its last block clears it)
-    uint32_t pad;
 };
-// k_segw reserves entries of both lists with one 64-bit atomic on (n_ord, n_long)
+// the segment pass reserves entries of both its lists with one 64-bit atomic on
+// (n_ord, n_long), the replay with one on (n_trig, n_tail)
 static_assert(offsetof(qs_dev_state, n_ord) % 8 == 0 && offsetof(qs_dev_state, n_long) == offsetof(qs_dev_state, n_ord) + 4,
               "n_ord and n_long form one aligned 64-bit word");
+static_assert(offsetof(qs_dev_state, n_trig) % 8 == 0 && offsetof(qs_dev_state, n_tail) == offsetof(qs_dev_state, n_trig) + 4,
+              "n_trig and n_tail form one aligned 64-bit word");
 
 // One allocation found by the in-order replay (filled before ids are known).
 struct qs_trig {
