@@ -138,18 +138,47 @@ struct sid_window {
     uint32_t sid0, cnt;
 };
 
+// find_sid by a wavefront, 64 offsets at a time: two reads deep for 512 sketches
+// where one lane's binary search is nine
+__device__ static inline uint32_t find_sid_wave(const uint64_t *__restrict__ offs, uint32_t nsk, uint64_t pos)
+{
+    const uint32_t lane = threadIdx.x & 63u;
+    uint32_t lo = 0, hi = nsk; // uniform; offs[lo] <= pos < offs[hi]
+    while (hi - lo > 1) {
+        const uint32_t step = (hi - lo + 63u) >> 6;
+        const uint64_t p = (uint64_t)lo + (uint64_t)(lane + 1u) * step;
+        // (offsets ascend: the lanes that hold are a prefix)
+        const uint32_t c = (uint32_t)__popcll(__ballot(p < hi && offs[p < hi ? p : hi] <= pos));
+        const uint32_t nl = lo + c * step;
+        hi = hi - nl > step ? nl + step : hi;
+        lo = nl;
+    }
+    return lo;
+}
+
 __device__ static inline void load_sid_window(const uint64_t *__restrict__ offs, uint32_t nsk, uint64_t lo,
                                               uint64_t hi, uint64_t *s_off, uint32_t *s_w)
 {
-    if (threadIdx.x == 0) {
-        const uint32_t a = find_sid(offs, nsk, lo), b = find_sid(offs, nsk, hi);
-        s_w[0] = a;
-        s_w[1] = (b - a + 1u) <= SIDW ? (b - a + 1u) : 0u;
+    const uint32_t wv = threadIdx.x >> 6;
+    if (wv < 2u) { // the first wavefront searches the first position, the second the last
+        const uint32_t a = find_sid_wave(offs, nsk, wv ? hi : lo);
+        if ((threadIdx.x & 63u) == 0)
+            s_w[wv] = a;
     }
     __syncthreads();
-    for (uint32_t j = threadIdx.x; s_w[1] && j <= s_w[1]; j += blockDim.x)
-        s_off[j] = offs[s_w[0] + j];
+    const uint32_t a = s_w[0], cnt = s_w[1] - a + 1u;
+    if (cnt > 1u && cnt <= SIDW)
+        for (uint32_t j = threadIdx.x; j <= cnt; j += blockDim.x)
+            s_off[j] = offs[a + j];
     __syncthreads();
+}
+
+// the window that load_sid_window left, in scalar registers
+__device__ static inline sid_window sid_window_of(const uint64_t *s_off, const uint32_t *s_w)
+{
+    const uint32_t a = (uint32_t)__builtin_amdgcn_readfirstlane((int)s_w[0]);
+    const uint32_t cnt = (uint32_t)__builtin_amdgcn_readfirstlane((int)s_w[1]) - a + 1u;
+    return sid_window{s_off, a, cnt <= SIDW ? cnt : 0u};
 }
 
 // bucket and mask fields of a key's item: h % n_low and h % n_masks, or in the
@@ -196,6 +225,36 @@ __device__ static inline uint64_t make_item(const KeyT<KB> key, uint32_t i, uint
     return bucket_mask_fields<KB>(key, d, pk) | ((uint64_t)sid << pk.bb) | ((pos - start) << pk.ishift);
 }
 
+// The items of a thread's OS_IPL keys, chunk positions i0, i0 + step, ...; past n
+// zero.  Most tiles of a batch lie in one sketch (uniform): its descriptor is then read
+// once, into scalar registers.  75 M keys of 512 sketches, with the search by
+// wavefronts and the key loads before it: tile counts 261 -> 135 us, first scatter
+// 535 -> 369.
+template <int KB, bool MULTI>
+__device__ static inline void make_items(uint64_t (&item)[OS_IPL], const KeyT<KB> (&raw)[OS_IPL], uint32_t i0,
+                                         uint32_t step, uint32_t n, uint64_t base, const qs_sdesc &d0,
+                                         const qs_sdesc *__restrict__ D, const uint64_t *__restrict__ offs,
+                                         uint32_t nsk, const qs_pack &pk, const sid_window &win)
+{
+    if (MULTI && win.cnt == 1u) {
+        const qs_sdesc d = D[win.sid0];
+        const uint64_t sstart = offs[win.sid0];
+        const uint32_t before = sstart > base ? (uint32_t)(sstart - base) : 0u; // chunk position of the sketch's part
+        const uint64_t cell = (uint64_t)win.sid0 << pk.bb;
+#pragma unroll
+        for (int r = 0; r < OS_IPL; ++r) {
+            const uint32_t i = i0 + r * step;
+            item[r] = i < n ? bucket_mask_fields<KB>(raw[r], d, pk) | cell | ((uint64_t)(i - before) << pk.ishift) : 0ull;
+        }
+        return;
+    }
+#pragma unroll
+    for (int r = 0; r < OS_IPL; ++r) {
+        const uint32_t i = i0 + r * step;
+        item[r] = i < n ? make_item<KB, MULTI>(raw[r], i, base, d0, D, offs, nsk, pk, win) : 0ull;
+    }
+}
+
 // what a radix pass reads per position: the key (first pass) or the item,
 // streamed once (non-temporal); positions past n read the last one
 template <int KB, bool FIRST> using RawT = typename std::conditional<FIRST, KeyT<KB>, uint64_t>::type;
@@ -232,30 +291,27 @@ __global__ __launch_bounds__(OS_THREADS) void k_bs_up(const void *__restrict__ i
         tbit[blockIdx.x * (OS_TILE / 32u) + t] = 0;
     if (t == 0 && tb % QS_TSPAN == 0)
         tsum[tb / QS_TSPAN] = 0;
-    sid_window win{s_off, 0u, 0u};
-    if (MULTI) {
-        const uint32_t te = (n - tb) < OS_TILE ? n : tb + OS_TILE;
-        load_sid_window(offs, nsk, base + tb, base + te - 1u, s_off, s_w);
-        win.sid0 = s_w[0];
-        win.cnt = s_w[1];
-    }
-    __syncthreads();
-    const uint32_t lane = t & 63u;
     // every load first, from clamped positions: a load inside a per-item branch
     // is issued and waited for one at a time
     KeyT<KB> raw[OS_IPL];
 #pragma unroll
     for (int r = 0; r < OS_IPL; ++r)
         raw[r] = load_raw<KB, true>(in, tb + r * OS_THREADS + t, n);
+    sid_window win{s_off, 0u, 0u};
+    if (MULTI) {
+        const uint32_t te = (n - tb) < OS_TILE ? n : tb + OS_TILE;
+        load_sid_window(offs, nsk, base + tb, base + te - 1u, s_off, s_w);
+        win = sid_window_of(s_off, s_w);
+    }
+    __syncthreads();
+    const uint32_t lane = t & 63u;
+    uint64_t item[OS_IPL];
+    make_items<KB, MULTI>(item, raw, tb + t, OS_THREADS, n, base, d0, D, offs, nsk, pk, win);
 #pragma unroll
     for (int r = 0; r < OS_IPL; ++r) {
         const uint32_t i = tb + r * OS_THREADS + t; // a wavefront's lanes hold consecutive items
         const bool valid = i < n;
-        uint32_t d = 0;
-        if (valid) {
-            const uint64_t c = it_cell(make_item<KB, MULTI>(raw[r], i, base, d0, D, offs, nsk, pk, win), pk);
-            d = (uint32_t)(c >> shift) & dmask;
-        }
+        const uint32_t d = valid ? (uint32_t)(it_cell(item[r], pk) >> shift) & dmask : 0u;
         // one LDS add per run of equal digits on adjacent lanes (a Zipf-hot
         // cell fills whole wavefronts, whose adds to one bin would serialise)
         // (both ballots are taken by the whole wavefront, outside any branch)
@@ -502,12 +558,17 @@ __global__ __launch_bounds__(OS_THREADS) void k_bs_down(
     const uint32_t xq = ntiles >> 3, xr = ntiles & 7u, xb = blockIdx.x & 7u;
     const uint32_t tile = xb * xq + min(xb, xr) + (blockIdx.x >> 3);
     const uint32_t tb = tile * OS_TILE;
+    const uint32_t i0 = tb + wv * OS_WAVE_ITEMS + lane; // lane's items: every 64th from here
+    // a batch's keys are in flight while its sketches are searched
+    RawT<KB, FIRST> raw[OS_IPL];
     sid_window win{s_off, 0u, 0u};
     if (FIRST && MULTI) {
+#pragma unroll
+        for (int r = 0; r < OS_IPL; ++r)
+            raw[r] = load_raw<KB, FIRST>(in, i0 + r * 64u, n);
         const uint32_t te = (n - tb) < OS_TILE ? n : tb + OS_TILE;
         load_sid_window(offs, nsk, base + tb, base + te - 1u, s_off, s_w);
-        win.sid0 = s_w[0];
-        win.cnt = s_w[1];
+        win = sid_window_of(s_off, s_w);
     }
     if (t < OS_BINS)
 #pragma unroll
@@ -540,25 +601,20 @@ __global__ __launch_bounds__(OS_THREADS) void k_bs_down(
     const int dbits = __builtin_popcount(dmask);
     uint64_t item[OS_IPL];
     uint32_t dr[OS_IPL]; // digit | wave-local position << 8 | valid << 31
-    {
-        // every load first (see k_bs_up)
-        RawT<KB, FIRST> raw[OS_IPL];
+    // every load first (see k_bs_up)
+    if (!(FIRST && MULTI))
 #pragma unroll
         for (int r = 0; r < OS_IPL; ++r)
-            raw[r] = load_raw<KB, FIRST>(in, tb + wv * OS_WAVE_ITEMS + r * 64u + lane, n);
+            raw[r] = load_raw<KB, FIRST>(in, i0 + r * 64u, n);
+    if constexpr (FIRST)
+        make_items<KB, MULTI>(item, raw, i0, 64u, n, base, d0, D, offs, nsk, pk, win);
+    else
 #pragma unroll
-        for (int r = 0; r < OS_IPL; ++r) {
-            const uint32_t i = tb + wv * OS_WAVE_ITEMS + r * 64u + lane;
-            if (FIRST)
-                item[r] = i < n ? make_item<KB, MULTI>((KeyT<KB>)raw[r], i, base, d0, D, offs, nsk, pk, win) : 0ull;
-            else
-                item[r] = i < n ? (uint64_t)raw[r] : 0ull;
-        }
-    }
+        for (int r = 0; r < OS_IPL; ++r)
+            item[r] = i0 + r * 64u < n ? raw[r] : 0ull;
 #pragma unroll
     for (int r = 0; r < OS_IPL; ++r) {
-        const uint32_t i = tb + wv * OS_WAVE_ITEMS + r * 64u + lane;
-        const bool valid = i < n;
+        const bool valid = i0 + r * 64u < n;
         const uint32_t d = (uint32_t)(it_cell(item[r], pk) >> shift) & dmask;
         // lanes sharing my digit: one ballot per digit bit (the bits above the
         // digit are 0 in every lane and leave m as it is)
