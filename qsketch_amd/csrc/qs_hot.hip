@@ -156,8 +156,8 @@ __device__ static inline void hot_buckets(uint32_t key, uint32_t &b1, uint32_t &
 // of the counts.  Which keys become candidates moves time only, never the
 // result, so a key that finds the LDS table crowded is simply left out.
 // (The sample was sorted before, and the candidates sorted again by count:
-// 29 launches, about 270 us with their gaps; these four kernels take 72 us at
-// Zipf 1.1, 48 of them the block whose bin holds the hottest key.)
+// 29 launches, about 270 us with their gaps; these four kernels take 65 us at
+// Zipf 1.1 over 2^24 keys, 43 of them the block whose bin holds the hottest key.)
 // ---------------------------------------------------------------------------
 #define SAMP_TILE 8192u // sample keys per block of the split
 #define SAMP_TILES (HOT_SAMPLE / SAMP_TILE)
@@ -275,8 +275,27 @@ __global__ __launch_bounds__(1024) void k_samp_count(const uint32_t *__restrict_
         s_n = 0;
     __syncthreads();
     const uint32_t b0 = start[blockIdx.x], b1 = start[blockIdx.x + 1];
-    // (a hot key's bin can hold most of the sample: the loads of SAMP_ROWS rows
-    // are in flight together)
+    // adds w to key k's count, if there is room for it
+    auto add = [&](uint32_t k, uint32_t w) {
+        uint32_t sl = (samp_hash(k) >> 11) & (SAMP_SLOTS - 1u);
+        for (uint32_t pr = 0; pr < SAMP_PROBES; ++pr, sl = (sl + 1u) & (SAMP_SLOTS - 1u)) {
+            uint32_t cur = s_key[sl];
+            if (cur == HOT_EMPTY)
+                cur = atomicCAS(&s_key[sl], HOT_EMPTY, k);
+            if (cur == HOT_EMPTY || cur == k) {
+                atomicAdd(&s_cnt[sl], w);
+                break;
+            }
+        }
+    };
+    // A hot key's bin can hold most of the sample, nearly all of it that key:
+    // one block walks 113 rows of the default workload's.  Each wavefront keeps one
+    // key and its count in scalar registers (the key that its latest row shared
+    // most, or was led by), so such a row costs a compare and a population count,
+    // and the LDS table only sees the other lanes: 95 -> 50 us with the default
+    // workload, 52 -> 43 with Zipf 1.1 over 2^24 keys.  The loads of SAMP_ROWS rows
+    // are in flight together.
+    uint32_t hk = HOT_EMPTY, hc = 0; // uniform
     for (uint32_t i0 = b0; i0 < b1; i0 += 1024u * SAMP_ROWS) {
         uint32_t kk[SAMP_ROWS];
 #pragma unroll
@@ -287,35 +306,37 @@ __global__ __launch_bounds__(1024) void k_samp_count(const uint32_t *__restrict_
 #pragma unroll
         for (uint32_t r = 0; r < SAMP_ROWS; ++r) {
             const uint32_t i = i0 + r * 1024u + t, k = kk[r];
-            // the lanes with the first lane's key, then those with the first key
-            // of the rest, are added by one lane each
-            uint32_t w = i < b1 && k != HOT_EMPTY ? 1u : 0u; // (the empty marker is never hot)
-            uint64_t left = __ballot(w != 0u);
-#pragma unroll
-            for (int peel = 0; peel < 2; ++peel) {
-                if (left == 0)
-                    break;
-                const uint32_t first = (uint32_t)__builtin_ctzll(left);
-                const uint32_t fk = (uint32_t)__shfl((int)k, (int)first, 64);
-                const uint64_t same = __ballot(k == fk) & left;
-                left &= ~same;
-                if ((same >> lane) & 1ull)
-                    w = lane == first ? (uint32_t)__popcll(same) : 0u;
-            }
-            if (!w)
+            uint64_t left = __ballot(i < b1 && k != HOT_EMPTY); // (the empty marker is never hot)
+            const uint64_t kept = __ballot(k == hk) & left;
+            hc += (uint32_t)__popcll(kept);
+            left &= ~kept;
+            if (left == 0)
                 continue;
-            uint32_t sl = (samp_hash(k) >> 11) & (SAMP_SLOTS - 1u);
-            for (uint32_t pr = 0; pr < SAMP_PROBES; ++pr, sl = (sl + 1u) & (SAMP_SLOTS - 1u)) {
-                uint32_t cur = s_key[sl];
-                if (cur == HOT_EMPTY)
-                    cur = atomicCAS(&s_key[sl], HOT_EMPTY, k);
-                if (cur == HOT_EMPTY || cur == k) {
-                    atomicAdd(&s_cnt[sl], w);
-                    break;
+            // the lanes with the first remaining lane's key are added by one lane,
+            // or take the kept key's place
+            const uint32_t first = (uint32_t)__builtin_ctzll(left);
+            const uint32_t fk = (uint32_t)__builtin_amdgcn_readlane((int)k, (int)first);
+            const uint64_t same = __ballot(k == fk) & left;
+            const uint32_t ns = (uint32_t)__popcll(same);
+            uint32_t w = (left >> lane) & 1ull;
+            if ((same >> lane) & 1ull)
+                w = lane == first ? ns : 0u;
+            uint32_t ak = k;
+            if (ns > (uint32_t)__popcll(kept)) {
+                // the first lane hands the old key's count over instead of its own
+                if (lane == first) {
+                    ak = hk;
+                    w = hc;
                 }
+                hk = fk;
+                hc = ns;
             }
+            if (w)
+                add(ak, w);
         }
     }
+    if (lane == 0 && hc)
+        add(hk, hc);
     __syncthreads();
     uint32_t mine = 0;
     for (uint32_t e = t; e < SAMP_SLOTS; e += 1024u)
