@@ -22,8 +22,8 @@
 // (bucket | sketch | mask index | stream index); later passes and kernels
 // only extract bit fields.  Digit ranks inside a wavefront come from a ballot
 // match (one ballot per digit bit gives each lane the mask of lanes sharing
-// its digit), which is stable; the group's lowest lane advances the digit's
-// running count with one LDS atomic.
+// its digit), which is stable; every lane reads the digit's running count and
+// the group's lowest lane adds the group to it (wave_digit_rank).
 //
 // Per chunk (a fixed launch sequence with no host synchronisation, so it can
 // be captured in a hipGraph; all counts stay on the device):
@@ -112,13 +112,16 @@ __device__ static inline uint32_t sid_chunk_start(const uint64_t *__restrict__ o
 // radix sort of the chunk by cell = (sketch, bucket)
 // ===========================================================================
 #ifndef QS_OS_THREADS
-#define QS_OS_THREADS 256
+#define QS_OS_THREADS 512
 #endif
 #define OS_THREADS QS_OS_THREADS
 #define OS_WAVES (OS_THREADS / 64)
-// items per lane: 8 measured best on MI355X (2^28-key Zipf insert: 16 items
-// per lane left the scatter at 4 waves/SIMD, 4 grew the scan of the tile
-// histograms more than the scatter gained)
+// Tiles of 512 * 8 items: a digit's run in a tile is what a scatter writes at a
+// time, 16 items of an 8-byte item's 128-byte line for 8-bit digits, and 24 wavefronts per
+// CU are still in flight.  A later pass of 134 M items (7-bit digits): 480 us with
+// 256 threads, 384 with 512, 556 with 1024 (one block per CU), 380 with 512 of 16
+// items, which loses elsewhere (a pass of 75 M items with 8-bit digits: 325, 297, 412, 302).
+// Non-temporal stores take 550: the runs of neighbouring tiles meet in the L2.
 #ifndef QS_OS_IPL
 #define QS_OS_IPL 8
 #endif
@@ -311,7 +314,7 @@ __global__ __launch_bounds__(OS_THREADS) void k_bs_up(const void *__restrict__ i
     for (int r = 0; r < OS_IPL; ++r) {
         const uint32_t i = tb + r * OS_THREADS + t; // a wavefront's lanes hold consecutive items
         const bool valid = i < n;
-        const uint32_t d = valid ? (uint32_t)(it_cell(item[r], pk) >> shift) & dmask : 0u;
+        const uint32_t d = valid ? (uint32_t)(item[r] >> shift) & dmask : 0u;
         // one LDS add per run of equal digits on adjacent lanes (a Zipf-hot
         // cell fills whole wavefronts, whose adds to one bin would serialise)
         // (both ballots are taken by the whole wavefront, outside any branch)
@@ -427,7 +430,7 @@ __global__ __launch_bounds__(OS_THREADS) void k_bs_up_dig(const uint8_t *__restr
 // (reads and writes are contiguous rows), and leaves group-local prefixes plus
 // the group's sums.  Level 2: one block per digit scans that digit's group
 // sums and writes its total.  The scatter adds the two levels.
-#define SCAN_TPB 32u
+#define SCAN_TPB 16u
 // The tile counts and their group-local prefixes are 16-bit: a count is at
 // most OS_TILE and a prefix at most (SCAN_TPB - 1) * OS_TILE.
 static_assert(SCAN_TPB * OS_TILE <= 65536u, "16-bit tile counts");
@@ -542,11 +545,10 @@ __global__ __launch_bounds__(OS_THREADS) void k_bs_down(
     const uint64_t *__restrict__ offs, uint32_t nsk, qs_pack pk, int shift, uint32_t dmask,
     uint32_t nbins, uint32_t ntiles, const uint16_t *__restrict__ hist, const uint32_t *__restrict__ gsum,
     const uint32_t *__restrict__ totals, int scan, uint64_t *__restrict__ out, uint8_t *__restrict__ dig,
-    int nshift, qs_dev_state *__restrict__ st)
+    int nshift, uint32_t ndmask, qs_dev_state *__restrict__ st)
 {
     __shared__ uint64_t s_item[OS_TILE];
     __shared__ uint32_t s_wh[OS_WAVES][OS_BINS];
-    __shared__ uint32_t s_ls[OS_BINS];
     __shared__ uint32_t s_goff[OS_BINS];
     __shared__ uint32_t s_red[OS_WAVES];
     __shared__ uint64_t s_off[MULTI ? SIDW + 1 : 1];
@@ -597,10 +599,8 @@ __global__ __launch_bounds__(OS_THREADS) void k_bs_down(
     }
     const uint32_t dbase = block_excl_scan(tot, s_red);
 
-    const uint64_t lt = (1ull << lane) - 1ull;
-    const int dbits = __builtin_popcount(dmask);
     uint64_t item[OS_IPL];
-    uint32_t dr[OS_IPL]; // digit | wave-local position << 8 | valid << 31
+    uint32_t dr[OS_IPL]; // digit | wave-local position << 8
     // every load first (see k_bs_up)
     if (!(FIRST && MULTI))
 #pragma unroll
@@ -615,67 +615,70 @@ __global__ __launch_bounds__(OS_THREADS) void k_bs_down(
 #pragma unroll
     for (int r = 0; r < OS_IPL; ++r) {
         const bool valid = i0 + r * 64u < n;
-        const uint32_t d = (uint32_t)(it_cell(item[r], pk) >> shift) & dmask;
-        // lanes sharing my digit: one ballot per digit bit (the bits above the
-        // digit are 0 in every lane and leave m as it is)
-        uint64_t m = __ballot(valid);
-#pragma unroll
-        for (int bit = 0; bit < 8; ++bit) {
-            if (bit < dbits) { // uniform: the digit width is a launch argument
-                const bool on = (d >> bit) & 1u;
-                const uint64_t bb = __ballot(on);
-                m &= on ? bb : ~bb;
-            }
-        }
-        const uint32_t rank = (uint32_t)__popcll(m & lt);
-        const int leader = valid ? (int)__builtin_ctzll(m) : 0;
-        // the group's lowest lane advances the wave's running count of the
-        // digit (LDS atomics of one wave complete in issue order)
-        uint32_t run = 0;
-        if (valid && rank == 0)
-            run = atomicAdd(&s_wh[wv][d], (uint32_t)__popcll(m));
-        run = (uint32_t)__shfl((int)run, leader, 64);
-        dr[r] = d | ((run + rank) << 8) | (valid ? 0x80000000u : 0u);
+        const uint32_t d = (uint32_t)(item[r] >> shift) & dmask;
+        dr[r] = d | wave_digit_rank(s_wh[wv], d, __ballot(valid), valid) << 8;
     }
     __syncthreads();
     {
         // this tile's count of digit t comes from the ranking itself; the
-        // per-wave counts become per-wave starts within the digit
-        uint32_t cnt = 0;
+        // per-wave counts become per-wave starts within the tile
+        uint32_t cnt = 0, c[OS_WAVES] = {};
         if (t < OS_BINS)
 #pragma unroll
             for (int w = 0; w < OS_WAVES; ++w) {
-                const uint32_t c = s_wh[w][t];
-                s_wh[w][t] = cnt;
-                cnt += c;
+                c[w] = s_wh[w][t];
+                cnt += c[w];
             }
         const uint32_t lstart = block_excl_scan(cnt, s_red);
         if (t < OS_BINS) {
-            s_ls[t] = lstart;
             s_goff[t] = dbase + hcur - lstart;
+            uint32_t at = lstart;
+#pragma unroll
+            for (int w = 0; w < OS_WAVES; ++w) {
+                s_wh[w][t] = at;
+                at += c[w];
+            }
         }
     }
     __syncthreads();
 #pragma unroll
-    for (int r = 0; r < OS_IPL; ++r) {
-        if (dr[r] & 0x80000000u) {
-            const uint32_t d = dr[r] & 0xffu;
-            s_item[s_ls[d] + s_wh[wv][d] + ((dr[r] >> 8) & 0x7fffffu)] = item[r];
-        }
-    }
+    for (int r = 0; r < OS_IPL; ++r)
+        if (i0 + r * 64u < n)
+            s_item[s_wh[wv][dr[r] & 0xffu] + (dr[r] >> 8)] = item[r];
     __syncthreads();
     const uint32_t tn = (n - tb) < OS_TILE ? (n - tb) : OS_TILE;
-    for (uint32_t q = t; q < tn; q += OS_THREADS) {
-        const uint64_t it = s_item[q];
-        const uint64_t c = it_cell(it, pk);
-        const uint32_t dst = s_goff[(uint32_t)(c >> shift) & dmask] + q;
-        if (dst < n) { // the tile counts and the ranking agree; checked, never trusted
-            out[dst] = it;
-            if (nshift >= 0) // the next pass's digit, for its tile counts
-                dig[dst] = (uint8_t)((uint32_t)(c >> nshift) & dmask);
-        } else
-            atomicOr(&st->err, QS_EF_SORT);
-    }
+    // (the tile counts and the ranking agree; checked, never trusted)
+    bool bad = false;
+    auto put = [&](uint64_t it, uint32_t dst) {
+        out[dst] = it;
+        if (nshift >= 0) // the next pass's digit, for its tile counts
+            dig[dst] = (uint8_t)((uint32_t)(it >> nshift) & ndmask);
+    };
+    if (tn == OS_TILE) { // every LDS read of a whole tile's rounds in flight together
+        uint32_t dst[OS_IPL];
+#pragma unroll
+        for (uint32_t r = 0; r < OS_IPL; ++r)
+            item[r] = s_item[r * OS_THREADS + t];
+#pragma unroll
+        for (uint32_t r = 0; r < OS_IPL; ++r) {
+            dst[r] = s_goff[(uint32_t)(item[r] >> shift) & dmask] + r * OS_THREADS + t;
+            bad = bad || dst[r] >= n;
+        }
+        if (!bad)
+#pragma unroll
+            for (uint32_t r = 0; r < OS_IPL; ++r)
+                put(item[r], dst[r]);
+    } else
+        for (uint32_t q = t; q < tn; q += OS_THREADS) {
+            const uint64_t it = s_item[q];
+            const uint32_t dst = s_goff[(uint32_t)(it >> shift) & dmask] + q;
+            if (dst < n)
+                put(it, dst);
+            else
+                bad = true;
+        }
+    if (bad)
+        atomicOr(&st->err, QS_EF_SORT);
 }
 
 // ===========================================================================
@@ -2208,22 +2211,7 @@ __global__ __launch_bounds__(SMALL_THREADS) void k_small(const KeyT<KB> *__restr
                 break;
             const bool valid = wave0 + r * 64u + lane < n;
             const uint32_t d = (uint32_t)(it_cell(item[r], pk) >> shift) & dmask;
-            uint64_t m = __ballot(valid);
-#pragma unroll
-            for (int bit = 0; bit < 8; ++bit) {
-                if (bit < dbits) {
-                    const bool on = (d >> bit) & 1u;
-                    const uint64_t bb = __ballot(on);
-                    m &= on ? bb : ~bb;
-                }
-            }
-            const uint32_t rank = (uint32_t)__popcll(m & lt);
-            const int leader = valid ? (int)__builtin_ctzll(m) : 0;
-            uint32_t run = 0;
-            if (valid && rank == 0)
-                run = atomicAdd(&s_wh[wv][d], (uint32_t)__popcll(m));
-            run = (uint32_t)__shfl((int)run, leader, 64);
-            dr[r] = d | ((run + rank) << 8);
+            dr[r] = d | wave_digit_rank(s_wh[wv], d, __ballot(valid), valid) << 8;
         }
         __syncthreads();
         // thread d < OS_BINS: digit d's start and each wavefront's within it
@@ -2393,7 +2381,9 @@ static int sort_chunk(qs_sketch *s, const KeyT<KB> *keys, uint32_t cn, uint64_t 
     const int bits = (int)(s->pk.bb + s->pk.sb);
     const int passes = (bits + 7) / 8;
     const int dbits = (bits + passes - 1) / passes; // <= 8
-    const uint32_t nbins = 1u << dbits, dmask = nbins - 1u;
+    const uint32_t nbins = 1u << dbits;
+    // (the digits of an item: the last pass's stops with the cell)
+    auto digit_mask = [&](int ps) { return (1u << (bits - dbits * ps < dbits ? bits - dbits * ps : dbits)) - 1u; };
     const uint32_t ngrp = (ntiles + SCAN_TPB - 1) / SCAN_TPB;
     const qs_scratch &sc = *bc.sc;
     uint16_t *tcount = reinterpret_cast<uint16_t *>(sc.hist); // 16-bit tile counts (half the region)
@@ -2407,6 +2397,7 @@ static int sort_chunk(qs_sketch *s, const KeyT<KB> *keys, uint32_t cn, uint64_t 
     for (int ps = 0; ps < passes; ++ps) {
         const int shift = dbits * ps;
         const int nshift = ps + 1 < passes ? shift + dbits : -1; // the scatter writes the next digit
+        const uint32_t dmask = digit_mask(ps), ndmask = nshift >= 0 ? digit_mask(ps + 1) : 0u;
         qs_evpair e0, e1, e2;
         if (bc.timed) {
             if (ps == 0)
@@ -2432,11 +2423,11 @@ static int sort_chunk(qs_sketch *s, const KeyT<KB> *keys, uint32_t cn, uint64_t 
         if (ps == 0)
             hipLaunchKernelGGL((k_bs_down<KB, true, MULTI>), dim3(ntiles), dim3(OS_THREADS), 0, stream, in, cn,
                                base, d0, s->d_desc, bc.d_offs, s->nsk, s->pk, shift, dmask, nbins, ntiles,
-                               tcount, gsum, totals, scan, sc.it[out], sc.dig, nshift, s->d_st);
+                               tcount, gsum, totals, scan, sc.it[out], sc.dig, nshift, ndmask, s->d_st);
         else
             hipLaunchKernelGGL((k_bs_down<KB, false, false>), dim3(ntiles), dim3(OS_THREADS), 0, stream, in, cn,
                                base, d0, s->d_desc, bc.d_offs, s->nsk, s->pk, shift, dmask, nbins, ntiles,
-                               tcount, gsum, totals, scan, sc.it[out], sc.dig, nshift, s->d_st);
+                               tcount, gsum, totals, scan, sc.it[out], sc.dig, nshift, ndmask, s->d_st);
         if (bc.timed) {
             if (ps + 1 == passes)
                 qs_tim_end(s, e2, stream);

@@ -203,7 +203,7 @@ __device__ static inline uint32_t sf_block_excl_scan(uint32_t v, uint32_t *s_red
 // Stable scatter of one tile.  Each wavefront ranks its keys round by round:
 // one ballot per digit bit gives every lane the lanes sharing its digit, and
 // the group's lowest lane advances the wavefront's running count of the
-// digit.  The tile is staged digit-sorted in LDS and written as contiguous
+// digit (wave_digit_rank).  The tile is staged digit-sorted in LDS and written as contiguous
 // digit runs.  hist holds the exclusive tile prefixes of every digit and
 // totals the digit totals (qs_scan_digits).
 template <int KB>
@@ -216,7 +216,6 @@ __global__ __launch_bounds__(SF_THREADS) void k_sfs_down(const KeyT<KB> *__restr
     using C = sfs_tile<KB>;
     __shared__ KeyT<KB> s_item[C::TILE];
     __shared__ uint32_t s_wh[SF_WAVES][256];
-    __shared__ uint32_t s_ls[256];
     __shared__ uint32_t s_goff[256];
     __shared__ uint32_t s_red[SF_WAVES];
     const uint32_t t = threadIdx.x, lane = t & 63u, wv = t >> 6;
@@ -229,9 +228,8 @@ __global__ __launch_bounds__(SF_THREADS) void k_sfs_down(const KeyT<KB> *__restr
     const uint32_t hcur = dv ? hist[(size_t)t * ntiles + tile] : 0u;
     const uint32_t dbase = sf_block_excl_scan(dv ? totals[t] : 0u, s_red);
 
-    const uint64_t lt = (1ull << lane) - 1ull;
     KeyT<KB> key[C::IPL];
-    uint32_t dr[C::IPL]; // digit | wave-local position << 8 | valid << 31
+    uint32_t dr[C::IPL]; // digit | wave-local position << 8
 #pragma unroll
     for (int r = 0; r < C::IPL; ++r) {
         const uint32_t i = tb + wv * C::WAVE_ITEMS + r * 64u + lane;
@@ -242,54 +240,60 @@ __global__ __launch_bounds__(SF_THREADS) void k_sfs_down(const KeyT<KB> *__restr
         const uint32_t i = tb + wv * C::WAVE_ITEMS + r * 64u + lane;
         const bool valid = i < n;
         const uint32_t d = sfs_digit<KB>(key[r], p, shift, dmask);
-        uint64_t m = __ballot(valid);
-#pragma unroll
-        for (int bit = 0; bit < 8; ++bit) {
-            if ((dmask >> bit) & 1u) { // uniform: the digit width is a launch argument
-                const bool on = (d >> bit) & 1u;
-                const uint64_t bb = __ballot(on);
-                m &= on ? bb : ~bb;
-            }
-        }
-        const uint32_t rank = (uint32_t)__popcll(m & lt);
-        const int leader = valid ? (int)__builtin_ctzll(m) : 0;
-        uint32_t run = 0;
-        if (valid && rank == 0)
-            run = atomicAdd(&s_wh[wv][d], (uint32_t)__popcll(m));
-        run = (uint32_t)__shfl((int)run, leader, 64);
-        dr[r] = d | ((run + rank) << 8) | (valid ? 0x80000000u : 0u);
+        dr[r] = d | wave_digit_rank(s_wh[wv], d, __ballot(valid), valid) << 8;
     }
     __syncthreads();
     {
-        // per-wavefront counts -> each wavefront's start within the digit
-        uint32_t cnt = 0;
+        // per-wavefront counts -> each wavefront's start within the tile
+        uint32_t cnt = 0, c[SF_WAVES];
 #pragma unroll
         for (int w = 0; w < SF_WAVES; ++w) {
-            const uint32_t c = s_wh[w][t];
-            s_wh[w][t] = cnt;
-            cnt += c;
+            c[w] = s_wh[w][t];
+            cnt += c[w];
         }
         const uint32_t lstart = sf_block_excl_scan(cnt, s_red);
-        s_ls[t] = lstart;
         s_goff[t] = dbase + hcur - lstart;
+        uint32_t at = lstart;
+#pragma unroll
+        for (int w = 0; w < SF_WAVES; ++w) {
+            s_wh[w][t] = at;
+            at += c[w];
+        }
     }
     __syncthreads();
 #pragma unroll
     for (int r = 0; r < C::IPL; ++r)
-        if (dr[r] & 0x80000000u) {
-            const uint32_t d = dr[r] & 0xffu;
-            s_item[s_ls[d] + s_wh[wv][d] + ((dr[r] >> 8) & 0x7fffffu)] = key[r];
-        }
+        if (tb + wv * C::WAVE_ITEMS + r * 64u + lane < n)
+            s_item[s_wh[wv][dr[r] & 0xffu] + (dr[r] >> 8)] = key[r];
     __syncthreads();
     const uint32_t tn = (n - tb) < C::TILE ? (n - tb) : C::TILE;
-    for (uint32_t q = t; q < tn; q += SF_THREADS) {
-        const KeyT<KB> k = s_item[q];
-        const uint32_t dst = s_goff[sfs_digit<KB>(k, p, shift, dmask)] + q;
-        if (dst < n) // the tile counts and the ranking agree; checked, never trusted
-            out[dst] = k;
-        else
-            atomicOr(err, 1u);
-    }
+    // (the tile counts and the ranking agree; checked, never trusted)
+    bool bad = false;
+    if (tn == C::TILE) { // every LDS read of a whole tile's rounds in flight together
+        uint32_t dst[C::IPL];
+#pragma unroll
+        for (uint32_t r = 0; r < C::IPL; ++r)
+            key[r] = s_item[r * SF_THREADS + t];
+#pragma unroll
+        for (uint32_t r = 0; r < C::IPL; ++r) {
+            dst[r] = s_goff[sfs_digit<KB>(key[r], p, shift, dmask)] + r * SF_THREADS + t;
+            bad = bad || dst[r] >= n;
+        }
+        if (!bad)
+#pragma unroll
+            for (uint32_t r = 0; r < C::IPL; ++r)
+                out[dst[r]] = key[r];
+    } else
+        for (uint32_t q = t; q < tn; q += SF_THREADS) {
+            const KeyT<KB> k = s_item[q];
+            const uint32_t dst = s_goff[sfs_digit<KB>(k, p, shift, dmask)] + q;
+            if (dst < n)
+                out[dst] = k;
+            else
+                bad = true;
+        }
+    if (bad)
+        atomicOr(err, 1u);
 }
 
 // ===========================================================================

@@ -1,5 +1,5 @@
 """Batched inserts whose sketches begin and end on the edges of the first radix
-pass's tiles (2048 keys): tiles of one sketch, of several, of more than the window of
+pass's tiles (4096 keys, and halves of them): tiles of one sketch, of several, of more than the window of
 64 holds, empty sketches between them, and sets that the search for a tile's
 sketches takes one, two and three rounds of 64 offsets to search."""
 from __future__ import annotations
@@ -14,7 +14,9 @@ pytestmark = pytest.mark.gpu
 
 LENGTHS = {
     "edges": [2048, 1, 2047, 4096, 0, 2049, 0, 0, 2047, 6143, 1],
+    "edges_whole": [4096, 1, 4095, 8192, 0, 4097, 0, 0, 4095, 12287, 1],
     "window_63_64_65": [32] * 64 + [2048] + [31] * 64 + [64] + [31, 30] * 33 + [33],
+    "window_whole": [64] * 64 + [4096] + [63] * 64 + [64] + [63, 62] * 33 + [65],
     "two_rounds": [0] * 63 + [5000] + [0] * 200 + [3000, 1, 0, 4095] + [7] * 300,
     "three_rounds": [1] * 2100 + [0] * 1500 + [4100, 0, 2] + [1] * 700,
 }
