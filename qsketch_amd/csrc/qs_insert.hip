@@ -2446,7 +2446,11 @@ template <bool MULTI, int W, int IPL>
 static void launch_segw(qs_sketch *s, const qs_scratch &sc, const uint64_t *IT, uint32_t cn, hipStream_t stream)
 {
     const uint64_t groups = ((uint64_t)cn + W * IPL - 1) / (W * IPL);
-    hipLaunchKernelGGL((k_segw<MULTI, W, IPL>), dim3(grid_cap((groups * W + SEG_THREADS - 1) / SEG_THREADS, 8)),
+    // Three blocks of the default shape fit a CU: 8 per CU left its last third of a
+    // round half empty, and 24 even out the windows' uneven cost (2^28 Zipf 1.1 keys: 1225
+    // and 1153 us, 75 M keys of 512 sketches 1020 and 970; 16, 32 and 48 lie between
+    // or level, and a window per wavefront, without the loads ahead, takes 1243 and 1067).
+    hipLaunchKernelGGL((k_segw<MULTI, W, IPL>), dim3(grid_cap((groups * W + SEG_THREADS - 1) / SEG_THREADS, 24)),
                        dim3(SEG_THREADS), 0, stream, IT, cn, s->d_desc, s->h_desc[0].n_masks, s->d_low, s->d_high,
                        s->d_masks, s->pk, s->d_longbm, sc.ord, sc.lng, s->d_st);
 }
