@@ -53,7 +53,8 @@
 #define SF_WAVES (SF_THREADS / 64)
 #define SF_ROW_WAVES 8192u      // wavefronts of k_sf_rows (32 per CU)
 #define SF_ROW_SPREAD 4096u     // work items that a short call is cut into
-#define SF_ROW_RANGE 4096u     // most keys per work item of k_sf_rows
+#define SF_ROW_RANGE 4096u      // most keys per work item of k_sf_rows
+#define SF_ROW_RANGE_COLD 512u  // and of a call whose frequent keys the filter took out
 #define SF_SORT_MIN (1u << 16)  // shorter inserts are applied unsorted
 #define SF_TILE_SMALL_MAX (1u << 17) // up to here the unsorted tiles hold 512 keys, then 2048
 #define SF_CHUNK4 (1u << 28)    // keys per radix chunk: 4-byte keys
@@ -854,21 +855,26 @@ static uint32_t sf_grid(uint64_t want)
 // after the other, so short calls take short ranges that occupy the chip; long
 // ones take the longest (each range's first and last bucket are shared, and
 // cost atomics).  Ranges of 4096 keys whatever the call took 290 us for 65536
-// keys (16 wavefronts), now 90.
-static uint64_t sf_range(uint64_t n)
+// keys (16 wavefronts), now 90.  Keys that come from the hot-key filter have no
+// frequent one left among them, whose bucket would be shared by thousands of ranges,
+// and are walked by twice the wavefronts in ranges of 512: 17 M keys 632 -> 531 us
+// (1024: 557, 2048: 590; unfiltered, 2^24 keys of Zipf 1.5 would take 789 us for 456).
+static uint64_t sf_range(uint64_t n, bool cold)
 {
+    const uint64_t most = cold ? SF_ROW_RANGE_COLD : SF_ROW_RANGE;
     const uint64_t r = (n / SF_ROW_SPREAD + 63) / 64 * 64;
-    return r < 64 ? 64 : r < SF_ROW_RANGE ? r : SF_ROW_RANGE;
+    return r < 64 ? 64 : r < most ? r : most;
 }
 
-// most ranges of any call of at most n keys
+// most ranges of any call of at most n keys (sf_range(m) is the longest, or a
+// multiple 64k of 64 with m < (64k + 1) * SPREAD)
 static uint64_t sf_max_ranges(uint64_t n)
 {
-    const uint64_t a = (n + SF_ROW_RANGE - 1) / SF_ROW_RANGE, b = (n + 63) / 64;
-    return a > SF_ROW_WAVES ? a : b < SF_ROW_WAVES ? b : SF_ROW_WAVES;
+    const uint64_t a = (n + SF_ROW_RANGE_COLD - 1) / SF_ROW_RANGE_COLD, b = (n + 63) / 64;
+    const uint64_t c = SF_ROW_SPREAD + SF_ROW_SPREAD / 64 + 1;
+    return a > c ? a : b < c ? b : c;
 }
 
-// radix scratch for chunks of up to `keys` keys (kept across calls)
 static int sf_ensure_scratch(qs_sf *s, uint64_t keys)
 {
     if (keys <= s->scratch_keys)
@@ -902,11 +908,11 @@ static int sf_ensure_scratch(qs_sf *s, uint64_t keys)
 // k_sf_tile (owned = false: any order, all atomics) or k_sf_rows (owned =
 // true: keys sorted by bucket)
 template <int KB>
-static void sf_launch_flush(qs_sf *s, const sf_par &p, const KeyT<KB> *keys, uint64_t n, bool owned)
+static void sf_launch_flush(qs_sf *s, const sf_par &p, const KeyT<KB> *keys, uint64_t n, bool owned, bool cold)
 {
     const dim3 block(SF_THREADS);
     if (owned) {
-        const uint64_t range = sf_range(n), ranges = (n + range - 1) / range;
+        const uint64_t range = sf_range(n, cold), ranges = (n + range - 1) / range;
         const uint64_t w = ranges < SF_ROW_WAVES ? ranges : SF_ROW_WAVES;
         (void)hipMemsetAsync(s->d_err + 1, 0, 4, 0);
         const dim3 g((uint32_t)((w + SF_WAVES - 1) / SF_WAVES));
@@ -934,7 +940,8 @@ static void sf_launch_flush(qs_sf *s, const sf_par &p, const KeyT<KB> *keys, uin
 }
 
 // one chunk: sort by bucket (8-bit digits at most), then flush
-template <int KB> static int sf_insert_chunk(qs_sf *s, const sf_par &p, const KeyT<KB> *keys, uint32_t cn);
+template <int KB>
+static int sf_insert_chunk(qs_sf *s, const sf_par &p, const KeyT<KB> *keys, uint32_t cn, bool cold);
 
 // One chunk of 4-byte keys through the hot-key filter: the frequent keys are
 // counted in LDS and added once each (k_sf_hot_flush), only the cold keys
@@ -950,7 +957,7 @@ static int sf_insert_hot(qs_sf *s, const sf_par &p, const uint32_t *keys, uint32
     if (hs.ncold > cn)
         return QS_ERR_INTERNAL;
     if (hs.ncold) {
-        rc = sf_insert_chunk<4>(s, p, hs.cold, (uint32_t)hs.ncold);
+        rc = sf_insert_chunk<4>(s, p, hs.cold, (uint32_t)hs.ncold, true);
         if (rc)
             return rc;
     }
@@ -960,11 +967,12 @@ static int sf_insert_hot(qs_sf *s, const sf_par &p, const uint32_t *keys, uint32
     return QS_OK;
 }
 
-template <int KB> static int sf_insert_chunk(qs_sf *s, const sf_par &p, const KeyT<KB> *keys, uint32_t cn)
+template <int KB>
+static int sf_insert_chunk(qs_sf *s, const sf_par &p, const KeyT<KB> *keys, uint32_t cn, bool cold)
 {
     const int bits = s->n > 1 ? 64 - __builtin_clzll(s->n - 1) : 0; // bits of the largest bucket
     if (cn < SF_SORT_MIN || bits == 0) { // unsorted (one bucket: nothing to sort)
-        sf_launch_flush<KB>(s, p, keys, cn, false);
+        sf_launch_flush<KB>(s, p, keys, cn, false, cold);
         CK(hipGetLastError());
         return QS_OK;
     }
@@ -983,7 +991,7 @@ template <int KB> static int sf_insert_chunk(qs_sf *s, const sf_par &p, const Ke
                            ntiles, s->d_hist, totals, out, s->d_err);
         in = out;
     }
-    sf_launch_flush<KB>(s, p, in, cn, true);
+    sf_launch_flush<KB>(s, p, in, cn, true, cold);
     CK(hipGetLastError());
     return QS_OK;
 }
@@ -1007,9 +1015,9 @@ extern "C" int qs_sf_insert(qs_sf *s, const void *d_keys, size_t n)
         if (s->key_bytes == 4) {
             rc = sf_insert_hot(s, p, static_cast<const uint32_t *>(d_keys) + off, cn, &done);
             if (rc == QS_OK && !done)
-                rc = sf_insert_chunk<4>(s, p, static_cast<const uint32_t *>(d_keys) + off, cn);
+                rc = sf_insert_chunk<4>(s, p, static_cast<const uint32_t *>(d_keys) + off, cn, false);
         } else {
-            rc = sf_insert_chunk<8>(s, p, static_cast<const uint64_t *>(d_keys) + off, cn);
+            rc = sf_insert_chunk<8>(s, p, static_cast<const uint64_t *>(d_keys) + off, cn, false);
         }
         if (rc != QS_OK)
             return rc;

@@ -38,3 +38,18 @@ def test_sf_work_split(gpu, key_bytes, times, n, n_buckets):
         assert np.array_equal(st["search"], o.search())
     uq = np.unique(keys)
     assert np.array_equal(to_host_u32(g.search(to_dev(uq))), o.query(uq))
+
+
+@pytest.mark.parametrize("n", [4096 * 65 - 1, 4096 * 65, 4096 * 449 - 63, 8192 * 512 + 4097])
+def test_sf_most_ranges(gpu, n):
+    """The most ranges of 64 keys, and the longest ranges, more than the wavefronts."""
+    import qsketch_amd as q
+    print("CASE sf ranges", n, flush=True)
+    keys = q.Zipf(0.8, 1 << 20, device=False).keys_u32_host(n, n)
+    g = q.Sketch_GPU_SF_Host_Sub_Warp(98297, 8, 3, 1, 1021, rng_seed=11)
+    o = po.OracleSF(98297, 8, 3, 1021, rng_seed=11)
+    g.insert(to_dev(keys))
+    o.insert(keys)
+    st = g.export_state()
+    assert np.array_equal(st["split"], o.split())
+    assert np.array_equal(st["search"], o.search())
