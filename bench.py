@@ -287,9 +287,9 @@ def main():
             "bound": "hbm",
             "kernel": "insert path: on the prefix and on the cold keys, per radix pass k_bs_up (first "
                       "pass) or k_bs_up_dig, k_hist_scan_local, k_hist_scan_groups, k_bs_down; then k_segw, "
-                      "k_ordered, k_trig_keys + pair sort, k_assign, k_tail, k_clear_long, k_next, k_reset; "
+                      "k_ordered, k_trig_scan, k_assign, k_tail, k_finish; "
                       "between them the hot-key filter (k_hot_build, k_hot_count, k_scan_*, k_hot_move, "
-                      "k_hot_flush).  The filter's candidate sample sort runs on a second stream beside the "
+                      "k_hot_flush).  The filter's candidate kernels run on a second stream beside the "
                       "prefix; any wait for it is counted in the filter's time",
             "achieved": round(achieved, 1),
             "peak": HBM_PEAK_GBS,

@@ -118,10 +118,10 @@ __device__ static inline uint32_t sid_chunk_start(const uint64_t *__restrict__ o
 #define OS_WAVES (OS_THREADS / 64)
 // Tiles of 512 * 8 items: a digit's run in a tile is what a scatter writes at a
 // time, 16 items of an 8-byte item's 128-byte line for 8-bit digits, and 24 wavefronts per
-// CU are still in flight.  A later pass of 134 M items (7-bit digits): 480 us with
-// 256 threads, 384 with 512, 556 with 1024 (one block per CU), 380 with 512 of 16
+// CU are still in flight.  A later pass of 134 M items (7-bit digits): 576 us with
+// 256 threads, 460 with 512, 668 with 1024 (one block per CU), 456 with 512 of 16
 // items, which loses elsewhere (a pass of 75 M items with 8-bit digits: 325, 297, 412, 302).
-// Non-temporal stores take 550: the runs of neighbouring tiles meet in the L2.
+// Non-temporal stores take 660: the runs of neighbouring tiles meet in the L2.
 #ifndef QS_OS_IPL
 #define QS_OS_IPL 8
 #endif
