@@ -241,8 +241,8 @@ int qs_multi_import_state(qs_sketch *s, uint32_t sketch, const uint32_t *low, co
  * graph reads d_keys and d_offs at replay time, so the caller may refill them
  * between replays with the same layout h_offs.  Destroy graphs before their
  * set; while a graph lives, import is refused (QS_ERR_STATE: the graph holds
- * the hash parameters) and so is a later batch that needs larger scratch
- * buffers than the graph's.  Build addition with no reference counterpart. */
+ * the hash parameters) and so is a later batch (inserted or captured) that
+ * needs larger scratch buffers than the graph's.  Build addition with no reference counterpart. */
 typedef struct qs_graph qs_graph;
 int qs_graph_capture_insert(qs_sketch *s, const void *d_keys, const uint64_t *h_offs,
                             const uint64_t *d_offs, qs_graph **out);

@@ -2346,6 +2346,8 @@ int qs_ensure_scratch(qs_sketch *s, uint64_t chunk)
     grid_cap(0, 1); // query the CU count now: never while a launch sequence is captured
     if (s->sc.chunk >= chunk)
         return QS_OK;
+    if (s->graphs > 0)
+        return QS_ERR_STATE; // a captured graph holds the current scratch buffers
     qs_free_scratch(s);
     const uint32_t tcap = qs_trig_cap(s, chunk);
     qs_scratch &sc = s->sc;
@@ -2620,8 +2622,6 @@ static int insert_impl(qs_sketch *s, const void *d_keys, const uint64_t *offs, c
         if (n > cap || n > fixed->chunk || qs_trig_cap(s, n) > fixed->trig_cap)
             return QS_ERR_PARAM;
     } else {
-        if (s->sc.chunk < need && s->graphs > 0)
-            return QS_ERR_STATE; // a captured graph holds the current scratch buffers
         rc = qs_ensure_scratch(s, need);
         if (rc)
             return rc;

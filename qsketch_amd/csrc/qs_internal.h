@@ -435,6 +435,8 @@ uint64_t qs_scan_sums(uint64_t n);
 // batch must then fit one chunk of it.
 int qs_insert_set(qs_sketch *s, const void *d_keys, const uint64_t *offs, const uint64_t *d_offs,
                   hipStream_t stream, bool blocking, bool capture, const qs_scratch *fixed = nullptr);
+// the handle's own scratch for chunks of `chunk` keys: grown if it is smaller, which
+// every caller is refused (QS_ERR_STATE) while a captured graph lives
 int qs_ensure_scratch(qs_sketch *s, uint64_t chunk);
 // allocation entries the insert scratch needs for a chunk of `chunk` keys
 uint32_t qs_trig_cap(const qs_sketch *s, uint64_t chunk);

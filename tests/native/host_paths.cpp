@@ -1,0 +1,222 @@
+// Host paths of the library on a HIP runtime made of host memory: the functions
+// below stand in for the runtime's (the executable's definitions come first), so
+// allocations can be made to fail, a second device can be current, and what is
+// launched, allocated and freed is known.  No kernel runs.  usage: host_paths CASE
+#include <hip/hip_runtime_api.h>
+#include <dlfcn.h>
+
+#include <cstdio>
+#include <cstdlib>
+#include <cstring>
+#include <map>
+#include <string>
+#include <vector>
+
+#include "../../include/qsketch.h"
+
+namespace {
+struct launch {
+    std::string kernel;
+    int device;
+};
+int g_device = 0;                    // current device
+uint64_t g_mallocs = 0, g_frees = 0; // device allocations made, live ones freed
+uint64_t g_fail_at = 0;              // the allocation of this number fails (0: none)
+hipError_t g_last = hipSuccess;      // sticky, as the runtime's
+std::map<void *, size_t> g_live;
+std::vector<launch> g_launches;
+uint64_t g_handles = 0;
+
+hipError_t fail(hipError_t e)
+{
+    g_last = e;
+    return e;
+}
+
+int g_bad = 0;
+void expect(bool ok, const char *what)
+{
+    if (!ok) {
+        printf("FAILED: %s\n", what);
+        g_bad = 1;
+    }
+}
+} // namespace
+
+extern "C" {
+hipError_t hipMalloc(void **p, size_t bytes)
+{
+    *p = nullptr;
+    if (++g_mallocs == g_fail_at)
+        return fail(hipErrorOutOfMemory);
+    *p = calloc(bytes ? bytes : 1, 1);
+    g_live[*p] = bytes;
+    return hipSuccess;
+}
+hipError_t hipFree(void *p)
+{
+    if (!p)
+        return hipSuccess;
+    if (!g_live.erase(p))
+        return fail(hipErrorInvalidValue);
+    ++g_frees;
+    free(p);
+    return hipSuccess;
+}
+hipError_t hipHostMalloc(void **p, size_t bytes, unsigned int)
+{
+    *p = calloc(bytes, 1);
+    return hipSuccess;
+}
+hipError_t hipHostFree(void *p)
+{
+    free(p);
+    return hipSuccess;
+}
+hipError_t hipMemcpy(void *d, const void *s, size_t n, hipMemcpyKind)
+{
+    memcpy(d, s, n);
+    return hipSuccess;
+}
+hipError_t hipMemcpyAsync(void *d, const void *s, size_t n, hipMemcpyKind, hipStream_t)
+{
+    memcpy(d, s, n);
+    return hipSuccess;
+}
+hipError_t hipMemset(void *d, int v, size_t n)
+{
+    memset(d, v, n);
+    return hipSuccess;
+}
+hipError_t hipMemsetAsync(void *d, int v, size_t n, hipStream_t)
+{
+    memset(d, v, n);
+    return hipSuccess;
+}
+hipError_t hipGetDeviceCount(int *n)
+{
+    *n = 2;
+    return hipSuccess;
+}
+hipError_t hipGetDevice(int *d)
+{
+    *d = g_device;
+    return hipSuccess;
+}
+hipError_t hipSetDevice(int d)
+{
+    g_device = d;
+    return hipSuccess;
+}
+hipError_t hipDeviceGetAttribute(int *v, hipDeviceAttribute_t, int)
+{
+    *v = 256;
+    return hipSuccess;
+}
+hipError_t hipGetDeviceProperties(hipDeviceProp_t *p, int) // (a macro names the current version of it)
+{
+    memset(p, 0, sizeof(*p));
+    p->multiProcessorCount = 256;
+    return hipSuccess;
+}
+hipError_t hipDeviceSynchronize() { return hipSuccess; }
+hipError_t hipStreamSynchronize(hipStream_t) { return hipSuccess; }
+hipError_t hipStreamQuery(hipStream_t) { return hipSuccess; }
+hipError_t hipStreamWaitEvent(hipStream_t, hipEvent_t, unsigned int) { return hipSuccess; }
+hipError_t hipStreamCreateWithFlags(hipStream_t *s, unsigned int)
+{
+    *s = reinterpret_cast<hipStream_t>(++g_handles);
+    return hipSuccess;
+}
+hipError_t hipStreamDestroy(hipStream_t) { return hipSuccess; }
+hipError_t hipEventCreateWithFlags(hipEvent_t *e, unsigned)
+{
+    *e = reinterpret_cast<hipEvent_t>(++g_handles);
+    return hipSuccess;
+}
+hipError_t hipEventDestroy(hipEvent_t) { return hipSuccess; }
+hipError_t hipEventRecord(hipEvent_t, hipStream_t) { return hipSuccess; }
+hipError_t hipStreamBeginCapture(hipStream_t, hipStreamCaptureMode) { return hipSuccess; }
+hipError_t hipStreamEndCapture(hipStream_t, hipGraph_t *g)
+{
+    *g = reinterpret_cast<hipGraph_t>(++g_handles);
+    return hipSuccess;
+}
+hipError_t hipGraphInstantiate(hipGraphExec_t *x, hipGraph_t, hipGraphNode_t *, char *, size_t)
+{
+    *x = reinterpret_cast<hipGraphExec_t>(++g_handles);
+    return hipSuccess;
+}
+hipError_t hipGraphDestroy(hipGraph_t) { return hipSuccess; }
+hipError_t hipGraphExecDestroy(hipGraphExec_t) { return hipSuccess; }
+hipError_t hipGetLastError()
+{
+    const hipError_t e = g_last;
+    g_last = hipSuccess;
+    return e;
+}
+hipError_t __hipPushCallConfiguration(dim3, dim3, size_t, hipStream_t) { return hipSuccess; }
+hipError_t __hipPopCallConfiguration(dim3 *g, dim3 *b, size_t *shared, hipStream_t *s)
+{
+    *g = dim3(1);
+    *b = dim3(1);
+    *shared = 0;
+    *s = nullptr;
+    return hipSuccess;
+}
+hipError_t hipLaunchKernel(const void *f, dim3, dim3, void **, size_t, hipStream_t)
+{
+    Dl_info info;
+    g_launches.push_back({dladdr(f, &info) && info.dli_sname ? info.dli_sname : "?", g_device});
+    return hipSuccess;
+}
+} // extern "C"
+
+static qs_params params(uint64_t n_low)
+{
+    qs_params p;
+    qs_default_params(&p, 1 << 16, 0.5);
+    p.n_low = n_low;
+    p.rng_seed = 1;
+    return p;
+}
+
+static uint32_t s_keys[1]; // stands for device keys: nothing reads them
+
+// While a captured graph lives, nothing may free the scratch it holds: a batch
+// that needs more is refused, whichever way it comes.
+static void case_graph()
+{
+    const qs_params p = params(1021);
+    qs_sketch *s = nullptr;
+    qs_graph *g = nullptr, *g2 = nullptr;
+    expect(qs_create(&p, &s) == QS_OK, "create");
+    const uint64_t small[2] = {0, 1500}, less[2] = {0, 1000}, more[2] = {0, 1501};
+    expect(qs_graph_capture_insert(s, s_keys, small, nullptr, &g) == QS_OK, "capture");
+    const uint64_t frees = g_frees;
+    expect(qs_graph_capture_insert(s, s_keys, more, nullptr, &g2) == QS_ERR_STATE && !g2, "larger capture refused");
+    expect(qs_insert(s, s_keys, 1501) == QS_ERR_STATE, "larger insert refused");
+    expect(qs_insert_async(s, s_keys, 1501, nullptr) == QS_ERR_STATE, "larger stream-ordered insert refused");
+    expect(qs_insert(s, s_keys, 1ull << 26) == QS_ERR_STATE, "filtered insert refused");
+    expect(g_frees == frees, "the graph's scratch is still allocated");
+    expect(qs_graph_capture_insert(s, s_keys, less, nullptr, &g2) == QS_OK, "smaller capture");
+    expect(qs_insert(s, s_keys, 1500) == QS_OK, "insert that fits");
+    qs_graph_destroy(g);
+    expect(qs_insert(s, s_keys, 1501) == QS_ERR_STATE, "refused while the second graph lives");
+    qs_graph_destroy(g2);
+    expect(qs_insert(s, s_keys, 1501) == QS_OK, "accepted without graphs");
+    qs_destroy(s);
+    expect(g_live.empty(), "everything freed");
+}
+
+int main(int argc, char **argv)
+{
+    const std::map<std::string, void (*)()> cases = {
+        {"graph", case_graph},
+    };
+    const auto c = cases.find(argc > 1 ? argv[1] : "");
+    if (c == cases.end())
+        return 2;
+    c->second();
+    return g_bad;
+}
