@@ -802,7 +802,6 @@ static int hot_alloc(void **state, uint64_t rest)
         h = (qs_hot *)calloc(1, sizeof(qs_hot));
         if (!h)
             return QS_ERR_NOMEM;
-        *state = h;
         int dev = 0, cu = 0;
         if (hipGetDevice(&dev) != hipSuccess ||
             hipDeviceGetAttribute(&cu, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cu <= 0)
@@ -821,18 +820,19 @@ static int hot_alloc(void **state, uint64_t rest)
              hipStreamCreateWithFlags(&h->side, hipStreamNonBlocking) == hipSuccess &&
              hipEventCreateWithFlags(&h->ev_fork, hipEventDisableTiming) == hipSuccess &&
              hipEventCreateWithFlags(&h->ev_cand, hipEventDisableTiming) == hipSuccess;
-        if (ok) {
-            h->scnt = h->samp + HOT_SAMPLE;
-            h->ccount = h->scnt + (SAMP_TILES + 2u) * SAMP_BINS;
-            h->ck = h->ccount + SAMP_COUNTS;
-            h->cv = h->ck + HOT_CAND_MAX;
-            h->cand = h->cv + HOT_CAND_MAX;
-            h->ccnt = h->cand + HOT_MAX;
-            memset(h->h_ctl, 0, 4ull * HOT_PUB_WORDS);
-            h->seq = 0;
-        }
-        if (!ok)
+        if (!ok) { // nothing half built is kept: a later call starts over
+            qs_hot_state_free(h);
             return QS_ERR_NOMEM;
+        }
+        h->scnt = h->samp + HOT_SAMPLE;
+        h->ccount = h->scnt + (SAMP_TILES + 2u) * SAMP_BINS;
+        h->ck = h->ccount + SAMP_COUNTS;
+        h->cv = h->ck + HOT_CAND_MAX;
+        h->cand = h->cv + HOT_CAND_MAX;
+        h->ccnt = h->cand + HOT_MAX;
+        memset(h->h_ctl, 0, 4ull * HOT_PUB_WORDS);
+        h->seq = 0;
+        *state = h;
     }
     const uint64_t chunks = (rest + HOT_CHUNK - 1) / HOT_CHUNK;
     if (h->chunk_cap < chunks) {

@@ -209,11 +209,40 @@ static void case_graph()
     expect(g_live.empty(), "everything freed");
 }
 
+// An allocation of the hot-key filter that fails leaves nothing half built: the call
+// after it allocates everything, as the first call of another sketch does.
+static void case_hot_alloc()
+{
+    const uint64_t n = 1ull << 26;
+    const qs_params p = params(1021);
+    uint64_t whole = 0; // allocations of a first filtered call
+    for (uint64_t k = 0; k <= 7; ++k) { // the k-th of the filter's own fails (0: none)
+        qs_sketch *s = nullptr;
+        expect(qs_create(&p, &s) == QS_OK, "create");
+        const size_t live = g_live.size();
+        if (k) {
+            g_fail_at = g_mallocs + k;
+            expect(qs_insert(s, s_keys, n) == QS_ERR_NOMEM, "a failed allocation is reported");
+            expect(g_live.size() == live, "what was allocated before it is freed");
+            g_fail_at = 0;
+            (void)hipGetLastError();
+        }
+        const uint64_t before = g_mallocs;
+        expect(qs_insert(s, s_keys, n) == QS_ERR_HIP, "no kernel publishes the candidates here");
+        whole = k ? whole : g_mallocs - before;
+        expect(g_mallocs - before == whole, "the next call allocates everything");
+        qs_destroy(s);
+        expect(g_live.empty(), "everything freed");
+    }
+}
+
 int main(int argc, char **argv)
 {
     const std::map<std::string, void (*)()> cases = {
         {"graph", case_graph},
+        {"hot_alloc", case_hot_alloc},
     };
+    setvbuf(stdout, nullptr, _IONBF, 0);
     const auto c = cases.find(argc > 1 ? argv[1] : "");
     if (c == cases.end())
         return 2;
