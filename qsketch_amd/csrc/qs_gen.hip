@@ -166,6 +166,7 @@ extern "C" int qs_zipf_create(double alpha, uint64_t universe, int with_device, 
             hipMemcpy(z->d_alias, z->h_alias, sizeof(uint32_t) * U, hipMemcpyHostToDevice) !=
                 hipSuccess) {
             qs_zipf_destroy(z);
+            (void)hipGetLastError(); // (reported here: the next launch check must not meet it)
             return QS_ERR_HIP;
         }
     }

@@ -822,7 +822,7 @@ static int hot_alloc(void **state, uint64_t rest)
              hipEventCreateWithFlags(&h->ev_cand, hipEventDisableTiming) == hipSuccess;
         if (!ok) { // nothing half built is kept: a later call starts over
             qs_hot_state_free(h);
-            return QS_ERR_NOMEM;
+            return qs_alloc_failed();
         }
         h->scnt = h->samp + HOT_SAMPLE;
         h->ccount = h->scnt + (SAMP_TILES + 2u) * SAMP_BINS;
@@ -846,7 +846,7 @@ static int hot_alloc(void **state, uint64_t rest)
         if (hipMalloc(&h->ccold, 4ull * (chunks + 1)) != hipSuccess ||
             hipMalloc(&h->stage, 4ull * HOT_CHUNK * chunks) != hipSuccess ||
             hipMalloc(&h->bsum, 4ull * ((chunks + SCAN_SPAN - 1) / SCAN_SPAN + 1)) != hipSuccess)
-            return QS_ERR_NOMEM;
+            return qs_alloc_failed();
         h->chunk_cap = chunks;
     }
     if (h->cold_cap < rest) {
@@ -854,7 +854,7 @@ static int hot_alloc(void **state, uint64_t rest)
         h->cold = nullptr;
         h->cold_cap = 0;
         if (hipMalloc(&h->cold, 4ull * rest) != hipSuccess)
-            return QS_ERR_NOMEM;
+            return qs_alloc_failed();
         h->cold_cap = rest;
     }
     return QS_OK;

@@ -2354,16 +2354,16 @@ int qs_ensure_scratch(qs_sketch *s, uint64_t chunk)
     sc.trig_cap = tcap;
     for (int k = 0; k < 2; ++k)
         if (hipMalloc(&sc.it[k], sizeof(uint64_t) * chunk) != hipSuccess)
-            return QS_ERR_NOMEM;
+            return qs_alloc_failed();
     if (hipMalloc(&sc.tbit, tbit_bytes(chunk)) != hipSuccess ||
         hipMalloc(&sc.tsum, sizeof(uint32_t) * tsum_words(chunk)) != hipSuccess)
-        return QS_ERR_NOMEM;
+        return qs_alloc_failed();
     if (hipMalloc(&sc.hist, sizeof(uint32_t) * qs_scratch_hist_words(chunk)) != hipSuccess ||
         hipMalloc(&sc.dig, (chunk + OS_TILE - 1) / OS_TILE * OS_TILE) != hipSuccess ||
         hipMalloc(&sc.ord, sizeof(uint32_t) * chunk) != hipSuccess ||
         hipMalloc(&sc.lng, sizeof(uint32_t) * (chunk / 8 + 64)) != hipSuccess ||
         hipMalloc(&sc.trig, sizeof(qs_trig) * tcap) != hipSuccess)
-        return QS_ERR_NOMEM;
+        return qs_alloc_failed();
     sc.chunk = chunk;
     return QS_OK;
 }

@@ -304,6 +304,14 @@ static inline int qs_err_code(uint32_t err)
     return (err & QS_EF_SORT) ? QS_ERR_INTERNAL : err ? QS_ERR_POOL : QS_OK;
 }
 
+// The code of a failed device allocation.  The runtime keeps its last error until it
+// is read, so the next launch check (torch's too) would report this one: it is taken back.
+static inline int qs_alloc_failed()
+{
+    (void)hipGetLastError();
+    return QS_ERR_NOMEM;
+}
+
 struct qs_dev_state {
     uint32_t n_ord;     // bucket segments queued for the in-order replay
     uint32_t n_long;    // long bucket segments found by the segment pass (for the windowed tail kernel)

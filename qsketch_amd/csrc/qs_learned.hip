@@ -1228,7 +1228,7 @@ extern "C" int qs_learned_create(const qs_params *p, uint32_t table_log2, uint64
               hipHostMalloc(&L->h_pin, 16, hipHostMallocDefault) == hipSuccess;
     if (!ok) {
         qs_learned_destroy(L);
-        return QS_ERR_NOMEM;
+        return qs_alloc_failed();
     }
     L->d_err = L->d_bins + 2u * HBINS;
     L->d_g = L->d_part + (size_t)PART_STRIDE * GRAD_BLOCKS;
@@ -1429,7 +1429,7 @@ static int ensure_route(qs_learned *L, uint64_t n)
         hipMalloc(&L->d_bsum, 4ull * qs_scan_sums(chunks)) != hipSuccess ||
         hipMalloc(&L->d_stage, chunks * ROUTE_CHUNK * L->key_bytes) != hipSuccess ||
         hipMalloc(&L->d_light, n * L->key_bytes) != hipSuccess)
-        return QS_ERR_NOMEM;
+        return qs_alloc_failed();
     L->rcap = n;
     return QS_OK;
 }

@@ -833,7 +833,7 @@ extern "C" int qs_sf_create(uint64_t n, uint32_t m, uint32_t times, uint32_t see
               hipMalloc(&s->d_search, 4ull * cells) == hipSuccess;
     if (!ok) {
         qs_sf_destroy(s);
-        return QS_ERR_NOMEM;
+        return qs_alloc_failed();
     }
     if (hipMemcpy(s->d_masks, s->h_masks, 4ull * n_masks, hipMemcpyHostToDevice) != hipSuccess ||
         hipMemcpy(s->d_index, s->h_index, 4ull * n_masks, hipMemcpyHostToDevice) != hipSuccess ||
@@ -895,10 +895,10 @@ static int sf_ensure_scratch(qs_sf *s, uint64_t keys)
         hipMalloc(&s->d_buf[1], keys * s->key_bytes) != hipSuccess ||
         hipMalloc(&s->d_hist, 4ull * 256 * (ntiles + 1)) != hipSuccess ||
         hipMalloc(&s->d_shared, 8ull * sf_max_ranges(keys)) != hipSuccess)
-        return QS_ERR_NOMEM;
+        return qs_alloc_failed();
     if (!s->d_err) {
         if (hipMalloc(&s->d_err, 8) != hipSuccess)
-            return QS_ERR_NOMEM;
+            return qs_alloc_failed();
         CK(hipMemset(s->d_err, 0, 8));
     }
     s->scratch_keys = keys;

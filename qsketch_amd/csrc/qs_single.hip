@@ -217,7 +217,7 @@ extern "C" int qs_sl_create(uint64_t n, uint32_t m, uint32_t seed_sz, uint32_t n
     const size_t tbytes = (size_t)n * m * 4u;
     if (hipMalloc(&s->d_masks, n_masks * 4u) != hipSuccess || hipMalloc(&s->d_table, tbytes) != hipSuccess) {
         qs_sl_destroy(s);
-        return QS_ERR_NOMEM;
+        return qs_alloc_failed();
     }
     if (hipMemcpy(s->d_masks, s->h_masks, n_masks * 4u, hipMemcpyHostToDevice) != hipSuccess ||
         hipMemset(s->d_table, 0, tbytes) != hipSuccess || hipDeviceSynchronize() != hipSuccess) {

@@ -578,7 +578,7 @@ static int create_set(const qs_params *ps, uint32_t nsk, qs_sketch **out)
               hipHostMalloc(&s->h_st, sizeof(qs_dev_state), hipHostMallocDefault) == hipSuccess;
     if (!ok) {
         qs_destroy(s);
-        return QS_ERR_NOMEM;
+        return qs_alloc_failed();
     }
     if (hipMemset(s->d_low, 0, low_w * 4) != hipSuccess || hipMemset(s->d_high, 0, high_w * 4) != hipSuccess ||
         hipMemset(s->d_longbm, 0, s->bm_words * 4) != hipSuccess ||

@@ -13,6 +13,9 @@
 #include <vector>
 
 #include "../../include/qsketch.h"
+#include "../../include/qsketch_learned.h"
+#include "../../include/qsketch_sf.h"
+#include "../../include/qsketch_single.h"
 
 namespace {
 struct launch {
@@ -225,7 +228,6 @@ static void case_hot_alloc()
             expect(qs_insert(s, s_keys, n) == QS_ERR_NOMEM, "a failed allocation is reported");
             expect(g_live.size() == live, "what was allocated before it is freed");
             g_fail_at = 0;
-            (void)hipGetLastError();
         }
         const uint64_t before = g_mallocs;
         expect(qs_insert(s, s_keys, n) == QS_ERR_HIP, "no kernel publishes the candidates here");
@@ -236,11 +238,51 @@ static void case_hot_alloc()
     }
 }
 
+// the k-th allocation of `call` fails, for every k: reported as such, with no error
+// left in the runtime for the next launch check, and the call works when repeated
+template <class F> static void each_allocation_fails(const char *what, F call)
+{
+    for (uint64_t k = 1;; ++k) {
+        const uint64_t before = g_mallocs;
+        g_fail_at = before + k;
+        const int rc = call();
+        g_fail_at = 0;
+        if (g_mallocs < before + k) { // it makes fewer than k
+            expect(k > 1 && rc == QS_OK, what);
+            return;
+        }
+        expect(rc == QS_ERR_NOMEM, what);
+        expect(hipGetLastError() == hipSuccess, what);
+    }
+}
+
+static void case_alloc_errors()
+{
+    const qs_params p = params(1021);
+    qs_sketch *s = nullptr;
+    qs_sf *f = nullptr;
+    qs_sl *l = nullptr;
+    qs_learned *L = nullptr;
+    each_allocation_fails("qs_create", [&] { return qs_create(&p, &s); });
+    each_allocation_fails("qs_sf_create", [&] { return qs_sf_create(1021, 8, 3, 1, 1021, 4, 1, &f); });
+    each_allocation_fails("qs_sl_create", [&] { return qs_sl_create(1021, 8, 1, 1021, 4, 1, &l); });
+    each_allocation_fails("qs_learned_create", [&] { return qs_learned_create(&p, 10, 1, &L); });
+    each_allocation_fails("qs_insert", [&] { return qs_insert(s, s_keys, 100000); });
+    each_allocation_fails("qs_sf_insert", [&] { return qs_sf_insert(f, s_keys, 100000); });
+    each_allocation_fails("qs_learned_insert", [&] { return qs_learned_insert(L, s_keys, 1 << 12, nullptr); });
+    qs_destroy(s);
+    qs_sf_destroy(f);
+    qs_sl_destroy(l);
+    qs_learned_destroy(L);
+    expect(g_live.empty(), "everything freed");
+}
+
 int main(int argc, char **argv)
 {
     const std::map<std::string, void (*)()> cases = {
         {"graph", case_graph},
         {"hot_alloc", case_hot_alloc},
+        {"alloc_errors", case_alloc_errors},
     };
     setvbuf(stdout, nullptr, _IONBF, 0);
     const auto c = cases.find(argc > 1 ? argv[1] : "");
