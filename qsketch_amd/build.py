@@ -69,7 +69,8 @@ def build(verbose: bool = False) -> str:
 
 def build_native_tests(verbose: bool = False) -> None:
     """C++ drivers used by the GPU tests: the include/qsketch.hpp interface
-    against the oracle, the exhaustive fastmod check and the item packing check."""
+    against the oracle, the exhaustive fastmod check, the item packing check and the
+    heavy keys' grouping on its own."""
     root = os.path.dirname(HERE)
     nat = os.path.join(root, "tests", "native")
     cmd = [HIPCC, "-O2", "-std=c++17", f"--offload-arch={ARCH}",
@@ -86,6 +87,9 @@ def build_native_tests(verbose: bool = False) -> None:
     _run(cmd)
     cmd = [HIPCC, "-O2", "-std=c++17", os.path.join(nat, "pack_check.cpp"),
            "-o", os.path.join(nat, "pack_check")]
+    _run(cmd)
+    cmd = [HIPCC, "-O2", *FLAGS[1:], *SOURCE_FLAGS["qs_learned.hip"], os.path.join(nat, "heavy_part_check.cpp"),
+           "-o", os.path.join(nat, "heavy_part_check")]
     _run(cmd)
 
 

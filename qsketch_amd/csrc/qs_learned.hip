@@ -50,6 +50,9 @@
 #define T_EMPTY 0xffffffffffffffffull
 #define T_NONE 0xffffffffu
 #define T_PROBES 4096u
+// error bits of one insert call
+#define LE_FULL 1u // the table turned a key away
+#define LE_SORT 2u // the grouping computed a position outside the call
 
 #define ROUTE_THREADS 1024
 #define ROUTE_CHUNK 1024u // keys per chunk, a wavefront's unit of routing
@@ -77,7 +80,7 @@ struct qs_learned {
     uint64_t *d_tkeys;
     uint32_t *d_tcnt;
     uint32_t *d_bins;  // heavy keys per bin and the bins' write cursors (both of one call)
-    uint32_t *d_err;   // (after them) [0] set when the table turned a key away, [1] slots in use
+    uint32_t *d_err;   // (after them) [0] error bits of one call (LE_*), [1] slots in use
     uint64_t inserted; // keys inserted since create / clear
     uint32_t full;     // the table has turned a key away since create / clear
     uint32_t used;     // table slots in use after the last insert
@@ -664,13 +667,13 @@ __device__ static inline uint32_t t_find(const uint64_t *tkeys, uint32_t tlog2, 
     return T_NONE;
 }
 
-// err[0]: set when the table has no slot for key
+// err[0] gets LE_FULL when the table has no slot for key
 __device__ static inline void t_add(uint64_t *tkeys, uint32_t *tcnt, uint32_t tlog2, uint64_t key, uint32_t c,
                                     uint32_t *err, uint32_t &claims)
 {
     const uint32_t s = t_insert(tkeys, tlog2, key, claims);
     if (s == T_NONE)
-        atomicOr(err, 1u);
+        atomicOr(err, LE_FULL);
     else
         atomicAdd(tcnt + s, c);
 }
@@ -886,7 +889,7 @@ __global__ __launch_bounds__(64 * HP_WAVES) void k_heavy_part(const KeyT<KB> *__
                                                               uint32_t nchunks, const uint32_t *__restrict__ ccount,
                                                               const uint32_t *__restrict__ bins,
                                                               uint32_t *__restrict__ cursor,
-                                                              KeyT<KB> *__restrict__ out)
+                                                              KeyT<KB> *__restrict__ out, uint32_t *__restrict__ err)
 {
     __shared__ KeyT<KB> s_key[HP_WAVES * ROUTE_CHUNK];
     __shared__ uint32_t s_cnt[HBINS], s_start[HBINS], s_goff[HBINS], s_red[2][4];
@@ -939,6 +942,8 @@ __global__ __launch_bounds__(64 * HP_WAVES) void k_heavy_part(const KeyT<KB> *__
         const uint32_t dst = s_goff[heavy_bin((uint64_t)v)] + q;
         if (dst < n) // the counts and the ranks agree; checked, never trusted
             out[dst] = v;
+        else
+            atomicOr(err, LE_SORT);
     }
 }
 
@@ -1437,6 +1442,8 @@ static int ensure_route(qs_learned *L, uint64_t n)
 template <int KB>
 static int learned_insert(qs_learned *L, const KeyT<KB> *keys, uint64_t n, uint64_t *n_heavy)
 {
+    if (L->sk->sticky_err == QS_ERR_INTERNAL)
+        return QS_ERR_INTERNAL;
     int rc = ensure_route(L, n);
     if (rc)
         return rc;
@@ -1452,7 +1459,7 @@ static int learned_insert(qs_learned *L, const KeyT<KB> *keys, uint64_t n, uint6
         // (grouped in the buffer that takes the light keys afterwards)
         KeyT<KB> *grouped = (KeyT<KB> *)L->d_light;
         hipLaunchKernelGGL(k_heavy_part<KB>, dim3((chunks + HP_WAVES - 1u) / HP_WAVES), dim3(64 * HP_WAVES), 0, 0,
-                           stage, n, chunks, L->d_count, L->d_bins, L->d_bins + HBINS, grouped);
+                           stage, n, chunks, L->d_count, L->d_bins, L->d_bins + HBINS, grouped, L->d_err);
         hipLaunchKernelGGL(k_heavy_sum<KB>, dim3((uint32_t)((n + HS_WINDOW - 1) / HS_WINDOW)), dim3(HS_THREADS), 0, 0,
                            grouped, L->d_bins, L->d_tkeys, L->d_tcnt, L->tlog2, L->d_err);
     }
@@ -1469,8 +1476,12 @@ static int learned_insert(qs_learned *L, const KeyT<KB> *keys, uint64_t n, uint6
     CK(hipMemcpy(L->h_pin, L->d_count + chunks, 4, hipMemcpyDeviceToHost));
     CK(hipMemcpy(L->h_pin + 1, L->d_err, 8, hipMemcpyDeviceToHost));
     const uint64_t n_light = L->h_pin[0];
-    if (L->h_pin[1])
+    if (L->h_pin[1] & LE_FULL)
         L->full = 1;
+    if (L->h_pin[1] & LE_SORT) {
+        L->sk->sticky_err = QS_ERR_INTERNAL; // keys are missing from the table: invalid until the clear
+        return QS_ERR_INTERNAL;
+    }
     L->used = L->h_pin[2];
     L->inserted += n;
     if (n_heavy)

@@ -29,6 +29,7 @@ hipError_t g_last = hipSuccess;      // sticky, as the runtime's
 std::map<void *, size_t> g_live;
 std::vector<launch> g_launches;
 uint64_t g_handles = 0;
+uint32_t g_word = 0; // the first word of every 8-byte copy to the host, unless 0
 
 hipError_t fail(hipError_t e)
 {
@@ -76,9 +77,11 @@ hipError_t hipHostFree(void *p)
     free(p);
     return hipSuccess;
 }
-hipError_t hipMemcpy(void *d, const void *s, size_t n, hipMemcpyKind)
+hipError_t hipMemcpy(void *d, const void *s, size_t n, hipMemcpyKind kind)
 {
     memcpy(d, s, n);
+    if (g_word && n == 8 && kind == hipMemcpyDeviceToHost)
+        memcpy(d, &g_word, 4);
     return hipSuccess;
 }
 hipError_t hipMemcpyAsync(void *d, const void *s, size_t n, hipMemcpyKind, hipStream_t)
@@ -277,12 +280,29 @@ static void case_alloc_errors()
     expect(g_live.empty(), "everything freed");
 }
 
+// the learned form's device check (error bit 2 of a call): an insert that lost keys
+// says so, and so do the following ones until the clear
+static void case_learned_error()
+{
+    const qs_params p = params(1021);
+    qs_learned *L = nullptr;
+    expect(qs_learned_create(&p, 10, 1, &L) == QS_OK, "create");
+    g_word = 2;
+    expect(qs_learned_insert(L, s_keys, 1 << 21, nullptr) == QS_ERR_INTERNAL, "the failed check is reported");
+    g_word = 0;
+    expect(!qs_learned_table_full(L), "the table is not full");
+    expect(qs_learned_insert(L, s_keys, 1 << 10, nullptr) == QS_ERR_INTERNAL, "invalid until the clear");
+    expect(qs_learned_clear(L) == QS_OK && qs_learned_insert(L, s_keys, 1 << 10, nullptr) == QS_OK, "valid after it");
+    qs_learned_destroy(L);
+}
+
 int main(int argc, char **argv)
 {
     const std::map<std::string, void (*)()> cases = {
         {"graph", case_graph},
         {"hot_alloc", case_hot_alloc},
         {"alloc_errors", case_alloc_errors},
+        {"learned_error", case_learned_error},
     };
     setvbuf(stdout, nullptr, _IONBF, 0);
     const auto c = cases.find(argc > 1 ? argv[1] : "");
