@@ -656,10 +656,32 @@ __global__ __launch_bounds__(256) void k_clear(uint4 *__restrict__ low, uint64_t
 // tables; k_clear's stores reach 5.65), below it joins the one kernel.
 #define CLEAR_FILL_MIN (64ull << 20)
 
+// makes a device current, and the caller's again at the end of the scope
+struct on_device {
+    int prev = -1;
+    bool ok, changed;
+    explicit on_device(int dev)
+    {
+        ok = hipGetDevice(&prev) == hipSuccess;
+        changed = ok && prev != dev;
+        if (changed)
+            ok = hipSetDevice(dev) == hipSuccess;
+    }
+    ~on_device()
+    {
+        if (changed)
+            (void)hipSetDevice(prev);
+    }
+};
+
 extern "C" int qs_clear(qs_sketch *s)
 {
     if (!s)
         return QS_ERR_PARAM;
+    // (the fills take the tables' addresses on any device, the kernel only on theirs)
+    const on_device here(s->device);
+    if (!here.ok)
+        return QS_ERR_HIP;
     // Blocking, as the reference's clear: every earlier use of the tables has
     // finished before the fills start, and the fills and the control block's
     // reset have finished when the call returns.  In between they are queued

@@ -296,6 +296,23 @@ static void case_learned_error()
     qs_learned_destroy(L);
 }
 
+// a sketch is cleared on its own device, whichever is current
+static void case_clear_device()
+{
+    const qs_params p = params(1021);
+    qs_sketch *s = nullptr;
+    expect(qs_create(&p, &s) == QS_OK, "create");
+    for (int current = 1; current >= 0; --current) {
+        g_device = current;
+        g_launches.clear();
+        expect(qs_clear(s) == QS_OK && g_launches.size() == 1, "clear");
+        for (const launch &l : g_launches)
+            expect(l.device == 0, l.kernel.c_str());
+        expect(g_device == current, "the current device is the caller's again");
+    }
+    qs_destroy(s);
+}
+
 int main(int argc, char **argv)
 {
     const std::map<std::string, void (*)()> cases = {
@@ -303,6 +320,7 @@ int main(int argc, char **argv)
         {"hot_alloc", case_hot_alloc},
         {"alloc_errors", case_alloc_errors},
         {"learned_error", case_learned_error},
+        {"clear_device", case_clear_device},
     };
     setvbuf(stdout, nullptr, _IONBF, 0);
     const auto c = cases.find(argc > 1 ? argv[1] : "");
