@@ -1333,11 +1333,11 @@ extern "C" int qs_mlp_step(qs_learned *L, const void *d_keys, const float *d_t, 
         return QS_ERR_PARAM;
     if (L->inserted)
         return QS_ERR_STATE; // the routing of the keys already in would change
-    L->step++;
-    const float c1 = 1.f - powf(beta1, (float)L->step), c2 = 1.f - powf(beta2, (float)L->step);
-    int rc = grad_launch(L, d_keys, d_t, n, true, lr, beta1, beta2, eps, c1, c2);
+    const float step = (float)(L->step + 1);
+    int rc = grad_launch(L, d_keys, d_t, n, true, lr, beta1, beta2, eps, 1.f - powf(beta1, step), 1.f - powf(beta2, step));
     if (rc)
         return rc;
+    L->step++;
     if (loss || h_grad)
         CK(hipDeviceSynchronize());
     if (h_grad)

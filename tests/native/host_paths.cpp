@@ -5,6 +5,7 @@
 #include <hip/hip_runtime_api.h>
 #include <dlfcn.h>
 
+#include <cmath>
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
@@ -29,6 +30,8 @@ hipError_t g_last = hipSuccess;      // sticky, as the runtime's
 std::map<void *, size_t> g_live;
 std::vector<launch> g_launches;
 uint64_t g_handles = 0;
+bool g_fail_launches = false;
+float g_correction = 0.f; // the first moment's bias correction of the last training step
 uint32_t g_word = 0; // the first word of every 8-byte copy to the host, unless 0
 
 hipError_t fail(hipError_t e)
@@ -170,11 +173,13 @@ hipError_t __hipPopCallConfiguration(dim3 *g, dim3 *b, size_t *shared, hipStream
     *s = nullptr;
     return hipSuccess;
 }
-hipError_t hipLaunchKernel(const void *f, dim3, dim3, void **, size_t, hipStream_t)
+hipError_t hipLaunchKernel(const void *f, dim3, dim3, void **args, size_t, hipStream_t)
 {
     Dl_info info;
     g_launches.push_back({dladdr(f, &info) && info.dli_sname ? info.dli_sname : "?", g_device});
-    return hipSuccess;
+    if (g_launches.back().kernel.find("k_grad_sum") != std::string::npos)
+        g_correction = *static_cast<float *>(args[12]);
+    return g_fail_launches ? fail(hipErrorLaunchFailure) : hipSuccess;
 }
 } // extern "C"
 
@@ -313,6 +318,23 @@ static void case_clear_device()
     qs_destroy(s);
 }
 
+// a training step whose launches fail is no step: the next one is the first
+static void case_failed_step()
+{
+    const qs_params p = params(1021);
+    qs_learned *L = nullptr;
+    expect(qs_learned_create(&p, 10, 1, &L) == QS_OK, "create");
+    const float t[1] = {0.f};
+    g_fail_launches = true;
+    expect(qs_mlp_step(L, s_keys, t, 64, 1e-3f, 0.9f, 0.999f, 1e-8f, nullptr, nullptr) == QS_ERR_HIP, "failed launch");
+    g_fail_launches = false;
+    for (int step = 1; step <= 2; ++step) {
+        expect(qs_mlp_step(L, s_keys, t, 64, 1e-3f, 0.9f, 0.999f, 1e-8f, nullptr, nullptr) == QS_OK, "step");
+        expect(g_correction == 1.f - powf(0.9f, (float)step), "bias correction");
+    }
+    qs_learned_destroy(L);
+}
+
 int main(int argc, char **argv)
 {
     const std::map<std::string, void (*)()> cases = {
@@ -321,6 +343,7 @@ int main(int argc, char **argv)
         {"alloc_errors", case_alloc_errors},
         {"learned_error", case_learned_error},
         {"clear_device", case_clear_device},
+        {"failed_step", case_failed_step},
     };
     setvbuf(stdout, nullptr, _IONBF, 0);
     const auto c = cases.find(argc > 1 ? argv[1] : "");

@@ -21,7 +21,8 @@ def exe(tmp_path_factory):
     return path
 
 
-@pytest.mark.parametrize("case", ["graph", "hot_alloc", "alloc_errors", "learned_error", "clear_device"])
+@pytest.mark.parametrize("case", ["graph", "hot_alloc", "alloc_errors", "learned_error", "clear_device",
+                                  "failed_step"])
 def test_host_path(exe, case):
     r = subprocess.run([exe, case], stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True, timeout=60)
     assert r.returncode == 0, r.stdout
