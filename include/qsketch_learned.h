@@ -86,7 +86,9 @@ int qs_learned_set_threshold(qs_learned *L, float threshold);
 float qs_learned_threshold(const qs_learned *L);
 /* Insert n keys (device pointer): route, count the heavy ones exactly, insert
  * the others into the sketch in stream order.  Blocking.  *n_heavy (may be
- * NULL) receives how many of the n went to the table. */
+ * NULL) receives how many of the n went to the table.  Device scratch, kept
+ * for the next call: 1 + 2 key_bytes per key, beside the sketch's own; a call
+ * for which that does not fit is routed in pieces, with the same result. */
 int qs_learned_insert(qs_learned *L, const void *d_keys, uint64_t n, uint64_t *n_heavy);
 int qs_learned_query(qs_learned *L, const void *d_keys, uint64_t n, uint32_t *d_counts);
 /* Zero the table and the sketch (the network is kept). */

@@ -1408,6 +1408,24 @@ extern "C" int qs_learned_clear(qs_learned *L)
     return QS_OK;
 }
 
+// the routing buffers freed; the light keys of the call may be kept
+static void free_route(qs_learned *L, bool keep_light)
+{
+    hipFree(L->d_flag);
+    hipFree(L->d_count);
+    hipFree(L->d_bsum);
+    hipFree(L->d_stage);
+    L->d_flag = nullptr;
+    L->d_count = nullptr;
+    L->d_bsum = nullptr;
+    L->d_stage = nullptr;
+    L->rcap = 0;
+    if (keep_light)
+        return;
+    hipFree(L->d_light);
+    L->d_light = nullptr;
+}
+
 static int ensure_route(qs_learned *L, uint64_t n)
 {
     if (!L->cus) {
@@ -1418,29 +1436,22 @@ static int ensure_route(qs_learned *L, uint64_t n)
     }
     if (L->rcap >= n)
         return QS_OK;
-    hipFree(L->d_flag);
-    hipFree(L->d_count);
-    hipFree(L->d_bsum);
-    hipFree(L->d_stage);
-    hipFree(L->d_light);
-    L->d_flag = nullptr;
-    L->d_count = nullptr;
-    L->d_bsum = nullptr;
-    L->d_stage = nullptr;
-    L->d_light = nullptr;
-    L->rcap = 0;
+    free_route(L, false);
     const uint64_t chunks = (n + ROUTE_CHUNK - 1) / ROUTE_CHUNK;
     if (hipMalloc(&L->d_flag, n) != hipSuccess || hipMalloc(&L->d_count, (chunks + 1) * 4) != hipSuccess ||
         hipMalloc(&L->d_bsum, 4ull * qs_scan_sums(chunks)) != hipSuccess ||
         hipMalloc(&L->d_stage, chunks * ROUTE_CHUNK * L->key_bytes) != hipSuccess ||
-        hipMalloc(&L->d_light, n * L->key_bytes) != hipSuccess)
+        hipMalloc(&L->d_light, n * L->key_bytes) != hipSuccess) {
+        free_route(L, false);
         return qs_alloc_failed();
+    }
     L->rcap = n;
     return QS_OK;
 }
 
+// one piece of a call; *n_heavy grows by its heavy keys
 template <int KB>
-static int learned_insert(qs_learned *L, const KeyT<KB> *keys, uint64_t n, uint64_t *n_heavy)
+static int learned_piece(qs_learned *L, const KeyT<KB> *keys, uint64_t n, uint64_t *n_heavy)
 {
     if (L->sk->sticky_err == QS_ERR_INTERNAL)
         return QS_ERR_INTERNAL;
@@ -1484,11 +1495,36 @@ static int learned_insert(qs_learned *L, const KeyT<KB> *keys, uint64_t n, uint6
     }
     L->used = L->h_pin[2];
     L->inserted += n;
-    if (n_heavy)
-        *n_heavy = n - n_light;
+    *n_heavy += n - n_light;
     if (n_light == 0)
         return QS_OK;
-    return qs_insert(L->sk, L->d_light, n_light);
+    rc = qs_insert(L->sk, L->d_light, n_light);
+    if (rc == QS_ERR_NOMEM) { // nothing was inserted: again without the buffers that the routing is done with
+        free_route(L, true);
+        rc = qs_insert(L->sk, L->d_light, n_light);
+    }
+    return rc;
+}
+
+// A call is one piece when the routing buffers for it fit the device, else as many as
+// it takes: the pieces one after the other are the same insert.  (The buffers hold a
+// flag and two copies of a key; a form that placed the light keys at once held one, so
+// calls that fitted then must not be refused for the second.)
+#define ROUTE_PIECE_MIN (1ull << 20)
+template <int KB>
+static int learned_insert(qs_learned *L, const KeyT<KB> *keys, uint64_t n, uint64_t *n_heavy)
+{
+    uint64_t piece = n, heavy = 0;
+    int rc = ensure_route(L, piece);
+    while (rc == QS_ERR_NOMEM && piece > ROUTE_PIECE_MIN) {
+        piece = (piece + 1) / 2;
+        rc = ensure_route(L, piece);
+    }
+    for (uint64_t off = 0; rc == QS_OK && off < n; off += piece)
+        rc = learned_piece<KB>(L, keys + off, n - off < piece ? n - off : piece, &heavy);
+    if (n_heavy)
+        *n_heavy = heavy;
+    return rc;
 }
 
 extern "C" int qs_learned_insert(qs_learned *L, const void *d_keys, uint64_t n, uint64_t *n_heavy)

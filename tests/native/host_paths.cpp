@@ -32,7 +32,14 @@ std::vector<launch> g_launches;
 uint64_t g_handles = 0;
 bool g_fail_launches = false;
 float g_correction = 0.f; // the first moment's bias correction of the last training step
-uint32_t g_word = 0; // the first word of every 8-byte copy to the host, unless 0
+uint32_t g_word = 0; // the first word of every g_word_bytes-byte copy to the host, unless 0
+size_t g_word_bytes = 8;
+size_t g_bytes = 0, g_budget = ~(size_t)0; // device memory in use and in all
+struct routed {
+    const void *keys;
+    uint64_t n;
+};
+std::vector<routed> g_routed; // the routing launches' keys
 
 hipError_t fail(hipError_t e)
 {
@@ -54,18 +61,22 @@ extern "C" {
 hipError_t hipMalloc(void **p, size_t bytes)
 {
     *p = nullptr;
-    if (++g_mallocs == g_fail_at)
+    if (++g_mallocs == g_fail_at || bytes > g_budget - g_bytes)
         return fail(hipErrorOutOfMemory);
     *p = calloc(bytes ? bytes : 1, 1);
     g_live[*p] = bytes;
+    g_bytes += bytes;
     return hipSuccess;
 }
 hipError_t hipFree(void *p)
 {
     if (!p)
         return hipSuccess;
-    if (!g_live.erase(p))
+    const auto it = g_live.find(p);
+    if (it == g_live.end())
         return fail(hipErrorInvalidValue);
+    g_bytes -= it->second;
+    g_live.erase(it);
     ++g_frees;
     free(p);
     return hipSuccess;
@@ -83,7 +94,7 @@ hipError_t hipHostFree(void *p)
 hipError_t hipMemcpy(void *d, const void *s, size_t n, hipMemcpyKind kind)
 {
     memcpy(d, s, n);
-    if (g_word && n == 8 && kind == hipMemcpyDeviceToHost)
+    if (g_word && n == g_word_bytes && kind == hipMemcpyDeviceToHost)
         memcpy(d, &g_word, 4);
     return hipSuccess;
 }
@@ -179,6 +190,8 @@ hipError_t hipLaunchKernel(const void *f, dim3, dim3, void **args, size_t, hipSt
     g_launches.push_back({dladdr(f, &info) && info.dli_sname ? info.dli_sname : "?", g_device});
     if (g_launches.back().kernel.find("k_grad_sum") != std::string::npos)
         g_correction = *static_cast<float *>(args[12]);
+    if (g_launches.back().kernel.find("k_route") != std::string::npos)
+        g_routed.push_back({*static_cast<void **>(args[0]), *static_cast<uint64_t *>(args[1])});
     return g_fail_launches ? fail(hipErrorLaunchFailure) : hipSuccess;
 }
 } // extern "C"
@@ -335,6 +348,48 @@ static void case_failed_step()
     qs_learned_destroy(L);
 }
 
+// A learned insert needs no more memory than a flag and one copy of each key beside
+// the sketch's scratch: with less than its buffers would like, it runs in pieces.
+static void case_learned_memory()
+{
+    const uint64_t n = (1 << 22) + 77;
+    static uint32_t keys[n];
+    const qs_params p = params(1021);
+    qs_sketch *s = nullptr;
+    expect(qs_create(&p, &s) == QS_OK, "create");
+    const size_t before = g_bytes;
+    expect(qs_insert(s, keys, n) == QS_OK, "insert");
+    const size_t scratch = g_bytes - before; // of the sketch, for n keys
+    qs_destroy(s);
+    qs_learned *L = nullptr;
+    expect(qs_learned_create(&p, 10, 1, &L) == QS_OK, "create");
+    g_budget = g_bytes + n * 5 + 65536;
+    for (int call = 0; call < 2; ++call) {
+        uint64_t heavy = 0, at = 0;
+        g_routed.clear();
+        expect(qs_learned_insert(L, keys, n, &heavy) == QS_OK && heavy == n, "insert in pieces");
+        for (const routed &r : g_routed) {
+            expect(r.keys == keys + at, "a piece starts where the last one ended");
+            at += r.n;
+        }
+        expect(at == n && g_routed.size() > 1, "the pieces make up the call");
+    }
+    g_budget = ~(size_t)0;
+    qs_learned_destroy(L);
+    // the sketch's scratch takes the place of buffers that the routing has done with
+    expect(qs_learned_create(&p, 10, 1, &L) == QS_OK, "create");
+    expect(qs_learned_insert(L, keys, n, nullptr) == QS_OK, "insert in one piece");
+    g_budget = g_bytes + scratch - n * 4;
+    g_word_bytes = 4;
+    g_word = (uint32_t)n; // every key light
+    expect(qs_learned_insert(L, keys, n, nullptr) == QS_OK, "room made for the sketch");
+    g_word = 0;
+    g_word_bytes = 8;
+    g_budget = ~(size_t)0;
+    qs_learned_destroy(L);
+    expect(g_live.empty(), "everything freed");
+}
+
 int main(int argc, char **argv)
 {
     const std::map<std::string, void (*)()> cases = {
@@ -344,6 +399,7 @@ int main(int argc, char **argv)
         {"learned_error", case_learned_error},
         {"clear_device", case_clear_device},
         {"failed_step", case_failed_step},
+        {"learned_memory", case_learned_memory},
     };
     setvbuf(stdout, nullptr, _IONBF, 0);
     const auto c = cases.find(argc > 1 ? argv[1] : "");
