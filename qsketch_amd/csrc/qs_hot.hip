@@ -889,8 +889,9 @@ static int hot_cand_result(qs_hot *h, hipStream_t stream, bool *skewed)
 }
 
 // Blocking insert of n 32-bit keys into a plain sketch through the hot-key
-// filter.  *used = 0 (and nothing inserted) when the call is too short or its
-// sample shows too little skew: the caller then runs the ordinary insert.
+// filter.  *used = 0 (and nothing inserted) when the call is too short, its sample
+// shows too little skew or the device has no room for the filter's buffers: the
+// caller then runs the ordinary insert.
 int qs_insert_hot(qs_sketch *s, const void *d_keys, uint64_t n, hipStream_t stream, int *used)
 {
     *used = 0;
@@ -898,9 +899,15 @@ int qs_insert_hot(qs_sketch *s, const void *d_keys, uint64_t n, hipStream_t stre
         return QS_OK;
     const uint32_t *keys = (const uint32_t *)d_keys;
     const uint64_t prefix = hot_prefix(n), rest = n - prefix;
+    // The filter only saves time, so no call is refused for its memory (8 bytes per
+    // key beside the insert's scratch): without room for both it is given back.
+    auto no_room = [&]() -> int {
+        qs_hot_free(s);
+        return QS_OK; // *used = 0: the caller runs the ordinary insert
+    };
     int rc = hot_alloc(&s->hot, rest);
     if (rc)
-        return rc;
+        return rc == QS_ERR_NOMEM ? no_room() : rc;
     qs_hot *h = (qs_hot *)s->hot;
     const qs_sdesc d0 = s->h_desc[0];
     qs_evpair e1, e2;
@@ -930,7 +937,7 @@ int qs_insert_hot(qs_sketch *s, const void *d_keys, uint64_t n, hipStream_t stre
         // sequential result, as for any call split into chunks.
         rc = size_scratch();
         if (rc)
-            return rc;
+            return rc == QS_ERR_NOMEM ? no_room() : rc;
         CK(hipEventRecord(h->ev_fork, stream));
         *used = 1;
         rc = qs_insert_set(s, keys, offs_p, nullptr, stream, false, false);
@@ -974,7 +981,7 @@ int qs_insert_hot(qs_sketch *s, const void *d_keys, uint64_t n, hipStream_t stre
             return QS_OK; // *used = 0: the caller runs the ordinary insert
         rc = size_scratch();
         if (rc)
-            return rc;
+            return rc == QS_ERR_NOMEM ? no_room() : rc;
         *used = 1;
         rc = qs_insert_set(s, keys, offs_p, nullptr, stream, false, false); // 2. the prefix
         if (rc)

@@ -233,8 +233,9 @@ static void case_graph()
     expect(g_live.empty(), "everything freed");
 }
 
-// An allocation of the hot-key filter that fails leaves nothing half built: the call
-// after it allocates everything, as the first call of another sketch does.
+// An allocation of the hot-key filter that fails leaves nothing half built: the call is
+// inserted the ordinary way, and the next one allocates all of the filter, as the first
+// call of another sketch does.
 static void case_hot_alloc()
 {
     const uint64_t n = 1ull << 26;
@@ -243,11 +244,12 @@ static void case_hot_alloc()
     for (uint64_t k = 0; k <= 7; ++k) { // the k-th of the filter's own fails (0: none)
         qs_sketch *s = nullptr;
         expect(qs_create(&p, &s) == QS_OK, "create");
+        expect(qs_insert_async(s, s_keys, n, nullptr) == QS_OK, "the insert's scratch");
         const size_t live = g_live.size();
         if (k) {
             g_fail_at = g_mallocs + k;
-            expect(qs_insert(s, s_keys, n) == QS_ERR_NOMEM, "a failed allocation is reported");
-            expect(g_live.size() == live, "what was allocated before it is freed");
+            expect(qs_insert(s, s_keys, n) == QS_OK, "the ordinary insert takes over");
+            expect(g_live.size() == live, "what was allocated before the failure is freed");
             g_fail_at = 0;
         }
         const uint64_t before = g_mallocs;
@@ -390,6 +392,32 @@ static void case_learned_memory()
     expect(g_live.empty(), "everything freed");
 }
 
+// The filter only saves time: a call for which it does not fit the device is inserted
+// the ordinary way.
+static void case_filter_memory()
+{
+    const uint64_t n = 1ull << 26;
+    const qs_params p = params(1021);
+    qs_sketch *s = nullptr;
+    expect(qs_create(&p, &s) == QS_OK && qs_set_hot_filter(s, 0) == QS_OK, "create");
+    const size_t before = g_bytes;
+    expect(qs_insert(s, s_keys, n) == QS_OK, "insert without the filter");
+    const size_t scratch = g_bytes - before;
+    qs_destroy(s);
+    for (size_t more : {(size_t)0, (size_t)100 << 20, (size_t)n * 9}) { // (the filter takes 8 bytes per key)
+        expect(qs_create(&p, &s) == QS_OK, "create");
+        g_budget = g_bytes + scratch + more;
+        const int want = more < n * 9 ? QS_OK : QS_ERR_HIP; // (QS_ERR_HIP: no kernel publishes the candidates here)
+        for (int call = 0; call < 2; ++call)
+            expect(qs_insert(s, s_keys, n) == want, "insert in what the ordinary way takes");
+        g_budget = g_bytes + 1;
+        expect(qs_insert(s, s_keys, 2 * n) == QS_ERR_NOMEM, "not in less");
+        g_budget = ~(size_t)0;
+        qs_destroy(s);
+        expect(g_live.empty(), "everything freed");
+    }
+}
+
 int main(int argc, char **argv)
 {
     const std::map<std::string, void (*)()> cases = {
@@ -400,6 +428,7 @@ int main(int argc, char **argv)
         {"clear_device", case_clear_device},
         {"failed_step", case_failed_step},
         {"learned_memory", case_learned_memory},
+        {"filter_memory", case_filter_memory},
     };
     setvbuf(stdout, nullptr, _IONBF, 0);
     const auto c = cases.find(argc > 1 ? argv[1] : "");

@@ -22,7 +22,7 @@ def exe(tmp_path_factory):
 
 
 @pytest.mark.parametrize("case", ["graph", "hot_alloc", "alloc_errors", "learned_error", "clear_device",
-                                  "failed_step", "learned_memory"])
+                                  "failed_step", "learned_memory", "filter_memory"])
 def test_host_path(exe, case):
     r = subprocess.run([exe, case], stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True, timeout=60)
     assert r.returncode == 0, r.stdout
