@@ -344,7 +344,9 @@ __global__ __launch_bounds__(INS_THREADS) void k_query(const KeyT<KB> *__restric
             continue;
         }
         for (uint32_t sid = sa; sid <= sz; ++sid) { // uniform
-            const uint64_t a = offs[sid] > i0 ? offs[sid] : i0, z = offs[sid + 1] < i1 ? offs[sid + 1] : i1;
+            // (offs[sa + 1 .. sz] lie inside the tile; keys before the first sketch's part and
+            // after the last one's are theirs, as in the search)
+            const uint64_t a = sid == sa ? i0 : offs[sid], z = sid == sz ? i1 : offs[sid + 1];
             if (a >= z)
                 continue;
             const qs_sdesc d = D[sid];
