@@ -1733,6 +1733,13 @@ __device__ static inline uint32_t trig_rank(const uint32_t *__restrict__ tbit, c
     return scanned ? tsum[span] + c : c;
 }
 
+// Sets of more sketches than this move their allocators on by the triggers, not sketch
+// by sketch (finish_pass): the closing kernel's 256 wavefronts took 386 us for 65536
+// sketches, 28 for 4096 of 512 keys, and take 5 and 6 so. With few sketches their
+// allocations meet on few words: 8 sketches of 10^6 keys 17 us so and 7 by sketch, 512
+// of 10^5 25 and 14, 1025 of 20000 12 and 13.
+#define FIN_SKETCHES 1024u
+
 // Ids in stream order of the triggering inserts, per sketch (the sequential
 // bump allocator of v3:68-85, next starting at 1025).  The sketches' parts of
 // a chunk follow one another, so a trigger's rank within its sketch is its
@@ -1742,7 +1749,7 @@ __device__ static inline uint32_t trig_rank(const uint32_t *__restrict__ tbit, c
 // bitmap costs one 8 us scan and no sort.)
 // block bid of nblk, of NW wavefronts
 template <int NW>
-__device__ __forceinline__ void assign_pass(uint32_t bid, uint32_t nblk, const qs_trig *__restrict__ trig, uint32_t trig_cap,
+__device__ __forceinline__ void assign_pass(uint32_t bid, uint32_t nblk, qs_trig *__restrict__ trig, uint32_t trig_cap,
                                             const uint32_t *__restrict__ tbit,
                                             const uint32_t *__restrict__ tsum, uint32_t cn,
                                             const uint64_t *__restrict__ offs, uint64_t base,
@@ -1758,7 +1765,7 @@ __device__ __forceinline__ void assign_pass(uint32_t bid, uint32_t nblk, const q
     const uint32_t gw = bid * (uint32_t)NW + (threadIdx.x >> 6);
     const uint32_t nw = nblk * (uint32_t)NW;
     for (uint32_t r = gw; r < n_trig; r += nw) {
-        const qs_trig *tr = trig + r;
+        qs_trig *tr = trig + r;
         const uint32_t sid = tr->sid;
         uint32_t rank = trig_rank(tbit, tsum, tr->idx, cn);
         if (nsk > 1)
@@ -1776,11 +1783,13 @@ __device__ __forceinline__ void assign_pass(uint32_t bid, uint32_t nblk, const q
         if (lane == 0) {
             low_pool[d.low_off + (size_t)tr->bucket * 8u + 7u] = id;
             tail_pool[d.tail_off + row] = tr->tail_start;
+            if (nsk > FIN_SKETCHES)
+                tr->idx = id; // for the chunk's last kernel
         }
     }
 }
 
-__global__ __launch_bounds__(256) void k_assign(const qs_trig *__restrict__ trig, uint32_t trig_cap,
+__global__ __launch_bounds__(256) void k_assign(qs_trig *__restrict__ trig, uint32_t trig_cap,
                                                 const uint32_t *__restrict__ tbit,
                                                 const uint32_t *__restrict__ tsum, uint32_t cn,
                                                 const uint64_t *__restrict__ offs, uint64_t base,
@@ -2076,7 +2085,8 @@ __global__ __launch_bounds__(256) void k_tail(const uint64_t *__restrict__ IT, u
 
 
 // The chunk's last kernel: the long-segment marks are taken back, next[sid]
-// moves on by the allocations of sid (a wavefront per sketch), and the block
+// moves on by the allocations of sid (a wavefront per sketch; in a large set a thread
+// per allocation raises its sketch's next above the id that k_assign left it), and the block
 // that finishes last resets the chunk's counters and leaves the error bits in
 // the host's pinned mirror, so that a blocking call needs no copy.
 #define FIN_BLOCKS 64u // at most: every block ends with one atomic on st->done
@@ -2084,7 +2094,8 @@ __global__ __launch_bounds__(256) void k_tail(const uint64_t *__restrict__ IT, u
 template <int NW>
 __device__ __forceinline__ void finish_pass(uint32_t bid, uint32_t nblk, const uint32_t *__restrict__ lng, const uint64_t *__restrict__ IT,
                                             const qs_sdesc *__restrict__ D, qs_pack pk,
-                                            uint32_t *__restrict__ longbm, const uint32_t *__restrict__ tbit,
+                                            uint32_t *__restrict__ longbm, const qs_trig *__restrict__ trig,
+                                            uint32_t trig_cap, const uint32_t *__restrict__ tbit,
                                             const uint32_t *__restrict__ tsum, uint32_t cn,
                                             const uint64_t *__restrict__ offs, uint64_t base, uint32_t nsk,
                                             uint32_t *__restrict__ next, qs_dev_state *__restrict__ st,
@@ -2096,7 +2107,15 @@ __device__ __forceinline__ void finish_pass(uint32_t bid, uint32_t nblk, const u
         const uint64_t bit = D[it_sid(it, pk)].bm_off + it_b(it, pk);
         atomicAnd(longbm + (bit >> 5), ~(1u << (bit & 31u)));
     }
-    if (n_trig && !st->err) {
+    if (nsk > FIN_SKETCHES) {
+        if (!st->err)
+            for (uint32_t r = bid * blockDim.x + threadIdx.x; r < min(n_trig, trig_cap); r += nblk * blockDim.x) {
+                uint32_t *nx = next + trig[r].sid;
+                const uint32_t after = trig[r].idx + 1u; // the id's successor
+                if (__hip_atomic_load(nx, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) < after)
+                    atomicMax(nx, after);
+            }
+    } else if (n_trig && !st->err) {
         const uint32_t lane = threadIdx.x & 63u;
         for (uint32_t sid = bid * (uint32_t)NW + (threadIdx.x >> 6); sid < nsk; sid += nblk * (uint32_t)NW) {
             uint32_t c = n_trig;
@@ -2133,13 +2152,14 @@ __device__ __forceinline__ void finish_pass(uint32_t bid, uint32_t nblk, const u
 
 __global__ __launch_bounds__(256) void k_finish(const uint32_t *__restrict__ lng, const uint64_t *__restrict__ IT,
                                                 const qs_sdesc *__restrict__ D, qs_pack pk,
-                                                uint32_t *__restrict__ longbm, const uint32_t *__restrict__ tbit,
+                                                uint32_t *__restrict__ longbm, const qs_trig *__restrict__ trig,
+                                                uint32_t trig_cap, const uint32_t *__restrict__ tbit,
                                                 const uint32_t *__restrict__ tsum, uint32_t cn,
                                                 const uint64_t *__restrict__ offs, uint64_t base, uint32_t nsk,
                                                 uint32_t *__restrict__ next, qs_dev_state *__restrict__ st,
                                                 uint32_t *__restrict__ h_err)
 {
-    finish_pass<4>(blockIdx.x, gridDim.x, lng, IT, D, pk, longbm, tbit, tsum, cn, offs, base, nsk, next, st, h_err);
+    finish_pass<4>(blockIdx.x, gridDim.x, lng, IT, D, pk, longbm, trig, trig_cap, tbit, tsum, cn, offs, base, nsk, next, st, h_err);
 }
 
 // ---------------------------------------------------------------------------
@@ -2265,7 +2285,7 @@ __global__ __launch_bounds__(SMALL_THREADS) void k_small(const KeyT<KB> *__restr
     tail_pass<false, uint64_t, SMALL_WAVES>(0u, 1u, s_item, n, D, s_masks, low, high, mask_pool, pk, longbm, tail_pool, next, lng, false,
                                64u * TAIL_PF, st);
     pass_fence();
-    finish_pass<SMALL_WAVES>(0u, 1u, lng, s_item, D, pk, longbm, tbit, tsum, n, nullptr, 0, 1u, next, st, h_err);
+    finish_pass<SMALL_WAVES>(0u, 1u, lng, s_item, D, pk, longbm, trig, trig_cap, tbit, tsum, n, nullptr, 0, 1u, next, st, h_err);
 }
 
 
@@ -2567,8 +2587,8 @@ static int insert_chunk(qs_sketch *s, const KeyT<KB> *keys, uint32_t cn, uint64_
                            short_runs, twin, s->d_st);
     const uint64_t fin = (uint64_t)cn / 64 / 256 > (uint64_t)s->nsk / 4 ? (uint64_t)cn / 64 / 256 : (uint64_t)s->nsk / 4;
     hipLaunchKernelGGL(k_finish, dim3((uint32_t)(fin < FIN_BLOCKS ? fin + 1 : FIN_BLOCKS)), dim3(256), 0, stream,
-                       sc.lng, IT, s->d_desc, s->pk, s->d_longbm, sc.tbit, sc.tsum, cn, bc.d_offs, base, s->nsk,
-                       s->d_next, s->d_st, &s->h_st->err);
+                       sc.lng, IT, s->d_desc, s->pk, s->d_longbm, sc.trig, sc.trig_cap, sc.tbit, sc.tsum, cn, bc.d_offs,
+                       base, s->nsk, s->d_next, s->d_st, &s->h_st->err);
     if (bc.timed)
         qs_tim_end(s, et, stream);
     CK(hipGetLastError());
