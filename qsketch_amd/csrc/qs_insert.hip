@@ -135,7 +135,10 @@ __device__ static inline uint32_t sid_chunk_start(const uint64_t *__restrict__ o
 // the owning sketch by binary search over the batch offsets.
 // The sketches a tile of a batch spans: their offsets offs[sid0 .. sid0 + cnt]
 // copied to LDS by the block (cnt = 0: too many, search the global array).
-#define SIDW 64u
+// (A tile of parts of 32 keys and more fits: with a window of 64 sketches, parts of 60
+// keys took 247 us for the first tile counts of 18 M keys and 292 for the first
+// scatter, with 128 they take 83 and 129.)
+#define SIDW 128u
 struct sid_window {
     const uint64_t *o;
     uint32_t sid0, cnt;
