@@ -283,10 +283,15 @@ __device__ static inline void query_bucket(uint32_t M, uint32_t b, const uint32_
 // Sketches of a tile that it takes one after the other; a tile of more (short
 // parts) finds each key's sketch by itself.
 #define QUERY_PARTS 8u
+// Batches of fewer keys are not cut into tiles: their keys are spread over the chip and
+// find their sketches each by itself, since a tile's search and its rounds of 128 keys are
+// one chain (2400 to 2^17 lookups in 8 to 8000 sketches: 10 to 19 us by tiles, 5 so;
+// 2^18 10 to 15 and 7 to 10; 2^19 11 to 16 and 12 to 20; 2^20 13 to 18 and 20 to 41).
+#define QUERY_TILES_MIN (1u << 19)
 // keys of a part from which its masks are worth copying to LDS
 #define QUERY_LDS_MIN 256u
 
-// A single sketch's blocks take keys in turn.  In a batch a block takes tiles of
+// A single sketch's blocks take keys in turn.  In a long batch a block takes tiles of
 // consecutive keys and, sketch by sketch, answers the tile's parts as a single
 // sketch's: descriptor in scalar registers, masks in LDS.  The tiles of one XCD's
 // blocks (blocks go to the 8 XCDs in turn) are consecutive, so at any time they
@@ -316,6 +321,16 @@ __global__ __launch_bounds__(INS_THREADS) void k_query(const KeyT<KB> *__restric
             const KeyT<KB> key = next;
             next = keys[i + stride < n ? i + stride : n - 1u]; // in flight beside this key's bucket
             query_bucket<NT>(s_masks[qs_maskidx_d(key, d0)], qs_bucket_d(key, d0), low_pool, high_pool, half, out + i);
+        }
+        return;
+    }
+    if (n < QUERY_TILES_MIN) {
+        const uint64_t step = (uint64_t)gridDim.x * (INS_THREADS / 2);
+        for (uint64_t i = (uint64_t)blockIdx.x * (INS_THREADS / 2) + (threadIdx.x >> 1); i < n; i += step) {
+            const KeyT<KB> key = keys[i];
+            const qs_sdesc &d = D[query_sid(offs, nsk, i)];
+            query_bucket<NT>(mask_pool[d.masks_off + qs_maskidx_d(key, d)], qs_bucket_d(key, d), low_pool + d.low_off,
+                             high_pool + d.high_off, half, out + i);
         }
         return;
     }
