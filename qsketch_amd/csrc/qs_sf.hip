@@ -56,7 +56,7 @@
 #define SF_ROW_RANGE 4096u      // most keys per work item of k_sf_rows
 #define SF_ROW_RANGE_COLD 512u  // and of a call whose frequent keys the filter took out
 #define SF_SORT_MIN (1u << 16)  // shorter inserts are applied unsorted
-#define SF_TILE_SMALL_MAX (1u << 17) // up to here the unsorted tiles hold 512 keys, then 2048
+#define SF_TILE_SMALL_MAX (1u << 17) // up to here the unsorted tiles hold 256 keys, then 2048
 #define SF_CHUNK4 (1u << 28)    // keys per radix chunk: 4-byte keys
 #define SF_CHUNK8 (1u << 27)    //                       8-byte keys
 
@@ -322,9 +322,13 @@ __device__ static inline void sf_add(uint32_t *__restrict__ split, uint32_t *__r
 
 // Short inserts, unsorted: a block counts a tile of 256 * IPT keys in an LDS
 // table and adds each distinct key's count with sf_add, so that a frequent key
-// costs its counters one atomic per tile (20000 Zipf 1.1 keys: 149 us when
-// every run of equal neighbours was added by itself, now 44).  The all-ones
-// key is the table's empty marker and is counted apart.
+// costs its counters one atomic per tile.  The thread that claimed a slot adds it, so
+// that a thread's chain of counter updates is no longer than its keys, and short calls
+// take tiles of one key per thread.  (Kernel times, every run of equal neighbours by
+// itself / tiles of 512 keys whose slots were walked / now: 4195 distinct keys 10, 21, 9 us,
+// 30000 12, 22, 12, 65535 21, 24, 19; 4195 Zipf 1.1 keys 31, 19, 9, 20000 127, 33, 19, 65535
+// 440, 81, 53.  Tiles of 512 with the claimers adding: 19 us for 30000 distinct keys, 39
+// for 65535 Zipf ones.)  The all-ones key is the table's empty marker and is counted apart.
 #define SF_RUN_PF 8
 template <int KB, int IPT>
 __global__ __launch_bounds__(SF_THREADS) void k_sf_tile(const KeyT<KB> *__restrict__ keys, uint64_t n, sf_par p,
@@ -350,6 +354,10 @@ __global__ __launch_bounds__(SF_THREADS) void k_sf_tile(const KeyT<KB> *__restri
     if (t == 0)
         s_cnt[SLOTS] = 0;
     __syncthreads();
+    uint32_t own[IPT]; // the slots this thread claimed
+#pragma unroll
+    for (int r = 0; r < IPT; ++r)
+        own[r] = SLOTS;
 #pragma unroll
     for (int r = 0; r < IPT; ++r) {
         const KeyT<KB> k = kk[r];
@@ -380,15 +388,18 @@ __global__ __launch_bounds__(SF_THREADS) void k_sf_tile(const KeyT<KB> *__restri
                                               (unsigned long long)k);
             }
             if (cur == EMPTY || cur == k) {
+                if (cur == EMPTY)
+                    own[r] = sl;
                 atomicAdd(&s_cnt[sl], w);
                 break;
             }
         }
     }
     __syncthreads();
-    for (uint32_t e = t; e < SLOTS; e += SF_THREADS)
-        if (s_cnt[e])
-            sf_add<KB>(split, search, p, index, (uint64_t)s_key[e], s_cnt[e]);
+#pragma unroll
+    for (int r = 0; r < IPT; ++r)
+        if (own[r] != SLOTS)
+            sf_add<KB>(split, search, p, index, (uint64_t)kk[r], s_cnt[own[r]]);
     if (t == 0 && s_cnt[SLOTS])
         sf_add<KB>(split, search, p, index, (uint64_t)EMPTY, s_cnt[SLOTS]);
 }
@@ -931,8 +942,8 @@ static void sf_launch_flush(qs_sf *s, const sf_par &p, const KeyT<KB> *keys, uin
         hipLaunchKernelGGL(k_sf_fix, dim3((listed + 255) / 256), dim3(256), 0, 0, s->d_shared, listed, p, s->d_split,
                            s->d_search);
     } else if (n <= SF_TILE_SMALL_MAX) {
-        hipLaunchKernelGGL((k_sf_tile<KB, 2>), dim3((uint32_t)((n + 2 * SF_THREADS - 1) / (2 * SF_THREADS))), block, 0, 0,
-                           keys, n, p, s->d_index, s->d_split, s->d_search);
+        hipLaunchKernelGGL((k_sf_tile<KB, 1>), dim3((uint32_t)((n + SF_THREADS - 1) / SF_THREADS)), block, 0, 0, keys, n, p,
+                           s->d_index, s->d_split, s->d_search);
     } else {
         hipLaunchKernelGGL((k_sf_tile<KB, 8>), dim3((uint32_t)((n + 8 * SF_THREADS - 1) / (8 * SF_THREADS))), block, 0, 0,
                            keys, n, p, s->d_index, s->d_split, s->d_search);
