@@ -111,10 +111,7 @@ __device__ static inline uint32_t sid_chunk_start(const uint64_t *__restrict__ o
 // ===========================================================================
 // radix sort of the chunk by cell = (sketch, bucket)
 // ===========================================================================
-#ifndef QS_OS_THREADS
-#define QS_OS_THREADS 512
-#endif
-#define OS_THREADS QS_OS_THREADS
+#define OS_THREADS 512
 #define OS_WAVES (OS_THREADS / 64)
 // Tiles of 512 * 8 items: a digit's run in a tile is what a scatter writes at a
 // time, 16 items of an 8-byte item's 128-byte line for 8-bit digits, and 24 wavefronts per
@@ -122,10 +119,7 @@ __device__ static inline uint32_t sid_chunk_start(const uint64_t *__restrict__ o
 // 256 threads, 460 with 512, 668 with 1024 (one block per CU), 456 with 512 of 16
 // items, which loses elsewhere (a pass of 75 M items with 8-bit digits: 325, 297, 412, 302).
 // Non-temporal stores take 660: the runs of neighbouring tiles meet in the L2.
-#ifndef QS_OS_IPL
-#define QS_OS_IPL 8
-#endif
-#define OS_IPL QS_OS_IPL
+#define OS_IPL 8
 #define OS_WAVE_ITEMS (64 * OS_IPL)       // items per wave
 #define OS_TILE (OS_THREADS * OS_IPL)     // items per tile
 #define OS_BINS 256                       // LDS capacity for digits up to 8 bits
@@ -990,31 +984,17 @@ __device__ static inline void add_words(uint32_t a[7], const uint32_t b[7])
         a[k] += b[k];
 }
 
-// one owner finishes a run: apply it, or queue it for the replay, or mark it
-// long; returns FR_* bits (a value, not references, so that the flags stay
-// in registers)
+// What an owner finds when it finishes a run: nothing more to do, or the run is queued
+// for the replay, or marked long (a value, not references, so that the flags stay in
+// registers)
 #define FR_RISKY 1u    // to the in-order replay
 #define FR_LONG 2u     // to the tail kernel
 #define FR_UNLINKED 4u // long and unlinked: to the replay first
-template <bool MULTI>
-__device__ static inline uint32_t finish_run(bool act, uint32_t sid, uint32_t b, uint64_t len, const uint32_t a[7],
-                                             const qs_sdesc *__restrict__ D, uint32_t *low_pool,
-                                             uint32_t *high_pool, const uint32_t *mask_pool, uint32_t *longbm)
-{
-    if (!act)
-        return 0u;
-    seg_tables tb = tables_of<MULTI>(sid, D, low_pool, high_pool, mask_pool);
-    if (len >= 256u) {
-        set_long<MULTI>(longbm, D, sid, b);
-        return FR_LONG | (tb.low[(size_t)b * 8u + 7u] <= QS_LINK_START ? FR_UNLINKED : 0u);
-    }
-    return apply_segment(tb.low, tb.high, b, a) ? FR_RISKY : 0u;
-}
 
-// The same finish in two phases, so that the bucket loads of all the runs a
+// A run is finished in two phases, so that the bucket loads of all the runs a
 // lane finishes in one window are in flight together (the runs are distinct
 // cells, so no load depends on another run's store): load_run reads the
-// bucket's two 16-byte words, apply_run then does what finish_run does.
+// bucket's two 16-byte words, apply_run then applies the run or says what is left.
 //
 // In a batch, a wavefront's windows nearly always lie in one sketch's part of
 // the sorted items; its descriptor is then read once, into scalar registers
@@ -2207,7 +2187,6 @@ __global__ __launch_bounds__(SMALL_THREADS) void k_small(const KeyT<KB> *__restr
     if (t == 0)
         tsum[0] = 0;
     const uint32_t rounds = (n + SMALL_THREADS - 1u) / SMALL_THREADS, wave0 = wv * rounds * 64u; // this wavefront's items
-    const uint64_t lt = (1ull << lane) - 1ull;
     const uint32_t dmask = (1u << dbits) - 1u;
     const sid_window win{nullptr, 0u, 0u};
     uint64_t item[SMALL_ROUNDS];

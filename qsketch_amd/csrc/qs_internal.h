@@ -159,8 +159,7 @@ __device__ static inline uint32_t qs_maskidx_d(uint64_t key, const qs_sdesc &d)
 //   [ bucket : bb | sketch : sb | mask field : bm | stream index : ib ]
 // The sort key is the low bb + sb bits (bucket within sketch), so a bucket
 // segment is a run of equal "cell" values.  The stream index is the position
-// within the sketch's part of the chunk, so allocations of one sketch can be
-// ordered by (sketch, index) in 32 bits.
+// within the sketch's part of the chunk.
 // The mask field holds the mask index h % n_masks, or (quotient form, 32-bit
 // keys only) the hash quotient q = h / n_low, from which h = q * n_low + b and
 // the mask index follow.  The quotient form is used when it is narrower: on
@@ -187,9 +186,11 @@ static inline uint32_t qs_bits_for(uint64_t n) // bits to hold 0 .. n-1 (at leas
 
 // Field widths for a set of nsk sketches whose tables have min_low .. max_low
 // buckets and at most max_masks masks, for keys of key_bytes bytes.  The
-// stream index gets what is left of 64 bits, but at most 32 - sb bits (the
-// allocation order key (sketch, index) is 32 bits) and at most 30 bits (device
-// code shifts 32-bit values by ib; a shift by 32 would wrap to a shift by 0).
+// stream index gets what is left of 64 bits, but at most 30 bits (device code shifts
+// 32-bit values by ib; a shift by 32 would wrap to a shift by 0) and at most 32 - sb
+// bits.  (Nothing sorts by (sketch, index) in 32 bits any more; the limit stays because it
+// fixes which batches of a large set are one chunk, and so their scratch and what
+// a captured graph takes.)
 // Returns false when fewer than 12 bits remain.  A single sketch's n_low and
 // n_masks go into the pack for the quotient form (set q_low, q_fd after).
 static inline bool qs_make_pack(uint64_t max_low, uint64_t min_low, uint32_t nsk, uint64_t max_masks,

@@ -492,8 +492,7 @@ static int create_set(const qs_params *ps, uint32_t nsk, qs_sketch **out)
         if (ps[i].key_bytes != ps[0].key_bytes)
             return QS_ERR_PARAM;
     }
-    // item packing: [bucket | sketch | mask field | stream index] in 64 bits,
-    // and (sketch, stream index) in 32 bits for the allocation order
+    // item packing: [bucket | sketch | mask field | stream index] in 64 bits
     uint64_t max_low = 0, min_low = ~0ull, max_masks = 0;
     for (uint32_t i = 0; i < nsk; ++i) {
         max_low = ps[i].n_low > max_low ? ps[i].n_low : max_low;
@@ -769,8 +768,8 @@ extern "C" int qs_insert_async(qs_sketch *s, const void *d_keys, size_t n, void 
 
 // ---------------------------------------------------------------------------
 // Allocation-free insert: the insert scratch (items, radix counts, digit
-// bytes, replay and long-segment lists, allocation records and their sort
-// buffers) is carved out of one static device array instead of the handle's
+// bytes, replay and long-segment lists, allocation records and their bitmap)
+// is carved out of one static device array instead of the handle's
 // own buffers.  Each GPU holds its own copy of the array from module load to
 // process end; its address on a device comes from hipGetSymbolAddress, taken
 // once per device with that device current.  The array's name is never used
