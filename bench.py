@@ -325,7 +325,7 @@ def main():
                   "long_segments_per_step": st["long_segments"],
                   "linked_buckets": st["linked_buckets"],
                   "pool_occupancy": round(st["linked_buckets"] / (a.n_high - 1), 4),
-                  "allocator": "ids assigned in stream order by a sort of the triggering inserts; "
+                  "allocator": "ids assigned in stream order from a bitmap of the triggering inserts; "
                                "no compare-and-swap loop, so no retries"},
     }
     # the measured ceilings of the two dominant access patterns, live

@@ -114,11 +114,13 @@ int qs_sync(qs_sketch *s);
 /* Hot-key filter of the blocking qs_insert (build addition; on by default).
  * A call of at least 2^26 32-bit keys into a plain sketch whose first 2^20
  * keys show skew (keys occurring 8 or more times there covering 30% or more
- * of them) inserts its first 2^25 keys the ordinary way; after that, the
- * inserts of those frequent keys whose bucket is now linked are counted and
- * added to their high rows at once (such inserts commute), and only the other
- * keys go through the ordered insert.  The result is the same state, bit for
- * bit.  enable = 0 turns it off for this handle. */
+ * of them) inserts its first sixteenth (2^22 to 2^24 keys) the ordinary way;
+ * after that, the inserts of those frequent keys whose bucket is now linked are
+ * counted and added to their high rows at once (such inserts commute), and only
+ * the other keys go through the ordered insert.  The result is the same state,
+ * bit for bit.  It takes 8 bytes of device memory per key beside the insert's
+ * scratch; where that does not fit, the call runs without it.  enable = 0 turns
+ * it off for this handle. */
 int qs_set_hot_filter(qs_sketch *s, int enable);
 
 /* Allocation-free insert.  No counterpart in the reference: it is for callers
@@ -179,7 +181,10 @@ int qs_get_stats(qs_sketch *s, qs_stats *st);
 /* ---- kernel timing (build addition) --------------------------------------
  * When enabled, the library records HIP events on the launch stream around
  * every kernel launch of the insert path and of the query (the reference only
- * timed whole blocking calls on the host, include/tool/tool.h:26-50).
+ * timed whole blocking calls on the host, include/tool/tool.h:26-50).  A chunk
+ * of up to 4096 keys of a single sketch is one launch when it is not timed; a
+ * timed one runs the launch sequence of longer chunks, which has the groups
+ * below (same state, but more time).
  * Enabling resets the totals; qs_get_timing synchronises and resolves them.
  * kernel_ms[k] / kernel_launches[k] per kernel group k:                      */
 #define QS_TK_SORT_UP   0  /* radix sort by bucket: digit histograms         */

@@ -13,7 +13,7 @@
 //   3. the hot set: the candidates whose bucket is linked now, in a table of
 //      HOT_BUCKETS buckets of 2 slots where each key may sit in one of two
 //      buckets (the emptier one when it is placed), so that a lookup is two
-//      16-byte reads and no loop; a key that finds both buckets full is left
+//      8-byte reads and no loop; a key that finds both buckets full is left
 //      out of the set (it then takes the ordered path, which is always exact);
 //   4. the rest of the call in one pass: a hot key is counted in LDS (per
 //      persistent block, summed over blocks at the end and added to its high
@@ -157,7 +157,9 @@ __device__ static inline void hot_buckets(uint32_t key, uint32_t &b1, uint32_t &
 // result, so a key that finds the LDS table crowded is simply left out.
 // (The sample was sorted before, and the candidates sorted again by count:
 // 29 launches, about 270 us with their gaps; these four kernels take 65 us at
-// Zipf 1.1 over 2^24 keys, 43 of them the block whose bin holds the hottest key.)
+// Zipf 1.1 over 2^24 keys, 43 of them the block whose bin holds the hottest key.
+// On the second stream, beside a prefix that fills the chip, k_samp_count's last
+// blocks wait for their turn and its launch spans 228 us, within the prefix's time.)
 // ---------------------------------------------------------------------------
 #define SAMP_TILE 8192u // sample keys per block of the split
 #define SAMP_TILES (HOT_SAMPLE / SAMP_TILE)
@@ -715,7 +717,7 @@ __global__ __launch_bounds__(1024) void k_scan_apply(uint32_t *__restrict__ a, u
 }
 
 // the hot counts summed over the persistent blocks and added to the high
-// rows: a block takes 64 slots, its four wavefronts a quarter of the rows each
+// rows: a block takes 64 slots, its wavefronts a share of the rows each
 #define FLUSH_WAVES 16u // wavefronts per block, each summing every 16th row of part
 __global__ __launch_bounds__(64 * FLUSH_WAVES) void k_hot_flush(const uint32_t *__restrict__ part, uint32_t nblk,
                                                                 const uint32_t *__restrict__ tkey,

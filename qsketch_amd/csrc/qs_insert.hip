@@ -414,8 +414,8 @@ __global__ __launch_bounds__(OS_THREADS) void k_bs_up_dig(const uint8_t *__restr
 //   SCAN_LOCAL  k_hist_scan_local only; the scatter sums at most SCAN_SUM_GROUPS
 //               group rows
 //   SCAN_NONE   no scan kernel; it sums at most SCAN_SUM_TILES tile rows
-// Summing 33 tile rows (65537 keys) costs a scatter 3 us and saves two
-// launches; summing 64 group rows (2^22 keys) cost it 12 us and saved 4.
+// Summing 33 tile rows (65537 keys in tiles of 2048; 17 rows now) cost a scatter 3 us and
+// saved two launches; summing 64 group rows (2^22 keys) cost it 12 us and saved 4.
 #define SCAN_FULL 0
 #define SCAN_LOCAL 1
 #define SCAN_NONE 2

@@ -704,7 +704,7 @@ __global__ __launch_bounds__(SF_THREADS) void k_sf_rows(const KeyT<KB> *__restri
 // The hot keys of a filtered call (qs_hot_split_keys): each slot's count
 // summed over the persistent blocks and added with sf_add (after the cold
 // keys' kernels, so no plain write of k_sf_rows runs beside these atomics).
-// A block takes 64 slots, its four wavefronts a quarter of the rows each.
+// A block takes 64 slots, its wavefronts a share of the rows each.
 #define SF_FLUSH_WAVES 16u // wavefronts per block, each summing every 16th row of part
 __global__ __launch_bounds__(64 * SF_FLUSH_WAVES) void k_sf_hot_flush(const uint32_t *__restrict__ part,
                                                                       uint32_t nblk,

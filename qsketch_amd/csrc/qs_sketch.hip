@@ -882,8 +882,10 @@ static int query_launch(qs_sketch *s, const void *d_keys, uint64_t n, const uint
     // (12.6 M Zipf 1.1 lookups: 165 us with non-temporal reads, 92 so).  A large
     // read-out of a table that it mostly touches once is the exception: with
     // at least two lines per key nothing is found again, and non-temporal reads take
-    // 380 us instead of 410 for 15.8 M distinct keys of a 6.4 GB table.  (Short
-    // calls are left cached: they are bound by latency either way.)
+    // 380 us instead of 410 for 15.8 M distinct keys of a 6.4 GB table.  Shorter
+    // calls are left cached, where a skewed stream gains more than distinct keys lose: in
+    // the same table 4.5 M keys take 66 us cached and 82 not at Zipf 1.1, 132 and 123
+    // distinct; 8.3 M 101 and 133, 231 and 214.  (Below 2^22 keys there is no difference.)
     const bool nt = !multi && nn >= QUERY_NT_MIN && s->low_words / 32u >= 2ull * nn;
 #define QS_QUERY(KB, MULTI, NT)                                                                                  \
     hipLaunchKernelGGL((k_query<KB, MULTI, NT>), grid, block, 0, stream, (const KeyT<KB> *)d_keys, nn, d0, s->d_desc, \
