@@ -158,8 +158,8 @@ __device__ static inline void hot_buckets(uint32_t key, uint32_t &b1, uint32_t &
 // (The sample was sorted before, and the candidates sorted again by count:
 // 29 launches, about 270 us with their gaps; these four kernels take 65 us at
 // Zipf 1.1 over 2^24 keys, 43 of them the block whose bin holds the hottest key.
-// On the second stream, beside a prefix that fills the chip, k_samp_count's last
-// blocks wait for their turn and its launch spans 228 us, within the prefix's time.)
+// On the second stream k_samp_count shares the chip with the prefix: its launch spans
+// 50 us in one trace of a 2^28-key call and 228 in another, within the prefix's time.)
 // ---------------------------------------------------------------------------
 #define SAMP_TILE 8192u // sample keys per block of the split
 #define SAMP_TILES (HOT_SAMPLE / SAMP_TILE)
